@@ -1,7 +1,7 @@
 // fft_radix.hpp -- in-register DFT butterflies used by the LDS transforms.
 //
 // dft<T, R, S>(v) overwrites v[0..R) with X_q = sum_r v_r exp(S*2*pi*i*r*q/R),
-// S = -1 forward, +1 inverse, for R in {2, 3, 4, 5, 6, 8, 12, 16}.  Radices 2-5
+// S = -1 forward, +1 inverse, for R in {2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16}.  Radices 2-5
 // are closed-form butterflies; the composite ones are a Cooley-Tukey split
 // R = A*B evaluated entirely in registers with constant twiddles.  All
 // constants are exact trigonometric values (rounded from 21 digits).
@@ -52,9 +52,34 @@ __host__ __device__ __forceinline__ double cos48(int t) {
   return c[t];
 }
 
-// exp(S*2*pi*i*m/R) for R dividing 48.
+// exp(S*2*pi*i*m/R) for R dividing 90 (radices 9, 10 and 15).
+template <typename T, int R, int S>
+__host__ __device__ __forceinline__ cpx<T> unit_root90(int m) {
+  constexpr double c[23] = {
+      1.000000000000000000000, 0.997564050259824247613, 0.990268068741570315084, 0.978147600733805637929,
+      0.961261695938318861916, 0.939692620785908384054, 0.913545457642600895502, 0.882947592858926942032,
+      0.848048096156425970386, 0.809016994374947424102, 0.766044443118978035202, 0.719339800338651139356,
+      0.669130606358858213826, 0.615661475325658279669, 0.559192903470746830160, 0.500000000000000000000,
+      0.438371146789077417453, 0.374606593415912035415, 0.309016994374947424102, 0.241921895599667722560,
+      0.173648177666930348852, 0.104528463267653471400, 0.034899496702500971646};
+  constexpr double s[23] = {
+      0.000000000000000000000, 0.069756473744125300776, 0.139173100960065444112, 0.207911690817759337102,
+      0.275637355816999185650, 0.342020143325668733044, 0.406736643075800207754, 0.469471562785890775959,
+      0.529919264233204954047, 0.587785252292473129169, 0.642787609686539326323, 0.694658370458997286656,
+      0.743144825477394235015, 0.788010753606721956694, 0.829037572555041692006, 0.866025403784438646764,
+      0.898794046299166992782, 0.927183854566787400806, 0.951056516295153572116, 0.970295726275996472306,
+      0.984807753012208059367, 0.994521895368273336923, 0.999390827019095730006};
+  const int t = ((m * (90 / R)) % 90 + 90) % 90;
+  const int h = t > 45 ? 90 - t : t;    // cos even, sin odd about a half turn
+  const int q = h > 22 ? 45 - h : h;    // cos odd, sin even about a quarter turn
+  const double cr = h > 22 ? -c[q] : c[q], sr = t > 45 ? -s[q] : s[q];
+  return cpx<T>{(T)cr, (T)(S * sr)};
+}
+
+// exp(S*2*pi*i*m/R) for R dividing 48 or 90.
 template <typename T, int R, int S>
 __host__ __device__ __forceinline__ cpx<T> unit_root(int m) {
+  if constexpr (48 % R != 0) return unit_root90<T, R, S>(m);
   const int t = ((m * (48 / R)) % 48 + 48) % 48;
   const int q = t / 12, r = t % 12;
   const double c = cos48(r), s = cos48((12 - r) % 12) * (r == 0 ? 0.0 : 1.0);
@@ -152,7 +177,8 @@ __host__ __device__ __forceinline__ void dft_split(cpx<T>* v) {
 
 template <typename T, int R, int S>
 __host__ __device__ __forceinline__ void dft(cpx<T>* v) {
-  static_assert(R == 2 || R == 3 || R == 4 || R == 5 || R == 6 || R == 8 || R == 12 || R == 16,
+  static_assert(R == 2 || R == 3 || R == 4 || R == 5 || R == 6 || R == 8 || R == 9 || R == 10 ||
+                    R == 12 || R == 15 || R == 16,
                 "unsupported radix");
   if constexpr (R == 2) dft2<T, S>(v);
   else if constexpr (R == 3) dft3<T, S>(v);
@@ -160,8 +186,47 @@ __host__ __device__ __forceinline__ void dft(cpx<T>* v) {
   else if constexpr (R == 5) dft5<T, S>(v);
   else if constexpr (R == 6) dft_split<T, 2, 3, S>(v);
   else if constexpr (R == 8) dft_split<T, 2, 4, S>(v);
+  else if constexpr (R == 9) dft_split<T, 3, 3, S>(v);
+  else if constexpr (R == 10) dft_split<T, 5, 2, S>(v);
   else if constexpr (R == 12) dft_split<T, 4, 3, S>(v);
+  else if constexpr (R == 15) dft_split<T, 5, 3, S>(v);
   else dft_split<T, 4, 4, S>(v);
+}
+
+// The radices of a length-L transform (a product of 2, 3 and 5), largest
+// first: the fewest passes, then the largest smallest radix (L / rmin threads
+// per sequence, at most max_threads), then the smallest largest one (fewest
+// registers).  Returns the number of passes, 0 when there is no plan.
+inline int fft_plan(int L, int max_threads, int* out, int max_pass = 8) {
+  constexpr int kR[] = {16, 15, 12, 10, 9, 8, 6, 5, 4, 3, 2};
+  constexpr int kN = sizeof(kR) / sizeof(int);
+  struct Search {
+    int L, max_threads, max_pass, best[8], nbest, cur[8];
+    void go(int m, int from, int n) {
+      if (m == 1) {
+        if (n == 0 || L / cur[n - 1] > max_threads) return;
+        const bool better = nbest == 0 || n < nbest ||
+                            (n == nbest && (cur[n - 1] > best[n - 1] ||
+                                            (cur[n - 1] == best[n - 1] && cur[0] < best[0])));
+        if (!better) return;
+        nbest = n;
+        for (int i = 0; i < n; ++i) best[i] = cur[i];
+        return;
+      }
+      if (n >= max_pass || (nbest && n >= nbest)) return;
+      for (int r = from; r < kN; ++r)
+        if (m % kR[r] == 0) {
+          cur[n] = kR[r];
+          go(m / kR[r], r, n + 1);
+        }
+    }
+  } s{};
+  s.L = L;
+  s.max_threads = max_threads;
+  s.max_pass = max_pass < 8 ? max_pass : 8;
+  if (L >= 2) s.go(L, 0, 0);
+  for (int i = 0; i < s.nbest; ++i) out[i] = s.best[i];
+  return s.nbest;
 }
 
 }  // namespace pll

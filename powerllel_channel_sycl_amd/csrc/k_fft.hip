@@ -14,12 +14,14 @@
 // reference's per-column real DFT (src/mod_fft.cc:122-187) computed two
 // columns at a time.
 //
-// Complex transforms use the Stockham autosort formulation with radix 4, 2,
-// 3 and 5 passes ping-ponging between two LDS buffers.  Twiddles are computed
-// on the host in long double and rounded to the field precision.
+// Complex transforms use the Stockham autosort formulation, in place in one
+// LDS buffer with the butterflies in registers: lengths in common use are
+// compiled in, every other product of 2, 3 and 5 runs from a plan.  Twiddles
+// are computed on the host in long double and rounded to the field precision.
 #include "fft_radix.hpp"
 #include "pll_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -27,258 +29,6 @@
 namespace pll {
 
 namespace {
-
-// One Stockham butterfly: sequence q, butterfly jj of a radix-R pass with span Ns.
-template <typename T, int R, int S>
-__device__ __forceinline__ void butterfly(const cpx<T>* __restrict__ a, cpx<T>* __restrict__ b,
-                                          const cpx<T>* __restrict__ tw, int jj, int q, int Ns,
-                                          int LR, int es, int ss) {
-  const int k = jj % Ns;
-  cpx<T> v[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) v[r] = a[q * ss + (jj + r * LR) * es];
-  if (Ns > 1) {
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      cpx<T> w = tw[k * (R - 1) + r - 1];
-      if (S > 0) w.im = -w.im;
-      v[r] = cmul(v[r], w);
-    }
-  }
-  dft<T, R, S>(v);
-  const int base = (jj / Ns) * Ns * R + k;
-#pragma unroll
-  for (int r = 0; r < R; ++r) b[q * ss + (base + r * Ns) * es] = v[r];
-}
-
-// All passes of a batch of nseq complex transforms of length pl.L in LDS.
-// Element m of sequence q lives at q*ss + m*es.  With seq_fast, consecutive
-// threads take consecutive sequences (for the y layout, where sequences are
-// adjacent in LDS); otherwise consecutive butterflies of one sequence.
-// Returns the buffer that holds the result.
-template <typename T, int S>
-__device__ cpx<T>* lds_fft(cpx<T>* a, cpx<T>* b, const FftPlan& pl, const cpx<T>* __restrict__ tw,
-                           int nseq, int es, int ss, bool seq_fast) {
-  for (int p = 0; p < pl.npass; ++p) {
-    const int R = pl.radix[p], Ns = pl.ns[p], LR = pl.L / R;
-    const cpx<T>* twp = tw + pl.twoff[p];
-    const int total = nseq * LR;
-    for (int t = threadIdx.x; t < total; t += blockDim.x) {
-      int q, jj;
-      if (seq_fast) {
-        q = t % nseq;
-        jj = t / nseq;
-      } else {
-        jj = t % LR;
-        q = t / LR;
-      }
-      switch (R) {
-        case 4: butterfly<T, 4, S>(a, b, twp, jj, q, Ns, LR, es, ss); break;
-        case 2: butterfly<T, 2, S>(a, b, twp, jj, q, Ns, LR, es, ss); break;
-        case 3: butterfly<T, 3, S>(a, b, twp, jj, q, Ns, LR, es, ss); break;
-        default: butterfly<T, 5, S>(a, b, twp, jj, q, Ns, LR, es, ss); break;
-      }
-    }
-    __syncthreads();
-    cpx<T>* t = a;
-    a = b;
-    b = t;
-  }
-  return a;
-}
-
-constexpr int kFftThreads = 256;
-
-// ---- x direction ------------------------------------------------------------------
-// execute_fft_fwd_xpen (src/mod_fft.cc:60-88): rows r = j + ny*k of p's interior.
-template <typename T>
-__global__ __launch_bounds__(kFftThreads) void k_fft_x_fwd(Geom g, const T* __restrict__ p,
-                                                           T* __restrict__ spec, FftPlan pl,
-                                                           const cpx<T>* __restrict__ tw,
-                                                           const cpx<T>* __restrict__ rtw,
-                                                           int batch) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int n = g.nx, h = n / 2;
-  cpx<T>* A = reinterpret_cast<cpx<T>*>(smem);
-  cpx<T>* B = A + (long)batch * h;
-  const long nrows = (long)g.ny * g.nz;
-  const long r0 = (long)blockIdx.x * batch;
-  T* Ar = reinterpret_cast<T*>(A);
-  for (int e = threadIdx.x; e < batch * n; e += blockDim.x) {
-    const int b = e / n, i = e - b * n;
-    const long r = r0 + b;
-    T val = T(0);
-    if (r < nrows) {
-      const int j = (int)(r % g.ny), k = (int)(r / g.ny);
-      val = p[g.idx(i + 1, j + 1, k + 1)];
-    }
-    Ar[e] = val;
-  }
-  __syncthreads();
-  const cpx<T>* Z = lds_fft<T, -1>(A, B, pl, tw, batch, 1, h, false);
-  for (int e = threadIdx.x; e < batch * h; e += blockDim.x) {
-    const int b = e / h, kk = e - b * h;
-    const long r = r0 + b;
-    if (r >= nrows) continue;
-    T* out = spec + r * n;
-    const cpx<T> zk = Z[b * h + kk];
-    if (kk == 0) {
-      out[0] = zk.re + zk.im;  // X0
-      out[1] = zk.re - zk.im;  // X(n/2)
-    } else {
-      const cpx<T> zm = Z[b * h + (h - kk)];
-      const T er = T(0.5) * (zk.re + zm.re), ei = T(0.5) * (zk.im - zm.im);
-      const T orr = T(0.5) * (zk.im + zm.im), oi = T(-0.5) * (zk.re - zm.re);
-      const cpx<T> w = rtw[kk];
-      out[2 * kk] = er + (w.re * orr - w.im * oi);
-      out[2 * kk + 1] = ei + (w.re * oi + w.im * orr);
-    }
-  }
-}
-
-// execute_fft_bwd_xpen (src/mod_fft.cc:90-120): perm rows -> p interior * norm.
-template <typename T>
-__global__ __launch_bounds__(kFftThreads) void k_fft_x_bwd(Geom g, const T* __restrict__ spec,
-                                                           T* __restrict__ p, FftPlan pl,
-                                                           const cpx<T>* __restrict__ tw,
-                                                           const cpx<T>* __restrict__ rtw,
-                                                           int batch, T norm) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int n = g.nx, h = n / 2;
-  cpx<T>* A = reinterpret_cast<cpx<T>*>(smem);
-  cpx<T>* B = A + (long)batch * h;
-  const long nrows = (long)g.ny * g.nz;
-  const long r0 = (long)blockIdx.x * batch;
-  T* Ar = reinterpret_cast<T*>(A);
-  for (int e = threadIdx.x; e < batch * n; e += blockDim.x) {
-    const int b = e / n;
-    const long r = r0 + b;
-    Ar[e] = (r < nrows) ? spec[r * n + (e - b * n)] : T(0);
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < batch * h; e += blockDim.x) {
-    const int b = e / h, kk = e - b * h;
-    const T* pr = Ar + (long)b * n;
-    cpx<T> xk, xm;
-    if (kk == 0) {
-      xk = cpx<T>{pr[0], T(0)};
-      xm = cpx<T>{pr[1], T(0)};
-    } else {
-      xk = cpx<T>{pr[2 * kk], pr[2 * kk + 1]};
-      xm = cpx<T>{pr[2 * (h - kk)], pr[2 * (h - kk) + 1]};
-    }
-    const cpx<T> s{xk.re + xm.re, xk.im - xm.im};  // Xk + conj(X(h-k))
-    const cpx<T> d{xk.re - xm.re, xk.im + xm.im};  // Xk - conj(X(h-k))
-    const cpx<T> w{rtw[kk].re, -rtw[kk].im};       // exp(+2 pi i k/n)
-    const cpx<T> wd = cmul(w, d);
-    B[b * h + kk] = cpx<T>{s.re - wd.im, s.im + wd.re};
-  }
-  __syncthreads();
-  const cpx<T>* z = lds_fft<T, +1>(B, A, pl, tw, batch, 1, h, false);
-  const T* zr = reinterpret_cast<const T*>(z);
-  for (int e = threadIdx.x; e < batch * n; e += blockDim.x) {
-    const int b = e / n, i = e - b * n;
-    const long r = r0 + b;
-    if (r >= nrows) continue;
-    const int j = (int)(r % g.ny), k = (int)(r / g.ny);
-    p[g.idx(i + 1, j + 1, k + 1)] = norm * zr[e];
-  }
-}
-
-// ---- y direction ------------------------------------------------------------------
-// execute_fft_fwd_ypen (src/mod_fft.cc:122-153) on a tile of `tile` perm columns.
-template <typename T>
-__global__ __launch_bounds__(kFftThreads) void k_fft_y_fwd(Geom g, T* __restrict__ spec,
-                                                           FftPlan pl,
-                                                           const cpx<T>* __restrict__ tw,
-                                                           int tile) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int n = g.ny, Q = tile / 2;
-  cpx<T>* A = reinterpret_cast<cpx<T>*>(smem);
-  cpx<T>* B = A + (long)n * Q;
-  const int k = blockIdx.y, i0 = blockIdx.x * tile;
-  T* plane = spec + (long)k * g.nx * g.ny + i0;
-  T* Ar = reinterpret_cast<T*>(A);
-  for (int e = threadIdx.x; e < n * tile; e += blockDim.x) {
-    const int j = e / tile, cidx = e - j * tile;
-    Ar[e] = plane[(long)j * g.nx + cidx];
-  }
-  __syncthreads();
-  const cpx<T>* Z = lds_fft<T, -1>(A, B, pl, tw, Q, Q, 1, true);
-  T* O = reinterpret_cast<T*>(Z == A ? B : A);
-  for (int e = threadIdx.x; e < Q * (n / 2 + 1); e += blockDim.x) {
-    const int q = e % Q, m = e / Q;
-    const cpx<T> zm = Z[m * Q + q];
-    const cpx<T> zc = Z[((n - m) % n) * Q + q];
-    const T ar = T(0.5) * (zm.re + zc.re), ai = T(0.5) * (zm.im - zc.im);
-    const T br = T(0.5) * (zm.im + zc.im), bi = T(-0.5) * (zm.re - zc.re);
-    if (m == 0) {
-      O[2 * q] = ar;
-      O[2 * q + 1] = br;
-    } else if (m == n / 2) {
-      O[tile + 2 * q] = ar;
-      O[tile + 2 * q + 1] = br;
-    } else {
-      O[(2 * m) * tile + 2 * q] = ar;
-      O[(2 * m + 1) * tile + 2 * q] = ai;
-      O[(2 * m) * tile + 2 * q + 1] = br;
-      O[(2 * m + 1) * tile + 2 * q + 1] = bi;
-    }
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < n * tile; e += blockDim.x) {
-    const int j = e / tile, cidx = e - j * tile;
-    plane[(long)j * g.nx + cidx] = O[e];
-  }
-}
-
-// execute_fft_bwd_ypen (src/mod_fft.cc:155-187), unscaled.
-template <typename T>
-__global__ __launch_bounds__(kFftThreads) void k_fft_y_bwd(Geom g, T* __restrict__ spec,
-                                                           FftPlan pl,
-                                                           const cpx<T>* __restrict__ tw,
-                                                           int tile) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int n = g.ny, Q = tile / 2;
-  cpx<T>* A = reinterpret_cast<cpx<T>*>(smem);
-  cpx<T>* B = A + (long)n * Q;
-  const int k = blockIdx.y, i0 = blockIdx.x * tile;
-  T* plane = spec + (long)k * g.nx * g.ny + i0;
-  T* Ar = reinterpret_cast<T*>(A);
-  for (int e = threadIdx.x; e < n * tile; e += blockDim.x) {
-    const int j = e / tile, cidx = e - j * tile;
-    Ar[e] = plane[(long)j * g.nx + cidx];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < Q * n; e += blockDim.x) {
-    const int q = e % Q, m = e / Q;
-    const T* pa = Ar + 2 * q;  // perm column 2q, stride tile
-    const T* pb = pa + 1;      // perm column 2q+1
-    cpx<T> z;
-    if (m == 0) {
-      z = cpx<T>{pa[0], pb[0]};
-    } else if (m == n / 2) {
-      z = cpx<T>{pa[tile], pb[tile]};
-    } else if (m < n / 2) {
-      const T are = pa[(2 * m) * tile], aim = pa[(2 * m + 1) * tile];
-      const T bre = pb[(2 * m) * tile], bim = pb[(2 * m + 1) * tile];
-      z = cpx<T>{are - bim, aim + bre};
-    } else {
-      const int mm = n - m;
-      const T are = pa[(2 * mm) * tile], aim = pa[(2 * mm + 1) * tile];
-      const T bre = pb[(2 * mm) * tile], bim = pb[(2 * mm + 1) * tile];
-      z = cpx<T>{are + bim, bre - aim};
-    }
-    B[m * Q + q] = z;
-  }
-  __syncthreads();
-  const cpx<T>* z = lds_fft<T, +1>(B, A, pl, tw, Q, Q, 1, true);
-  const T* zr = reinterpret_cast<const T*>(z);
-  for (int e = threadIdx.x; e < n * tile; e += blockDim.x) {
-    const int j = e / tile, cidx = e - j * tile;
-    plane[(long)j * g.nx + cidx] = zr[e];
-  }
-}
 
 // ============================================================================
 // Compile-time transforms for the lengths of the supported grids.  One
@@ -416,6 +166,15 @@ struct RhsSrc {
   // on planes 0 and nz (src/mod_updateBound.cc:32-144)
   int bcfold;
 };
+
+template <typename T>
+RhsSrc<T> rhs_src(const pll_context* c) {
+  const double dti = 1.0 / c->dt;  // src/mod_calcRHS.cc:11-13
+  return RhsSrc<T>{static_cast<const T*>(c->fld[PLL_U]), static_cast<const T*>(c->fld[PLL_V]),
+                   static_cast<const T*>(c->fld[PLL_W]),
+                   static_cast<const T*>(c->d_mesh) + (c->g.nz + 2),  // dzf_inv
+                   (T)dti, (T)(dti * c->dx_inv), (T)(dti * c->dy_inv), c->rhs_bcfold};
+}
 
 // execute_fft_fwd_xpen (src/mod_fft.cc:60-88), L = nx/2 points per row.  With
 // RHS the rows are calcRHS's output computed on load (nothing is stored in p).
@@ -719,33 +478,376 @@ __global__ __launch_bounds__((y_seqs<T, L>() * tps<L>())) void k_yb(Geom g, T* _
   store_tile<T, L * Q, NT, Q>(buf, plane, g.nx);
 }
 
+// ============================================================================
+// Run-time-plan transforms for every other length: the same one-buffer Stockham
+// passes with the radices of an FftPlan (fft_plan in fft_radix.hpp: the fewest
+// passes of radices 2..16, then the largest smallest radix), one butterfly per
+// thread and pass, so L = 100 takes two passes (10, 10) and one LDS buffer.
+// They are bound by HBM like the fixed-length kernels, so what matters is loads
+// in flight: kGenChunk loads per thread are issued before the first LDS write,
+// and blocks of about 256 threads and at most 32 KiB of LDS leave five or more
+// of them on a CU.  Against radix 4/2/3/5 passes ping-ponging in 64 KiB blocks:
+// the FP64 step at 200x90x176 294 -> 246 us (its four transforms 136 -> 88 us).
+// ============================================================================
+// n / d by multiplication, m = ceil(2^32 / d): exact for n * d < 2^32, d > 1
+__device__ __forceinline__ int div_by(int n, unsigned m) { return (int)__umulhi((unsigned)n, m); }
+
+template <typename T, int S, int R>
+__device__ __forceinline__ void plan_pass(cpx<T>* buf, const cpx<T>* __restrict__ twL, int soff,
+                                          int es, int jj, bool on, int LR, int ns, unsigned mns,
+                                          int tws) {
+  cpx<T> v[R];
+  const bool active = on && jj < LR;
+  if (active) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = buf[pad(soff + (jj + r * LR) * es)];
+  }
+  __syncthreads();
+  if (active) {
+    int hi = jj, k = 0;
+    if (ns > 1) {
+      hi = div_by(jj, mns);
+      k = jj - hi * ns;
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        cpx<T> w = twL[r * k * tws];
+        if (S > 0) w.im = -w.im;
+        v[r] = cmul(v[r], w);
+      }
+    }
+    dft<T, R, S>(v);
+    const int base = hi * ns * R + k;
+#pragma unroll
+    for (int r = 0; r < R; ++r) buf[pad(soff + (base + r * ns) * es)] = v[r];
+  }
+  __syncthreads();
+}
+
+// All passes in place; `on` is false for threads without a sequence.
+template <typename T, int S>
+__device__ __forceinline__ void plan_fft(cpx<T>* buf, const FftPlan& pl,
+                                         const cpx<T>* __restrict__ twL, int soff, int es, int jj,
+                                         bool on) {
+  for (int p = 0; p < pl.npass; ++p) {
+    const int LR = pl.lr[p], ns = pl.ns[p], tws = pl.tws[p];
+    const unsigned mns = pl.mns[p];
+#define PLL_PASS(R) \
+  case R: plan_pass<T, S, R>(buf, twL, soff, es, jj, on, LR, ns, mns, tws); break;
+    switch (pl.radix[p]) {
+      PLL_PASS(2)
+      PLL_PASS(3)
+      PLL_PASS(4)
+      PLL_PASS(5)
+      PLL_PASS(6)
+      PLL_PASS(8)
+      PLL_PASS(9)
+      PLL_PASS(10)
+      PLL_PASS(12)
+      PLL_PASS(15)
+      default: plan_pass<T, S, 16>(buf, twL, soff, es, jj, on, LR, ns, mns, tws); break;
+    }
+#undef PLL_PASS
+  }
+}
+
+constexpr int kGenChunk = 8;      // loads in flight per thread
+constexpr int kGenRows = 64;      // most rows of an x block
+constexpr int kGenThreads = 1024; // most threads of a block
+
+// Launch shape of an x transform: nb rows per block, magic divisors.
+struct XShape {
+  int nb, tps;
+  unsigned mN, mtps;  // dividing by nx and tps (tps = 1: unused)
+};
+
+// k_xf's transform (src/mod_fft.cc:60-88) with a run-time plan.
+template <typename T, bool RHS>
+__global__ __launch_bounds__(kGenThreads) void k_gxf(Geom g, const T* __restrict__ p,
+                                                     T* __restrict__ spec, FftPlan pl, XShape xs,
+                                                     const cpx<T>* __restrict__ twL,
+                                                     const cpx<T>* __restrict__ rtw, long nrows,
+                                                     RhsSrc<T> rs) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
+  __shared__ long rowbase[kGenRows];
+  __shared__ T rowdz[kGenRows];
+  __shared__ long rowvs[kGenRows];           // offset of the v row below (j-1, or its image)
+  __shared__ unsigned char roww[kGenRows];   // bit 0: w below is the wall 0; bit 1: w is the wall 0
+  const int N = g.nx, L = N / 2, NT = blockDim.x;
+  const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * xs.nb;
+  if ((int)threadIdx.x < xs.nb) {
+    const long r = row0 + threadIdx.x;
+    const int j = (int)(r % g.ny), k = (int)(r / g.ny);
+    rowbase[threadIdx.x] = r < nrows ? g.idx(1, j + 1, k + 1) : -1;
+    if (RHS) {
+      rowdz[threadIdx.x] = r < nrows ? rs.dti * rs.dzf_inv[k + 1] : T(0);
+      const bool f = rs.bcfold != 0;
+      rowvs[threadIdx.x] = (f && j == 0) ? (long)(g.ny - 1) * g.sx : -g.sx;
+      roww[threadIdx.x] = (unsigned char)((f && k == 0 ? 1 : 0) | (f && k + 1 == g.nz ? 2 : 0));
+    }
+  }
+  __syncthreads();
+  constexpr int CH = RHS ? kGenChunk / 2 : kGenChunk;
+  const int total = xs.nb * N;
+  for (int e0 = threadIdx.x; e0 < total; e0 += CH * NT) {
+    T a0[CH], a1[CH], a2[CH], a3[CH], a4[CH], a5[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT;
+      a0[u] = a1[u] = a2[u] = a3[u] = a4[u] = a5[u] = T(0);
+      if (e < total) {
+        const int s = div_by(e, xs.mN), i = e - s * N;
+        const long b = rowbase[s];
+        if (b >= 0) {
+          const long c = b + i;
+          if (RHS) {
+            const long cw = (i == 0 && rs.bcfold) ? b + (N - 1) : c - 1;  // u(0) = u(nx)
+            const unsigned char wf = roww[s];
+            a0[u] = rs.u[c];
+            a1[u] = rs.u[cw];
+            a2[u] = rs.v[c];
+            a3[u] = rs.v[c + rowvs[s]];
+            if (!(wf & 2)) a4[u] = rs.w[c];
+            if (!(wf & 1)) a5[u] = rs.w[c - g.sxy];
+          } else {
+            a0[u] = p[c];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT;
+      if (e < total) {
+        T val = a0[u];
+        if (RHS) {
+          // src/mod_calcRHS.cc:21-28, same association as k_calc_rhs
+          val = (a0[u] - a1[u]) * rs.dtidxi + (a2[u] - a3[u]) * rs.dtidyi +
+                (a4[u] - a5[u]) * rowdz[div_by(e, xs.mN)];
+        }
+        real_at(buf, e) = val;  // row s starts at element s * N
+      }
+    }
+  }
+  __syncthreads();
+  const int s = xs.tps > 1 ? div_by(threadIdx.x, xs.mtps) : (int)threadIdx.x;
+  const int jj = (int)threadIdx.x - s * xs.tps;
+  const bool on = s < xs.nb;
+  plan_fft<T, -1>(buf, pl, twL, s * L, 1, jj, on);
+  const long r = row0 + s;
+  if (!on || r >= nrows) return;
+  cpx<T>* out = reinterpret_cast<cpx<T>*>(spec + r * N);
+  for (int kk = jj; kk < L; kk += xs.tps) {
+    const cpx<T> zk = buf[pad(s * L + kk)];
+    if (kk == 0) {
+      out[0] = cpx<T>{zk.re + zk.im, zk.re - zk.im};  // X0, X(n/2)
+    } else {
+      const cpx<T> zm = buf[pad(s * L + (L - kk))];
+      const T er = T(0.5) * (zk.re + zm.re), ei = T(0.5) * (zk.im - zm.im);
+      const T orr = T(0.5) * (zk.im + zm.im), oi = T(-0.5) * (zk.re - zm.re);
+      const cpx<T> w = rtw[kk];
+      out[kk] = cpx<T>{er + (w.re * orr - w.im * oi), ei + (w.re * oi + w.im * orr)};
+    }
+  }
+}
+
+// k_xb's transform (src/mod_fft.cc:90-120) with a run-time plan.  One thread
+// merges slots kk and L - kk, so the merge runs in place without a barrier.
+template <typename T, bool HALO>
+__global__ __launch_bounds__(kGenThreads) void k_gxb(Geom g, const T* __restrict__ spec,
+                                                     T* __restrict__ p, FftPlan pl, XShape xs,
+                                                     const cpx<T>* __restrict__ twL,
+                                                     const cpx<T>* __restrict__ rtw, long nrows,
+                                                     unsigned mP, T norm) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
+  __shared__ long rowbase[kGenRows];
+  const int N = g.nx, L = N / 2, NT = blockDim.x;
+  const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * xs.nb;
+  if ((int)threadIdx.x < xs.nb) {
+    const long r = row0 + threadIdx.x;
+    const int j = (int)(r % g.ny), k = (int)(r / g.ny);
+    rowbase[threadIdx.x] = r < nrows ? g.idx(HALO ? 0 : 1, j + 1, k + 1) : -1;
+  }
+  const cpx<T>* specc = reinterpret_cast<const cpx<T>*>(spec) + row0 * L;
+  const int slots = xs.nb * L;
+  const long have = (nrows - row0) * L;  // slots of rows that exist
+  for (int e0 = threadIdx.x; e0 < slots; e0 += kGenChunk * NT) {
+    cpx<T> t[kGenChunk];
+#pragma unroll
+    for (int u = 0; u < kGenChunk; ++u) {
+      const int e = e0 + u * NT;
+      t[u] = e < slots && e < have ? specc[e] : cpx<T>{T(0), T(0)};
+    }
+#pragma unroll
+    for (int u = 0; u < kGenChunk; ++u) {
+      const int e = e0 + u * NT;
+      if (e < slots) buf[pad(e)] = t[u];
+    }
+  }
+  __syncthreads();
+  const int s = xs.tps > 1 ? div_by(threadIdx.x, xs.mtps) : (int)threadIdx.x;
+  const int jj = (int)threadIdx.x - s * xs.tps;
+  const bool on = s < xs.nb;
+  // perm slot kk holds (Re Xkk, Im Xkk); slot 0 holds (X0, X(n/2))
+  if (on) {
+    auto merge = [&](cpx<T> xk, cpx<T> xm, int kk) {
+      const cpx<T> sm{xk.re + xm.re, xk.im - xm.im};  // Xk + conj(X(h-k))
+      const cpx<T> d{xk.re - xm.re, xk.im + xm.im};   // Xk - conj(X(h-k))
+      const cpx<T> w{rtw[kk].re, -rtw[kk].im};        // exp(+2 pi i k/n)
+      const cpx<T> wd = cmul(w, d);
+      return cpx<T>{sm.re - wd.im, sm.im + wd.re};
+    };
+    for (int kk = jj; kk <= L / 2; kk += xs.tps) {
+      cpx<T>& lo = buf[pad(s * L + kk)];
+      const cpx<T> a = lo;
+      if (kk == 0) {
+        lo = merge(cpx<T>{a.re, T(0)}, cpx<T>{a.im, T(0)}, 0);
+      } else {
+        cpx<T>& hi = buf[pad(s * L + (L - kk))];
+        const cpx<T> b = hi;
+        lo = merge(a, b, kk);
+        if (2 * kk != L) hi = merge(b, a, L - kk);
+      }
+    }
+  }
+  __syncthreads();
+  plan_fft<T, +1>(buf, pl, twL, s * L, 1, jj, on);
+  if (HALO) {
+    // pair q = (p(2q), p(2q+1)); p(i) is element i-1 of the row, p(0) = p(nx), p(nx+1) = p(1)
+    const int NP = L + 1;
+    for (int e = threadIdx.x; e < xs.nb * NP; e += NT) {
+      const int s2 = div_by(e, mP), q = e - s2 * NP;
+      if (rowbase[s2] < 0) continue;
+      const int i0 = q == 0 ? N - 1 : 2 * q - 1, i1 = q == L ? 0 : 2 * q;
+      reinterpret_cast<cpx<T>*>(p + rowbase[s2])[q] =
+          cpx<T>{norm * real_at(buf, s2 * N + i0), norm * real_at(buf, s2 * N + i1)};
+    }
+  } else {
+    for (int e = threadIdx.x; e < xs.nb * N; e += NT) {
+      const int s2 = div_by(e, xs.mN);
+      if (rowbase[s2] >= 0) p[rowbase[s2] + (e - s2 * N)] = norm * real_at(buf, e);
+    }
+  }
+}
+
+// k_yf's transform (src/mod_fft.cc:122-153) with a run-time plan: a tile of
+// 2^lq column pairs of one k plane, the last tile of a plane possibly ragged.
+template <typename T>
+__global__ __launch_bounds__(kGenThreads) void k_gyf(Geom g, T* __restrict__ spec, FftPlan pl,
+                                                     const cpx<T>* __restrict__ twL, int lq,
+                                                     int ntiles) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
+  const int L = g.ny, Q = 1 << lq, NT = blockDim.x;
+  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = (int)(b % (unsigned)ntiles), k = (int)(b / (unsigned)ntiles);
+  T* plane = spec + (long)k * g.nx * g.ny + ((long)tile << (lq + 1));
+  const int have = g.nx / 2 - (tile << lq);  // column pairs of this tile that exist
+  const int total = L << lq;
+  for (int e0 = threadIdx.x; e0 < total; e0 += kGenChunk * NT) {
+    cpx<T> t[kGenChunk];
+#pragma unroll
+    for (int u = 0; u < kGenChunk; ++u) {
+      const int e = e0 + u * NT, q = e & (Q - 1);
+      t[u] = e < total && q < have ? reinterpret_cast<const cpx<T>*>(plane + (long)(e >> lq) * g.nx)[q]
+                                   : cpx<T>{T(0), T(0)};
+    }
+#pragma unroll
+    for (int u = 0; u < kGenChunk; ++u) {
+      const int e = e0 + u * NT;
+      if (e < total) buf[pad(e)] = t[u];
+    }
+  }
+  __syncthreads();
+  const int q = (int)threadIdx.x & (Q - 1), jj = (int)threadIdx.x >> lq;
+  plan_fft<T, -1>(buf, pl, twL, q, Q, jj, jj < pl.tps);
+  if (q >= have) return;
+  for (int m = jj; m <= L / 2; m += NT >> lq) {
+    const cpx<T> zm = buf[pad(m * Q + q)];
+    const cpx<T> zc = buf[pad((m == 0 ? 0 : L - m) * Q + q)];
+    const T ar = T(0.5) * (zm.re + zc.re), ai = T(0.5) * (zm.im - zc.im);
+    const T br = T(0.5) * (zm.im + zc.im), bi = T(-0.5) * (zm.re - zc.re);
+    if (m == 0) {
+      reinterpret_cast<cpx<T>*>(plane)[q] = cpx<T>{ar, br};
+    } else if (m == L / 2) {
+      reinterpret_cast<cpx<T>*>(plane + g.nx)[q] = cpx<T>{ar, br};
+    } else {
+      reinterpret_cast<cpx<T>*>(plane + (long)(2 * m) * g.nx)[q] = cpx<T>{ar, br};
+      reinterpret_cast<cpx<T>*>(plane + (long)(2 * m + 1) * g.nx)[q] = cpx<T>{ai, bi};
+    }
+  }
+}
+
+// k_yb's transform (src/mod_fft.cc:155-187, unscaled) with a run-time plan.
+template <typename T>
+__global__ __launch_bounds__(kGenThreads) void k_gyb(Geom g, T* __restrict__ spec, FftPlan pl,
+                                                     const cpx<T>* __restrict__ twL, int lq,
+                                                     int ntiles) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
+  const int L = g.ny, Q = 1 << lq, NT = blockDim.x;
+  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = (int)(b % (unsigned)ntiles), k = (int)(b / (unsigned)ntiles);
+  T* plane = spec + (long)k * g.nx * g.ny + ((long)tile << (lq + 1));
+  const int have = g.nx / 2 - (tile << lq);
+  // rows 2m and 2m+1 unpack into the complex inputs Z[m] and Z[L-m] (k_yb)
+  constexpr int CH = kGenChunk / 2;
+  const int total = (L / 2) << lq;
+  for (int e0 = threadIdx.x; e0 < total; e0 += CH * NT) {
+    cpx<T> r0[CH], r1[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT, mm = e >> lq, q = e & (Q - 1);
+      r0[u] = r1[u] = cpx<T>{T(0), T(0)};
+      if (e < total && q < have) {
+        r0[u] = reinterpret_cast<const cpx<T>*>(plane + (long)(2 * mm) * g.nx)[q];
+        r1[u] = reinterpret_cast<const cpx<T>*>(plane + (long)(2 * mm + 1) * g.nx)[q];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT, mm = e >> lq, q = e & (Q - 1);
+      if (e < total) {
+        if (mm == 0) {
+          buf[pad(q)] = r0[u];
+          buf[pad((L / 2) * Q + q)] = r1[u];
+        } else {
+          buf[pad(mm * Q + q)] = cpx<T>{r0[u].re - r1[u].im, r1[u].re + r0[u].im};
+          buf[pad((L - mm) * Q + q)] = cpx<T>{r0[u].re + r1[u].im, r0[u].im - r1[u].re};
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const int q = (int)threadIdx.x & (Q - 1), jj = (int)threadIdx.x >> lq;
+  plan_fft<T, +1>(buf, pl, twL, q, Q, jj, jj < pl.tps);
+  if (q >= have) return;
+  for (int j = jj; j < L; j += NT >> lq)
+    reinterpret_cast<cpx<T>*>(plane + (long)j * g.nx)[q] = buf[pad(j * Q + q)];
+}
+
 // ---- host side -------------------------------------------------------------------
-bool build_plan(int L, FftPlan& pl, std::vector<std::complex<long double>>& tw) {
+unsigned magic(int d) { return (unsigned)((0x100000000ULL + (unsigned)d - 1) / (unsigned)d); }
+
+bool build_plan(int L, FftPlan& pl) {
+  int rad[kMaxPass];
+  const int np = fft_plan(L, kGenThreads, rad);
+  if (np < 1) return false;
   pl.L = L;
-  pl.npass = 0;
-  int m = L;
-  std::vector<int> rad;
-  while (m % 4 == 0) { rad.push_back(4); m /= 4; }
-  while (m % 2 == 0) { rad.push_back(2); m /= 2; }
-  while (m % 3 == 0) { rad.push_back(3); m /= 3; }
-  while (m % 5 == 0) { rad.push_back(5); m /= 5; }
-  if (m != 1 || (int)rad.size() > kMaxPass) return false;
-  const long double two_pi = 6.283185307179586476925286766559005768L;
-  int ns = 1;
-  for (int R : rad) {
-    const int p = pl.npass++;
+  pl.npass = np;
+  int ns = 1, rmin = L;
+  for (int p = 0; p < np; ++p) {
+    const int R = rad[p];
     pl.radix[p] = R;
     pl.ns[p] = ns;
-    pl.twoff[p] = (int)tw.size();
-    for (int k = 0; k < ns; ++k)
-      for (int r = 1; r < R; ++r) {
-        const long t = ((long)r * k) % ((long)ns * R);
-        const long double ang = -two_pi * (long double)t / (long double)(ns * R);
-        tw.emplace_back(cosl(ang), sinl(ang));
-      }
+    pl.lr[p] = L / R;
+    pl.tws[p] = L / (ns * R);
+    pl.mns[p] = ns > 1 ? magic(ns) : 0;
     ns *= R;
+    rmin = R < rmin ? R : rmin;
   }
-  if (tw.empty()) tw.emplace_back(1.0L, 0.0L);
+  pl.tps = L / rmin;
   return true;
 }
 
@@ -758,81 +860,93 @@ int upload_table(pll_context* c, const std::vector<std::complex<long double>>& s
   return PLL_OK;
 }
 
-constexpr size_t kLdsBudget = 64 * 1024;  // bytes per block for the two ping-pong buffers
+// The longest lengths taken: two complex rows (or column pairs) of 64 KiB.
+constexpr size_t kLdsBudget = 64 * 1024;
+// LDS of a run-time-plan block: several blocks per CU
+constexpr size_t kGenLds = 32 * 1024;
 
 template <typename T>
 int setup_t(pll_context* c) {
   const int nx = c->g.nx, ny = c->g.ny;
-  std::vector<std::complex<long double>> twx, twy, rtw;
-  if (!build_plan(nx / 2, c->plan_x, twx)) return fail(PLL_ERR_ARG, "nx/2 must factor into 2, 3, 5");
-  if (!build_plan(ny, c->plan_y, twy)) return fail(PLL_ERR_ARG, "ny must factor into 2, 3, 5");
+  if ((size_t)nx * sizeof(T) * 2 > kLdsBudget)
+    return fail(PLL_ERR_ARG, "nx too large for one LDS row transform");
+  if ((size_t)ny * sizeof(T) * 4 > kLdsBudget)
+    return fail(PLL_ERR_ARG, "ny too large for one LDS column transform");
+  if (!build_plan(nx / 2, c->plan_x)) return fail(PLL_ERR_ARG, "nx/2 must factor into 2, 3, 5");
+  if (!build_plan(ny, c->plan_y)) return fail(PLL_ERR_ARG, "ny must factor into 2, 3, 5");
+  std::vector<std::complex<long double>> rtw;
   const long double two_pi = 6.283185307179586476925286766559005768L;
   for (int k = 0; k <= nx / 2; ++k) {
     const long double ang = -two_pi * (long double)k / (long double)nx;
     rtw.emplace_back(cosl(ang), sinl(ang));
   }
   int rc;
-  if ((rc = upload_table<T>(c, twx, &c->d_tw_x))) return rc;
-  if ((rc = upload_table<T>(c, twy, &c->d_tw_y))) return rc;
   if ((rc = upload_table<T>(c, rtw, &c->d_rtw_x))) return rc;
-  const size_t rowbytes = (size_t)nx * sizeof(T) * 2;  // two buffers
-  long batch = (long)(kLdsBudget / rowbytes);
-  if (batch < 1) return fail(PLL_ERR_ARG, "nx too large for one LDS row transform");
-  if (batch > 64) batch = 64;
-  c->x_batch = (int)batch;
-  const size_t colbytes = (size_t)ny * sizeof(T) * 2;
-  int tile = 2;
-  while (tile * 2 <= 64 && (size_t)(tile * 2) * colbytes <= kLdsBudget && nx % (tile * 2) == 0)
-    tile *= 2;
-  if ((size_t)tile * colbytes > kLdsBudget) return fail(PLL_ERR_ARG, "ny too large for one LDS column transform");
-  c->y_tile = tile;
+  // rows per block of the x transforms: about 256 threads within kGenLds, fewer
+  // where that would leave the chip with under two blocks per CU
+  const long nrows = (long)ny * c->g.nz;
+  int nb = std::max(1, std::min(kGenRows, 256 / c->plan_x.tps));
+  while (nb > 1 && (size_t)padded(nb * (nx / 2)) * 2 * sizeof(T) > kGenLds) --nb;
+  while (nb > 1 && nrows / nb < 512) nb = (nb + 1) / 2;
+  c->x_batch = nb;
+  // column pairs per block of the y transforms: 128-byte rows within 1024
+  // threads and kLdsBudget, no more than the plane has
+  int lq = sizeof(T) == 8 ? 3 : 4;
+  while (lq > 0 && ((c->plan_y.tps << lq) > kGenThreads ||
+                    (size_t)padded(ny << lq) * 2 * sizeof(T) > kLdsBudget ||
+                    (1 << (lq - 1)) >= nx / 2))
+    --lq;
+  c->y_tile = lq;
   return PLL_OK;
 }
 
-template <typename T>
-int x_fwd_generic(pll_context* c) {
-  const long nrows = (long)c->g.ny * c->g.nz;
-  const unsigned blocks = (unsigned)((nrows + c->x_batch - 1) / c->x_batch);
-  const size_t sh = (size_t)c->x_batch * c->g.nx * sizeof(T) * 2;
-  TimerScope ts(c, K_FFT_X_FWD);
-  hipLaunchKernelGGL((k_fft_x_fwd<T>), dim3(blocks), dim3(kFftThreads), sh, c->stream, c->g,
-                     static_cast<const T*>(c->fld[PLL_P]), static_cast<T*>(c->spec), c->plan_x,
-                     static_cast<const cpx<T>*>(c->d_tw_x), static_cast<const cpx<T>*>(c->d_rtw_x),
-                     c->x_batch);
-  PLL_HIP_TRY(hipGetLastError());
-  return PLL_OK;
+int round_wave(int n) { return (n + 63) / 64 * 64; }
+
+XShape x_shape(const pll_context* c) {
+  const int tps = c->plan_x.tps;
+  return XShape{c->x_batch, tps, magic(c->g.nx), tps > 1 ? magic(tps) : 0};
 }
 
 template <typename T>
-int x_bwd_generic(pll_context* c) {
+int x_generic(pll_context* c, bool fwd, bool step) {
   const long nrows = (long)c->g.ny * c->g.nz;
-  const unsigned blocks = (unsigned)((nrows + c->x_batch - 1) / c->x_batch);
-  const size_t sh = (size_t)c->x_batch * c->g.nx * sizeof(T) * 2;
-  const double norm = 1.0 / (c->g.nx * c->g.ny);  // src/mod_fft.cc:57
-  TimerScope ts(c, K_FFT_X_BWD);
-  hipLaunchKernelGGL((k_fft_x_bwd<T>), dim3(blocks), dim3(kFftThreads), sh, c->stream, c->g,
-                     static_cast<const T*>(c->spec), static_cast<T*>(c->fld[PLL_P]), c->plan_x,
-                     static_cast<const cpx<T>*>(c->d_tw_x), static_cast<const cpx<T>*>(c->d_rtw_x),
-                     c->x_batch, (T)norm);
+  const XShape xs = x_shape(c);
+  const int L = c->g.nx / 2;
+  const dim3 blocks((unsigned)((nrows + xs.nb - 1) / xs.nb)), threads(round_wave(xs.nb * xs.tps));
+  const size_t sh = (size_t)padded(xs.nb * L) * 2 * sizeof(T);
+  const cpx<T>* tw = static_cast<const cpx<T>*>(c->d_twl_x);
+  const cpx<T>* rtw = static_cast<const cpx<T>*>(c->d_rtw_x);
+  T* p = static_cast<T*>(c->fld[PLL_P]);
+  T* spec = static_cast<T*>(c->spec);
+  if (fwd && step) {
+    TimerScope ts(c, K_FFT_X_FWD_RHS);
+    hipLaunchKernelGGL((k_gxf<T, true>), blocks, threads, sh, c->stream, c->g,
+                       static_cast<const T*>(nullptr), spec, c->plan_x, xs, tw, rtw, nrows,
+                       rhs_src<T>(c));
+  } else if (fwd) {
+    TimerScope ts(c, K_FFT_X_FWD);
+    hipLaunchKernelGGL((k_gxf<T, false>), blocks, threads, sh, c->stream, c->g,
+                       static_cast<const T*>(p), spec, c->plan_x, xs, tw, rtw, nrows, RhsSrc<T>{});
+  } else {
+    const double norm = 1.0 / (c->g.nx * c->g.ny);  // src/mod_fft.cc:57
+    TimerScope ts(c, K_FFT_X_BWD);
+    hipLaunchKernelGGL((step ? k_gxb<T, true> : k_gxb<T, false>), blocks, threads, sh, c->stream,
+                       c->g, static_cast<const T*>(spec), p, c->plan_x, xs, tw, rtw, nrows,
+                       magic(L + 1), (T)norm);
+  }
   PLL_HIP_TRY(hipGetLastError());
   return PLL_OK;
 }
 
 template <typename T>
 int y_generic(pll_context* c, bool fwd) {
-  const dim3 grid(c->g.nx / c->y_tile, c->g.nz);
-  const size_t sh = (size_t)c->y_tile * c->g.ny * sizeof(T) * 2;
-  if (fwd) {
-    TimerScope ts(c, K_FFT_Y_FWD);
-    hipLaunchKernelGGL((k_fft_y_fwd<T>), grid, dim3(kFftThreads), sh, c->stream, c->g,
-                       static_cast<T*>(c->spec), c->plan_y, static_cast<const cpx<T>*>(c->d_tw_y),
-                       c->y_tile);
-  } else {
-    TimerScope ts(c, K_FFT_Y_BWD);
-    hipLaunchKernelGGL((k_fft_y_bwd<T>), grid, dim3(kFftThreads), sh, c->stream, c->g,
-                       static_cast<T*>(c->spec), c->plan_y, static_cast<const cpx<T>*>(c->d_tw_y),
-                       c->y_tile);
-  }
+  const int lq = c->y_tile, ntiles = (c->g.nx / 2 + (1 << lq) - 1) >> lq;
+  const dim3 blocks((unsigned)ntiles * c->g.nz), threads(round_wave(c->plan_y.tps << lq));
+  const size_t sh = (size_t)padded(c->g.ny << lq) * 2 * sizeof(T);
+  TimerScope ts(c, fwd ? K_FFT_Y_FWD : K_FFT_Y_BWD);
+  hipLaunchKernelGGL((fwd ? k_gyf<T> : k_gyb<T>), blocks, threads, sh, c->stream, c->g,
+                     static_cast<T*>(c->spec), c->plan_y, static_cast<const cpx<T>*>(c->d_twl_y),
+                     lq, ntiles);
   PLL_HIP_TRY(hipGetLastError());
   return PLL_OK;
 }
@@ -846,11 +960,7 @@ int x_fixed(pll_context* c, bool fwd, bool rhs = false) {
   const cpx<T>* tw = static_cast<const cpx<T>*>(c->d_twl_x);
   const cpx<T>* rtw = static_cast<const cpx<T>*>(c->d_rtw_x);
   if (fwd && rhs) {
-    const double dti = 1.0 / c->dt;  // src/mod_calcRHS.cc:11-13
-    RhsSrc<T> rs{static_cast<const T*>(c->fld[PLL_U]), static_cast<const T*>(c->fld[PLL_V]),
-                 static_cast<const T*>(c->fld[PLL_W]),
-                 static_cast<const T*>(c->d_mesh) + (c->g.nz + 2),  // dzf_inv
-                 (T)dti, (T)(dti * c->dx_inv), (T)(dti * c->dy_inv), c->rhs_bcfold};
+    const RhsSrc<T> rs = rhs_src<T>(c);
     TimerScope ts(c, K_FFT_X_FWD_RHS);
     hipLaunchKernelGGL((k_xf<T, L, true>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
                        static_cast<const T*>(nullptr), static_cast<T*>(c->spec), tw, rtw, nrows, rs);
@@ -919,17 +1029,18 @@ bool y_has_fixed(const pll_context* c, int L) {
   return false;
 }
 
+// step: calcRHS in the forward loads, periodic halos in the inverse's stores
 template <typename T>
-int x_t(pll_context* c, bool fwd) {
+int x_t(pll_context* c, bool fwd, bool step = false) {
   if (c->x_fixed) {
     switch (c->g.nx / 2) {
-#define PLL_CASE(n) case n: return x_fixed<T, n>(c, fwd);
+#define PLL_CASE(n) case n: return x_fixed<T, n>(c, fwd, step);
       PLL_X_SIZES(PLL_CASE)
 #undef PLL_CASE
       default: break;
     }
   }
-  return fwd ? x_fwd_generic<T>(c) : x_bwd_generic<T>(c);
+  return x_generic<T>(c, fwd, step);
 }
 
 template <typename T>
@@ -978,40 +1089,15 @@ int fft_setup(pll_context* c) {
 }
 int launch_fft_x_fwd(pll_context* c) { return c->prec == PLL_FP64 ? x_t<double>(c, true) : x_t<float>(c, true); }
 
-template <typename T>
-int x_rhs_t(pll_context* c) {
-  switch (c->g.nx / 2) {
-#define PLL_CASE(n) case n: return x_fixed<T, n>(c, true, true);
-    PLL_X_SIZES(PLL_CASE)
-#undef PLL_CASE
-    default: break;
-  }
-  return fail(PLL_ERR_UNSUPPORTED, "no fixed-length x transform for calcRHS fusion");
-}
-
-bool fft_x_rhs_available(const pll_context* c) { return c->x_fixed; }
-
-template <typename T>
-int x_bwd_halo_t(pll_context* c) {
-  switch (c->g.nx / 2) {
-#define PLL_CASE(n) case n: return x_fixed<T, n>(c, false, true);
-    PLL_X_SIZES(PLL_CASE)
-#undef PLL_CASE
-    default: break;
-  }
-  return x_bwd_generic<T>(c);
-}
-
-int launch_fft_x_bwd_step(pll_context* c) {
-  if (!c->x_fixed) return launch_fft_x_bwd(c);
-  return c->prec == PLL_FP64 ? x_bwd_halo_t<double>(c) : x_bwd_halo_t<float>(c);
-}
-
 int launch_fft_x_fwd_rhs(pll_context* c) {
-  if (!c->x_fixed) return fail(PLL_ERR_UNSUPPORTED, "no fixed-length x transform for calcRHS fusion");
-  return c->prec == PLL_FP64 ? x_rhs_t<double>(c) : x_rhs_t<float>(c);
+  return c->prec == PLL_FP64 ? x_t<double>(c, true, true) : x_t<float>(c, true, true);
+}
+int launch_fft_x_bwd_step(pll_context* c) {
+  return c->prec == PLL_FP64 ? x_t<double>(c, false, true) : x_t<float>(c, false, true);
 }
 int launch_fft_x_bwd(pll_context* c) { return c->prec == PLL_FP64 ? x_t<double>(c, false) : x_t<float>(c, false); }
+int launch_fft_y_fwd(pll_context* c) { return c->prec == PLL_FP64 ? y_t<double>(c, true) : y_t<float>(c, true); }
+int launch_fft_y_bwd(pll_context* c) { return c->prec == PLL_FP64 ? y_t<double>(c, false) : y_t<float>(c, false); }
 
 int launch_poisson_step(pll_context* c, bool rhs) {
   int rc;
@@ -1021,7 +1107,5 @@ int launch_poisson_step(pll_context* c, bool rhs) {
   if ((rc = launch_fft_y_bwd(c))) return rc;
   return launch_fft_x_bwd_step(c);
 }
-int launch_fft_y_fwd(pll_context* c) { return c->prec == PLL_FP64 ? y_t<double>(c, true) : y_t<float>(c, true); }
-int launch_fft_y_bwd(pll_context* c) { return c->prec == PLL_FP64 ? y_t<double>(c, false) : y_t<float>(c, false); }
 
 }  // namespace pll

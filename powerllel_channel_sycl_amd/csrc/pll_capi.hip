@@ -146,7 +146,7 @@ void release(pll_context* c) {
   for (double*& p : c->d_stat)
     if (p) (void)hipFree(p);
   void* bufs[] = {c->spec,   c->d_mesh, c->d_mesh64, c->d_a,    c->d_c,       c->d_piv, c->d_seg,
-                  c->d_tw_x, c->d_tw_y,    c->d_rtw_x, c->d_twl_x, c->d_twl_y, c->d_rkcoef,
+                  c->d_rtw_x, c->d_twl_x, c->d_twl_y, c->d_rkcoef,
                   c->d_partial, c->d_scalar, c->d_red, c->d_feat, c->d_nut};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
@@ -306,7 +306,7 @@ int step_impl(pll_context* c, bool first, bool last) {
   int rc;
   const bool fused = !c->is_forced[1] && !c->is_forced[2];
   const int fold = (fused && !first) ? 1 : 0;
-  if (c->closure && fused && fft_x_rhs_available(c) && closure_fused_available(c)) {
+  if (c->closure && fused && closure_fused_available(c)) {
     // the closure stages (eddy viscosity evaluated on every cell of the
     // stage's source) in a deferred sequence: the previous step's projection,
     // forcing and boundary update (:145-153) in one pass before stage 1, u1's
@@ -336,7 +336,7 @@ int step_impl(pll_context* c, bool first, bool last) {
     if ((rc = launch_poisson_step(c, false))) return rc;  // :137
     return finish_step(c, false, last);
   }
-  if (fused && c->prec != PLL_FP64 && fft_x_rhs_available(c)) {
+  if (fused && c->prec != PLL_FP64) {
     // FP32-mixed: the projection of step n (:145), its forcing (:149) and
     // boundary update (:153) are applied by step n+1's stage loads (corr);
     // stage 2 sums the bulk mean of the predictor for that forcing, and
@@ -373,7 +373,7 @@ int step_impl(pll_context* c, bool first, bool last) {
     if ((rc = launch_poisson_step(c, false))) return rc;       // :137
     return finish_deferred(c, last);
   }
-  // unfused, or FP32-mixed without the calcRHS transform
+  // unfused: v or w is forced
   if ((rc = launch_rk(c, 1, fold))) return rc;  // src/main.cc:117
   if ((rc = launch_bc_vel(c, 1))) return rc;    // :121
   if ((rc = launch_rk(c, 2, fold))) return rc;  // :125

@@ -28,13 +28,16 @@ struct MeshT {
 };
 
 // Stockham plan of a complex transform of length L held in LDS.
-constexpr int kMaxPass = 20;
+constexpr int kMaxPass = 8;
 struct FftPlan {
   int L;
   int npass;
+  int tps;  // threads per sequence: one butterfly of the smallest radix each
   int radix[kMaxPass];
-  int ns[kMaxPass];     // span before the pass (product of earlier radices)
-  int twoff[kMaxPass];  // offset of the pass' twiddles: tw[off + k*(R-1) + r-1]
+  int ns[kMaxPass];        // span before the pass (product of earlier radices)
+  int lr[kMaxPass];        // butterflies of the pass, L / radix
+  int tws[kMaxPass];       // twiddle stride, L / (ns * radix)
+  unsigned mns[kMaxPass];  // ceil(2^32 / ns): division by ns
 };
 
 // Blocks are dispatched round-robin over the 8 XCDs of the GPU; this gives each
@@ -124,14 +127,13 @@ struct pll_context {
   // FFT plans and twiddles (in field precision)
   pll::FftPlan plan_x;  // complex length nx/2
   pll::FftPlan plan_y;  // complex length ny
-  void* d_tw_x = nullptr;
-  void* d_tw_y = nullptr;
   void* d_rtw_x = nullptr;  // exp(-2 pi i k/nx), k = 0..nx/2
-  void* d_twl_x = nullptr;  // exp(-2 pi i t/L), L = nx/2 (fixed-length kernels)
+  void* d_twl_x = nullptr;  // exp(-2 pi i t/L), L = nx/2 
   void* d_twl_y = nullptr;  // exp(-2 pi i t/L), L = ny
   bool x_fixed = false, y_fixed = false;
   int rhs_bcfold = 0;  // calcRHS in the x transform reads halos through the boundary rules
-  int x_batch = 1, y_tile = 2;
+  int x_batch = 1;  // rows per block of the run-time-plan x transforms
+  int y_tile = 0;   // log2 of the column pairs per block of the y transforms
 
   // reductions
   double* d_partial = nullptr;
@@ -249,7 +251,6 @@ int launch_check_nan(pll_context* c, int field, int* passed);
 int fft_setup(pll_context* c);
 int launch_fft_x_fwd(pll_context* c);
 // calcRHS fused into the forward x transform (reads u, v, w; p is not written)
-bool fft_x_rhs_available(const pll_context* c);
 int launch_fft_x_fwd_rhs(pll_context* c);
 // inverse x transform inside the step (x halos of p written with their periodic values)
 int launch_fft_x_bwd_step(pll_context* c);

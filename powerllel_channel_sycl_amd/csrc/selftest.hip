@@ -30,8 +30,16 @@ extern "C" int pll_selftest_dft(int radix, int sign, const double* in, double* o
     case 5: return run_sign<5>(sign, in, out);
     case 6: return run_sign<6>(sign, in, out);
     case 8: return run_sign<8>(sign, in, out);
+    case 9: return run_sign<9>(sign, in, out);
+    case 10: return run_sign<10>(sign, in, out);
     case 12: return run_sign<12>(sign, in, out);
+    case 15: return run_sign<15>(sign, in, out);
     case 16: return run_sign<16>(sign, in, out);
     default: return 1;
   }
+}
+
+// The radices fft_plan takes for a length; returns their number (0: none).
+extern "C" int pll_selftest_plan(int L, int max_threads, int* radices) {
+  return pll::fft_plan(L, max_threads, radices);
 }
