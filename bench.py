@@ -39,19 +39,19 @@ WORKLOADS = {
 DEFAULT_WORKLOAD = "retau550_768x384x384"
 
 # Algorithmic (compulsory) HBM bytes per grid point per launch.  Inside a run
-# the previous step's projection is applied on load, so stage 1 reads u,v,w,p
-# and writes u1,v1,w1.  FP64: stage 2 fused with calcRHS reads u1,v1,w1,u,v,w,p
-# and writes u,v,w and the right-hand side; each transform and the tridiagonal
-# solve read and write the work array once; correctVel (last step of a run)
-# reads p,u,v,w and writes u,v,w (the bulk mean of u rides along); the separate
-# bulk mean reads u; the force update reads and writes u.  FP32-mixed (4-byte
-# fields): inside a run both stages run in one kernel (rk12: reads u,v,w,p,
-# writes u,v,w; u1 stays on chip); the first and last step of a run take the
-# separate stages, where stage 2 reads u1,v1,w1,u,v,w,p and writes u,v,w.
-# calcRHS runs inside the forward x transform (reads u,v,w, writes the work
-# array).
+# both RK stages run in one kernel (rk12) with the previous step's projection
+# applied on load: it reads u, v, w, p and writes u, v, w; u1 stays on chip.
+# calcRHS runs inside the forward x transform (reads u, v, w, writes the work
+# array); each other transform and the tridiagonal solve read and write the work
+# array once; correctVel (last step of a run) reads p, u, v, w and writes u, v, w;
+# the separate bulk mean reads u; the force update reads and writes u.  The
+# separate stages (rk1, rk2: first step of a run) are listed with the deferred
+# projection's p among their reads (FP64 stage 1, FP32 stage 2), and rk2_rhs is
+# FP64 stage 2 with calcRHS and the projection in one kernel: forms that earlier
+# measurements were made in and that no run launches any more.
 BYTES_PER_POINT = {
-    "fp64": {"rk1": 56, "rk2": 72, "calc_rhs": 32, "rk2_rhs": 88, "fft_x_fwd": 16,
+    "fp64": {"rk1": 56, "rk2": 72, "calc_rhs": 32, "rk2_rhs": 88, "rk12": 56,
+             "fft_x_fwd": 16, "fft_x_fwd_rhs": 32,
              "fft_y_fwd": 16, "solve_trid": 16, "fft_y_bwd": 16, "fft_x_bwd": 16,
              "correct_vel": 56, "mean_partial": 8, "force_add": 16},
     "fp32_mixed": {"rk1": 28, "rk2": 40, "rk12": 28, "calc_rhs": 16, "fft_x_fwd": 8,

@@ -9,6 +9,7 @@
 #include "pll_internal.hpp"
 #include "stencil_ops.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -37,122 +38,119 @@ struct PlaneAcc {
   }
 };
 
-// FP32-mixed form of the same operator, scaled by S (dt in stage 1, dt/2 in
-// stage 2): algebraically equal to S*(visc - conv) above, with the mesh factors
-// gathered into per-plane coefficients (RkCoef) and the viscous terms written
-// as second differences.  It is not bit-identical to the reference order and
-// is used only by the FP32-mixed path, whose error is measured against the
-// FP64 oracle.
+// The momentum operator with fewer operations, scaled by S (dt in stage 1, dt/2
+// in stage 2): algebraically equal to S*(visc - conv) of tendency_z, with the
+// mesh factors gathered into per-plane coefficients (RkCoef), the viscous terms
+// written as second differences and products fused into FMAs: about 85
+// operations for the three components instead of 150.  It rounds differently
+// from the reference's order (no less accurately), so only the FP32-mixed
+// stages and the fused stages inside a run use it.
+template <typename T>
 struct RkCoef {
-  float a1, a2, b1, b2;  // (u,v) face interpolation to k+1/2 and k-1/2
-  float zuv, cp, cm;     // S*0.25*dzf_inv(k); S*re_inv*dzc_inv(k|k-1)*dzf_inv(k)
-  float zw, dp, dm;      // S*0.25*dzc_inv(k); S*re_inv*dzf_inv(k+1|k)*dzc_inv(k)
-  float cdu, cdw;        // diagonal of the viscous operator: 2 vx + 2 vy + cp + cm (u, v), + dp + dm (w)
+  T a1, a2, b1, b2;  // (u,v) face interpolation to k+1/2 and k-1/2
+  T zuv, cp, cm;     // S*0.25*dzf_inv(k); S*re_inv*dzc_inv(k|k-1)*dzf_inv(k)
+  T zw, dp, dm;      // S*0.25*dzc_inv(k); S*re_inv*dzf_inv(k+1|k)*dzc_inv(k)
+  T cdu, cdw;        // diagonal of the viscous operator: 2 vx + 2 vy + cp + cm (u, v), + dp + dm (w)
 };
+template <typename T>
+__device__ __forceinline__ RkCoef<T> load_coef(const RkCoef<T>* p, int k) {
+  static_assert(sizeof(RkCoef<T>) == 12 * sizeof(T), "twelve coefficients");
+  const T* f = reinterpret_cast<const T*>(p + k);
+  auto c = [&](int n) { return uniform_load(f, n); };
+  return RkCoef<T>{c(0), c(1), c(2), c(3), c(4), c(5), c(6), c(7), c(8), c(9), c(10), c(11)};
+}
+template <typename T>
 struct RkUniform {
-  float cx, cy, vx, vy, crf;  // S*0.25*dxi, S*0.25*dyi, S*re_inv*dxi^2, S*re_inv*dyi^2, S*0.5*u_crf*dxi
+  T cx, cy, vx, vy, crf;  // S*0.25*dxi, S*0.25*dyi, S*re_inv*dxi^2, S*re_inv*dyi^2, S*0.5*u_crf*dxi
 };
 
-// The lower z-face convective products of the three components (ab*wb,
-// wb*ab, ab*ab): the upper-face products of the cell below up to FP32
-// rounding (the face interpolation coefficients of plane k-1's upper face are
-// plane k's lower ones), carried up a column like the FP64 ZFace.
+// The z-face value of u or v between cells below and above the face, with the
+// upper-face weights (a1, a2) of the lower cell, which are the lower-face
+// weights (b2, b1) of the upper one: one expression for both.
+__device__ __forceinline__ float zface_value(float below, float above, float wb, float wa) {
+  return __builtin_fmaf(below, wb, above * wa);
+}
+__device__ __forceinline__ double zface_value(double below, double above, double wb, double wa) {
+  return __builtin_fma(below, wb, above * wa);
+}
+
+// The lower z-face convective products of the three components: the
+// upper-face products of the cell below, bit for bit, carried up a column like
+// tendency_z's ZFace.
+template <typename T>
 struct ZConv {
-  float u, v, w;
+  T u, v, w;
 };
 
-template <class A>
-__device__ __forceinline__ ZConv zconv_lower(const A& U, const A& V, const A& W, const RkCoef& q) {
-#pragma clang fp contract(fast)
-  ZConv z;
-  const float ub = U(0, 0, 0) * q.b1 + U(0, 0, -1) * q.b2;
-  z.u = ub * (W(0, 0, -1) + W(1, 0, -1));
-  const float vb = V(0, 0, 0) * q.b1 + V(0, 0, -1) * q.b2;
-  z.v = (W(0, 0, -1) + W(0, 1, -1)) * vb;
-  const float wb = W(0, 0, 0) + W(0, 0, -1);
+template <typename T, class A>
+__device__ __forceinline__ ZConv<T> zconv_lower(const A& U, const A& V, const A& W,
+                                                const RkCoef<T>& q) {
+  ZConv<T> z;
+  z.u = zface_value(U(0, 0, -1), U(0, 0, 0), q.b2, q.b1) * (W(0, 0, -1) + W(1, 0, -1));
+  z.v = zface_value(V(0, 0, -1), V(0, 0, 0), q.b2, q.b1) * (W(0, 0, -1) + W(0, 1, -1));
+  const T wb = W(0, 0, -1) + W(0, 0, 0);
   z.w = wb * wb;
   return z;
 }
 
-// The upper z-face convective products of the cell at the accessor's plane
-// (at*wt, wt*at, at*at), the expressions of tendency_fast: what its CARRY form
-// hands to the plane above.
-template <class A>
-__device__ __forceinline__ ZConv zconv_upper(const A& U, const A& V, const A& W, const RkCoef& q) {
+// The lower-face products come from zc, which then receives the upper ones.
+template <bool CRF, typename T, class A>
+__device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W,
+                                              const RkCoef<T>& q, const RkUniform<T>& cu, T& iu,
+                                              T& iv, T& iw, ZConv<T>& zc) {
+  // not held to the reference's rounding: let products fuse into FMAs
 #pragma clang fp contract(fast)
-  ZConv z;
+  // FP64: one component at a time, or the compiler reads the LDS values of all
+  // three ahead and the registers of a wave no longer fit three waves per SIMD
+  // (k_rk12 at 768x384x384: 2442 us without the fence, 2348 us with it; FP32
+  // loses 5 % to it)
+  auto fence = [] {
+    if constexpr (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
+  };
   {
-    const float at = U(0, 0, 0) * q.a1 + U(0, 0, 1) * q.a2;
-    const float wt = W(0, 0, 0) + W(1, 0, 0);
-    z.u = at * wt;
-  }
-  {
-    const float at = V(0, 0, 0) * q.a1 + V(0, 0, 1) * q.a2;
-    const float wt = W(0, 0, 0) + W(0, 1, 0);
-    z.v = wt * at;
-  }
-  {
-    const float at = W(0, 0, 0) + W(0, 0, 1);
-    z.w = at * at;
-  }
-  return z;
-}
-
-// CARRY: the lower-face products come from zc, which then receives the upper ones.
-template <bool CRF, bool CARRY = false, class A>
-__device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W, const RkCoef& q,
-                                              const RkUniform& cu, float& iu, float& iv,
-                                              float& iw, ZConv* zc = nullptr) {
-  // the FP32 form is not held to the reference's rounding: let products fuse into FMAs
-#pragma clang fp contract(fast)
-  {
-    const float q0 = U(0, 0, 0), qe = U(1, 0, 0), qw = U(-1, 0, 0), qn = U(0, 1, 0);
-    const float qs = U(0, -1, 0), qt = U(0, 0, 1), qb = U(0, 0, -1);
-    const float ae = q0 + qe, aw = qw + q0, an = q0 + qn, as = qs + q0;
-    const float at = q0 * q.a1 + qt * q.a2;
-    const float vn = V(0, 0, 0) + V(1, 0, 0), vs = V(0, -1, 0) + V(1, -1, 0);
-    const float wt = W(0, 0, 0) + W(1, 0, 0);
-    const float ct = at * wt;
-    const float cb = CARRY ? zc->u : (q0 * q.b1 + qb * q.b2) * (W(0, 0, -1) + W(1, 0, -1));
-    if (CARRY) zc->u = ct;
-    float conv = cu.cx * (ae * ae - aw * aw) + cu.cy * (an * vn - as * vs) + q.zuv * (ct - cb);
+    const T q0 = U(0, 0, 0), qe = U(1, 0, 0), qw = U(-1, 0, 0), qn = U(0, 1, 0);
+    const T qs = U(0, -1, 0), qt = U(0, 0, 1), qb = U(0, 0, -1);
+    const T ae = q0 + qe, aw = qw + q0, an = q0 + qn, as = qs + q0;
+    const T at = zface_value(q0, qt, q.a1, q.a2);
+    const T vn = V(0, 0, 0) + V(1, 0, 0), vs = V(0, -1, 0) + V(1, -1, 0);
+    const T wt = W(0, 0, 0) + W(1, 0, 0);
+    const T ct = at * wt;
+    const T cb = zc.u;
+    zc.u = ct;
+    T conv = cu.cx * (ae * ae - aw * aw) + cu.cy * (an * vn - as * vs) + q.zuv * (ct - cb);
     if (CRF) conv += cu.crf * (ae - aw);
     // viscous part as neighbour sums minus the diagonal: fewer operations
     iu = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.cp * qt + q.cm * qb - q.cdu * q0 - conv;
   }
+  fence();
   {
-    const float q0 = V(0, 0, 0), qe = V(1, 0, 0), qw = V(-1, 0, 0), qn = V(0, 1, 0);
-    const float qs = V(0, -1, 0), qt = V(0, 0, 1), qb = V(0, 0, -1);
-    const float ae = q0 + qe, aw = qw + q0, an = q0 + qn, as = qs + q0;
-    const float at = q0 * q.a1 + qt * q.a2;
-    const float ue = U(0, 0, 0) + U(0, 1, 0), uw = U(-1, 0, 0) + U(-1, 1, 0);
-    const float wt = W(0, 0, 0) + W(0, 1, 0);
-    const float ct = wt * at;
-    const float cb = CARRY ? zc->v : (W(0, 0, -1) + W(0, 1, -1)) * (q0 * q.b1 + qb * q.b2);
-    if (CARRY) zc->v = ct;
-    float conv = cu.cx * (ue * ae - uw * aw) + cu.cy * (an * an - as * as) + q.zuv * (ct - cb);
+    const T q0 = V(0, 0, 0), qe = V(1, 0, 0), qw = V(-1, 0, 0), qn = V(0, 1, 0);
+    const T qs = V(0, -1, 0), qt = V(0, 0, 1), qb = V(0, 0, -1);
+    const T ae = q0 + qe, aw = qw + q0, an = q0 + qn, as = qs + q0;
+    const T at = zface_value(q0, qt, q.a1, q.a2);
+    const T ue = U(0, 0, 0) + U(0, 1, 0), uw = U(-1, 0, 0) + U(-1, 1, 0);
+    const T wt = W(0, 0, 0) + W(0, 1, 0);
+    const T ct = wt * at;
+    const T cb = zc.v;
+    zc.v = ct;
+    T conv = cu.cx * (ue * ae - uw * aw) + cu.cy * (an * an - as * as) + q.zuv * (ct - cb);
     if (CRF) conv += cu.crf * (ae - aw);
     iv = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.cp * qt + q.cm * qb - q.cdu * q0 - conv;
   }
+  fence();
   {
-    const float q0 = W(0, 0, 0), qe = W(1, 0, 0), qw = W(-1, 0, 0), qn = W(0, 1, 0);
-    const float qs = W(0, -1, 0), qt = W(0, 0, 1), qb = W(0, 0, -1);
-    const float ae = q0 + qe, aw = qw + q0, an = q0 + qn, as = qs + q0;
-    const float at = q0 + qt;
-    const float ue = U(0, 0, 0) * q.a1 + U(0, 0, 1) * q.a2;
-    const float uw = U(-1, 0, 0) * q.a1 + U(-1, 0, 1) * q.a2;
-    const float vn = V(0, 0, 0) * q.a1 + V(0, 0, 1) * q.a2;
-    const float vs = V(0, -1, 0) * q.a1 + V(0, -1, 1) * q.a2;
-    const float ct = at * at;
-    float cb;
-    if (CARRY) {
-      cb = zc->w;
-      zc->w = ct;
-    } else {
-      const float ab = q0 + qb;
-      cb = ab * ab;
-    }
-    float conv = cu.cx * (ue * ae - uw * aw) + cu.cy * (vn * an - vs * as) + q.zw * (ct - cb);
+    const T q0 = W(0, 0, 0), qe = W(1, 0, 0), qw = W(-1, 0, 0), qn = W(0, 1, 0);
+    const T qs = W(0, -1, 0), qt = W(0, 0, 1), qb = W(0, 0, -1);
+    const T ae = q0 + qe, aw = qw + q0, an = q0 + qn, as = qs + q0;
+    const T at = q0 + qt;
+    const T ue = U(0, 0, 0) * q.a1 + U(0, 0, 1) * q.a2;
+    const T uw = U(-1, 0, 0) * q.a1 + U(-1, 0, 1) * q.a2;
+    const T vn = V(0, 0, 0) * q.a1 + V(0, 0, 1) * q.a2;
+    const T vs = V(0, -1, 0) * q.a1 + V(0, -1, 1) * q.a2;
+    const T ct = at * at;
+    const T cb = zc.w;
+    zc.w = ct;
+    T conv = cu.cx * (ue * ae - uw * aw) + cu.cy * (vn * an - vs * as) + q.zw * (ct - cb);
     if (CRF) conv += cu.crf * (ae - aw);
     iw = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.dp * qt + q.dm * qb - q.cdw * q0 - conv;
   }
@@ -162,73 +160,125 @@ __device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W
 constexpr int kRkTx = 64;  // tile width along x (one wavefront per row)
 constexpr int kRkTy = 8;   // tile rows along y
 
-// Tile rows of the stage and projection kernels: 4 for the FP64 projection
-// (4-7 % faster than 8 at 768x384x384 on MI355X), 8 elsewhere (the FP32 stages
-// lose 10-28 % with 4 and 28 % with 16; the FP64 stage 1, which applies the
-// deferred projection on load, is 4 % faster with 8 than with 4).  The fused FP64 stage 2 +
-// calcRHS takes 12 rows where that still gives kRhsTallBlocks blocks (fewer
-// y-halo rows per output row than 8) and 8 on smaller grids, where taller tiles
-// would leave too few blocks (4 % slower at 96x64x64).  12 rows (768 threads,
-// up to 168 VGPRs, one block per CU) rather than 16: at 1024 threads its
-// deferred-projection variant is held to 128 VGPRs and spills.
-constexpr int kRhsTallTy = 12;
-constexpr long kRhsTallBlocks = 1024;
+// Tile rows of the projection kernel: 4 in FP64 (4-7 % faster than 8 at
+// 768x384x384), 8 in FP32.
 template <typename T>
 constexpr int correct_ty() {
   return std::is_same<T, double>::value ? 4 : kRkTy;
 }
 
-// Stage 1: d = s + dt*F(s).  Stage 2: d = (s + dt*F(s) + d)/2.
+// The stencil coefficients of both stages: the mesh and the uniform factors of
+// the reference's formulas, and the per-plane tables of tendency_fast.
+template <typename T>
+struct RkParam {
+  MeshT<T> m;
+  T dxi, dyi, rei, dt, ucrf, dtdxi, dtdyi, bc_u;
+  const RkCoef<T>* coef1;
+  const RkCoef<T>* coef2;
+  RkUniform<T> cu1, cu2;
+};
+
+// What a thread of k_rk12 carries up its column from one plane to the next:
+// the lower convective products and the values of the plane below, which the
+// viscous terms read.  With them a stage reads only the planes k and k+1.
+template <typename T>
+struct ZCarry {
+  ZConv<T> z;
+  T u, v, w;
+};
+
+template <typename T, int STAGE, class A>
+__device__ __forceinline__ ZCarry<T> carry_start(const A& U, const A& V, const A& W,
+                                                 const RkParam<T>& q, int k) {
+  return ZCarry<T>{zconv_lower(U, V, W, load_coef(STAGE == 1 ? q.coef1 : q.coef2, k)),
+                   U(0, 0, -1), V(0, 0, -1), W(0, 0, -1)};
+}
+
+// A stencil accessor whose value below the centre is carried in a register.
+template <typename T, int SX>
+struct CarryAcc {
+  PlaneAcc<T, SX> a;
+  T below;
+  __device__ __forceinline__ T operator()(int di, int dj, int dk) const {
+    return dk < 0 ? below : a(di, dj, dk);
+  }
+};
+
+// Stage 1: o = s + dt*F(s); stage 2: o = (s + old)/2 + dt/2*F(s), with the
+// carry replaced by the next plane's.
+template <typename T, int STAGE, bool CRF, int SX>
+__device__ __forceinline__ void stage_update(const PlaneAcc<T, SX>& U, const PlaneAcc<T, SX>& V,
+                                             const PlaneAcc<T, SX>& W, const RkParam<T>& q, int k,
+                                             T ou, T ov, T ow, ZCarry<T>& z, T& o1, T& o2, T& o3) {
+  const RkCoef<T> cq = load_coef(STAGE == 1 ? q.coef1 : q.coef2, k);
+  const CarryAcc<T, SX> Uc{U, z.u}, Vc{V, z.v}, Wc{W, z.w};
+  T iu, iv, iw;
+  tendency_fast<CRF>(Uc, Vc, Wc, cq, STAGE == 1 ? q.cu1 : q.cu2, iu, iv, iw, z.z);
+  z.u = U(0, 0, 0);
+  z.v = V(0, 0, 0);
+  z.w = W(0, 0, 0);
+  if (STAGE == 1) {
+    o1 = z.u + iu;
+    o2 = z.v + iv;
+    o3 = z.w + iw;
+  } else {
+    o1 = (z.u + ou) * T(0.5) + iu;
+    o2 = (z.v + ov) * T(0.5) + iv;
+    o3 = (z.w + ow) * T(0.5) + iw;
+  }
+}
+
+// The block's FP64 partial of the bulk mean into partial[b], through NT doubles
+// of LDS that every thread is done with; the block size is folded onto its
+// largest power of two first.
+template <int NT>
+__device__ __forceinline__ void block_partial(double* red, double s, double* partial, unsigned b) {
+  constexpr int P2 = NT >= 1024 ? 1024 : (NT >= 512 ? 512 : 256);
+  static_assert(NT >= P2 && NT < 2 * P2, "block size");
+  const int t = threadIdx.x;
+  red[t] = s;
+  __syncthreads();
+  if (t < NT - P2) red[t] += red[t + P2];
+  __syncthreads();
+  for (int h = P2 / 2; h > 0; h >>= 1) {
+    if (t < h) red[t] += red[t + h];
+    __syncthreads();
+  }
+  if (t == 0) partial[b] = red[0];
+}
+
+// One RK stage.  Stage 1: d = s + dt*F(s).  Stage 2: d = (s + dt*F(s) + d)/2.
 // A block owns a 64 x 8 (i,j) tile and marches a chunk of k planes.  The three
 // source fields of planes k-1, k, k+1 (tile plus a one-cell halo) sit in an
 // LDS ring; plane k+2 is fetched into registers while plane k is computed and
 // replaces plane k-1 afterwards, so every source value leaves HBM once per block.
+// These stages run where u1 goes through HBM: the reference's routines one by
+// one, the first step of a run (nothing of a previous step to apply) and steps
+// that force v or w.
 //
-// Inside a multi-step run the previous step's forcing and final boundary
-// update are folded into the loads (`fold`): `force` (device scalars, one per
-// forced component) is added to every source value, and every halo cell is
-// rebuilt from interior cells by the reference's closed-form rules -- x/y
-// halos are periodic images, the z ghost planes are 2*bc - (u + f) for u,
-// -(v + f) for v and 0 for w, and w on plane nz is 0
-// (src/mod_updateBound.cc:11-144) -- so the result is bit-identical to forcing,
-// updating the boundary and then running the stage.  Stage 2 adds the
-// deferred forcing to the point value of u it reads.
-//
-// With `corr` the previous step's projection is deferred as well: the stored
-// velocity is the predictor u* and every value read becomes
-// u* - dt*grad(p) (src/mod_calcVel.cc:272-274) before the force and the
-// boundary rules apply; p carries valid halos (updateBoundP ran).  With `acc`
-// stage 2 also sums its new u times dzflzi(k) in FP64 into partial[block]: the
-// bulk mean of the next projected velocity, since the projection changes every
-// x-row's sum only by p(nx+1) - p(1) = 0.
-// k_rk is the FP32-mixed form (tendency_fast, per-plane coefficients);
-// k_rk_late below is the FP64 form in the reference's arithmetic.  PROJ
-// compiles the deferred projection in; stage 1 launches the PROJ variant when
-// the projection is deferred.
-template <typename T, int STAGE, bool PROJ = true>
+// With `bcload` every halo cell of the source is rebuilt on load from interior
+// cells by the reference's closed-form rules, for a source whose boundary
+// update was not run: x/y halos are periodic images, the z ghost planes are
+// 2*bc - u for u, -v for v and 0 for w, and w on plane nz is 0
+// (src/mod_updateBound.cc:11-144).  With `acc` stage 2 also sums its new u
+// times dzflzi(k) in FP64 into partial[block]: the bulk mean of the next
+// projected velocity, since the projection changes every x-row's sum only by
+// p(nx+1) - p(1) = 0.
+// k_rk is the FP32-mixed form (tendency_fast, per-plane coefficients): at up to
+// 8 waves per SIMD the other waves cover the wait for a fetch's loads, and the
+// late form's registers cost it 6-9 %.
+template <typename T, int STAGE, bool CRF>
 __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restrict__ su,
                                                      const T* __restrict__ sv,
                                                      const T* __restrict__ sw, T* __restrict__ du,
                                                      T* __restrict__ dv, T* __restrict__ dw,
-                                                     MeshT<T> m, T dxi, T dyi, T rei, T dt,
-                                                     T ucrf, int kchunk, int ntx, int nty,
-                                                     int fold, int defer, T bc_u,
-                                                     const double* __restrict__ force,
-                                                     int forced_mask,
-                                                     const RkCoef* __restrict__ coef,
-                                                     RkUniform cu, int crf,
-                                                     const T* __restrict__ pp, int corr,
-                                                     T dtdxi, T dtdyi, int acc,
-                                                     const double* __restrict__ dzflzi,
+                                                     RkParam<T> q0, int kchunk, int ntx, int nty,
+                                                     int acc, const double* __restrict__ dzflzi,
                                                      double* __restrict__ partial, int bcload) {
   constexpr int TX = kRkTx, TY = kRkTy, SX = TX + 2, SY = TY + 2, PL = SX * SY,
                 NT = TX * TY;
   constexpr int NPF = (PL + NT - 1) / NT;
   static_assert(std::is_same<T, float>::value, "the FP64 stages run k_rk_late");
-  corr = PROJ ? corr : 0;
-  // halo cells from the boundary rules on load: with the folded forcing, or
-  // alone (bcload) for a source whose boundary update was not run
-  bcload = (fold || bcload) ? 1 : 0;
   __shared__ T sh[3][3][PL];  // [field][ring slot][tile cell]
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
   const int ti = (int)(b % (unsigned)ntx), tj = (int)((b / (unsigned)ntx) % (unsigned)nty);
@@ -238,21 +288,12 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   const int i = i0 + tx + 1, j = j0 + ty + 1;
   const bool active = i <= g.nx && j <= g.ny;
-  // deferred forcing of the three components (applied only where forced):
-  // to every loaded value when folding, to the point value of stage 2 when deferring
-  const bool any = fold || defer;
-  const bool fu = any && (forced_mask & 1), fv = any && (forced_mask & 2),
-             fw = any && (forced_mask & 4);
-  const T f_u = fu ? (T)force[0] : T(0), f_v = fv ? (T)force[1] : T(0),
-          f_w = fw ? (T)force[2] : T(0);
 
   long gaddr[NPF];  // plane-relative source address of this thread's tile cells (-1: outside)
-  int cell[NPF];
 #pragma unroll
   for (int n = 0; n < NPF; ++n) {
     const int e = threadIdx.x + n * NT;
     int gx = i0 + e % SX, gy = j0 + e / SX;
-    cell[n] = e;
     const bool inside = e < PL && gx <= g.nx + 1 && gy <= g.ny + 1;
     if (bcload) {  // halo cells read their periodic image
       gx = gx == 0 ? g.nx : (gx == g.nx + 1 ? 1 : gx);
@@ -261,51 +302,33 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
     gaddr[n] = inside ? gx + g.sx * gy : -1;
   }
   T pre[3][NPF];
-  T pabove[NPF];      // p of plane ks+1 from the previous fetch (corr)
-  int pabove_k = -1;  // the plane pabove belongs to
   auto fetch = [&](int kk) {
     const bool ghost = bcload && (kk == 0 || kk == g.nz + 1);
     const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
     const bool wzero = bcload && (kk == 0 || kk >= g.nz);
-    // the stage-1 source is the stored velocity; stage 2's source u1 is not projected
-    const bool pj = STAGE == 1 && corr;
-    const T dzci = pj ? m.dzc_inv[ks] : T(0);
-    const bool reuse = pabove_k == ks;
 #pragma unroll
     for (int n = 0; n < NPF; ++n)
       if (gaddr[n] >= 0) {
         const long a = gaddr[n] + g.sxy * ks;
-        T qu = su[a], qv = sv[a], qw = wzero ? T(0) : sw[a];
-        if (pj) {
-          const T p0 = reuse ? pabove[n] : pp[a];
-          pabove[n] = pp[a + g.sxy];
-          qu = qu - (pp[a + 1] - p0) * dtdxi;
-          qv = qv - (pp[a + g.sx] - p0) * dtdyi;
-          // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
-          if (!wzero) qw = qw - (pabove[n] - p0) * dt * dzci;
-        }
-        if (fold) {
-          if (fu) qu = qu + f_u;
-          if (fv) qv = qv + f_v;
-          if (fw && !wzero) qw = qw + f_w;
-        }
+        T qu = su[a], qv = sv[a];
+        const T qw = wzero ? T(0) : sw[a];
         if (ghost) {
-          qu = T(2) * bc_u - qu;  // src/mod_updateBound.cc:92,123
+          qu = T(2) * q0.bc_u - qu;  // src/mod_updateBound.cc:92,123
           qv = T(2) * T(0) - qv;
         }
         pre[0][n] = qu;
         pre[1][n] = qv;
         pre[2][n] = qw;
       }
-    pabove_k = pj ? ks + 1 : -1;
   };
   auto commit = [&](int slot) {
 #pragma unroll
     for (int n = 0; n < NPF; ++n)
       if (gaddr[n] >= 0) {
-        sh[0][slot][cell[n]] = pre[0][n];
-        sh[1][slot][cell[n]] = pre[1][n];
-        sh[2][slot][cell[n]] = pre[2][n];
+        const int e = threadIdx.x + n * NT;
+        sh[0][slot][e] = pre[0][n];
+        sh[1][slot][e] = pre[1][n];
+        sh[2][slot][e] = pre[2][n];
       }
   };
   if (k0 > k1) {
@@ -322,75 +345,42 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
   __syncthreads();
   int sm = 0, s0 = 1, sp = 2;
   const int c = (ty + 1) * SX + tx + 1;
-  // stage 2's point values and, with corr, the pressures around the point
-  // (fetching them a plane ahead costs more in occupancy than it saves)
-  struct Point {
-    T u, v, w, p0, pe, pn, pt;
-  };
-  auto load_point = [&](int kk, Point& q) {
-    const long a = g.idx(i, j, kk);
-    q.u = du[a];
-    q.v = dv[a];
-    q.w = dw[a];
-    if (corr) {
-      q.p0 = pp[a];
-      q.pe = pp[a + 1];
-      q.pn = pp[a + g.sx];
-      q.pt = pp[a + g.sxy];
-    }
-  };
-  Point qc{};
-  ZConv zc{};  // the carried lower-face convective products of the thread's column
+  ZConv<T> zc{};  // the carried lower-face convective products of the thread's column
+  const RkCoef<T>* coef = STAGE == 1 ? q0.coef1 : q0.coef2;
+  const RkUniform<T> cu = STAGE == 1 ? q0.cu1 : q0.cu2;
   if (active) {
     const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
     const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
     const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
-    zc = zconv_lower(U, V, W, coef[k0]);
+    zc = zconv_lower(U, V, W, load_coef(coef, k0));
   }
   for (int k = k0; k <= k1; ++k) {
     const bool more = k + 2 <= k1 + 1;
     if (more) fetch(k + 2);
-    if (STAGE == 2 && active) load_point(k, qc);
     if (active) {
-      const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
-      const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
-      const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
       const long a = g.idx(i, j, k);
       T ou = T(0), ov = T(0), ow = T(0);
       if (STAGE == 2) {
-        ou = qc.u;
-        ov = qc.v;
-        ow = qc.w;
-        if (corr) {
-          ou = ou - (qc.pe - qc.p0) * dtdxi;
-          ov = ov - (qc.pn - qc.p0) * dtdyi;
-          ow = ow - (qc.pt - qc.p0) * dt * m.dzc_inv[k];
-        }
-        if (defer) {
-          if (fu) ou = ou + f_u;
-          if (fv) ov = ov + f_v;
-          if (fw) ow = ow + f_w;
-          if (k == g.nz) ow = T(0);  // the wall value of the boundary update
-        }
+        ou = du[a];
+        ov = dv[a];
+        ow = dw[a];
       }
-      {
-        const RkCoef q = coef[k];
-        float iu, iv, iw;
-        if (crf)
-          tendency_fast<true, true>(U, V, W, q, cu, iu, iv, iw, &zc);
-        else
-          tendency_fast<false, true>(U, V, W, q, cu, iu, iv, iw, &zc);
-        if (STAGE == 1) {
-          du[a] = U(0, 0, 0) + iu;
-          dv[a] = V(0, 0, 0) + iv;
-          dw[a] = W(0, 0, 0) + iw;
-        } else {
-          const T nu = (U(0, 0, 0) + ou) * 0.5f + iu;
-          du[a] = nu;
-          dv[a] = (V(0, 0, 0) + ov) * 0.5f + iv;
-          dw[a] = (W(0, 0, 0) + ow) * 0.5f + iw;
-          if (acc) msum += (double)nu * dzflzi[k];
-        }
+      const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
+      const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
+      const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
+      const RkCoef<T> q = load_coef(coef, k);
+      float iu, iv, iw;
+      tendency_fast<CRF>(U, V, W, q, cu, iu, iv, iw, zc);
+      if (STAGE == 1) {
+        du[a] = U(0, 0, 0) + iu;
+        dv[a] = V(0, 0, 0) + iv;
+        dw[a] = W(0, 0, 0) + iw;
+      } else {
+        const T nu = (U(0, 0, 0) + ou) * 0.5f + iu;
+        du[a] = nu;
+        dv[a] = (V(0, 0, 0) + ov) * 0.5f + iv;
+        dw[a] = (W(0, 0, 0) + ow) * 0.5f + iw;
+        if (acc) msum += (double)nu * uniform_load(dzflzi, k);
       }
     }
     __syncthreads();
@@ -401,58 +391,41 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
     s0 = sp;
     sp = t;
   }
-  if (acc) {
-    // the ring is free after the last barrier of the loop
-    double* red = reinterpret_cast<double*>(&sh[0][0][0]);
-    static_assert(sizeof(sh) >= NT * sizeof(double), "reduction scratch");
-    red[threadIdx.x] = msum;
-    __syncthreads();
-    for (int h = NT / 2; h > 0; h >>= 1) {
-      if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[b] = red[0];
-  }
+  // the ring is free after the last barrier of the loop
+  static_assert(sizeof(sh) >= NT * sizeof(double), "reduction scratch");
+  if (acc) block_partial<NT>(reinterpret_cast<double*>(&sh[0][0][0]), msum, partial, b);
 }
 
-// The FP64 stages: k_rk's ring, folding and deferred projection, in the
-// reference's arithmetic and operation order (tendency_z, src/mod_calcVel.cc:
-// 81,103,125 and :194,216,238; bit-identical to the reference's stages), with
-// the plane loads scheduled late.  A fetch only issues the loads of plane k+2
-// into registers; the projection, forcing and boundary rules apply when that
-// plane is committed to the ring, after plane k has been computed, and plane
-// k's new values are stored after the commit.  With that arithmetic inside the
-// fetch (k_rk's form) every wave waits for its loads there, and a commit after
-// the stores waits for their completion too: that form ran 4-5 % slower in FP64
-// at 768x384x384 (4 waves per SIMD).  Every plane load is unconditional (a
-// thread without a tile cell loads the corner cell (0, 0) and writes LDS slot
-// PL; w is loaded on every plane and replaced by the wall value where it
-// applies): loads that some paths skip leave the compiler's wait counting
-// unsure which are still in flight, and it then waits for them before the next
-// fetch reuses their registers.  The FP64 tendency carries the lower z face,
-// so plane k-1 is not read while plane k is computed and one barrier per plane
-// suffices.  Stage 2 issues the point values of plane k before the fetch, so
-// that waiting for them leaves the plane in flight.
-// tile rows of k_rk_late: 8 (two 512-thread blocks per CU at 126 VGPRs); 4 rows
-// measured 9 % and 16 rows 5 % slower at 768x384x384
+// The FP64 stages: k_rk's ring and loads in the reference's arithmetic and
+// operation order (tendency_z, src/mod_calcVel.cc:81,103,125 and :194,216,238;
+// bit-identical to the reference's stages), with the plane loads scheduled
+// late.  A fetch only issues the loads of plane k+2 into registers; the
+// boundary rules apply when that plane is committed to the ring, after plane k
+// has been computed, and plane k's new values are stored after the commit.
+// With that arithmetic inside the fetch (k_rk's form) every wave waits for its
+// loads there, and a commit after the stores waits for their completion too:
+// that form ran 4-5 % slower in FP64 at 768x384x384 (4 waves per SIMD).  Every
+// plane load is unconditional (a thread without a tile cell loads the corner
+// cell (0, 0) and writes LDS slot PL; w is loaded on every plane and replaced
+// by the wall value where it applies): loads that some paths skip leave the
+// compiler's wait counting unsure which are still in flight, and it then waits
+// for them before the next fetch reuses their registers.  The FP64 tendency
+// carries the lower z face, so plane k-1 is not read while plane k is computed
+// and one barrier per plane suffices.  Stage 2 issues the point values of plane
+// k before the fetch, so that waiting for them leaves the plane in flight.
+// tile rows of k_rk_late: 8; 4 rows measured 9 % and 16 rows 5 % slower at
+// 768x384x384
 constexpr int kLateTy = 8;
-template <int STAGE, bool PROJ>
-__global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
+template <int STAGE, bool CRF>
+__global__ __launch_bounds__(kRkTx * kLateTy, 4) void k_rk_late(
     Geom g, const double* __restrict__ su, const double* __restrict__ sv,
     const double* __restrict__ sw, double* __restrict__ du, double* __restrict__ dv,
-    double* __restrict__ dw, MeshT<double> m, double dxi, double dyi, double rei, double dt,
-    double ucrf, int kchunk, int ntx, int nty, int fold, int defer, double bc_u,
-    const double* __restrict__ force, int forced_mask, const RkCoef* __restrict__,
-    RkUniform, int crf, const double* __restrict__ pp, int corr, double dtdxi, double dtdyi,
-    int, const double* __restrict__, double* __restrict__, int) {
+    double* __restrict__ dw, RkParam<double> q0, int kchunk, int ntx, int nty, int acc,
+    const double* __restrict__ dzflzi, double* __restrict__ partial, int bcload) {
   using T = double;
   constexpr int TX = kRkTx, TY = kLateTy, SX = TX + 2, SY = TY + 2, PL = SX * SY,
                 NT = TX * TY;
   constexpr int NPF = (PL + NT - 1) / NT;
-  // stage 1 launches the PROJ variant exactly when the projection is deferred
-  constexpr bool PJ = STAGE == 1 && PROJ;
-  corr = PROJ ? corr : 0;
-  const int bcload = fold;
   __shared__ T sh[3][3][PL + 1];  // [field][ring slot][tile cell]; slot PL: no cell
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
   const int ti = (int)(b % (unsigned)ntx), tj = (int)((b / (unsigned)ntx) % (unsigned)nty);
@@ -462,10 +435,6 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   const int i = i0 + tx + 1, j = j0 + ty + 1;
   const bool active = i <= g.nx && j <= g.ny;
-  const bool any = fold || defer;
-  const bool fu = any && (forced_mask & 1), fv = any && (forced_mask & 2),
-             fw = any && (forced_mask & 4);
-  const T f_u = fu ? force[0] : T(0), f_v = fv ? force[1] : T(0), f_w = fw ? force[2] : T(0);
 
   long gaddr[NPF];  // plane-relative source address of this thread's tile cells
   int cell[NPF];
@@ -482,51 +451,26 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
     cell[n] = inside ? e : PL;
   }
   T ru[NPF], rv[NPF], rw[NPF];
-  T rp0[NPF], rpe[NPF], rpn[NPF], rpt[NPF];  // p at the cell, +x, +y, +z (PJ)
-  auto plane_src = [&](int kk) {
-    const bool ghost = bcload && (kk == 0 || kk == g.nz + 1);
-    return ghost ? (kk == 0 ? 1 : g.nz) : kk;
-  };
   auto fetch = [&](int kk) {
-    const long pofs = g.sxy * plane_src(kk);
+    const bool ghost = bcload && (kk == 0 || kk == g.nz + 1);
+    const long pofs = g.sxy * (ghost ? (kk == 0 ? 1 : g.nz) : kk);
 #pragma unroll
     for (int n = 0; n < NPF; ++n) {
       const long a = gaddr[n] + pofs;
       ru[n] = su[a];
       rv[n] = sv[a];
       rw[n] = sw[a];
-      if constexpr (PJ) {
-        rp0[n] = pp[a];
-        rpe[n] = pp[a + 1];
-        rpn[n] = pp[a + g.sx];
-        rpt[n] = pp[a + g.sxy];
-      }
     }
   };
-  // k_rk's fetch arithmetic, applied to the loaded registers of plane kk
   auto commit = [&](int kk, int slot) {
     const bool ghost = bcload && (kk == 0 || kk == g.nz + 1);
-    const int ks = plane_src(kk);
     const bool wzero = bcload && (kk == 0 || kk >= g.nz);
-    const T dzci = PJ ? m.dzc_inv[ks] : T(0);
 #pragma unroll
     for (int n = 0; n < NPF; ++n) {
       T qu = ru[n], qv = rv[n], qw = rw[n];
-      if constexpr (PJ) {
-        const T p0 = rp0[n];
-        qu = qu - (rpe[n] - p0) * dtdxi;
-        qv = qv - (rpn[n] - p0) * dtdyi;
-        // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
-        qw = qw - (rpt[n] - p0) * dt * dzci;
-      }
-      if (fold) {
-        if (fu) qu = qu + f_u;
-        if (fv) qv = qv + f_v;
-        if (fw) qw = qw + f_w;
-      }
       if (wzero) qw = T(0);
       if (ghost) {
-        qu = T(2) * bc_u - qu;  // src/mod_updateBound.cc:92,123
+        qu = T(2) * q0.bc_u - qu;  // src/mod_updateBound.cc:92,123
         qv = T(2) * T(0) - qv;
       }
       sh[0][slot][cell[n]] = qu;
@@ -534,7 +478,10 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
       sh[2][slot][cell[n]] = qw;
     }
   };
-  if (k0 > k1) return;
+  if (k0 > k1) {
+    if (acc && threadIdx.x == 0) partial[b] = 0.0;
+    return;
+  }
   fetch(k0 - 1);
   commit(k0 - 1, 0);
   fetch(k0);
@@ -544,20 +491,14 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
   __syncthreads();
   int sm = 0, s0 = 1, sp = 2;
   const int c = (ty + 1) * SX + tx + 1;
-  // stage 2's point values and, with corr, the pressures around the point,
-  // loaded for every thread (a thread without a point reads cell (1, 1))
-  T qu0 = T(0), qv0 = T(0), qw0 = T(0), qp0 = T(0), qpe = T(0), qpn = T(0), qpt = T(0);
+  // stage 2's point values, loaded for every thread (a thread without a point
+  // reads cell (1, 1))
+  T qu0 = T(0), qv0 = T(0), qw0 = T(0);
   auto load_point = [&](int kk) {
     const long a = active ? g.idx(i, j, kk) : g.idx(1, 1, kk);
     qu0 = du[a];
     qv0 = dv[a];
     qw0 = dw[a];
-    if (corr) {
-      qp0 = pp[a];
-      qpe = pp[a + 1];
-      qpn = pp[a + g.sx];
-      qpt = pp[a + g.sxy];
-    }
   };
   // the lower z-face terms of the thread's cell, carried up the column
   ZFace<T> zf{};
@@ -565,10 +506,11 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
     const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
     const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
     const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
-    zf = zface_lower<T>(U, V, W, m, k0);
+    zf = zface_lower<T>(U, V, W, q0.m, k0);
   }
   __syncthreads();  // plane k0-1 is read above and rewritten in the loop
   T nu = T(0), nv = T(0), nw = T(0);  // plane k's new values until they are stored
+  double msum = 0.0;                  // FP64 partial of the bulk mean (acc)
   auto compute = [&](int k) {
     if (!active) return;
     const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
@@ -576,31 +518,16 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
     const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
     // reference arithmetic, src/mod_calcVel.cc:81,103,125 and :194,216,238
     T tu, tv, tw;
-    if (crf)
-      tendency_z<T, true, true>(U, V, W, m, k, dxi, dyi, rei, ucrf, tu, tv, tw, zf);
-    else
-      tendency_z<T, false, true>(U, V, W, m, k, dxi, dyi, rei, ucrf, tu, tv, tw, zf);
-    if (STAGE == 1) {
-      nu = U(0, 0, 0) + dt * tu;
-      nv = V(0, 0, 0) + dt * tv;
-      nw = W(0, 0, 0) + dt * tw;
-    } else {
-      T ou = qu0, ov = qv0, ow = qw0;
-      if (corr) {
-        ou = ou - (qpe - qp0) * dtdxi;
-        ov = ov - (qpn - qp0) * dtdyi;
-        ow = ow - (qpt - qp0) * dt * m.dzc_inv[k];
-      }
-      if (defer) {
-        if (fu) ou = ou + f_u;
-        if (fv) ov = ov + f_v;
-        if (fw) ow = ow + f_w;
-        if (k == g.nz) ow = T(0);  // the wall value of the boundary update
-      }
-      nu = (U(0, 0, 0) + dt * tu + ou) * T(0.5);
-      nv = (V(0, 0, 0) + dt * tv + ov) * T(0.5);
-      nw = (W(0, 0, 0) + dt * tw + ow) * T(0.5);
+    tendency_z<T, CRF, true>(U, V, W, q0.m, k, q0.dxi, q0.dyi, q0.rei, q0.ucrf, tu, tv, tw, zf);
+    nu = U(0, 0, 0) + q0.dt * tu;
+    nv = V(0, 0, 0) + q0.dt * tv;
+    nw = W(0, 0, 0) + q0.dt * tw;
+    if (STAGE == 2) {
+      nu = (nu + qu0) * T(0.5);
+      nv = (nv + qv0) * T(0.5);
+      nw = (nw + qw0) * T(0.5);
     }
+    if (STAGE == 2 && acc) msum += nu * uniform_load(dzflzi, k);
   };
   auto store = [&](int k) {
     if (active) {
@@ -626,32 +553,63 @@ __global__ __launch_bounds__(kRkTx * kLateTy) void k_rk_late(
   if (STAGE == 2) load_point(k1);
   compute(k1);
   store(k1);
+  if (STAGE == 2 && acc) {
+    __syncthreads();
+    static_assert(sizeof(sh) >= NT * sizeof(double), "reduction scratch");
+    block_partial<NT>(&sh[0][0][0], msum, partial, b);
+  }
 }
 
-// Both RK stages of an FP32-mixed step inside a run (src/mod_calcVel.cc:61-125
-// then :174-238) in one pass.  The stored velocity is the previous step's
+// Tile rows of k_rk12: one block of them fills a CU either way.  FP64 12 (160
+// VGPRs: three waves per SIMD; 8 and 10 rows ran 3021 and 2679 against 2348 us
+// at 768x384x384, 16 rows spill), FP32 16 (1302 against 1312 us with 8 and 1440
+// with 12; 6934 against 7111 us with 8 at 1536x768x512).
+template <typename T>
+constexpr int kRk12Ty() {
+  return std::is_same<T, double>::value ? 12 : 16;
+}
+constexpr int kRk12Slots = 256;  // blocks of k_rk12 that run at once: one per CU
+
+// Both RK stages of a step inside a run (src/mod_calcVel.cc:61-125 then
+// :174-238) in one pass.  The stored velocity is the previous step's
 // predictor u*; its projection, forcing and boundary update are applied on
-// load as in k_rk's stage 1 (fold and corr).  A block owns a 64 x 8 tile of
-// stage-2 points and marches a chunk of k planes.  Stage 1 runs on the tile
-// plus a one-cell ring (66 x 10 cells) from a three-plane LDS ring of the
-// loaded source (68 x 12 cells); its result u1 goes to a second three-plane
-// LDS ring and never to HBM.  The u1 values on the ring are stage 1 at the
-// periodic position -- the x/y boundary update of u1 -- and the planes 0 and
-// nz+1 of u1 and w1 on plane nz follow the boundary rules
-// (src/mod_updateBound.cc:92,123,137), as the stage-2 loads of k_rk rebuild
-// them.  Stage 2's point values are the loaded source at the tile point: the
-// same projection and forcing k_rk's stage 2 applies to them.  Per point, u,
-// v, w and p are read once and the new u, v, w written once.  The result goes
-// to separate arrays, since other blocks still read the source.  With `acc`
-// the block sums the new u times dzflzi(k) in FP64 into partial[block].
-template <int TY>
+// load as in the separate stage 1 (fold and corr).  A block owns a 64 x TY
+// tile of stage-2 points and marches a chunk of k planes.  Stage 1 runs on the
+// tile plus a one-cell ring (each thread its tile point, the first threads one
+// ring cell more) from a two-plane LDS ring of the loaded source (tile plus two
+// cells); its result u1 goes to a second two-plane LDS ring and, except on the
+// last step of a run (U1OUT), never to HBM.  The u1 values on the ring are
+// stage 1 at the periodic position -- the x/y boundary update of u1 -- and the
+// planes 0 and nz+1 of u1 and w1 on plane nz follow the boundary rules
+// (src/mod_updateBound.cc:92,123,137).  Stage 2's point values are the loaded
+// source at the tile point.  Per point u, v, w and p are read once and the new
+// u, v, w written once; the result goes to separate arrays, since other blocks
+// still read the source.  With `acc` the block sums the new u times dzflzi(k)
+// in FP64 into partial[block].
+//
+// Two planes suffice in each ring because the carry holds what plane k-1 would
+// be read for.  The fetch only issues the loads of a plane; the projection,
+// forcing and boundary rules apply at its commit, after stage 2 of the plane
+// below has been computed, and stage 2's results are stored after the commit:
+// arithmetic on the loaded values in the fetch, or stores ahead of the commit,
+// would make a wave wait there.  p on the y halo is read at its image, so only
+// its x halos (written by the inverse x transform) have to be valid.
+//
+// Bound by latency between its two barriers per plane, at one block per CU: per
+// point about 240 (FP64) VALU operations and 60 LDS reads, each near 0.9 ms of
+// pure issue at 768x384x384, beside 56 B of HBM traffic (1.3 ms).  Measured there,
+// FP64: 2348 us for both stages against 1646 + 2331 us for the two kernels it
+// replaces (stage 2 with calcRHS; calcRHS in the transform's loads costs 440 us
+// more there), 141 against 121 + 176 us at 256x192x128.  The reference's
+// operation order instead of tendency_fast took 3058 us.  FP32: 1302 us, 1456
+// with three planes in each ring and 8 rows; 230 against 309 us at 384x256x192,
+// half of which is the chunk rule of rk12_grid.
+template <typename T, int TY, bool U1OUT, bool CRF>
 __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
-    Geom g, const float* __restrict__ su, const float* __restrict__ sv,
-    const float* __restrict__ sw, const float* __restrict__ pp, float* __restrict__ du,
-    float* __restrict__ dv, float* __restrict__ dw, const float* __restrict__ dzc_inv, float dt,
-    float dtdxi, float dtdyi, float bc_u, const double* __restrict__ force, int forced_mask,
-    const RkCoef* __restrict__ coef1, const RkCoef* __restrict__ coef2, RkUniform cu1,
-    RkUniform cu2, int crf, int kchunk, int ntx, int nty, int acc,
+    Geom g, const T* __restrict__ su, const T* __restrict__ sv, const T* __restrict__ sw,
+    const T* __restrict__ pp, T* __restrict__ du, T* __restrict__ dv, T* __restrict__ dw,
+    T* __restrict__ u1, T* __restrict__ v1, T* __restrict__ w1, RkParam<T> q0,
+    const double* __restrict__ force, int forced_mask, int kchunk, int ntx, int nty, int acc,
     const double* __restrict__ dzflzi, double* __restrict__ partial) {
   constexpr int TX = kRkTx, NT = TX * TY;
   constexpr int RX = TX + 2, RY = TY + 2, RPL = RX * RY;  // u1 region: tile + 1
@@ -659,8 +617,9 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   constexpr int NPF = (UPL + NT - 1) / NT;
   constexpr int NRING = RPL - NT;  // region cells outside the tile
   static_assert(NRING == 2 * RX + 2 * TY && NRING <= NT, "one ring cell per thread");
-  __shared__ float ssrc[3][3][UPL];  // [field][slot][cell]; cell (cx, cy) = (i0-1+cx, j0-1+cy)
-  __shared__ float su1[3][3][RPL];   // [field][plane % 3][cell]; cell (rx, ry) = (i0+rx, j0+ry)
+  __shared__ T ssrc[3][2][UPL];  // [field][plane & 1][cell]; cell (cx, cy) = (i0-1+cx, j0-1+cy)
+  __shared__ ZCarry<T> szb[NRING];  // the ring cells' carry: few threads have one
+  __shared__ T su1[3][2][RPL];   // [field][plane & 1][cell]; cell (rx, ry) = (i0+rx, j0+ry)
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
   const int ti = (int)(b % (unsigned)ntx), tj = (int)((b / (unsigned)ntx) % (unsigned)nty);
   const int kc = (int)(b / (unsigned)(ntx * nty));
@@ -670,61 +629,59 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   const int i = i0 + tx + 1, j = j0 + ty + 1;
   const bool active = i <= g.nx && j <= g.ny;
   const bool fu = forced_mask & 1, fv = forced_mask & 2, fw = forced_mask & 4;
-  const float f_u = fu ? (float)force[0] : 0.f, f_v = fv ? (float)force[1] : 0.f,
-              f_w = fw ? (float)force[2] : 0.f;
+  const T f_u = fu ? (T)force[0] : T(0), f_v = fv ? (T)force[1] : T(0),
+          f_w = fw ? (T)force[2] : T(0);
   if (k0 > k1) {
     if (acc && t == 0) partial[b] = 0.0;
     return;
   }
   auto wrap = [](int x, int n) { return ((x - 1) % n + n) % n + 1; };
-  int gaddr[NPF];  // plane-relative address of the periodic image (-1: past the tile)
+  int gaddr[NPF], gnorth[NPF];  // plane-relative address of the periodic image (-1: past the tile), its j+1
 #pragma unroll
   for (int n = 0; n < NPF; ++n) {
     const int e = t + n * NT;
-    gaddr[n] = e < UPL ? wrap(i0 - 1 + e % UX, g.nx) + (int)g.sx * wrap(j0 - 1 + e / UX, g.ny) : -1;
+    const int y = wrap(j0 - 1 + e / UX, g.ny);
+    gaddr[n] = e < UPL ? wrap(i0 - 1 + e % UX, g.nx) + (int)g.sx * y : -1;
+    gnorth[n] = gaddr[n] + (int)g.sx * (y == g.ny ? 1 - g.ny : 1);
   }
-  // Source plane kk with the rules of k_rk's folded, projected stage-1 loads.
-  // The fetch only issues the loads (w on every plane, from plane 1 or nz for
-  // the ghost planes); the projection, forcing and boundary rules apply at the
-  // commit, after stage 2 of the plane below has been computed, and stage 2's
-  // results are stored after the commit: arithmetic on the loaded values in the
-  // fetch, or stores ahead of the commit, would make a wave wait there.
-  float ru[NPF], rv[NPF], rw[NPF], rp0[NPF], rpe[NPF], rpn[NPF], rpt[NPF];
+  T ru[NPF], rv[NPF], rw[NPF], rp0[NPF], rpe[NPF], rpn[NPF], rpt[NPF];
   auto fetch = [&](int kk) {
     const bool ghost = kk == 0 || kk == g.nz + 1;
     const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
+    const long o = g.sxy * ks;
 #pragma unroll
     for (int n = 0; n < NPF; ++n)
       if (gaddr[n] >= 0) {
-        const long a = gaddr[n] + g.sxy * ks;
+        const long a = gaddr[n] + o;
         ru[n] = su[a];
         rv[n] = sv[a];
         rw[n] = sw[a];
         rp0[n] = pp[a];
         rpe[n] = pp[a + 1];
-        rpn[n] = pp[a + g.sx];
+        rpn[n] = pp[gnorth[n] + o];
         rpt[n] = pp[a + g.sxy];
       }
   };
-  auto commit = [&](int kk, int slot) {
+  auto commit = [&](int kk) {
     const bool ghost = kk == 0 || kk == g.nz + 1;
-    const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
+    const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk, slot = kk & 1;
     const bool wzero = kk == 0 || kk >= g.nz;
-    const float dzci = dzc_inv[ks];
+    const T dzci = uniform_load(q0.m.dzc_inv, ks);
 #pragma unroll
     for (int n = 0; n < NPF; ++n)
       if (gaddr[n] >= 0) {
-        const float p0 = rp0[n];
-        float qu = ru[n] - (rpe[n] - p0) * dtdxi;
-        float qv = rv[n] - (rpn[n] - p0) * dtdyi;
-        float qw = rw[n] - (rpt[n] - p0) * dt * dzci;
+        const T p0 = rp0[n];
+        T qu = ru[n] - (rpe[n] - p0) * q0.dtdxi;
+        T qv = rv[n] - (rpn[n] - p0) * q0.dtdyi;
+        // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
+        T qw = rw[n] - (rpt[n] - p0) * q0.dt * dzci;
         if (fu) qu = qu + f_u;
         if (fv) qv = qv + f_v;
         if (fw) qw = qw + f_w;
-        if (wzero) qw = 0.f;
+        if (wzero) qw = T(0);
         if (ghost) {
-          qu = 2.f * bc_u - qu;  // src/mod_updateBound.cc:92,123
-          qv = 2.f * 0.f - qv;
+          qu = T(2) * q0.bc_u - qu;  // src/mod_updateBound.cc:92,123
+          qv = T(2) * T(0) - qv;
         }
         const int e = t + n * NT;
         ssrc[0][slot][e] = qu;
@@ -750,81 +707,71 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   }
   const bool has_b = t < NRING;
   const int rb = by * RX + bx;
-  int sm = 0, s0 = 1, sp = 2;  // source slots of planes q-1, q, q+1
+  const int ca = (ty + 2) * UX + tx + 2, cb = (by + 1) * UX + bx + 1;  // in the source ring
   const int qs = max(k0 - 1, 1), qe = k1 + 1;  // u1 planes formed: stage 1 up to nz, rules at nz+1
-  fetch(qs - 1);
-  commit(qs - 1, 0);
-  fetch(qs);
-  commit(qs, 1);
-  fetch(qs + 1);
-  commit(qs + 1, 2);
-  __syncthreads();
-  ZConv za{}, zb{}, z2{};  // carried lower-face products: stage 1 at A and B, stage 2
-  // stage 1 of region cell (rx, ry) on plane q, w1 = 0 on the wall plane nz.
-  // The carry restarts where k_rk's stage 1 restarts it (the first plane of
-  // each chunk of kchunk planes), and plane k0-1 continues the chain of the
-  // chunk below, so u1 is bit-identical to k_rk's.
-  auto stage1 = [&](int q, int rx, int ry, ZConv& z, float& o1, float& o2, float& o3) {
-    const int c = (ry + 1) * UX + rx + 1;
-    const PlaneAcc<float, UX> U{ssrc[0][sm], ssrc[0][s0], ssrc[0][sp], c};
-    const PlaneAcc<float, UX> V{ssrc[1][sm], ssrc[1][s0], ssrc[1][sp], c};
-    const PlaneAcc<float, UX> W{ssrc[2][sm], ssrc[2][s0], ssrc[2][sp], c};
-    const RkCoef cq = coef1[q];
-    if ((q - 1) % kchunk == 0) {
-      z = zconv_lower(U, V, W, cq);
-    } else if (q == qs) {
-      const PlaneAcc<float, UX> Ub{ssrc[0][sm], ssrc[0][sm], ssrc[0][s0], c};
-      const PlaneAcc<float, UX> Vb{ssrc[1][sm], ssrc[1][sm], ssrc[1][s0], c};
-      const PlaneAcc<float, UX> Wb{ssrc[2][sm], ssrc[2][sm], ssrc[2][s0], c};
-      z = zconv_upper(Ub, Vb, Wb, coef1[q - 1]);
-    }
-    float iu, iv, iw;
-    if (crf)
-      tendency_fast<true, true>(U, V, W, cq, cu1, iu, iv, iw, &z);
-    else
-      tendency_fast<false, true>(U, V, W, cq, cu1, iu, iv, iw, &z);
-    o1 = U(0, 0, 0) + iu;
-    o2 = V(0, 0, 0) + iv;
-    o3 = q >= g.nz ? 0.f : W(0, 0, 0) + iw;
+  auto src = [&](int f, int q, int c) {
+    return PlaneAcc<T, UX>{ssrc[f][(q + 1) & 1], ssrc[f][q & 1], ssrc[f][(q + 1) & 1], c};
   };
+  auto reg = [&](int f, int q, int c) {
+    return PlaneAcc<T, RX>{su1[f][(q + 1) & 1], su1[f][q & 1], su1[f][(q + 1) & 1], c};
+  };
+  fetch(qs - 1);
+  commit(qs - 1);
+  fetch(qs);
+  commit(qs);
+  fetch(qs + 1);
+  __syncthreads();
+  // the carries of the first plane, while plane qs-1 is in the slot of qs+1
+  ZCarry<T> za{}, z2{};
+  za = carry_start<T, 1>(src(0, qs, ca), src(1, qs, ca), src(2, qs, ca), q0, qs);
+  if (has_b) szb[t] = carry_start<T, 1>(src(0, qs, cb), src(1, qs, cb), src(2, qs, cb), q0, qs);
+  __syncthreads();
+  commit(qs + 1);
+  __syncthreads();
   // u1 of plane q at region cell r; with q == 1 also plane 0 by the rules
-  auto put1 = [&](int q, int r, float o1, float o2, float o3) {
-    const int s = q % 3;
+  auto put1 = [&](int q, int r, T o1, T o2, T o3) {
+    const int s = q & 1;
     su1[0][s][r] = o1;
     su1[1][s][r] = o2;
     su1[2][s][r] = o3;
     if (q == 1) {
-      su1[0][0][r] = 2.f * bc_u - o1;
-      su1[1][0][r] = 2.f * 0.f - o2;
-      su1[2][0][r] = 0.f;
+      su1[0][0][r] = T(2) * q0.bc_u - o1;
+      su1[1][0][r] = T(2) * T(0) - o2;
+      su1[2][0][r] = T(0);
     }
   };
   // plane nz+1 of u1 by the rules from plane nz (the same thread wrote cell r of it)
   auto ghost_top = [&](int r) {
-    const int s = g.nz % 3, d = (g.nz + 1) % 3;
-    su1[0][d][r] = 2.f * bc_u - su1[0][s][r];
-    su1[1][d][r] = 2.f * 0.f - su1[1][s][r];
-    su1[2][d][r] = 0.f;
+    const int s = g.nz & 1, d = s ^ 1;
+    su1[0][d][r] = T(2) * q0.bc_u - su1[0][s][r];
+    su1[1][d][r] = T(2) * T(0) - su1[1][s][r];
+    su1[2][d][r] = T(0);
   };
-  const int cp = (ty + 2) * UX + tx + 2;  // the tile point in the source ring
   double msum = 0.0;
   for (int q = qs; q <= qe; ++q) {
-    // the next iteration's stage 1 reads source planes q .. q+2
+    // the next iteration's stage 1 reads source planes q+1, q+2
     const bool more = q + 1 <= qe && q + 1 <= g.nz;
     const int k = q - 1;  // stage-2 plane
     const bool s2 = k >= k0;
-    float pu = 0.f, pv = 0.f, pw = 0.f;
-    if (s2) {
-      pu = ssrc[0][sm][cp];
-      pv = ssrc[1][sm][cp];
-      pw = ssrc[2][sm][cp];
-    }
+    const T pu = za.u, pv = za.v, pw = za.w;  // the source at the tile point of plane k
     if (q <= g.nz) {
-      float o1, o2, o3;
-      stage1(q, tx + 1, ty + 1, za, o1, o2, o3);
+      T o1, o2, o3;
+      stage_update<T, 1, CRF, UX>(src(0, q, ca), src(1, q, ca), src(2, q, ca), q0, q, T(0), T(0), T(0),
+                             za, o1, o2, o3);
+      if (q == g.nz) o3 = T(0);
       put1(q, ra, o1, o2, o3);
+      if (U1OUT && active && q >= k0 && q <= k1) {
+        const long a = g.idx(i, j, q);
+        u1[a] = o1;
+        v1[a] = o2;
+        w1[a] = o3;
+      }
       if (has_b) {
-        stage1(q, bx, by, zb, o1, o2, o3);
+        ZCarry<T> zb = szb[t];
+        stage_update<T, 1, CRF, UX>(src(0, q, cb), src(1, q, cb), src(2, q, cb), q0, q, T(0), T(0),
+                                    T(0), zb, o1, o2, o3);
+        szb[t] = zb;
+        if (q == g.nz) o3 = T(0);
         put1(q, rb, o1, o2, o3);
       }
     } else {
@@ -835,24 +782,15 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
     // fetched here rather than before stage 1: its registers are then not
     // live across both stages
     if (more) fetch(q + 2);
-    float nu = 0.f, nv = 0.f, nw = 0.f;
+    T nu = T(0), nv = T(0), nw = T(0);
     if (s2 && active) {
-      const PlaneAcc<float, RX> U{su1[0][(k + 2) % 3], su1[0][k % 3], su1[0][(k + 1) % 3], ra};
-      const PlaneAcc<float, RX> V{su1[1][(k + 2) % 3], su1[1][k % 3], su1[1][(k + 1) % 3], ra};
-      const PlaneAcc<float, RX> W{su1[2][(k + 2) % 3], su1[2][k % 3], su1[2][(k + 1) % 3], ra};
-      const RkCoef cq = coef2[k];
-      if (k == k0) z2 = zconv_lower(U, V, W, cq);
-      float iu, iv, iw;
-      if (crf)
-        tendency_fast<true, true>(U, V, W, cq, cu2, iu, iv, iw, &z2);
-      else
-        tendency_fast<false, true>(U, V, W, cq, cu2, iu, iv, iw, &z2);
-      nu = (U(0, 0, 0) + pu) * 0.5f + iu;
-      nv = (V(0, 0, 0) + pv) * 0.5f + iv;
-      nw = (W(0, 0, 0) + pw) * 0.5f + iw;
-      if (acc) msum += (double)nu * dzflzi[k];
+      stage_update<T, 2, CRF, RX>(reg(0, k, ra), reg(1, k, ra), reg(2, k, ra), q0, k, pu, pv, pw, z2,
+                             nu, nv, nw);
+      if (acc) msum += (double)nu * uniform_load(dzflzi, k);
+    } else if (q == k0 && active) {
+      z2 = carry_start<T, 2>(reg(0, k0, ra), reg(1, k0, ra), reg(2, k0, ra), q0, k0);
     }
-    if (more) commit(q + 2, sm);  // source plane q+2 replaces q-1
+    if (more) commit(q + 2);
     if (s2 && active) {
       const long a = g.idx(i, j, k);
       du[a] = nu;
@@ -860,299 +798,9 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
       dw[a] = nw;
     }
     __syncthreads();
-    const int tmp = sm;
-    sm = s0;
-    s0 = sp;
-    sp = tmp;
   }
-  if (acc) {
-    // the block size is folded onto its largest power of two first
-    double* red = reinterpret_cast<double*>(&ssrc[0][0][0]);
-    static_assert(sizeof(ssrc) >= NT * sizeof(double), "reduction scratch");
-    constexpr int P2 = NT >= 1024 ? 1024 : (NT >= 512 ? 512 : 256);
-    static_assert(NT >= P2 && NT < 2 * P2, "block size");
-    red[t] = msum;
-    __syncthreads();
-    if (t < NT - P2) red[t] += red[t + P2];
-    __syncthreads();
-    for (int h = P2 / 2; h > 0; h >>= 1) {
-      if (t < h) red[t] += red[t + h];
-      __syncthreads();
-    }
-    if (t == 0) partial[b] = red[0];
-  }
-}
-
-// RK stage 2 fused with calcRHS (src/mod_calcVel.cc:140-242 then
-// src/mod_calcRHS.cc:27-29) for the step sequence.  Besides its 64x8 interior
-// the block evaluates u_new on the column i0 and v_new on the row j0 (the
-// backward neighbours calcRHS needs); at the domain edge these are computed
-// from periodic images of the stencil and equal the boundary copy bit for bit.
-// w_new(k-1) is carried in a register (a chunk first recomputes it for its
-// plane k0-1; below the wall it is the boundary value 0).  Loads rebuild the
-// u1 halos from interior cells (so the boundary update of u1 is not needed),
-// w_new on plane nz is the wall value 0 (the middle boundary update's only
-// effect on the interior), and the deferred force of the previous step is
-// added to the point values of u.  The new state goes to separate buffers
-// (nu, nv, nw): the backward neighbours read old values of cells that other
-// blocks update, so the update cannot be in place.
-//
-// With PROJ the previous step's projection is deferred into this kernel as
-// well: the stored u, v, w are the predictor u* and every point value read is
-// u* - dt*grad(p) (src/mod_calcVel.cc:272-274, k_correct's association) before
-// the force applies; p (pin, valid halos) is the previous pressure, held in a
-// fourth field of the LDS ring, and the right-hand side goes to a separate
-// buffer (pout).  With `acc` the block sums
-// its new u times dzflzi(k) in FP64 into partial[block]: the bulk mean of the
-// next projected velocity (the projection changes every x-row's sum only by
-// p(nx+1) - p(1) = 0).
-template <typename T, int TY, bool PROJ>
-__global__ __launch_bounds__(kRkTx* TY) void k_rk2_rhs(
-    Geom g, const T* __restrict__ su, const T* __restrict__ sv, const T* __restrict__ sw,
-    const T* __restrict__ du, const T* __restrict__ dv, const T* __restrict__ dw,
-    T* __restrict__ nu_out, T* __restrict__ nv_out, T* __restrict__ nw_out,
-    const T* __restrict__ pin, T* __restrict__ pout, MeshT<T> m, T dxi, T dyi, T rei, T dt,
-    T ucrf, int kchunk, int ntx, int nty, int defer, T bc_u, const double* __restrict__ force,
-    int forced_mask, const RkCoef* __restrict__ coef, RkUniform cu, int crf, T dti, T dtidxi,
-    T dtidyi, T pdx, T pdy, int acc, const double* __restrict__ dzflzi,
-    double* __restrict__ partial) {
-  constexpr int TX = kRkTx, SX = TX + 3, SY = TY + 3, PL = SX * SY, NT = TX * TY;
-  constexpr int NPF = (PL + NT - 1) / NT;
-  constexpr int NF = PROJ ? 4 : 3;
-  __shared__ T sh[NF][3][PL];  // u1, v1, w1 (and p) ring; cell (cx, cy) = (i0-1+cx, j0-1+cy)
-  __shared__ T un[TY][TX + 1];          // u_new at i = i0 .. i0+TX of the tile rows
-  __shared__ T vn[TY + 1][TX];          // v_new at j = j0 .. j0+TY of the tile columns
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const int ti = (int)(b % (unsigned)ntx), tj = (int)((b / (unsigned)ntx) % (unsigned)nty);
-  const int kc = (int)(b / (unsigned)(ntx * nty));
-  const int i0 = ti * TX, j0 = tj * TY;
-  const int k0 = kc * kchunk + 1, k1 = min(k0 + kchunk - 1, g.nz);
-  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-  const int i = i0 + tx + 1, j = j0 + ty + 1;
-  const bool active = i <= g.nx && j <= g.ny;
-  const bool fu = defer && (forced_mask & 1), fv = defer && (forced_mask & 2),
-             fw = defer && (forced_mask & 4);
-  const T f_u = fu ? (T)force[0] : T(0), f_v = fv ? (T)force[1] : T(0),
-          f_w = fw ? (T)force[2] : T(0);
-  auto wrapx = [&](int x) { return x < 1 ? x + g.nx : (x > g.nx ? x - g.nx : x); };
-  auto wrapy = [&](int y) { return y < 1 ? y + g.ny : (y > g.ny ? y - g.ny : y); };
-
-  long gaddr[NPF];
-  int cell[NPF];
-#pragma unroll
-  for (int n = 0; n < NPF; ++n) {
-    const int e = threadIdx.x + n * NT;
-    const int gx = i0 - 1 + e % SX, gy = j0 - 1 + e / SX;
-    cell[n] = e;
-    const bool inside = e < PL && gx <= g.nx + 1 && gy <= g.ny + 1;
-    gaddr[n] = inside ? wrapx(gx) + g.sx * wrapy(gy) : -1;
-  }
-  T pre[NF][NPF];
-  // u1, v1, w1 of plane kk with the boundary rules applied, and p of plane kk as
-  // stored (updateBoundP ran; x/y halo cells read their periodic image, which
-  // holds the same value).  The fetch only issues the loads (w on every plane,
-  // from plane 1 or nz for the ghost planes); the boundary rules apply at the
-  // commit, after the plane below has been computed: arithmetic on the loaded
-  // values inside the fetch would make every wave wait for its loads there.
-  auto fetch = [&](int kk) {
-    const bool ghost = kk == 0 || kk == g.nz + 1;
-    const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
-#pragma unroll
-    for (int n = 0; n < NPF; ++n)
-      if (gaddr[n] >= 0) {
-        const long a = gaddr[n] + g.sxy * ks;
-        pre[0][n] = su[a];
-        pre[1][n] = sv[a];
-        pre[2][n] = sw[a];
-        if constexpr (PROJ) pre[NF - 1][n] = pin[gaddr[n] + g.sxy * kk];
-      }
-  };
-  auto commit = [&](int kk, int slot) {
-    const bool ghost = kk == 0 || kk == g.nz + 1;
-    const bool wzero = kk == 0 || kk >= g.nz;
-#pragma unroll
-    for (int n = 0; n < NPF; ++n)
-      if (gaddr[n] >= 0) {
-        T qu = pre[0][n], qv = pre[1][n], qw = pre[2][n];
-        if (wzero) qw = T(0);
-        if (ghost) {
-          qu = T(2) * bc_u - qu;  // src/mod_updateBound.cc:92,123
-          qv = T(2) * T(0) - qv;
-        }
-        sh[0][slot][cell[n]] = qu;
-        sh[1][slot][cell[n]] = qv;
-        sh[2][slot][cell[n]] = qw;
-        if constexpr (PROJ) sh[NF - 1][slot][cell[n]] = pre[NF - 1][n];
-      }
-  };
-  // the projection's pressure differences at tile cell c of ring slots s0
-  // (plane k) and sp (plane k+1)
-  auto dpx = [&](int s0, int c) { return sh[NF - 1][s0][c + 1] - sh[NF - 1][s0][c]; };
-  auto dpy = [&](int s0, int c) { return sh[NF - 1][s0][c + SX] - sh[NF - 1][s0][c]; };
-  auto dpz = [&](int s0, int sp, int c) { return sh[NF - 1][sp][c] - sh[NF - 1][s0][c]; };
-  // old u at tile cell (1, cy), old v at (cx, 1) of plane kk (slot s0), with
-  // the deferred projection and force; x/y halo cells wrap
-  auto old_u = [&](int s0, int cy, int x, int y, int kk) {
-    T q = du[g.idx(wrapx(x), wrapy(y), kk)];
-    if constexpr (PROJ) q = q - dpx(s0, cy * SX + 1) * pdx;
-    return fu ? q + f_u : q;
-  };
-  auto old_v = [&](int s0, int cx, int x, int y, int kk) {
-    T q = dv[g.idx(wrapx(x), wrapy(y), kk)];
-    if constexpr (PROJ) q = q - dpy(s0, SX + cx) * pdy;
-    return fv ? q + f_v : q;
-  };
-  // the three stage-2 updates at tile cell (cx, cy) of plane kk.  FP64: zf
-  // receives the upper z-face terms; with `carry` it also supplies the lower
-  // ones (the thread's own column, marching up)
-  auto update = [&](int sm, int s0, int sp, int cx, int cy, int kk, T& nu, T& nv, T& nw,
-                    T ou, T ov, T ow, ZFace<T>& zf, bool carry) {
-    const int c = cy * SX + cx;
-    const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
-    const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
-    const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
-    if constexpr (std::is_same<T, double>::value) {
-      T tu, tv, tw;
-      if (!carry)
-        tendency_z<T, true, false>(U, V, W, m, kk, dxi, dyi, rei, ucrf, tu, tv, tw, zf);
-      else if (crf)
-        tendency_z<T, true, true>(U, V, W, m, kk, dxi, dyi, rei, ucrf, tu, tv, tw, zf);
-      else
-        tendency_z<T, false, true>(U, V, W, m, kk, dxi, dyi, rei, ucrf, tu, tv, tw, zf);
-      nu = (U(0, 0, 0) + dt * tu + ou) * T(0.5);
-      nv = (V(0, 0, 0) + dt * tv + ov) * T(0.5);
-      nw = (W(0, 0, 0) + dt * tw + ow) * T(0.5);
-    } else {
-      const RkCoef q = coef[kk];
-      float iu, iv, iw;
-      if (crf)
-        tendency_fast<true>(U, V, W, q, cu, iu, iv, iw);
-      else
-        tendency_fast<false>(U, V, W, q, cu, iu, iv, iw);
-      nu = (U(0, 0, 0) + ou) * 0.5f + iu;
-      nv = (V(0, 0, 0) + ov) * 0.5f + iv;
-      nw = (W(0, 0, 0) + ow) * 0.5f + iw;
-    }
-  };
-  if (k0 > k1) {
-    if (acc && threadIdx.x == 0) partial[b] = 0.0;
-    return;
-  }
-  const int cxi = tx + 2, cyi = ty + 2;  // tile cell of the thread's interior point
-  double msum = 0.0;  // FP64 partial of the bulk mean (acc)
-  ZFace<T> zf{}, zx{};  // the column's carried z-face terms; scratch of the extra cells
-  int sm = 0, s0 = 1, sp = 2;
-  T wprev = T(0);  // w_new(i, j, k-1); 0 below the wall (w(0) = 0)
-  if (k0 > 1) {
-    // recompute w_new on plane k0-1 from u1 planes k0-2, k0-1, k0
-    fetch(k0 - 2);
-    commit(k0 - 2, 0);
-    fetch(k0 - 1);
-    commit(k0 - 1, 1);
-    fetch(k0);
-    commit(k0, 2);
-    __syncthreads();
-    if (active) {
-      T nu, nv, nw;
-      T ow = dw[g.idx(i, j, k0 - 1)];
-      // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
-      if constexpr (PROJ) ow = ow - dpz(1, 2, cyi * SX + cxi) * dt * m.dzc_inv[k0 - 1];
-      if (fw) ow = (k0 - 1 == g.nz) ? T(0) : ow + f_w;
-      update(0, 1, 2, cxi, cyi, k0 - 1, nu, nv, nw, T(0), T(0), ow, zf, false);
-      wprev = (k0 - 1 == g.nz) ? T(0) : nw;
-    }
-    __syncthreads();
-    fetch(k0 + 1);
-    commit(k0 + 1, 0);  // slot 0 held plane k0-2
-    __syncthreads();
-    sm = 1;
-    s0 = 2;
-    sp = 0;
-  } else {
-    fetch(k0 - 1);
-    commit(k0 - 1, 0);
-    fetch(k0);
-    commit(k0, 1);
-    fetch(k0 + 1);
-    commit(k0 + 1, 2);
-    __syncthreads();
-    if (active) {
-      const int c = cyi * SX + cxi;
-      const PlaneAcc<T, SX> U{sh[0][0], sh[0][1], sh[0][2], c};
-      const PlaneAcc<T, SX> V{sh[1][0], sh[1][1], sh[1][2], c};
-      const PlaneAcc<T, SX> W{sh[2][0], sh[2][1], sh[2][2], c};
-      zf = zface_lower<T>(U, V, W, m, k0);
-    }
-  }
-  for (int k = k0; k <= k1; ++k) {
-    const bool more = k + 2 <= k1 + 1;
-    if (more) fetch(k + 2);
-    T nw = T(0);
-    if (active) {
-      const long a = g.idx(i, j, k);
-      T ou = du[a], ov = dv[a], ow = dw[a];
-      if constexpr (PROJ) {
-        // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
-        const int c = cyi * SX + cxi;
-        ou = ou - dpx(s0, c) * pdx;
-        ov = ov - dpy(s0, c) * pdy;
-        ow = ow - dpz(s0, sp, c) * dt * m.dzc_inv[k];
-      }
-      if (fu) ou = ou + f_u;
-      if (fv) ov = ov + f_v;
-      if (fw) ow = (k == g.nz) ? T(0) : ow + f_w;
-      T nu, nv;
-      update(sm, s0, sp, cxi, cyi, k, nu, nv, nw, ou, ov, ow, zf, true);
-      if (k == g.nz) nw = T(0);  // src/mod_updateBound.cc:137 (w(nz) = 0)
-      un[ty][tx + 1] = nu;
-      vn[ty + 1][tx] = nv;
-      if (acc) msum += (double)nu * dzflzi[k];
-      nu_out[a] = nu;
-      nv_out[a] = nv;
-      nw_out[a] = nw;
-    }
-    // backward neighbours: v_new on row j0 (wave 0), u_new on column i0 (wave 1)
-    if (ty == 0 && i <= g.nx) {
-      T nu, nv, nw2;
-      update(sm, s0, sp, cxi, 1, k, nu, nv, nw2, T(0), old_v(s0, cxi, i, j0, k), T(0), zx, false);
-      vn[0][tx] = nv;
-    } else if (ty == 1 && tx < TY && j0 + tx + 1 <= g.ny) {
-      T nu, nv, nw2;
-      update(sm, s0, sp, 1, tx + 2, k, nu, nv, nw2, old_u(s0, tx + 2, i0, j0 + tx + 1, k), T(0),
-             T(0), zx, false);
-      un[tx][0] = nu;
-    }
-    __syncthreads();
-    if (active) {
-      // calcRHS, src/mod_calcRHS.cc:27-29
-      pout[g.idx(i, j, k)] = (un[ty][tx + 1] - un[ty][tx]) * dtidxi +
-                             (vn[ty + 1][tx] - vn[ty][tx]) * dtidyi + (nw - wprev) * dti * m.dzf_inv[k];
-      wprev = nw;
-    }
-    if (more) commit(k + 2, sm);
-    __syncthreads();
-    const int t = sm;
-    sm = s0;
-    s0 = sp;
-    sp = t;
-  }
-  if (acc) {
-    // the ring is free after the last barrier of the loop; the block size
-    // (64 x TY) is folded onto its largest power of two first
-    double* red = reinterpret_cast<double*>(&sh[0][0][0]);
-    static_assert(sizeof(sh) >= NT * sizeof(double), "reduction scratch");
-    constexpr int P2 = NT >= 1024 ? 1024 : (NT >= 512 ? 512 : 256);
-    static_assert(NT >= P2 && NT < 2 * P2, "block size");
-    red[threadIdx.x] = msum;
-    __syncthreads();
-    if ((int)threadIdx.x < NT - P2) red[threadIdx.x] += red[threadIdx.x + P2];
-    __syncthreads();
-    for (int h = P2 / 2; h > 0; h >>= 1) {
-      if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[b] = red[0];
-  }
+  static_assert(sizeof(ssrc) >= NT * sizeof(double), "reduction scratch");
+  if (acc) block_partial<NT>(reinterpret_cast<double*>(&ssrc[0][0][0]), msum, partial, b);
 }
 
 // calcRHS, src/mod_calcRHS.cc:27-29.  w(k-1) is carried from the previous plane.
@@ -1208,7 +856,7 @@ __global__ __launch_bounds__(kRkTx* correct_ty<T>()) void k_correct(Geom g, cons
       u[c] = un;
       v[c] -= (p[c + g.sx] - p0) * dtdyi;
       w[c] -= (pt - p0) * dt * dzc_inv[k];
-      if (ACC) acc += (double)un * dzflzi[k];
+      if (ACC) acc += (double)un * uniform_load(dzflzi, k);
       p0 = pt;
     }
   }
@@ -1608,199 +1256,138 @@ inline int forced_mask(const pll_context* c) {
   return (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0) | (c->is_forced[2] ? 4 : 0);
 }
 
-// Per-plane coefficients of the FP32-mixed operator for stage `stage`
-// (S = dt or dt/2), computed in FP64 and rounded once.
-RkUniform rk_uniform(const pll_context* c, int stage) {
+// Coefficients of tendency_fast for stage `stage` (S = dt or dt/2), computed in
+// FP64 and rounded once.
+template <typename T>
+RkUniform<T> rk_uniform(const pll_context* c, int stage) {
   const double S = stage == 1 ? c->dt : 0.5 * c->dt;
-  return RkUniform{(float)(S * 0.25 * c->dx_inv), (float)(S * 0.25 * c->dy_inv),
-                   (float)(S * c->re_inv * c->dx_inv * c->dx_inv),
-                   (float)(S * c->re_inv * c->dy_inv * c->dy_inv),
-                   (float)(S * 0.5 * c->u_crf * c->dx_inv)};
+  return RkUniform<T>{(T)(S * 0.25 * c->dx_inv), (T)(S * 0.25 * c->dy_inv),
+                      (T)(S * c->re_inv * c->dx_inv * c->dx_inv),
+                      (T)(S * c->re_inv * c->dy_inv * c->dy_inv),
+                      (T)(S * 0.5 * c->u_crf * c->dx_inv)};
 }
 
+template <typename T>
 int rk_coef_setup(pll_context* c) {
   const int nz = c->g.nz;
-  std::vector<RkCoef> h(2 * (size_t)(nz + 2));
+  std::vector<RkCoef<T>> h(2 * (size_t)(nz + 2));
   for (int stage = 1; stage <= 2; ++stage) {
     const double S = stage == 1 ? c->dt : 0.5 * c->dt, rei = c->re_inv;
     for (int k = 1; k <= nz; ++k) {
       const double* f = c->dzf.data();
       const double* fi = c->dzf_inv.data();
       const double* ci = c->dzc_inv.data();
-      RkCoef& q = h[(stage - 1) * (size_t)(nz + 2) + k];
-      q.a1 = (float)(f[k + 1] * ci[k]);
-      q.a2 = (float)(f[k] * ci[k]);
-      q.b1 = (float)(f[k - 1] * ci[k - 1]);
-      q.b2 = (float)(f[k] * ci[k - 1]);
-      q.zuv = (float)(S * 0.25 * fi[k]);
-      q.cp = (float)(S * rei * ci[k] * fi[k]);
-      q.cm = (float)(S * rei * ci[k - 1] * fi[k]);
-      q.zw = (float)(S * 0.25 * ci[k]);
-      q.dp = (float)(S * rei * fi[k + 1] * ci[k]);
-      q.dm = (float)(S * rei * fi[k] * ci[k]);
-      // the diagonal from the rounded FP32 coefficients (one rounding off their sum)
-      const RkUniform cu = rk_uniform(c, stage);
+      RkCoef<T>& q = h[(stage - 1) * (size_t)(nz + 2) + k];
+      q.a1 = (T)(f[k + 1] * ci[k]);
+      q.a2 = (T)(f[k] * ci[k]);
+      q.b1 = (T)(f[k - 1] * ci[k - 1]);
+      q.b2 = (T)(f[k] * ci[k - 1]);
+      q.zuv = (T)(S * 0.25 * fi[k]);
+      q.cp = (T)(S * rei * ci[k] * fi[k]);
+      q.cm = (T)(S * rei * ci[k - 1] * fi[k]);
+      q.zw = (T)(S * 0.25 * ci[k]);
+      q.dp = (T)(S * rei * fi[k + 1] * ci[k]);
+      q.dm = (T)(S * rei * fi[k] * ci[k]);
+      // the diagonal from the rounded coefficients (one rounding off their sum)
+      const RkUniform<T> cu = rk_uniform<T>(c, stage);
       const double vxy = 2.0 * (double)cu.vx + 2.0 * (double)cu.vy;
-      q.cdu = (float)(vxy + (double)q.cp + (double)q.cm);
-      q.cdw = (float)(vxy + (double)q.dp + (double)q.dm);
+      q.cdu = (T)(vxy + (double)q.cp + (double)q.cm);
+      q.cdw = (T)(vxy + (double)q.dp + (double)q.dm);
     }
   }
-  PLL_HIP_TRY(ctx_malloc(c, &c->d_rkcoef, h.size() * sizeof(RkCoef)));
-  PLL_HIP_TRY(hipMemcpy(c->d_rkcoef, h.data(), h.size() * sizeof(RkCoef), hipMemcpyHostToDevice));
+  PLL_HIP_TRY(ctx_malloc(c, &c->d_rkcoef, h.size() * sizeof(RkCoef<T>)));
+  PLL_HIP_TRY(hipMemcpy(c->d_rkcoef, h.data(), h.size() * sizeof(RkCoef<T>), hipMemcpyHostToDevice));
   return PLL_OK;
 }
 
 template <typename T>
-int rk_t(pll_context* c, int stage, int fold, int corr, int acc, int bcload) {
-  const int ty = std::is_same<T, double>::value ? kLateTy : kRkTy;
-  const TileGrid t = tile_grid(c, ty);
-  if (acc && (long)t.blocks() > c->npartial)
-    return fail(PLL_ERR_STATE, "reduction scratch smaller than the stencil grid");
-  // the projected loads read p at the periodic image of halo cells, which only
-  // the folded (image-addressed) loads provide
-  if (corr && !fold) return fail(PLL_ERR_STATE, "deferred projection needs folded loads");
-  const double* dzflzi = c->d_mesh64 + 3 * (c->g.nz + 2);
-  const T dtdxi = (T)(c->dt * c->dx_inv), dtdyi = (T)(c->dt * c->dy_inv);  // src/mod_calcVel.cc:256-258
-  const MeshT<T> m = mesh_of<T>(c);
-  const T bc_u = (T)(0.0 - c->u_crf);  // src/mod_updateBound.cc:80
-  const double* force = c->d_scalar + 3;
-  const RkCoef* coef = static_cast<const RkCoef*>(c->d_rkcoef) + (stage - 1) * (c->g.nz + 2);
-  const RkUniform cu = rk_uniform(c, stage);
-  const int crf = c->u_crf != 0.0;
-  // FP64 runs the late-commit form of the stages (k_rk_late), FP32 k_rk
+RkParam<T> rk_param(const pll_context* c) {
+  const RkCoef<T>* coef = static_cast<const RkCoef<T>*>(c->d_rkcoef);
+  return RkParam<T>{mesh_of<T>(c), (T)c->dx_inv, (T)c->dy_inv, (T)c->re_inv, (T)c->dt, (T)c->u_crf,
+                    (T)(c->dt * c->dx_inv), (T)(c->dt * c->dy_inv),  // src/mod_calcVel.cc:256-258
+                    (T)(0.0 - c->u_crf),                             // src/mod_updateBound.cc:80
+                    coef, coef + (c->g.nz + 2), rk_uniform<T>(c, 1), rk_uniform<T>(c, 2)};
+}
+
+template <typename T>
+int rk_t(pll_context* c, int stage, int acc, int bcload) {
   constexpr bool kF64 = std::is_same<T, double>::value;
-  if (stage == 1) {
-    TimerScope ts(c, K_RK1);
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream, c->g,
-                         F<T>(c, PLL_U), F<T>(c, PLL_V), F<T>(c, PLL_W), F<T>(c, PLL_U1),
-                         F<T>(c, PLL_V1), F<T>(c, PLL_W1), m, (T)c->dx_inv, (T)c->dy_inv,
-                         (T)c->re_inv, (T)c->dt, (T)c->u_crf, t.kchunk, t.ntx, t.nty, fold, 0,
-                         bc_u, force, forced_mask(c), coef, cu, crf, F<T>(c, PLL_P), corr,
-                         dtdxi, dtdyi, 0, dzflzi, c->d_partial, fold);
-    };
-    // the deferred projection is compiled into its own variant of stage 1
-    if constexpr (kF64)
-      go(corr ? k_rk_late<1, true> : k_rk_late<1, false>);
-    else
-      go(corr ? k_rk<T, 1, true> : k_rk<T, 1>);
-  } else {
-    TimerScope ts(c, K_RK2);
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream, c->g,
-                         F<T>(c, PLL_U1), F<T>(c, PLL_V1), F<T>(c, PLL_W1), F<T>(c, PLL_U),
-                         F<T>(c, PLL_V), F<T>(c, PLL_W), m, (T)c->dx_inv, (T)c->dy_inv,
-                         (T)c->re_inv, (T)c->dt, (T)c->u_crf, t.kchunk, t.ntx, t.nty, 0, fold,
-                         bc_u, force, forced_mask(c), coef, cu, crf, F<T>(c, PLL_P), corr,
-                         dtdxi, dtdyi, acc, dzflzi, c->d_partial, bcload);
-    };
-    if constexpr (kF64)
-      go(k_rk_late<2, false>);
-    else
-      go(k_rk<T, 2>);
-  }
-  PLL_HIP_TRY(hipGetLastError());
-  if (acc) {
-    // forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297)
-    TimerScope ts(c, K_MEAN_FINAL);
-    hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kRedThreads), 0, c->stream, c->d_partial,
-                       (long)t.blocks(), (double)c->g.nx, (double)c->g.ny, c->d_scalar + 0,
-                       c->vel_force[0], c->d_scalar + 3);
-    PLL_HIP_TRY(hipGetLastError());
-  }
-  return PLL_OK;
-}
-
-// RK stage 2 + calcRHS into the spare velocity and pressure buffers, then
-// swap them in.  corr: the previous step's projection is applied on load;
-// acc: the bulk mean of the new u and the force of u go to d_scalar[0], [3].
-template <typename T>
-int rk2_rhs_t(pll_context* c, int defer, int corr, int acc) {
-  constexpr int kTall = std::is_same<T, double>::value ? kRhsTallTy : kRkTy;
-  const bool tall = (long)tile_grid(c, kTall).blocks() >= kRhsTallBlocks;
-  const int ty = tall ? kTall : kRkTy;
+  const int ty = kF64 ? kLateTy : kRkTy;
   const TileGrid t = tile_grid(c, ty);
   if (acc && (long)t.blocks() > c->npartial)
     return fail(PLL_ERR_STATE, "reduction scratch smaller than the stencil grid");
-  if (!c->fld_alt[3]) return fail(PLL_ERR_STATE, "no spare pressure buffer");
-  // the projection reads p at the periodic image of halo cells, which only the
-  // folded loads of stage 2 provide
-  if (corr && !defer) return fail(PLL_ERR_STATE, "deferred projection needs folded loads");
-  auto kernel = corr ? (tall ? k_rk2_rhs<T, kTall, true> : k_rk2_rhs<T, kRkTy, true>)
-                     : (tall ? k_rk2_rhs<T, kTall, false> : k_rk2_rhs<T, kRkTy, false>);
-  const MeshT<T> m = mesh_of<T>(c);
-  const T bc_u = (T)(0.0 - c->u_crf);  // src/mod_updateBound.cc:80
-  const RkCoef* coef = static_cast<const RkCoef*>(c->d_rkcoef) + (c->g.nz + 2);
-  const RkUniform cu = rk_uniform(c, 2);
-  const double dti = 1.0 / c->dt;  // src/mod_calcRHS.cc:11-13
-  const double dtidxi = dti * c->dx_inv;
-  const double dtidyi = dti * c->dy_inv;
-  const double pdx = c->dt * c->dx_inv, pdy = c->dt * c->dy_inv;  // src/mod_calcVel.cc:256-258
   const double* dzflzi = c->d_mesh64 + 3 * (c->g.nz + 2);
   {
-    TimerScope ts(c, K_RK2_RHS);
-    hipLaunchKernelGGL(kernel, dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream, c->g,
-                       F<T>(c, PLL_U1), F<T>(c, PLL_V1), F<T>(c, PLL_W1), F<T>(c, PLL_U),
-                       F<T>(c, PLL_V), F<T>(c, PLL_W), static_cast<T*>(c->fld_alt[0]),
-                       static_cast<T*>(c->fld_alt[1]), static_cast<T*>(c->fld_alt[2]),
-                       F<T>(c, PLL_P), static_cast<T*>(c->fld_alt[3]), m, (T)c->dx_inv,
-                       (T)c->dy_inv, (T)c->re_inv, (T)c->dt, (T)c->u_crf, t.kchunk, t.ntx, t.nty,
-                       defer, bc_u, c->d_scalar + 3, forced_mask(c), coef, cu,
-                       (int)(c->u_crf != 0.0), (T)dti, (T)dtidxi, (T)dtidyi, (T)pdx, (T)pdy, acc,
-                       dzflzi, c->d_partial);
+    TimerScope ts(c, stage == 1 ? K_RK1 : K_RK2);
+    auto go = [&](auto kernel, int src, int dst) {
+      hipLaunchKernelGGL(kernel, dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream, c->g,
+                         F<T>(c, src), F<T>(c, src + 1), F<T>(c, src + 2), F<T>(c, dst),
+                         F<T>(c, dst + 1), F<T>(c, dst + 2), rk_param<T>(c), t.kchunk, t.ntx,
+                         t.nty, acc, dzflzi, c->d_partial, bcload);
+    };
+    // FP64 runs the late-commit form of the stages (k_rk_late), FP32 k_rk
+    const bool crf = c->u_crf != 0.0;
+    if constexpr (kF64)
+      stage == 1 ? go(crf ? k_rk_late<1, true> : k_rk_late<1, false>, PLL_U, PLL_U1)
+                 : go(crf ? k_rk_late<2, true> : k_rk_late<2, false>, PLL_U1, PLL_U);
+    else
+      stage == 1 ? go(crf ? k_rk<T, 1, true> : k_rk<T, 1, false>, PLL_U, PLL_U1)
+                 : go(crf ? k_rk<T, 2, true> : k_rk<T, 2, false>, PLL_U1, PLL_U);
   }
   PLL_HIP_TRY(hipGetLastError());
-  for (int d = 0; d < 3; ++d) std::swap(c->fld[PLL_U + d], c->fld_alt[d]);
-  std::swap(c->fld[PLL_P], c->fld_alt[3]);
-  if (acc) {
-    // forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297)
-    TimerScope ts(c, K_MEAN_FINAL);
-    hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kRedThreads), 0, c->stream, c->d_partial,
-                       (long)t.blocks(), (double)c->g.nx, (double)c->g.ny, c->d_scalar + 0,
-                       c->vel_force[0], c->d_scalar + 3);
-    PLL_HIP_TRY(hipGetLastError());
-  }
-  return PLL_OK;
+  return acc ? launch_force_from_partials(c, (long)t.blocks()) : PLL_OK;
 }
 
-// Both stages of an FP32-mixed step inside a run (the previous step's
-// projection, forcing and boundary update applied on load) into the spare
-// velocity buffers, then swapped in; acc: the bulk mean of the new u and the
-// force of u go to d_scalar[0], [3].
-constexpr int kRk12Ty = 8;  // tile rows of the fused stages
-int rk12_f32(pll_context* c, int acc) {
-  const TileGrid t = tile_grid(c, kRk12Ty);
+// Launch shape of the fused stages: `slots` blocks run at once, and a block
+// costs its chunk's planes and about three more (two of stage 1 alone and the
+// ring's start), so the chunk is the one with the least rounds x (chunk + 3);
+// of equal costs the shortest, whose last round is spread the most.  Against
+// chunks for about 1024 blocks: 230 against 255 us at 384x256x192 (FP32), 30
+// against 39 us at 160x96x96.
+TileGrid rk12_grid(const pll_context* c, int ty, int slots) {
+  TileGrid t;
+  t.ntx = (c->g.nx + kRkTx - 1) / kRkTx;
+  t.nty = (c->g.ny + ty - 1) / ty;
+  const long cols = (long)t.ntx * t.nty;
+  long best = 0;
+  for (int kc = std::min(4, c->g.nz); kc <= c->g.nz; ++kc) {
+    const long nkc = (c->g.nz + kc - 1) / kc;
+    const long cost = ((cols * nkc + slots - 1) / slots) * (kc + 3);
+    if (best && cost >= best) continue;
+    best = cost;
+    t.kchunk = kc;
+    t.nkc = (int)nkc;
+  }
+  return t;
+}
+
+// Both stages of a step inside a run (the previous step's projection, forcing
+// and boundary update applied on load) into the spare velocity buffers, then
+// swapped in; u1out: u1 goes to its arrays as well; acc: the bulk mean of the
+// new u and the force of u go to d_scalar[0], [3].
+template <typename T>
+int rk12_t(pll_context* c, int acc, int u1out) {
+  constexpr int ty = kRk12Ty<T>();
+  const TileGrid t = rk12_grid(c, ty, kRk12Slots);
   if (acc && (long)t.blocks() > c->npartial)
     return fail(PLL_ERR_STATE, "reduction scratch smaller than the stencil grid");
   if (!c->fld_alt[0] || !c->fld_alt[1] || !c->fld_alt[2])
     return fail(PLL_ERR_STATE, "no spare velocity buffers");
-  const MeshT<float> m = mesh_of<float>(c);
-  const RkCoef* coef = static_cast<const RkCoef*>(c->d_rkcoef);
-  const double* dzflzi = c->d_mesh64 + 3 * (c->g.nz + 2);
   {
     TimerScope ts(c, K_RK12);
-    hipLaunchKernelGGL(k_rk12<kRk12Ty>, dim3(t.blocks()), dim3(kRkTx * kRk12Ty), 0, c->stream, c->g,
-                       F<float>(c, PLL_U), F<float>(c, PLL_V), F<float>(c, PLL_W),
-                       F<float>(c, PLL_P), static_cast<float*>(c->fld_alt[0]),
-                       static_cast<float*>(c->fld_alt[1]), static_cast<float*>(c->fld_alt[2]),
-                       m.dzc_inv, (float)c->dt, (float)(c->dt * c->dx_inv),
-                       (float)(c->dt * c->dy_inv),  // src/mod_calcVel.cc:256-258
-                       (float)(0.0 - c->u_crf),     // src/mod_updateBound.cc:80
-                       c->d_scalar + 3, forced_mask(c), coef, coef + (c->g.nz + 2),
-                       rk_uniform(c, 1), rk_uniform(c, 2), (int)(c->u_crf != 0.0), t.kchunk,
-                       t.ntx, t.nty, acc, dzflzi, c->d_partial);
+    const auto kernel =
+        c->u_crf != 0.0 ? (u1out ? k_rk12<T, ty, true, true> : k_rk12<T, ty, false, true>)
+                        : (u1out ? k_rk12<T, ty, true, false> : k_rk12<T, ty, false, false>);
+    hipLaunchKernelGGL(kernel, dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream, c->g, F<T>(c, PLL_U), F<T>(c, PLL_V),
+                       F<T>(c, PLL_W), F<T>(c, PLL_P), static_cast<T*>(c->fld_alt[0]),
+                       static_cast<T*>(c->fld_alt[1]), static_cast<T*>(c->fld_alt[2]),
+                       F<T>(c, PLL_U1), F<T>(c, PLL_V1), F<T>(c, PLL_W1), rk_param<T>(c),
+                       c->d_scalar + 3, forced_mask(c), t.kchunk, t.ntx, t.nty, acc,
+                       c->d_mesh64 + 3 * (c->g.nz + 2), c->d_partial);
   }
   PLL_HIP_TRY(hipGetLastError());
   for (int d = 0; d < 3; ++d) std::swap(c->fld[PLL_U + d], c->fld_alt[d]);
-  if (acc) {
-    // forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297)
-    TimerScope ts(c, K_MEAN_FINAL);
-    hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kRedThreads), 0, c->stream, c->d_partial,
-                       (long)t.blocks(), (double)c->g.nx, (double)c->g.ny, c->d_scalar + 0,
-                       c->vel_force[0], c->d_scalar + 3);
-    PLL_HIP_TRY(hipGetLastError());
-  }
-  return PLL_OK;
+  return acc ? launch_force_from_partials(c, (long)t.blocks()) : PLL_OK;
 }
 
 template <typename T>
@@ -2012,12 +1599,14 @@ int nan_t(pll_context* c, int field, int* passed) {
 #define PLL_DISPATCH(c, call_fp64, call_fp32) \
   ((c)->prec == PLL_FP64 ? (call_fp64) : (call_fp32))
 
-int rk_setup(pll_context* c) { return c->prec == PLL_FP64 ? PLL_OK : rk_coef_setup(c); }
+int rk_setup(pll_context* c) {
+  return PLL_DISPATCH(c, rk_coef_setup<double>(c), rk_coef_setup<float>(c));
+}
 
 int launch_rk(pll_context* c, int stage, int fold, int corr, int acc, int bcload) {
   if (c->closure) return launch_rk_closure(c, stage, fold, corr, acc, bcload);
-  return PLL_DISPATCH(c, rk_t<double>(c, stage, fold, corr, acc, bcload),
-                      rk_t<float>(c, stage, fold, corr, acc, bcload));
+  if (fold || corr) return fail(PLL_ERR_STATE, "the separate stages take no deferred updates");
+  return PLL_DISPATCH(c, rk_t<double>(c, stage, acc, bcload), rk_t<float>(c, stage, acc, bcload));
 }
 int launch_calc_rhs(pll_context* c) { return PLL_DISPATCH(c, rhs_t<double>(c), rhs_t<float>(c)); }
 int launch_force_from_partials(pll_context* c, long n) {
@@ -2030,13 +1619,8 @@ int launch_force_from_partials(pll_context* c, long n) {
   PLL_HIP_TRY(hipGetLastError());
   return PLL_OK;
 }
-int launch_rk12(pll_context* c, int acc) {
-  if (c->prec != PLL_FP32_MIXED) return fail(PLL_ERR_STATE, "the fused stages are the FP32-mixed step's");
-  return rk12_f32(c, acc);
-}
-int launch_rk2_rhs(pll_context* c, int defer, int corr, int acc) {
-  if (c->prec != PLL_FP64) return fail(PLL_ERR_STATE, "the fused stage 2 + calcRHS is the FP64 step's");
-  return rk2_rhs_t<double>(c, defer, corr, acc);
+int launch_rk12(pll_context* c, int acc, int u1out) {
+  return PLL_DISPATCH(c, rk12_t<double>(c, acc, u1out), rk12_t<float>(c, acc, u1out));
 }
 int launch_correct_vel(pll_context* c, bool with_mean) {
   return PLL_DISPATCH(c, correct_t<double>(c, with_mean), correct_t<float>(c, with_mean));

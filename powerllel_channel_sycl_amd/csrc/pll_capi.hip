@@ -14,7 +14,7 @@ namespace pll {
 const char* const kKernelNames[K_COUNT] = {
     "rk1",         "rk2",       "calc_rhs",   "fft_x_fwd",    "fft_y_fwd", "solve_trid",
     "fft_y_bwd",   "fft_x_bwd", "correct_vel", "mean_partial", "mean_final", "force_add",
-    "bc_vel",      "bc_p",      "check",      "init",         "misc",        "rk2_rhs",
+    "bc_vel",      "bc_p",      "check",      "init",         "misc",
     "fft_x_fwd_rhs", "rk_closure", "rk12"};
 
 namespace {
@@ -251,9 +251,8 @@ int create_impl(const pll_config* cfg, const double* dzf_global, pll_context** o
     e = hipMemsetAsync(c->fld[f], 0, c->nfield * c->esz, c->stream);
     if (e != hipSuccess) return bail(hip_fail(e, "hipMemsetAsync(field)"));
   }
-  // spare u, v, w (and p for the FP64 step's fused stage 2 + calcRHS)
-  const int nspare = c->prec == PLL_FP64 ? 4 : 3;
-  for (int d = 0; d < nspare; ++d) {
+  // spare u, v, w for the stages that cannot update in place
+  for (int d = 0; d < 3; ++d) {
     e = ctx_malloc(c, &c->fld_alt[d], c->nfield * c->esz);
     if (e != hipSuccess) return bail(hip_fail(e, "hipMalloc(spare field)"));
     e = hipMemsetAsync(c->fld_alt[d], 0, c->nfield * c->esz, c->stream);
@@ -299,7 +298,7 @@ int poisson_impl(pll_context* c) {
 // (`corr`, `fold`) and the bulk mean of the forcing is reduced by stage 2 from
 // the predictor; the last step of a run applies them explicitly, so every run
 // ends in the reference's state.
-int finish_step(pll_context* c, bool fused, bool last);
+int finish_step(pll_context* c);
 int finish_deferred(pll_context* c, bool last);
 
 int step_impl(pll_context* c, bool first, bool last) {
@@ -334,25 +333,23 @@ int step_impl(pll_context* c, bool first, bool last) {
     if ((rc = launch_bc_vel(c, 0))) return rc;  // :129
     if ((rc = launch_calc_rhs(c))) return rc;   // :133
     if ((rc = launch_poisson_step(c, false))) return rc;  // :137
-    return finish_step(c, false, last);
+    return finish_step(c);
   }
-  if (fused && c->prec != PLL_FP64) {
-    // FP32-mixed: the projection of step n (:145), its forcing (:149) and
-    // boundary update (:153) are applied by step n+1's stage loads (corr);
-    // stage 2 sums the bulk mean of the predictor for that forcing, and
-    // calcRHS runs inside the forward x transform's loads (:133-137).
-    // The boundary updates of u1 (:121) and u (:129) are not run either:
-    // stage 2 and calcRHS rebuild the halos they read from the boundary rules.
-    // Inside a run both stages run in one kernel (u1 stays in LDS); the
-    // first step (nothing deferred) and the last (u1 is left in its arrays)
-    // run them separately.
-    const int corr = fold;
+  if (fused) {
+    // The projection of step n (:145), its forcing (:149) and boundary update
+    // (:153) are applied by step n+1's stage loads; stage 2 sums the bulk mean
+    // of the predictor for that forcing, and calcRHS runs inside the forward x
+    // transform's loads (:133-137).  The boundary updates of u1 (:121) and u
+    // (:129) are not run either: stage 2 and calcRHS rebuild the halos they
+    // read from the boundary rules.  Both stages run in one kernel (u1 stays
+    // in LDS; the last step of a run also writes it to its arrays), but for
+    // the first step, which takes the velocity with its halos as it stands.
     const int acc = (!last && c->is_forced[0]) ? 1 : 0;
-    if (fold && !last) {
-      if ((rc = launch_rk12(c, acc))) return rc;  // :117-125
+    if (fold) {
+      if ((rc = launch_rk12(c, acc, last))) return rc;  // :117-125
     } else {
-      if ((rc = launch_rk(c, 1, fold, corr, 0))) return rc;       // :117
-      if ((rc = launch_rk(c, 2, fold, corr, acc, 1))) return rc;  // :125
+      if ((rc = launch_rk(c, 1, 0))) return rc;             // :117
+      if ((rc = launch_rk(c, 2, 0, 0, acc, 1))) return rc;  // :125
     }
     c->rhs_bcfold = 1;
     rc = launch_poisson_step(c, true);  // :133-137
@@ -360,27 +357,14 @@ int step_impl(pll_context* c, bool first, bool last) {
     if (rc) return rc;
     return finish_deferred(c, last);
   }
-  if (fused && c->prec == PLL_FP64) {
-    // FP64: the projection of step n (:145) and its forcing (:149) are applied
-    // by step n+1's loads (corr, fold); :121-133 run in one kernel: the u1
-    // boundary is rebuilt on load, the middle boundary update only matters for
-    // calcRHS (computed in the same kernel) and for w(nz) = 0 (written there).
-    // That kernel sums the predictor's bulk mean for the forcing.
-    const int corr = fold;
-    const int acc = (!last && c->is_forced[0]) ? 1 : 0;
-    if ((rc = launch_rk(c, 1, fold, corr))) return rc;        // :117
-    if ((rc = launch_rk2_rhs(c, fold, corr, acc))) return rc;  // :121-133
-    if ((rc = launch_poisson_step(c, false))) return rc;       // :137
-    return finish_deferred(c, last);
-  }
   // unfused: v or w is forced
-  if ((rc = launch_rk(c, 1, fold))) return rc;  // src/main.cc:117
+  if ((rc = launch_rk(c, 1, 0))) return rc;     // src/main.cc:117
   if ((rc = launch_bc_vel(c, 1))) return rc;    // :121
-  if ((rc = launch_rk(c, 2, fold))) return rc;  // :125
+  if ((rc = launch_rk(c, 2, 0))) return rc;     // :125
   if ((rc = launch_bc_vel(c, 0))) return rc;    // :129
   if ((rc = launch_calc_rhs(c))) return rc;     // :133
   if ((rc = launch_poisson_step(c, false))) return rc;  // :137
-  return finish_step(c, fused, last);
+  return finish_step(c);
 }
 
 // src/main.cc:141 after the pressure solve of a step whose projection, forcing
@@ -398,18 +382,12 @@ int finish_deferred(pll_context* c, bool last) {
 }
 
 // src/main.cc:141-153 after the pressure solve.
-int finish_step(pll_context* c, bool fused, bool last) {
+int finish_step(pll_context* c) {
   int rc;
-  if ((rc = launch_bc_p(c))) return rc;           // :141
-  if (!fused) {
-    if ((rc = launch_correct_vel(c, false))) return rc;  // :145
-    if ((rc = launch_force(c))) return rc;               // :149
-    return launch_bc_vel(c, 0);                          // :153
-  }
-  if ((rc = launch_correct_vel(c, c->is_forced[0] != 0))) return rc;  // :145 (+ mean of :149)
-  if (!last) return PLL_OK;
-  if (c->is_forced[0] && (rc = launch_add_force_u(c))) return rc;     // :149
-  return launch_bc_vel(c, 0);                                          // :153
+  if ((rc = launch_bc_p(c))) return rc;                // :141
+  if ((rc = launch_correct_vel(c, false))) return rc;  // :145
+  if ((rc = launch_force(c))) return rc;               // :149
+  return launch_bc_vel(c, 0);                          // :153
 }
 
 }  // namespace

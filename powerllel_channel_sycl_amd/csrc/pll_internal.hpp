@@ -27,6 +27,17 @@ struct MeshT {
   const T* dzflzi;
 };
 
+// Element k of a table that no kernel of the launch writes, k uniform over the
+// wave: a scalar load.  Through an ordinary pointer the compiler cannot rule
+// out that the kernel's stores change the table and loads it per lane, in order
+// behind every plane load in flight, so that using the coefficient waits for
+// all of them.
+template <typename T>
+__device__ __forceinline__ T uniform_load(const T* p, long k) {
+  using C = const __attribute__((address_space(4))) T;
+  return reinterpret_cast<C*>(reinterpret_cast<uintptr_t>(p))[k];
+}
+
 // Stockham plan of a complex transform of length L held in LDS.
 constexpr int kMaxPass = 8;
 struct FftPlan {
@@ -75,10 +86,9 @@ enum KernelId {
   K_CHECK,
   K_INIT,
   K_MISC,
-  K_RK2_RHS,        // stage 2 fused with calcRHS
   K_FFT_X_FWD_RHS,  // calcRHS fused into the forward x transform
   K_RK_CLOSURE,     // RK stage with the learned eddy viscosity
-  K_RK12,           // both RK stages of the FP32-mixed step
+  K_RK12,           // both RK stages of a step inside a run
   K_COUNT
 };
 extern const char* const kKernelNames[K_COUNT];
@@ -101,7 +111,7 @@ struct pll_context {
   hipStream_t stream = nullptr;
 
   void* fld[PLL_NFIELD] = {};
-  void* fld_alt[4] = {};  // spare u, v, w, p (FP64): the fused stage 2 writes here, then the roles swap
+  void* fld_alt[3] = {};  // spare u, v, w: the fused stages write here, then the roles swap
   void* spec = nullptr;
 
   // host mesh in FP64 (index 0..nz+1)
@@ -111,7 +121,7 @@ struct pll_context {
   int is_forced[3];
 
   void* d_mesh = nullptr;      // 4*(nz+2) in field precision: dzf, dzf_inv, dzc_inv, dzflzi
-  void* d_rkcoef = nullptr;    // FP32-mixed stencil coefficients, 2 stages x (nz+2)
+  void* d_rkcoef = nullptr;    // tendency_fast coefficients, 2 stages x (nz+2)
   double* d_mesh64 = nullptr;  // same, FP64
 
   // tridiagonal solve: a, c (nz), pre-factored pivot table [k][cy][cx]
@@ -223,14 +233,11 @@ bool closure_fused_available(const pll_context* c);
 // d_partial, into d_scalar[0] and d_scalar[3] (k_stencil.hip)
 int launch_force_from_partials(pll_context* c, long n);
 
-int rk_setup(pll_context* c);  // per-plane coefficients of the FP32-mixed stencil
+int rk_setup(pll_context* c);  // per-plane coefficients of the stages
 int launch_calc_rhs(pll_context* c);
-// RK stage 2 fused with calcRHS (FP64 step sequence only): writes the new u, v,
-// w and the right-hand side to the spare buffers and swaps them in; defer adds
-// the previous step's force, corr applies its projection on load, acc reduces
-// the bulk mean of the new u and the force of u into d_scalar[0], [3].
-int launch_rk2_rhs(pll_context* c, int defer, int corr = 0, int acc = 0);
-int launch_rk12(pll_context* c, int acc);
+// Both RK stages of a step inside a run, the previous step's projection,
+// forcing and boundary update applied on load; u1out: u1 is left in its arrays.
+int launch_rk12(pll_context* c, int acc, int u1out);
 // with_mean: also reduce the bulk mean of the corrected u and store the force
 // of u (vel_force[0] - mean) on the device.
 int launch_correct_vel(pll_context* c, bool with_mean);

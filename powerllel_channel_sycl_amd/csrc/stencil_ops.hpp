@@ -31,9 +31,9 @@ __device__ __forceinline__ void tendency_z(const A& U, const A& V, const A& W, c
                                            int k, T dxi, T dyi, T rei, T ucrf, T& tu, T& tv,
                                            T& tw, ZFace<T>& zf) {
   const T quarter = T(0.25), half = T(0.5);
-  const T dzf_k = m.dzf[k], dzf_p = m.dzf[k + 1], dzf_m = m.dzf[k - 1];
-  const T dci_k = m.dzc_inv[k], dci_m = m.dzc_inv[k - 1];
-  const T dfi_k = m.dzf_inv[k], dfi_p = m.dzf_inv[k + 1];
+  const T dzf_k = uniform_load(m.dzf, k), dzf_p = uniform_load(m.dzf, k + 1), dzf_m = uniform_load(m.dzf, k - 1);
+  const T dci_k = uniform_load(m.dzc_inv, k), dci_m = uniform_load(m.dzc_inv, k - 1);
+  const T dfi_k = uniform_load(m.dzf_inv, k), dfi_p = uniform_load(m.dzf_inv, k + 1);
 
   // ---- x-momentum at the u face ----
   {
@@ -144,8 +144,8 @@ __device__ __forceinline__ void tendency(const A& U, const A& V, const A& W, con
 template <typename T, class A>
 __device__ __forceinline__ ZFace<T> zface_lower(const A& U, const A& V, const A& W,
                                                 const MeshT<T>& m, int k) {
-  const T dzf_k = m.dzf[k], dzf_m = m.dzf[k - 1];
-  const T dci_m = m.dzc_inv[k - 1], dfi_k = m.dzf_inv[k];
+  const T dzf_k = uniform_load(m.dzf, k), dzf_m = uniform_load(m.dzf, k - 1);
+  const T dci_m = uniform_load(m.dzc_inv, k - 1), dfi_k = uniform_load(m.dzf_inv, k);
   ZFace<T> zf;
   {
     const T q0 = U(0, 0, 0), qb = U(0, 0, -1);
