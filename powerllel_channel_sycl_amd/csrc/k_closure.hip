@@ -1388,7 +1388,7 @@ int rk_closure_t(pll_context* c, int stage, int fold, int corr, int acc, int bcl
   }
   PLL_HIP_TRY(hipGetLastError());
   // forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297)
-  return acc ? launch_force_from_partials(c, (long)grid.x) : PLL_OK;
+  return acc ? force_from_partials(c, (long)grid.x) : PLL_OK;
 }
 
 // Blocks of the closure stage kernel (its bulk-mean partials must fit d_partial).

@@ -167,6 +167,41 @@ struct RhsSrc {
   int bcfold;
 };
 
+// forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297) from n block
+// partials of stage 2, as a block of its own in the forward transform that
+// follows: a launch of one block costs more than its work (5-6 us, of which a
+// step of 256x192x128 has 284).
+struct MeanJob {
+  const double* partial;
+  long n;  // 0: nothing to do
+  double nxg, nyg, vel_force;
+  double* mean;
+  double* force;
+};
+__device__ __forceinline__ void mean_job(const MeanJob& m) {
+  __shared__ double red[64];
+  const int W = blockDim.x < 64 ? (int)blockDim.x : 64, t = threadIdx.x;
+  if (t < W) {
+    double s = 0.0;
+    for (long i = t; i < m.n; i += 8 * W) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = i + u * W < m.n ? m.partial[i + u * W] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    red[t] = s;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double s = 0.0;
+    for (int i = 0; i < W; ++i) s += red[i];
+    const double mean = s / m.nxg / m.nyg;
+    *m.mean = mean;
+    *m.force = m.vel_force - mean;
+  }
+}
+
 template <typename T>
 RhsSrc<T> rhs_src(const pll_context* c) {
   const double dti = 1.0 / c->dt;  // src/mod_calcRHS.cc:11-13
@@ -183,14 +218,24 @@ __global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xf(Geom g, cons
                                                                T* __restrict__ spec,
                                                                const cpx<T>* __restrict__ twL,
                                                                const cpx<T>* __restrict__ rtw,
-                                                               long nrows, RhsSrc<T> rs) {
+                                                               long nrows, RhsSrc<T> rs,
+                                                               MeanJob mj) {
+  unsigned bid = blockIdx.x, nblk = gridDim.x;
+  if (RHS && mj.n) {
+    if (bid == 0) {
+      mean_job(mj);
+      return;
+    }
+    --bid;
+    --nblk;
+  }
   constexpr int TPS = tps<L>(), NB = x_rows<T, L>(), NT = NB * TPS, N = 2 * L;
   __shared__ cpx<T> buf[padded(NB * L)];
   __shared__ long rowbase[NB];
   __shared__ T rowdz[NB];
   __shared__ long rowvs[NB];     // offset of the v row below (j-1, or its image)
   __shared__ unsigned char roww[NB];  // bit 0: w below is the wall 0; bit 1: w is the wall 0
-  const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * NB;
+  const long row0 = (long)xcd_remap(bid, nblk) * NB;
   if (threadIdx.x < NB) {
     const long r = row0 + threadIdx.x;
     const int j = (int)(r % g.ny), k = (int)(r / g.ny);
@@ -267,7 +312,26 @@ __global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xf(Geom g, cons
 // execute_fft_bwd_xpen (src/mod_fft.cc:90-120): perm rows -> p interior * norm.
 // With HALO (the step sequence, where updateBoundP follows at once) a row is
 // stored as aligned pairs p(0..nx+1), the two x-halo cells holding their
-// periodic values p(nx) and p(1) -- what updateBoundP writes there.
+// periodic values p(nx) and p(1), and a row whose copies updateBoundP puts on
+// the y halo or a wall's ghost plane is stored there too (row_images), so that
+// boundary update (src/mod_updateBound.cc:253-296) needs no pass of its own.
+// Offsets of row (j, k)'s copies (0: none): y the periodic image on the y halo,
+// z the zero-gradient ghost plane (src/mod_updateBound.cc:253-296).
+struct RowImage {
+  long y, z;
+};
+__device__ __forceinline__ RowImage row_images(const Geom& g, int j, int k) {
+  return RowImage{j == 0 ? (long)g.ny * g.sx : (j == g.ny - 1 ? -(long)g.ny * g.sx : 0),
+                  k == 0 ? -g.sxy : (k == g.nz - 1 ? g.sxy : 0)};
+}
+template <typename V>
+__device__ __forceinline__ void store_images(V* at, long stride, const RowImage& im, V val) {
+  at[0] = val;
+  if (im.y) at[im.y / stride] = val;
+  if (im.z) at[im.z / stride] = val;
+  if (im.y && im.z) at[(im.y + im.z) / stride] = val;
+}
+
 template <typename T, int L, bool HALO>
 __global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xb(Geom g, const T* __restrict__ spec,
                                                                T* __restrict__ p,
@@ -278,11 +342,13 @@ __global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xb(Geom g, cons
   constexpr int RMIN = shape_rmin<Shape<L>>();
   __shared__ cpx<T> buf[padded(NB * L)];
   __shared__ long rowbase[NB];
+  __shared__ RowImage rowimg[NB];
   const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * NB;
   if (threadIdx.x < NB) {
     const long r = row0 + threadIdx.x;
     const int j = (int)(r % g.ny), k = (int)(r / g.ny);
     rowbase[threadIdx.x] = r < nrows ? g.idx(HALO ? 0 : 1, j + 1, k + 1) : -1;
+    if (HALO) rowimg[threadIdx.x] = row_images(g, j, k);
   }
   const cpx<T>* specc = reinterpret_cast<const cpx<T>*>(spec);
   {
@@ -342,7 +408,8 @@ __global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xb(Geom g, cons
     for (int u = 0; u < NST; ++u) {
       const int e = threadIdx.x + u * NT;
       const int s2 = e / NP, q = e % NP;
-      if (e < NB * NP && rowbase[s2] >= 0) reinterpret_cast<cpx<T>*>(p + rowbase[s2])[q] = t[u];
+      if (e < NB * NP && rowbase[s2] >= 0)
+        store_images(reinterpret_cast<cpx<T>*>(p + rowbase[s2]) + q, 2, rowimg[s2], t[u]);
     }
   } else {
     constexpr int NST = NB * N / NT;
@@ -566,7 +633,16 @@ __global__ __launch_bounds__(kGenThreads) void k_gxf(Geom g, const T* __restrict
                                                      T* __restrict__ spec, FftPlan pl, XShape xs,
                                                      const cpx<T>* __restrict__ twL,
                                                      const cpx<T>* __restrict__ rtw, long nrows,
-                                                     RhsSrc<T> rs) {
+                                                     RhsSrc<T> rs, MeanJob mj) {
+  unsigned bid = blockIdx.x, nblk = gridDim.x;
+  if (RHS && mj.n) {
+    if (bid == 0) {
+      mean_job(mj);
+      return;
+    }
+    --bid;
+    --nblk;
+  }
   extern __shared__ __align__(16) unsigned char smem[];
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
   __shared__ long rowbase[kGenRows];
@@ -574,7 +650,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gxf(Geom g, const T* __restrict
   __shared__ long rowvs[kGenRows];           // offset of the v row below (j-1, or its image)
   __shared__ unsigned char roww[kGenRows];   // bit 0: w below is the wall 0; bit 1: w is the wall 0
   const int N = g.nx, L = N / 2, NT = blockDim.x;
-  const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * xs.nb;
+  const long row0 = (long)xcd_remap(bid, nblk) * xs.nb;
   if ((int)threadIdx.x < xs.nb) {
     const long r = row0 + threadIdx.x;
     const int j = (int)(r % g.ny), k = (int)(r / g.ny);
@@ -662,12 +738,14 @@ __global__ __launch_bounds__(kGenThreads) void k_gxb(Geom g, const T* __restrict
   extern __shared__ __align__(16) unsigned char smem[];
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
   __shared__ long rowbase[kGenRows];
+  __shared__ RowImage rowimg[kGenRows];
   const int N = g.nx, L = N / 2, NT = blockDim.x;
   const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * xs.nb;
   if ((int)threadIdx.x < xs.nb) {
     const long r = row0 + threadIdx.x;
     const int j = (int)(r % g.ny), k = (int)(r / g.ny);
     rowbase[threadIdx.x] = r < nrows ? g.idx(HALO ? 0 : 1, j + 1, k + 1) : -1;
+    if (HALO) rowimg[threadIdx.x] = row_images(g, j, k);
   }
   const cpx<T>* specc = reinterpret_cast<const cpx<T>*>(spec) + row0 * L;
   const int slots = xs.nb * L;
@@ -720,8 +798,8 @@ __global__ __launch_bounds__(kGenThreads) void k_gxb(Geom g, const T* __restrict
       const int s2 = div_by(e, mP), q = e - s2 * NP;
       if (rowbase[s2] < 0) continue;
       const int i0 = q == 0 ? N - 1 : 2 * q - 1, i1 = q == L ? 0 : 2 * q;
-      reinterpret_cast<cpx<T>*>(p + rowbase[s2])[q] =
-          cpx<T>{norm * real_at(buf, s2 * N + i0), norm * real_at(buf, s2 * N + i1)};
+      store_images(reinterpret_cast<cpx<T>*>(p + rowbase[s2]) + q, 2, rowimg[s2],
+                   cpx<T>{norm * real_at(buf, s2 * N + i0), norm * real_at(buf, s2 * N + i1)});
     }
   } else {
     for (int e = threadIdx.x; e < xs.nb * N; e += NT) {
@@ -900,6 +978,14 @@ int setup_t(pll_context* c) {
   return PLL_OK;
 }
 
+// The bulk mean that stage 2 left partials of, for the transform that runs next.
+MeanJob take_mean(pll_context* c) {
+  const long n = c->mean_pending;
+  c->mean_pending = 0;
+  return MeanJob{c->d_partial, n, (double)c->g.nx, (double)c->g.ny, c->vel_force[0], c->d_scalar,
+                 c->d_scalar + 3};
+}
+
 int round_wave(int n) { return (n + 63) / 64 * 64; }
 
 XShape x_shape(const pll_context* c) {
@@ -919,14 +1005,16 @@ int x_generic(pll_context* c, bool fwd, bool step) {
   T* p = static_cast<T*>(c->fld[PLL_P]);
   T* spec = static_cast<T*>(c->spec);
   if (fwd && step) {
+    const MeanJob mj = take_mean(c);
     TimerScope ts(c, K_FFT_X_FWD_RHS);
-    hipLaunchKernelGGL((k_gxf<T, true>), blocks, threads, sh, c->stream, c->g,
+    hipLaunchKernelGGL((k_gxf<T, true>), dim3(blocks.x + (mj.n ? 1 : 0)), threads, sh, c->stream, c->g,
                        static_cast<const T*>(nullptr), spec, c->plan_x, xs, tw, rtw, nrows,
-                       rhs_src<T>(c));
+                       rhs_src<T>(c), mj);
   } else if (fwd) {
     TimerScope ts(c, K_FFT_X_FWD);
     hipLaunchKernelGGL((k_gxf<T, false>), blocks, threads, sh, c->stream, c->g,
-                       static_cast<const T*>(p), spec, c->plan_x, xs, tw, rtw, nrows, RhsSrc<T>{});
+                       static_cast<const T*>(p), spec, c->plan_x, xs, tw, rtw, nrows, RhsSrc<T>{},
+                       MeanJob{});
   } else {
     const double norm = 1.0 / (c->g.nx * c->g.ny);  // src/mod_fft.cc:57
     TimerScope ts(c, K_FFT_X_BWD);
@@ -961,14 +1049,15 @@ int x_fixed(pll_context* c, bool fwd, bool rhs = false) {
   const cpx<T>* rtw = static_cast<const cpx<T>*>(c->d_rtw_x);
   if (fwd && rhs) {
     const RhsSrc<T> rs = rhs_src<T>(c);
+    const MeanJob mj = take_mean(c);
     TimerScope ts(c, K_FFT_X_FWD_RHS);
-    hipLaunchKernelGGL((k_xf<T, L, true>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
-                       static_cast<const T*>(nullptr), static_cast<T*>(c->spec), tw, rtw, nrows, rs);
+    hipLaunchKernelGGL((k_xf<T, L, true>), dim3(blocks + (mj.n ? 1 : 0)), dim3(NT), 0, c->stream, c->g,
+                       static_cast<const T*>(nullptr), static_cast<T*>(c->spec), tw, rtw, nrows, rs, mj);
   } else if (fwd) {
     TimerScope ts(c, K_FFT_X_FWD);
     hipLaunchKernelGGL((k_xf<T, L, false>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
                        static_cast<const T*>(c->fld[PLL_P]), static_cast<T*>(c->spec), tw, rtw,
-                       nrows, RhsSrc<T>{});
+                       nrows, RhsSrc<T>{}, MeanJob{});
   } else {
     const double norm = 1.0 / (c->g.nx * c->g.ny);  // src/mod_fft.cc:57
     TimerScope ts(c, K_FFT_X_BWD);

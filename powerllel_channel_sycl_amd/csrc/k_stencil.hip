@@ -592,8 +592,7 @@ constexpr int kRk12Slots = 256;  // blocks of k_rk12 that run at once: one per C
 // forcing and boundary rules apply at its commit, after stage 2 of the plane
 // below has been computed, and stage 2's results are stored after the commit:
 // arithmetic on the loaded values in the fetch, or stores ahead of the commit,
-// would make a wave wait there.  p on the y halo is read at its image, so only
-// its x halos (written by the inverse x transform) have to be valid.
+// would make a wave wait there.
 //
 // Bound by latency between its two barriers per plane, at one block per CU: per
 // point about 240 (FP64) VALU operations and 60 LDS reads, each near 0.9 ms of
@@ -636,13 +635,11 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
     return;
   }
   auto wrap = [](int x, int n) { return ((x - 1) % n + n) % n + 1; };
-  int gaddr[NPF], gnorth[NPF];  // plane-relative address of the periodic image (-1: past the tile), its j+1
+  int gaddr[NPF];  // plane-relative address of the periodic image (-1: past the tile)
 #pragma unroll
   for (int n = 0; n < NPF; ++n) {
     const int e = t + n * NT;
-    const int y = wrap(j0 - 1 + e / UX, g.ny);
-    gaddr[n] = e < UPL ? wrap(i0 - 1 + e % UX, g.nx) + (int)g.sx * y : -1;
-    gnorth[n] = gaddr[n] + (int)g.sx * (y == g.ny ? 1 - g.ny : 1);
+    gaddr[n] = e < UPL ? wrap(i0 - 1 + e % UX, g.nx) + (int)g.sx * wrap(j0 - 1 + e / UX, g.ny) : -1;
   }
   T ru[NPF], rv[NPF], rw[NPF], rp0[NPF], rpe[NPF], rpn[NPF], rpt[NPF];
   auto fetch = [&](int kk) {
@@ -658,7 +655,7 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
         rw[n] = sw[a];
         rp0[n] = pp[a];
         rpe[n] = pp[a + 1];
-        rpn[n] = pp[gnorth[n] + o];
+        rpn[n] = pp[a + g.sx];
         rpt[n] = pp[a + g.sxy];
       }
   };
@@ -829,16 +826,15 @@ __global__ __launch_bounds__(kRkTx* kRkTy) void k_calc_rhs(Geom g, const T* __re
 }
 
 // correctVel, src/mod_calcVel.cc:272-274.  p(k+1) becomes the next plane's p(k).
-// With ACC the block also sums the corrected u times dzflzi(k) (FP64) into
-// partial[block] -- the first half of the bulk mean that forceVel needs.
-template <typename T, bool ACC>
-__global__ __launch_bounds__(kRkTx* correct_ty<T>()) void k_correct(Geom g, const T* __restrict__ p,
-                                                          T* __restrict__ u, T* __restrict__ v,
-                                                          T* __restrict__ w,
-                                                          const T* __restrict__ dzc_inv, T dtdxi,
-                                                          T dtdyi, T dt, int kchunk, int ntx,
-                                                          int nty, const double* __restrict__ dzflzi,
-                                                          double* __restrict__ partial) {
+// With fmask the force that is on the device is added to those components
+// (forceVel, :299-315), which saves the end of a run its pass over u.  The
+// boundary update stays a launch of its own: written by the cells that the halo
+// copies, in this loop, it took the loads of the next planes out of flight (one
+// 128^3 step 183 us, 1536x768x512 FP32 4 steps 74.3 ms; as it is 132 us, 69.9 ms).
+template <typename T>
+__global__ __launch_bounds__(kRkTx* correct_ty<T>()) void k_correct(
+    Geom g, const T* __restrict__ p, T* __restrict__ u, T* __restrict__ v, T* __restrict__ w,
+    RkParam<T> q, const double* __restrict__ force, int fmask, int kchunk, int ntx, int nty) {
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
   const int ti = (int)(b % (unsigned)ntx), tj = (int)((b / (unsigned)ntx) % (unsigned)nty);
   const int kc = (int)(b / (unsigned)(ntx * nty));
@@ -846,29 +842,24 @@ __global__ __launch_bounds__(kRkTx* correct_ty<T>()) void k_correct(Geom g, cons
   const int i = ti * kRkTx + (int)(threadIdx.x % kRkTx) + 1;
   const int j = tj * TY + (int)(threadIdx.x / kRkTx) + 1;
   const int k0 = kc * kchunk + 1, k1 = min(k0 + kchunk - 1, g.nz);
-  double acc = 0.0;
-  if (i <= g.nx && j <= g.ny && k0 <= k1) {
-    long c = g.idx(i, j, k0);
-    T p0 = p[c];
-    for (int k = k0; k <= k1; ++k, c += g.sxy) {
-      const T pt = p[c + g.sxy];
-      const T un = u[c] - (p[c + 1] - p0) * dtdxi;
-      u[c] = un;
-      v[c] -= (p[c + g.sx] - p0) * dtdyi;
-      w[c] -= (pt - p0) * dt * dzc_inv[k];
-      if (ACC) acc += (double)un * uniform_load(dzflzi, k);
-      p0 = pt;
-    }
-  }
-  if (ACC) {
-    __shared__ double sh[kRkTx * TY];
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int h = kRkTx * TY / 2; h > 0; h >>= 1) {
-      if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[b] = sh[0];
+  if (i > g.nx || j > g.ny || k0 > k1) return;
+  const bool fu = fmask & 1, fv = fmask & 2, fw = fmask & 4;
+  const T f_u = fu ? (T)force[0] : T(0), f_v = fv ? (T)force[1] : T(0),
+          f_w = fw ? (T)force[2] : T(0);
+  long c = g.idx(i, j, k0);
+  T p0 = p[c];
+  for (int k = k0; k <= k1; ++k, c += g.sxy) {
+    const T pt = p[c + g.sxy];
+    T nu = u[c] - (p[c + 1] - p0) * q.dtdxi;
+    T nv = v[c] - (p[c + g.sx] - p0) * q.dtdyi;
+    T nw = w[c] - (pt - p0) * q.dt * uniform_load(q.m.dzc_inv, k);
+    if (fu) nu = nu + f_u;
+    if (fv) nv = nv + f_v;
+    if (fw) nw = nw + f_w;
+    u[c] = nu;
+    v[c] = nv;
+    w[c] = nw;
+    p0 = pt;
   }
 }
 
@@ -981,9 +972,17 @@ __device__ __forceinline__ void perimeter(int q, int nx, int ny, int& i, int& j)
   }
 }
 
+// blockIdx.y 0 updates u, v, w, 1 the second set u2, v2, w2.
 template <typename T>
 __global__ __launch_bounds__(256) void k_bc_vel(Geom g, T* __restrict__ u, T* __restrict__ v,
-                                                T* __restrict__ w, T bc_u, int walls_only) {
+                                                T* __restrict__ w, T* __restrict__ u2,
+                                                T* __restrict__ v2, T* __restrict__ w2, T bc_u,
+                                                int walls_only) {
+  if (blockIdx.y) {
+    u = u2;
+    v = v2;
+    w = w2;
+  }
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const int nper = 2 * (g.nx + 2) + 2 * g.ny;
   const long nside = walls_only ? 0 : (long)nper * g.nz;
@@ -1335,7 +1334,7 @@ int rk_t(pll_context* c, int stage, int acc, int bcload) {
                  : go(crf ? k_rk<T, 2, true> : k_rk<T, 2, false>, PLL_U1, PLL_U);
   }
   PLL_HIP_TRY(hipGetLastError());
-  return acc ? launch_force_from_partials(c, (long)t.blocks()) : PLL_OK;
+  return acc ? force_from_partials(c, (long)t.blocks()) : PLL_OK;
 }
 
 // Launch shape of the fused stages: `slots` blocks run at once, and a block
@@ -1387,7 +1386,7 @@ int rk12_t(pll_context* c, int acc, int u1out) {
   }
   PLL_HIP_TRY(hipGetLastError());
   for (int d = 0; d < 3; ++d) std::swap(c->fld[PLL_U + d], c->fld_alt[d]);
-  return acc ? launch_force_from_partials(c, (long)t.blocks()) : PLL_OK;
+  return acc ? force_from_partials(c, (long)t.blocks()) : PLL_OK;
 }
 
 template <typename T>
@@ -1405,45 +1404,14 @@ int rhs_t(pll_context* c) {
 }
 
 template <typename T>
-int correct_t(pll_context* c, bool with_mean) {
+int correct_t(pll_context* c, bool with_force) {
   constexpr int ty = correct_ty<T>();
   const TileGrid t = tile_grid(c, ty);
-  const double dtdxi = c->dt * c->dx_inv;  // src/mod_calcVel.cc:256-258
-  const double dtdyi = c->dt * c->dy_inv;
-  const double* dzflzi = c->d_mesh64 + 3 * (c->g.nz + 2);
-  if (with_mean && (long)t.blocks() > c->npartial)
-    return fail(PLL_ERR_STATE, "reduction scratch smaller than the projection grid");
-  {
-    TimerScope ts(c, K_CORRECT);
-    if (with_mean)
-      hipLaunchKernelGGL((k_correct<T, true>), dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream,
-                         c->g, F<T>(c, PLL_P), F<T>(c, PLL_U), F<T>(c, PLL_V), F<T>(c, PLL_W),
-                         mesh_of<T>(c).dzc_inv, (T)dtdxi, (T)dtdyi, (T)c->dt, t.kchunk, t.ntx,
-                         t.nty, dzflzi, c->d_partial);
-    else
-      hipLaunchKernelGGL((k_correct<T, false>), dim3(t.blocks()), dim3(kRkTx * ty), 0,
-                         c->stream, c->g, F<T>(c, PLL_P), F<T>(c, PLL_U), F<T>(c, PLL_V),
-                         F<T>(c, PLL_W), mesh_of<T>(c).dzc_inv, (T)dtdxi, (T)dtdyi, (T)c->dt,
-                         t.kchunk, t.ntx, t.nty, dzflzi, c->d_partial);
-  }
-  if (with_mean) {
-    // forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297)
-    TimerScope ts(c, K_MEAN_FINAL);
-    hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kRedThreads), 0, c->stream, c->d_partial,
-                       (long)t.blocks(), (double)c->g.nx, (double)c->g.ny, c->d_scalar + 0,
-                       c->vel_force[0], c->d_scalar + 3);
-  }
-  PLL_HIP_TRY(hipGetLastError());
-  return PLL_OK;
-}
-
-// forceVel's update of u with the force already on the device.
-template <typename T>
-int add_force_u_t(pll_context* c) {
-  const int kc = kchunk_for(c);
-  TimerScope ts(c, K_FORCE);
-  hipLaunchKernelGGL((k_add_force<T>), col_grid(c, kc), dim3(kTx, kTy), 0, c->stream, c->g,
-                     F<T>(c, PLL_U), c->d_scalar + 3, kc);
+  TimerScope ts(c, K_CORRECT);
+  hipLaunchKernelGGL((k_correct<T>), dim3(t.blocks()), dim3(kRkTx * ty), 0, c->stream, c->g,
+                     F<T>(c, PLL_P), F<T>(c, PLL_U), F<T>(c, PLL_V), F<T>(c, PLL_W),
+                     rk_param<T>(c), c->d_scalar + 3, with_force ? forced_mask(c) : 0, t.kchunk,
+                     t.ntx, t.nty);
   PLL_HIP_TRY(hipGetLastError());
   return PLL_OK;
 }
@@ -1494,15 +1462,16 @@ inline long bc_threads(const pll_context* c) {
   return nper * c->g.nz + (long)(c->g.nx + 2) * (c->g.ny + 2);
 }
 
+// which: 0 (u, v, w), 1 (u1, v1, w1), 2 both
 template <typename T>
 int bc_vel_t(pll_context* c, int which, int walls_only) {
   const long n = walls_only ? (long)(c->g.nx + 2) * (c->g.ny + 2) : bc_threads(c);
-  const int base = which ? PLL_U1 : PLL_U;
+  const int a = which == 1 ? PLL_U1 : PLL_U, b = which == 0 ? PLL_U : PLL_U1;
   const double bc_u = 0.0 - c->u_crf;  // src/mod_updateBound.cc:80
   TimerScope ts(c, K_BC_VEL);
-  hipLaunchKernelGGL((k_bc_vel<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
-                     c->g, F<T>(c, base), F<T>(c, base + 1), F<T>(c, base + 2), (T)bc_u,
-                     walls_only);
+  hipLaunchKernelGGL((k_bc_vel<T>), dim3((unsigned)((n + 255) / 256), which == 2 ? 2 : 1),
+                     dim3(256), 0, c->stream, c->g, F<T>(c, a), F<T>(c, a + 1), F<T>(c, a + 2),
+                     F<T>(c, b), F<T>(c, b + 1), F<T>(c, b + 2), (T)bc_u, walls_only);
   PLL_HIP_TRY(hipGetLastError());
   return PLL_OK;
 }
@@ -1609,24 +1578,17 @@ int launch_rk(pll_context* c, int stage, int fold, int corr, int acc, int bcload
   return PLL_DISPATCH(c, rk_t<double>(c, stage, acc, bcload), rk_t<float>(c, stage, acc, bcload));
 }
 int launch_calc_rhs(pll_context* c) { return PLL_DISPATCH(c, rhs_t<double>(c), rhs_t<float>(c)); }
-int launch_force_from_partials(pll_context* c, long n) {
+int force_from_partials(pll_context* c, long n) {
   if (n < 1 || n > c->npartial || !c->d_partial)
     return fail(PLL_ERR_STATE, "bulk-mean partials do not fit the scratch");
-  TimerScope ts(c, K_MEAN_FINAL);
-  hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kRedThreads), 0, c->stream, c->d_partial, n,
-                     (double)c->g.nx, (double)c->g.ny, c->d_scalar + 0, c->vel_force[0],
-                     c->d_scalar + 3);
-  PLL_HIP_TRY(hipGetLastError());
+  c->mean_pending = n;
   return PLL_OK;
 }
 int launch_rk12(pll_context* c, int acc, int u1out) {
   return PLL_DISPATCH(c, rk12_t<double>(c, acc, u1out), rk12_t<float>(c, acc, u1out));
 }
-int launch_correct_vel(pll_context* c, bool with_mean) {
-  return PLL_DISPATCH(c, correct_t<double>(c, with_mean), correct_t<float>(c, with_mean));
-}
-int launch_add_force_u(pll_context* c) {
-  return PLL_DISPATCH(c, add_force_u_t<double>(c), add_force_u_t<float>(c));
+int launch_correct_vel(pll_context* c, bool with_force) {
+  return PLL_DISPATCH(c, correct_t<double>(c, with_force), correct_t<float>(c, with_force));
 }
 int launch_mean(pll_context* c, int field, double nxg, double nyg, double* d_out) {
   return PLL_DISPATCH(c, mean_t<double>(c, field, nxg, nyg, d_out, 0.0, nullptr),

@@ -299,7 +299,7 @@ int poisson_impl(pll_context* c) {
 // the predictor; the last step of a run applies them explicitly, so every run
 // ends in the reference's state.
 int finish_step(pll_context* c);
-int finish_deferred(pll_context* c, bool last);
+int finish_run(pll_context* c, int bc);
 
 int step_impl(pll_context* c, bool first, bool last) {
   int rc;
@@ -313,16 +313,14 @@ int step_impl(pll_context* c, bool first, bool last) {
     // forcing summed by stage 2, and calcRHS inside the forward x transform
     // (which rebuilds u's boundary on load)
     const int corr = fold;
-    const int acc = (!last && c->is_forced[0]) ? 1 : 0;
+    const int acc = c->is_forced[0] ? 1 : 0;
     if ((rc = launch_rk(c, 1, fold, corr, 0, 1))) return rc;  // :145-153, :117, :121
     if ((rc = launch_rk(c, 2, 0, 0, acc, 0))) return rc;      // :125
     c->rhs_bcfold = 1;
-    rc = launch_poisson_step(c, true);  // :133-137
+    rc = launch_poisson_step(c, true);  // :133-141
     c->rhs_bcfold = 0;
     if (rc) return rc;
-    // inside a run p's boundary update (:141) is left to the next step's
-    // deferred pass, which reads p's halos through their rules
-    return last ? finish_deferred(c, last) : PLL_OK;
+    return last ? finish_run(c, 0) : PLL_OK;  // :145-153
   }
   if (c->closure) {
     // the closure stages (eddy viscosity evaluated in the stage kernel), then
@@ -332,7 +330,7 @@ int step_impl(pll_context* c, bool first, bool last) {
     if ((rc = launch_rk(c, 2, 0))) return rc;  // :125
     if ((rc = launch_bc_vel(c, 0))) return rc;  // :129
     if ((rc = launch_calc_rhs(c))) return rc;   // :133
-    if ((rc = launch_poisson_step(c, false))) return rc;  // :137
+    if ((rc = launch_poisson_step(c, false))) return rc;  // :137-141
     return finish_step(c);
   }
   if (fused) {
@@ -344,7 +342,7 @@ int step_impl(pll_context* c, bool first, bool last) {
     // read from the boundary rules.  Both stages run in one kernel (u1 stays
     // in LDS; the last step of a run also writes it to its arrays), but for
     // the first step, which takes the velocity with its halos as it stands.
-    const int acc = (!last && c->is_forced[0]) ? 1 : 0;
+    const int acc = c->is_forced[0] ? 1 : 0;
     if (fold) {
       if ((rc = launch_rk12(c, acc, last))) return rc;  // :117-125
     } else {
@@ -352,10 +350,12 @@ int step_impl(pll_context* c, bool first, bool last) {
       if ((rc = launch_rk(c, 2, 0, 0, acc, 1))) return rc;  // :125
     }
     c->rhs_bcfold = 1;
-    rc = launch_poisson_step(c, true);  // :133-137
+    rc = launch_poisson_step(c, true);  // :133-141
     c->rhs_bcfold = 0;
     if (rc) return rc;
-    return finish_deferred(c, last);
+    // the last step of a run applies what the next one's loads would (:121 for
+    // u1's halos, :145-153)
+    return last ? finish_run(c, 2) : PLL_OK;
   }
   // unfused: v or w is forced
   if ((rc = launch_rk(c, 1, 0))) return rc;     // src/main.cc:117
@@ -363,31 +363,23 @@ int step_impl(pll_context* c, bool first, bool last) {
   if ((rc = launch_rk(c, 2, 0))) return rc;     // :125
   if ((rc = launch_bc_vel(c, 0))) return rc;    // :129
   if ((rc = launch_calc_rhs(c))) return rc;     // :133
-  if ((rc = launch_poisson_step(c, false))) return rc;  // :137
+  if ((rc = launch_poisson_step(c, false))) return rc;  // :137-141
   return finish_step(c);
 }
 
-// src/main.cc:141 after the pressure solve of a step whose projection, forcing
-// and final boundary update (:145-153) the next step's loads apply; the last
-// step of a run refreshes u1's halos (its boundary update :121 was not run)
-// and applies them explicitly.
-int finish_deferred(pll_context* c, bool last) {
-  int rc;
-  if ((rc = launch_bc_p(c))) return rc;  // :141
-  if (!last) return PLL_OK;
-  if ((rc = launch_bc_vel(c, 1))) return rc;                          // :121, u1's halos
-  if ((rc = launch_correct_vel(c, c->is_forced[0] != 0))) return rc;  // :145 (+ mean of :149)
-  if (c->is_forced[0] && (rc = launch_add_force_u(c))) return rc;     // :149
-  return launch_bc_vel(c, 0);                                          // :153
+// The last step of a run: projection and forcing, then the boundary updates
+// (bc: launch_bc_vel's which).
+int finish_run(pll_context* c, int bc) {
+  const int rc = launch_correct_vel(c, true);  // src/main.cc:145-149
+  return rc ? rc : launch_bc_vel(c, bc);       // :153 (and :121)
 }
 
-// src/main.cc:141-153 after the pressure solve.
+// src/main.cc:145-153 after the pressure solve.
 int finish_step(pll_context* c) {
   int rc;
-  if ((rc = launch_bc_p(c))) return rc;                // :141
   if ((rc = launch_correct_vel(c, false))) return rc;  // :145
-  if ((rc = launch_force(c))) return rc;               // :149
-  return launch_bc_vel(c, 0);                          // :153
+  if ((rc = launch_force(c))) return rc;        // :149
+  return launch_bc_vel(c, 0);                   // :153
 }
 
 }  // namespace

@@ -149,6 +149,7 @@ struct pll_context {
   double* d_partial = nullptr;
   long npartial = 0;
   int mean_chunks = 1;
+  long mean_pending = 0;  // partials of the bulk mean that the next transform adds up
   double* d_scalar = nullptr;  // [0..2] means, [3..5] forces, [6..] scratch
   void* d_red = nullptr;       // check-reduction scratch
   long nred = 0;
@@ -230,20 +231,20 @@ int launch_rk_closure(pll_context* c, int stage, int fold = 0, int corr = 0, int
 // the closure stages' bulk-mean partials fit d_partial (the fused step sequence)
 bool closure_fused_available(const pll_context* c);
 // forceVel's bulk mean of u and its force from n FP64 block partials in
-// d_partial, into d_scalar[0] and d_scalar[3] (k_stencil.hip)
-int launch_force_from_partials(pll_context* c, long n);
+// d_partial, into d_scalar[0] and d_scalar[3]: left to the forward x transform
+// with calcRHS, which follows every stage 2 that sums partials
+int force_from_partials(pll_context* c, long n);
 
 int rk_setup(pll_context* c);  // per-plane coefficients of the stages
 int launch_calc_rhs(pll_context* c);
 // Both RK stages of a step inside a run, the previous step's projection,
 // forcing and boundary update applied on load; u1out: u1 is left in its arrays.
 int launch_rk12(pll_context* c, int acc, int u1out);
-// with_mean: also reduce the bulk mean of the corrected u and store the force
-// of u (vel_force[0] - mean) on the device.
-int launch_correct_vel(pll_context* c, bool with_mean);
-int launch_add_force_u(pll_context* c);
+// with_force: the force that is on the device is added as well (forceVel)
+int launch_correct_vel(pll_context* c, bool with_force);
 int launch_mean(pll_context* c, int field, double nxg, double nyg, double* d_out);
 int launch_force(pll_context* c);
+// which: 0 u, v, w; 1 u1, v1, w1; 2 both
 int launch_bc_vel(pll_context* c, int which, int walls_only = 0);
 int launch_bc_p(pll_context* c);
 int launch_add_scalar(pll_context* c, int field, double value);
@@ -257,9 +258,10 @@ int launch_check_nan(pll_context* c, int field, int* passed);
 // transforms and the tridiagonal solve (k_fft.hip, k_trid.hip)
 int fft_setup(pll_context* c);
 int launch_fft_x_fwd(pll_context* c);
-// calcRHS fused into the forward x transform (reads u, v, w; p is not written)
+// calcRHS fused into the forward x transform (reads u, v, w; p is not written);
+// takes along the bulk mean that force_from_partials left
 int launch_fft_x_fwd_rhs(pll_context* c);
-// inverse x transform inside the step (x halos of p written with their periodic values)
+// inverse x transform inside the step (p's boundary update included)
 int launch_fft_x_bwd_step(pll_context* c);
 int launch_fft_x_bwd(pll_context* c);
 int launch_fft_y_fwd(pll_context* c);
@@ -270,7 +272,7 @@ int launch_trid(pll_context* c);
 int launch_trid_step(pll_context* c);
 // The pressure solve of the step (src/mod_poisson_solver.cc:454-510) from p
 // (or, with rhs, from calcRHS computed in the x transform's loads) back to p
-// with its periodic x halos.
+// with its boundary update.
 int launch_poisson_step(pll_context* c, bool rhs);
 
 }  // namespace pll
