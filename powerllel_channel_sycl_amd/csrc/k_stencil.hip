@@ -38,8 +38,8 @@ struct PlaneAcc {
   }
 };
 
-// The momentum operator with fewer operations, scaled by S (dt in stage 1, dt/2
-// in stage 2): algebraically equal to S*(visc - conv) of tendency_z, with the
+// The momentum operator with fewer operations, scaled by S = dt (stage 2 halves
+// its result): algebraically equal to S*(visc - conv) of tendency_z, with the
 // mesh factors gathered into per-plane coefficients (RkCoef), the viscous terms
 // written as second differences and products fused into FMAs: about 85
 // operations for the three components instead of 150.  It rounds differently
@@ -173,9 +173,8 @@ template <typename T>
 struct RkParam {
   MeshT<T> m;
   T dxi, dyi, rei, dt, ucrf, dtdxi, dtdyi, bc_u;
-  const RkCoef<T>* coef1;
-  const RkCoef<T>* coef2;
-  RkUniform<T> cu1, cu2;
+  const RkCoef<T>* coef;  // tendency_fast's, scaled by dt
+  RkUniform<T> cu;
 };
 
 // What a thread of k_rk12 carries up its column from one plane to the next:
@@ -187,11 +186,10 @@ struct ZCarry {
   T u, v, w;
 };
 
-template <typename T, int STAGE, class A>
+template <typename T, class A>
 __device__ __forceinline__ ZCarry<T> carry_start(const A& U, const A& V, const A& W,
                                                  const RkParam<T>& q, int k) {
-  return ZCarry<T>{zconv_lower(U, V, W, load_coef(STAGE == 1 ? q.coef1 : q.coef2, k)),
-                   U(0, 0, -1), V(0, 0, -1), W(0, 0, -1)};
+  return ZCarry<T>{zconv_lower(U, V, W, load_coef(q.coef, k)), U(0, 0, -1), V(0, 0, -1), W(0, 0, -1)};
 }
 
 // A stencil accessor whose value below the centre is carried in a register.
@@ -204,16 +202,16 @@ struct CarryAcc {
   }
 };
 
-// Stage 1: o = s + dt*F(s); stage 2: o = (s + old)/2 + dt/2*F(s), with the
+// Stage 1: o = s + dt*F(s); stage 2: o = ((s + old) + dt*F(s))/2, with the
 // carry replaced by the next plane's.
 template <typename T, int STAGE, bool CRF, int SX>
 __device__ __forceinline__ void stage_update(const PlaneAcc<T, SX>& U, const PlaneAcc<T, SX>& V,
                                              const PlaneAcc<T, SX>& W, const RkParam<T>& q, int k,
                                              T ou, T ov, T ow, ZCarry<T>& z, T& o1, T& o2, T& o3) {
-  const RkCoef<T> cq = load_coef(STAGE == 1 ? q.coef1 : q.coef2, k);
+  const RkCoef<T> cq = load_coef(q.coef, k);
   const CarryAcc<T, SX> Uc{U, z.u}, Vc{V, z.v}, Wc{W, z.w};
   T iu, iv, iw;
-  tendency_fast<CRF>(Uc, Vc, Wc, cq, STAGE == 1 ? q.cu1 : q.cu2, iu, iv, iw, z.z);
+  tendency_fast<CRF>(Uc, Vc, Wc, cq, q.cu, iu, iv, iw, z.z);
   z.u = U(0, 0, 0);
   z.v = V(0, 0, 0);
   z.w = W(0, 0, 0);
@@ -222,9 +220,9 @@ __device__ __forceinline__ void stage_update(const PlaneAcc<T, SX>& U, const Pla
     o2 = z.v + iv;
     o3 = z.w + iw;
   } else {
-    o1 = (z.u + ou) * T(0.5) + iu;
-    o2 = (z.v + ov) * T(0.5) + iv;
-    o3 = (z.w + ow) * T(0.5) + iw;
+    o1 = ((z.u + ou) + iu) * T(0.5);
+    o2 = ((z.v + ov) + iv) * T(0.5);
+    o3 = ((z.w + ow) + iw) * T(0.5);
   }
 }
 
@@ -346,13 +344,11 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
   int sm = 0, s0 = 1, sp = 2;
   const int c = (ty + 1) * SX + tx + 1;
   ZConv<T> zc{};  // the carried lower-face convective products of the thread's column
-  const RkCoef<T>* coef = STAGE == 1 ? q0.coef1 : q0.coef2;
-  const RkUniform<T> cu = STAGE == 1 ? q0.cu1 : q0.cu2;
   if (active) {
     const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
     const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
     const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
-    zc = zconv_lower(U, V, W, load_coef(coef, k0));
+    zc = zconv_lower(U, V, W, load_coef(q0.coef, k0));
   }
   for (int k = k0; k <= k1; ++k) {
     const bool more = k + 2 <= k1 + 1;
@@ -368,18 +364,18 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
       const PlaneAcc<T, SX> U{sh[0][sm], sh[0][s0], sh[0][sp], c};
       const PlaneAcc<T, SX> V{sh[1][sm], sh[1][s0], sh[1][sp], c};
       const PlaneAcc<T, SX> W{sh[2][sm], sh[2][s0], sh[2][sp], c};
-      const RkCoef<T> q = load_coef(coef, k);
+      const RkCoef<T> q = load_coef(q0.coef, k);
       float iu, iv, iw;
-      tendency_fast<CRF>(U, V, W, q, cu, iu, iv, iw, zc);
+      tendency_fast<CRF>(U, V, W, q, q0.cu, iu, iv, iw, zc);
       if (STAGE == 1) {
         du[a] = U(0, 0, 0) + iu;
         dv[a] = V(0, 0, 0) + iv;
         dw[a] = W(0, 0, 0) + iw;
       } else {
-        const T nu = (U(0, 0, 0) + ou) * 0.5f + iu;
+        const T nu = ((U(0, 0, 0) + ou) + iu) * 0.5f;
         du[a] = nu;
-        dv[a] = (V(0, 0, 0) + ov) * 0.5f + iv;
-        dw[a] = (W(0, 0, 0) + ow) * 0.5f + iw;
+        dv[a] = ((V(0, 0, 0) + ov) + iv) * 0.5f;
+        dw[a] = ((W(0, 0, 0) + ow) + iw) * 0.5f;
         if (acc) msum += (double)nu * uniform_load(dzflzi, k);
       }
     }
@@ -561,9 +557,9 @@ __global__ __launch_bounds__(kRkTx * kLateTy, 4) void k_rk_late(
 }
 
 // Tile rows of k_rk12: one block of them fills a CU either way.  FP64 12 (160
-// VGPRs: three waves per SIMD; 8 and 10 rows ran 3021 and 2679 against 2348 us
-// at 768x384x384, 16 rows spill), FP32 16 (1302 against 1312 us with 8 and 1440
-// with 12; 6934 against 7111 us with 8 at 1536x768x512).
+// VGPRs: three waves per SIMD; with two barriers a plane 8 and 10 rows ran 3021
+// and 2679 against 2348 us at 768x384x384, 16 rows spill), FP32 16 (1302 against
+// 1312 us with 8 and 1440 with 12; 6934 against 7111 us with 8 at 1536x768x512).
 template <typename T>
 constexpr int kRk12Ty() {
   return std::is_same<T, double>::value ? 12 : 16;
@@ -576,8 +572,8 @@ constexpr int kRk12Slots = 256;  // blocks of k_rk12 that run at once: one per C
 // load as in the separate stage 1 (fold and corr).  A block owns a 64 x TY
 // tile of stage-2 points and marches a chunk of k planes.  Stage 1 runs on the
 // tile plus a one-cell ring (each thread its tile point, the first threads one
-// ring cell more) from a two-plane LDS ring of the loaded source (tile plus two
-// cells); its result u1 goes to a second two-plane LDS ring and, except on the
+// ring cell more) from an LDS ring of the loaded source (tile plus two
+// cells); its result u1 goes to a second LDS ring and, except on the
 // last step of a run (U1OUT), never to HBM.  The u1 values on the ring are
 // stage 1 at the periodic position -- the x/y boundary update of u1 -- and the
 // planes 0 and nz+1 of u1 and w1 on plane nz follow the boundary rules
@@ -587,28 +583,31 @@ constexpr int kRk12Slots = 256;  // blocks of k_rk12 that run at once: one per C
 // still read the source.  With `acc` the block sums the new u times dzflzi(k)
 // in FP64 into partial[block].
 //
-// Two planes suffice in each ring because the carry holds what plane k-1 would
-// be read for.  The fetch only issues the loads of a plane; the projection,
-// forcing and boundary rules apply at its commit, after stage 2 of the plane
-// below has been computed, and stage 2's results are stored after the commit:
+// One barrier per plane: in iteration q a wave runs stage 1 on plane q, stage 2
+// on plane q-2 (its neighbours' u1 of q-1 is behind the last barrier) and the
+// commit of source plane q+2, so the waves of a block drift apart within it and
+// one's LDS reads overlap another's arithmetic.  The carry holds what plane k-1
+// would be read for, so each ring is two planes and the one being written.  The
+// fetch only issues the loads of a plane; the projection, forcing and boundary
+// rules apply at its commit, and stage 2's results are stored after the commit:
 // arithmetic on the loaded values in the fetch, or stores ahead of the commit,
 // would make a wave wait there.
 //
-// Bound by latency between its two barriers per plane, at one block per CU: per
-// point about 240 (FP64) VALU operations and 60 LDS reads, each near 0.9 ms of
-// pure issue at 768x384x384, beside 56 B of HBM traffic (1.3 ms).  Measured there,
-// FP64: 2348 us for both stages against 1646 + 2331 us for the two kernels it
-// replaces (stage 2 with calcRHS; calcRHS in the transform's loads costs 440 us
-// more there), 141 against 121 + 176 us at 256x192x128.  The reference's
-// operation order instead of tendency_fast took 3058 us.  FP32: 1302 us, 1456
-// with three planes in each ring and 8 rows; 230 against 309 us at 384x256x192,
-// half of which is the chunk rule of rk12_grid.
+// Bound by issue and LDS together at one block per CU: FP64 at 768x384x384 keeps
+// the VALU 44 % and the LDS 52 % busy at three waves per SIMD, with 56 B a point
+// of HBM traffic (2.8 TB/s).  2229 us for both stages there against 1646 + 2331
+// us for the two kernels it replaces (stage 2 with calcRHS; calcRHS in the
+// transform's loads costs 440 us more); 2348 us with two barriers a plane, 3058
+// with the reference's operation order as well.  135 us against 121 + 176 at
+// 256x192x128.  FP32: 1243 us (1456 with 8 rows, two barriers and
+// coefficients loaded per lane), 222 against 309 us at 384x256x192, half of which is
+// the chunk rule of rk12_grid.
 template <typename T, int TY, bool U1OUT, bool CRF>
 __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
     Geom g, const T* __restrict__ su, const T* __restrict__ sv, const T* __restrict__ sw,
     const T* __restrict__ pp, T* __restrict__ du, T* __restrict__ dv, T* __restrict__ dw,
     T* __restrict__ u1, T* __restrict__ v1, T* __restrict__ w1, RkParam<T> q0,
-    const double* __restrict__ force, int forced_mask, int kchunk, int ntx, int nty, int acc,
+    const double* __restrict__ force, int kchunk, int ntx, int nty, int acc,
     const double* __restrict__ dzflzi, double* __restrict__ partial) {
   constexpr int TX = kRkTx, NT = TX * TY;
   constexpr int RX = TX + 2, RY = TY + 2, RPL = RX * RY;  // u1 region: tile + 1
@@ -616,9 +615,9 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   constexpr int NPF = (UPL + NT - 1) / NT;
   constexpr int NRING = RPL - NT;  // region cells outside the tile
   static_assert(NRING == 2 * RX + 2 * TY && NRING <= NT, "one ring cell per thread");
-  __shared__ T ssrc[3][2][UPL];  // [field][plane & 1][cell]; cell (cx, cy) = (i0-1+cx, j0-1+cy)
+  __shared__ T ssrc[3][3][UPL];  // [field][plane % 3][cell]; cell (cx, cy) = (i0-1+cx, j0-1+cy)
   __shared__ ZCarry<T> szb[NRING];  // the ring cells' carry: few threads have one
-  __shared__ T su1[3][2][RPL];   // [field][plane & 1][cell]; cell (rx, ry) = (i0+rx, j0+ry)
+  __shared__ T su1[3][3][RPL];   // [field][plane % 3][cell]; cell (rx, ry) = (i0+rx, j0+ry)
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
   const int ti = (int)(b % (unsigned)ntx), tj = (int)((b / (unsigned)ntx) % (unsigned)nty);
   const int kc = (int)(b / (unsigned)(ntx * nty));
@@ -627,9 +626,7 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   const int t = threadIdx.x, tx = t % TX, ty = t / TX;
   const int i = i0 + tx + 1, j = j0 + ty + 1;
   const bool active = i <= g.nx && j <= g.ny;
-  const bool fu = forced_mask & 1, fv = forced_mask & 2, fw = forced_mask & 4;
-  const T f_u = fu ? (T)force[0] : T(0), f_v = fv ? (T)force[1] : T(0),
-          f_w = fw ? (T)force[2] : T(0);
+  const T f_u = force ? (T)force[0] : T(0);
   if (k0 > k1) {
     if (acc && t == 0) partial[b] = 0.0;
     return;
@@ -659,9 +656,9 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
         rpt[n] = pp[a + g.sxy];
       }
   };
-  auto commit = [&](int kk) {
+  auto commit = [&](int kk, int slot) {
     const bool ghost = kk == 0 || kk == g.nz + 1;
-    const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk, slot = kk & 1;
+    const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
     const bool wzero = kk == 0 || kk >= g.nz;
     const T dzci = uniform_load(q0.m.dzc_inv, ks);
 #pragma unroll
@@ -672,9 +669,7 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
         T qv = rv[n] - (rpn[n] - p0) * q0.dtdyi;
         // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
         T qw = rw[n] - (rpt[n] - p0) * q0.dt * dzci;
-        if (fu) qu = qu + f_u;
-        if (fv) qv = qv + f_v;
-        if (fw) qw = qw + f_w;
+        qu = qu + f_u;
         if (wzero) qw = T(0);
         if (ghost) {
           qu = T(2) * q0.bc_u - qu;  // src/mod_updateBound.cc:92,123
@@ -706,56 +701,61 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   const int rb = by * RX + bx;
   const int ca = (ty + 2) * UX + tx + 2, cb = (by + 1) * UX + bx + 1;  // in the source ring
   const int qs = max(k0 - 1, 1), qe = k1 + 1;  // u1 planes formed: stage 1 up to nz, rules at nz+1
-  auto src = [&](int f, int q, int c) {
-    return PlaneAcc<T, UX>{ssrc[f][(q + 1) & 1], ssrc[f][q & 1], ssrc[f][(q + 1) & 1], c};
+  // stencil accessors: centre plane in slot z, the plane above in slot p
+  auto src = [&](int f, int z, int p, int c) {
+    return PlaneAcc<T, UX>{ssrc[f][z], ssrc[f][z], ssrc[f][p], c};
   };
-  auto reg = [&](int f, int q, int c) {
-    return PlaneAcc<T, RX>{su1[f][(q + 1) & 1], su1[f][q & 1], su1[f][(q + 1) & 1], c};
+  auto reg = [&](int f, int z, int p) {
+    return PlaneAcc<T, RX>{su1[f][z], su1[f][z], su1[f][p], ra};
   };
+  // slots of planes q, q+1 and q+2 (= q-1) of either ring, at q = qs
+  int s0 = 0, s1 = 1, s2 = 2;
   fetch(qs - 1);
-  commit(qs - 1);
+  commit(qs - 1, s2);
   fetch(qs);
-  commit(qs);
+  commit(qs, s0);
   fetch(qs + 1);
+  commit(qs + 1, s1);
   __syncthreads();
-  // the carries of the first plane, while plane qs-1 is in the slot of qs+1
   ZCarry<T> za{}, z2{};
-  za = carry_start<T, 1>(src(0, qs, ca), src(1, qs, ca), src(2, qs, ca), q0, qs);
-  if (has_b) szb[t] = carry_start<T, 1>(src(0, qs, cb), src(1, qs, cb), src(2, qs, cb), q0, qs);
-  __syncthreads();
-  commit(qs + 1);
-  __syncthreads();
-  // u1 of plane q at region cell r; with q == 1 also plane 0 by the rules
+  {
+    auto below = [&](int f, int c) { return PlaneAcc<T, UX>{ssrc[f][s2], ssrc[f][s0], ssrc[f][s0], c}; };
+    za = carry_start<T>(below(0, ca), below(1, ca), below(2, ca), q0, qs);
+    if (has_b) szb[t] = carry_start<T>(below(0, cb), below(1, cb), below(2, cb), q0, qs);
+  }
+  __syncthreads();  // plane qs-1's slot is rewritten by the first commit
+  // u1 of plane q (slot s0) at region cell r; with q == 1 also plane 0 by the rules
   auto put1 = [&](int q, int r, T o1, T o2, T o3) {
-    const int s = q & 1;
-    su1[0][s][r] = o1;
-    su1[1][s][r] = o2;
-    su1[2][s][r] = o3;
+    if (q == g.nz) o3 = T(0);
+    su1[0][s0][r] = o1;
+    su1[1][s0][r] = o2;
+    su1[2][s0][r] = o3;
     if (q == 1) {
-      su1[0][0][r] = T(2) * q0.bc_u - o1;
-      su1[1][0][r] = T(2) * T(0) - o2;
-      su1[2][0][r] = T(0);
+      su1[0][s2][r] = T(2) * q0.bc_u - o1;
+      su1[1][s2][r] = T(2) * T(0) - o2;
+      su1[2][s2][r] = T(0);
     }
   };
   // plane nz+1 of u1 by the rules from plane nz (the same thread wrote cell r of it)
   auto ghost_top = [&](int r) {
-    const int s = g.nz & 1, d = s ^ 1;
-    su1[0][d][r] = T(2) * q0.bc_u - su1[0][s][r];
-    su1[1][d][r] = T(2) * T(0) - su1[1][s][r];
-    su1[2][d][r] = T(0);
+    su1[0][s0][r] = T(2) * q0.bc_u - su1[0][s2][r];
+    su1[1][s0][r] = T(2) * T(0) - su1[1][s2][r];
+    su1[2][s0][r] = T(0);
   };
   double msum = 0.0;
-  for (int q = qs; q <= qe; ++q) {
+  T nextu = T(0), nextv = T(0), nextw = T(0);  // the source at the tile point of plane q-2
+  for (int q = qs; q <= qe + 1; ++q) {
+    const int k = q - 2;  // stage-2 plane
     // the next iteration's stage 1 reads source planes q+1, q+2
-    const bool more = q + 1 <= qe && q + 1 <= g.nz;
-    const int k = q - 1;  // stage-2 plane
-    const bool s2 = k >= k0;
-    const T pu = za.u, pv = za.v, pw = za.w;  // the source at the tile point of plane k
-    if (q <= g.nz) {
+    const bool more = q < qe && q < g.nz;
+    const T pu = nextu, pv = nextv, pw = nextw;
+    nextu = za.u;
+    nextv = za.v;
+    nextw = za.w;
+    if (q <= qe && q <= g.nz) {
       T o1, o2, o3;
-      stage_update<T, 1, CRF, UX>(src(0, q, ca), src(1, q, ca), src(2, q, ca), q0, q, T(0), T(0), T(0),
-                             za, o1, o2, o3);
-      if (q == g.nz) o3 = T(0);
+      stage_update<T, 1, CRF, UX>(src(0, s0, s1, ca), src(1, s0, s1, ca), src(2, s0, s1, ca), q0,
+                                  q, T(0), T(0), T(0), za, o1, o2, o3);
       put1(q, ra, o1, o2, o3);
       if (U1OUT && active && q >= k0 && q <= k1) {
         const long a = g.idx(i, j, q);
@@ -765,36 +765,40 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
       }
       if (has_b) {
         ZCarry<T> zb = szb[t];
-        stage_update<T, 1, CRF, UX>(src(0, q, cb), src(1, q, cb), src(2, q, cb), q0, q, T(0), T(0),
-                                    T(0), zb, o1, o2, o3);
+        stage_update<T, 1, CRF, UX>(src(0, s0, s1, cb), src(1, s0, s1, cb), src(2, s0, s1, cb), q0,
+                                    q, T(0), T(0), T(0), zb, o1, o2, o3);
         szb[t] = zb;
-        if (q == g.nz) o3 = T(0);
         put1(q, rb, o1, o2, o3);
       }
-    } else {
+    } else if (q == g.nz + 1) {
       ghost_top(ra);
       if (has_b) ghost_top(rb);
     }
-    __syncthreads();
     // fetched here rather than before stage 1: its registers are then not
     // live across both stages
     if (more) fetch(q + 2);
     T nu = T(0), nv = T(0), nw = T(0);
-    if (s2 && active) {
-      stage_update<T, 2, CRF, RX>(reg(0, k, ra), reg(1, k, ra), reg(2, k, ra), q0, k, pu, pv, pw, z2,
-                             nu, nv, nw);
+    if (k >= k0 && active) {
+      // u1 planes k = q-2 and q-1 are in the slots of q+1 and q+2
+      stage_update<T, 2, CRF, RX>(reg(0, s1, s2), reg(1, s1, s2), reg(2, s1, s2), q0, k, pu, pv,
+                                  pw, z2, nu, nv, nw);
       if (acc) msum += (double)nu * uniform_load(dzflzi, k);
-    } else if (q == k0 && active) {
-      z2 = carry_start<T, 2>(reg(0, k0, ra), reg(1, k0, ra), reg(2, k0, ra), q0, k0);
+    } else if (k == k0 - 1 && active) {
+      auto below = [&](int f) { return PlaneAcc<T, RX>{su1[f][s1], su1[f][s2], su1[f][s2], ra}; };
+      z2 = carry_start<T>(below(0), below(1), below(2), q0, k0);
     }
-    if (more) commit(q + 2);
-    if (s2 && active) {
+    if (more) commit(q + 2, s2);
+    if (k >= k0 && active) {
       const long a = g.idx(i, j, k);
       du[a] = nu;
       dv[a] = nv;
       dw[a] = nw;
     }
     __syncthreads();
+    const int r = s0;
+    s0 = s1;
+    s1 = s2;
+    s2 = r;
   }
   static_assert(sizeof(ssrc) >= NT * sizeof(double), "reduction scratch");
   if (acc) block_partial<NT>(reinterpret_cast<double*>(&ssrc[0][0][0]), msum, partial, b);
@@ -1255,11 +1259,10 @@ inline int forced_mask(const pll_context* c) {
   return (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0) | (c->is_forced[2] ? 4 : 0);
 }
 
-// Coefficients of tendency_fast for stage `stage` (S = dt or dt/2), computed in
-// FP64 and rounded once.
+// Coefficients of tendency_fast (S = dt), computed in FP64 and rounded once.
 template <typename T>
-RkUniform<T> rk_uniform(const pll_context* c, int stage) {
-  const double S = stage == 1 ? c->dt : 0.5 * c->dt;
+RkUniform<T> rk_uniform(const pll_context* c) {
+  const double S = c->dt;
   return RkUniform<T>{(T)(S * 0.25 * c->dx_inv), (T)(S * 0.25 * c->dy_inv),
                       (T)(S * c->re_inv * c->dx_inv * c->dx_inv),
                       (T)(S * c->re_inv * c->dy_inv * c->dy_inv),
@@ -1269,30 +1272,28 @@ RkUniform<T> rk_uniform(const pll_context* c, int stage) {
 template <typename T>
 int rk_coef_setup(pll_context* c) {
   const int nz = c->g.nz;
-  std::vector<RkCoef<T>> h(2 * (size_t)(nz + 2));
-  for (int stage = 1; stage <= 2; ++stage) {
-    const double S = stage == 1 ? c->dt : 0.5 * c->dt, rei = c->re_inv;
-    for (int k = 1; k <= nz; ++k) {
-      const double* f = c->dzf.data();
-      const double* fi = c->dzf_inv.data();
-      const double* ci = c->dzc_inv.data();
-      RkCoef<T>& q = h[(stage - 1) * (size_t)(nz + 2) + k];
-      q.a1 = (T)(f[k + 1] * ci[k]);
-      q.a2 = (T)(f[k] * ci[k]);
-      q.b1 = (T)(f[k - 1] * ci[k - 1]);
-      q.b2 = (T)(f[k] * ci[k - 1]);
-      q.zuv = (T)(S * 0.25 * fi[k]);
-      q.cp = (T)(S * rei * ci[k] * fi[k]);
-      q.cm = (T)(S * rei * ci[k - 1] * fi[k]);
-      q.zw = (T)(S * 0.25 * ci[k]);
-      q.dp = (T)(S * rei * fi[k + 1] * ci[k]);
-      q.dm = (T)(S * rei * fi[k] * ci[k]);
-      // the diagonal from the rounded coefficients (one rounding off their sum)
-      const RkUniform<T> cu = rk_uniform<T>(c, stage);
-      const double vxy = 2.0 * (double)cu.vx + 2.0 * (double)cu.vy;
-      q.cdu = (T)(vxy + (double)q.cp + (double)q.cm);
-      q.cdw = (T)(vxy + (double)q.dp + (double)q.dm);
-    }
+  std::vector<RkCoef<T>> h((size_t)(nz + 2));
+  const double S = c->dt, rei = c->re_inv;
+  for (int k = 1; k <= nz; ++k) {
+    const double* f = c->dzf.data();
+    const double* fi = c->dzf_inv.data();
+    const double* ci = c->dzc_inv.data();
+    RkCoef<T>& q = h[k];
+    q.a1 = (T)(f[k + 1] * ci[k]);
+    q.a2 = (T)(f[k] * ci[k]);
+    q.b1 = (T)(f[k - 1] * ci[k - 1]);
+    q.b2 = (T)(f[k] * ci[k - 1]);
+    q.zuv = (T)(S * 0.25 * fi[k]);
+    q.cp = (T)(S * rei * ci[k] * fi[k]);
+    q.cm = (T)(S * rei * ci[k - 1] * fi[k]);
+    q.zw = (T)(S * 0.25 * ci[k]);
+    q.dp = (T)(S * rei * fi[k + 1] * ci[k]);
+    q.dm = (T)(S * rei * fi[k] * ci[k]);
+    // the diagonal from the rounded coefficients (one rounding off their sum)
+    const RkUniform<T> cu = rk_uniform<T>(c);
+    const double vxy = 2.0 * (double)cu.vx + 2.0 * (double)cu.vy;
+    q.cdu = (T)(vxy + (double)q.cp + (double)q.cm);
+    q.cdw = (T)(vxy + (double)q.dp + (double)q.dm);
   }
   PLL_HIP_TRY(ctx_malloc(c, &c->d_rkcoef, h.size() * sizeof(RkCoef<T>)));
   PLL_HIP_TRY(hipMemcpy(c->d_rkcoef, h.data(), h.size() * sizeof(RkCoef<T>), hipMemcpyHostToDevice));
@@ -1301,11 +1302,10 @@ int rk_coef_setup(pll_context* c) {
 
 template <typename T>
 RkParam<T> rk_param(const pll_context* c) {
-  const RkCoef<T>* coef = static_cast<const RkCoef<T>*>(c->d_rkcoef);
   return RkParam<T>{mesh_of<T>(c), (T)c->dx_inv, (T)c->dy_inv, (T)c->re_inv, (T)c->dt, (T)c->u_crf,
                     (T)(c->dt * c->dx_inv), (T)(c->dt * c->dy_inv),  // src/mod_calcVel.cc:256-258
                     (T)(0.0 - c->u_crf),                             // src/mod_updateBound.cc:80
-                    coef, coef + (c->g.nz + 2), rk_uniform<T>(c, 1), rk_uniform<T>(c, 2)};
+                    static_cast<const RkCoef<T>*>(c->d_rkcoef), rk_uniform<T>(c)};
 }
 
 template <typename T>
@@ -1381,7 +1381,7 @@ int rk12_t(pll_context* c, int acc, int u1out) {
                        F<T>(c, PLL_W), F<T>(c, PLL_P), static_cast<T*>(c->fld_alt[0]),
                        static_cast<T*>(c->fld_alt[1]), static_cast<T*>(c->fld_alt[2]),
                        F<T>(c, PLL_U1), F<T>(c, PLL_V1), F<T>(c, PLL_W1), rk_param<T>(c),
-                       c->d_scalar + 3, forced_mask(c), t.kchunk, t.ntx, t.nty, acc,
+                       c->is_forced[0] ? c->d_scalar + 3 : nullptr, t.kchunk, t.ntx, t.nty, acc,
                        c->d_mesh64 + 3 * (c->g.nz + 2), c->d_partial);
   }
   PLL_HIP_TRY(hipGetLastError());

@@ -121,7 +121,7 @@ struct pll_context {
   int is_forced[3];
 
   void* d_mesh = nullptr;      // 4*(nz+2) in field precision: dzf, dzf_inv, dzc_inv, dzflzi
-  void* d_rkcoef = nullptr;    // tendency_fast coefficients, 2 stages x (nz+2)
+  void* d_rkcoef = nullptr;    // tendency_fast coefficients, nz+2 planes
   double* d_mesh64 = nullptr;  // same, FP64
 
   // tridiagonal solve: a, c (nz), pre-factored pivot table [k][cy][cx]
