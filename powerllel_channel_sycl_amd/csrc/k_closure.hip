@@ -3,24 +3,20 @@
 // weights and FP32 accumulation on the MFMA units of gfx950, its training
 // (forward, backward, Adam) and its inference.  The reference has no closure.
 //
-// Tiles.  A wave owns 32 samples at a time.  The hidden layers are
+// Tiles.  A wave owns 32 samples at a time.  The layers are
 // v_mfma_f32_32x32x16_bf16 products: A is 32 x 16 (lane l holds row l%32,
 // k = 8*(l/32) .. +7), B is 16 x 32 (lane l holds column l%32, the same k),
 // D is 32 x 32 FP32 (lane l holds column l%32, rows 8*(j/4) + 4*(l/32) + j%4
-// for j = 0..15).  In training and batch inference activations pass between
-// layers through LDS as BF16 (the A operand of the next product), the output
-// layer is one more product with W3 in every B column, and the weight
-// gradients take both operands from the accumulator registers.  The closure
-// stage computes the layers transposed, entirely in registers, with the
-// output layer as BF16 dot products.  Rounding to BF16 is round-to-nearest-
-// even at fixed points -- the inputs, the weights, the activations h1 and h2
-// and the back-propagated deltas -- so a CPU restatement can follow it
-// exactly; only the FP32 summation order differs.
+// for j = 0..15).  Activations and deltas pass between the products in
+// registers (see "register-resident network" below).  Rounding to BF16 is
+// round-to-nearest-even at fixed points -- the inputs, the weights, the
+// activations h1 and h2 and the back-propagated deltas -- so a CPU restatement
+// can follow it exactly; only the FP32 summation order differs.
 //
 // Training is deterministic: each wave accumulates its gradient over its
-// tiles in registers, a block sums its waves' partials in LDS in wave order
-// and writes one partial, and two more levels sum the partials in a fixed
-// order, the last inside the Adam update.
+// tiles in registers, a block sums its waves' partials in LDS in a fixed order
+// and writes one partial, and one more kernel sums the partials in a fixed
+// order, in a training step with the Adam update.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -43,9 +39,9 @@ constexpr int kH = 64;    // hidden width
 // parameter vector (FP32 master): W1[16][64], b1[64], W2[64][64], b2[64], W3[64], b3
 constexpr int oW1 = 0, oB1 = oW1 + kInP * kH, oW2 = oB1 + kH, oB2 = oW2 + kH * kH,
               oW3 = oB2 + kH, oB3 = oW3 + kH, kNParam = oB3 + 1;
-constexpr int kWaves = 4;          // waves per block
-constexpr long kMaxWaves = 1024;   // training grid: one wave per SIMD (one partial per kWaves waves)
-constexpr int kRedChunk = 32;      // block partials summed per chunk in the first reduction level
+constexpr int kWaves = 4;          // waves per block of the closure stage's kernels
+constexpr int kMlpWaves = 8;       // waves per block of training and batch inference
+constexpr long kMaxWaves = 2048;   // their grid: two waves per SIMD (one partial per block)
 
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
@@ -80,360 +76,454 @@ struct Mlp {
   const uint16_t* w1;  // BF16 W1 [16][64]
   const uint16_t* w2;  // BF16 W2 [64][64]
   const uint16_t* w3;  // BF16 W3 [64]
-  // the same BF16 weights as each lane's B operand of the forward products,
-  // 8 values (16 bytes) per lane: b1[t][lane][e] = W1[8h + e][32t + c] and
-  // b2[t][kb][lane][e] = W2[16kb + 8h + e][32t + c], h = lane/32, c = lane%32
-  const uint16_t* b1;
-  const uint16_t* b2;
 };
 
-// Layout of the BF16 weight buffer: W1 | W2 | W3 | b1 | b2 (element offsets).
-constexpr int kWb1 = 0, kWb2 = kWb1 + kInP * kH, kWb3 = kWb2 + kH * kH, kWbB1 = kWb3 + kH,
-              kWbB2 = kWbB1 + 2 * 64 * 8, kWbLen = kWbB2 + 2 * 4 * 64 * 8;
-static_assert(kWbB1 % 8 == 0 && kWbB2 % 8 == 0, "operand copies start on 16-byte boundaries");
+// Layout of the BF16 weight buffer: W1 | W2 | W3 (element offsets).
+constexpr int kWb1 = 0, kWb2 = kWb1 + kInP * kH, kWb3 = kWb2 + kH * kH, kWbLen = kWb3 + kH;
 
-// BF16 of parameter i (already computed as v) into the plain and operand copies.
+// BF16 of parameter i (already computed as v) into the weight copies.
 __device__ inline void store_bf16_weight(uint16_t* __restrict__ wb, int i, float v) {
   const uint16_t b = to_bf16(v);
-  if (i < oB1) {
-    const int r = (i - oW1) / kH, c = (i - oW1) % kH;
+  if (i < oB1)
     wb[kWb1 + i - oW1] = b;
-    const int t = c / 32, lane = 32 * ((r % 16) / 8) + c % 32;
-    wb[kWbB1 + (t * 64 + lane) * 8 + r % 8] = b;
-  } else if (i >= oW2 && i < oB2) {
-    const int r = (i - oW2) / kH, c = (i - oW2) % kH;
+  else if (i >= oW2 && i < oB2)
     wb[kWb2 + i - oW2] = b;
-    const int t = c / 32, kb = r / 16, lane = 32 * ((r % 16) / 8) + c % 32;
-    wb[kWbB2 + ((t * 4 + kb) * 64 + lane) * 8 + r % 8] = b;
-  } else if (i >= oW3 && i < oB3) {
+  else if (i >= oW3 && i < oB3)
     wb[kWb3 + i - oW3] = b;
-  }
 }
 
 // Orders a wave's LDS writes before its lanes' later LDS reads of them.  A
 // wave's LDS instructions execute in order, so this only has to keep the
-// compiler from moving memory operations across it: the training and predict
-// kernels share no LDS between waves and need no block barrier.
+// compiler from moving memory operations across it.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Per-wave LDS: X (32 x 16), h1, h2 and delta2 (32 x 64), all BF16.
-struct WaveLds {
-  uint16_t x[32][kInP];
-  uint16_t h1[32][kH];
-  uint16_t h2[32][kH];
-  uint16_t d2[32][kH];
-  float o[32];    // network output per sample
-  float g[32];    // dL/do per sample
-  float red[64];  // lane exchange
-};
+// ---- register-resident network ---------------------------------------------
+// A 32 x 32 accumulator leaves lane l (half h = l/32) with one column and the
+// 16 rows hid_unit(j, h) (+32 per row block).  Used as the next product's A or B
+// operand, packed eight at a time, its rows become that product's K: numbering
+// the k-slots (kb, h, e) of a product over the hidden units as unit_of(kb, h, e)
+// makes every lane's own results its next operand, with no LDS and no barrier
+// between the layers.
+//
+// The batch kernels run every hidden layer in both orientations (the matrix
+// cores have the room): hidden x samples, whose packed result is the operand
+// over the hidden units, and samples x hidden, from the same operand registers
+// with A and B exchanged, whose packed result is the operand over the samples
+// that the weight gradients take.  In either, lane l reads W2 fragments of one
+// form: index l%32 + 32t fixed, the eight units unit_of(kb, h, .) of the other.
+__device__ __forceinline__ int hid_unit(int j, int h) { return 8 * (j / 4) + 4 * h + (j % 4); }
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ inline bf16x8 load8(const uint16_t* p) {
+// Two FP32 values rounded to BF16 (nearest, ties to even) in one dword, lo | hi << 16.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
+}
+// BF16 of relu(lo), relu(hi), packed: a negative value rounds to a BF16 with
+// its sign bit set, which a 16-bit signed max against 0 clears to +0, so this
+// is the BF16 of max(x, 0) in two instructions for the pair.
+__device__ __forceinline__ uint32_t pack_relu_bf16(float lo, float hi) {
+  const s16x2 q = __builtin_bit_cast(s16x2, pack_bf16(lo, hi));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(q, (s16x2){0, 0}));
+}
+
+// hidden unit of k-slot (kb, h, e) of a product over the hidden units
+__device__ __forceinline__ int unit_of(int kb, int h, int e) {
+  return hid_unit(8 * (kb % 2) + e, h) + 32 * (kb / 2);
+}
+
+// The hidden biases b1 (lb[0..63]) and b2 (lb[64..127]) are read from LDS into
+// the accumulator rows of lane half h, row block t, when a tile starts: the
+// rows j = 4q .. 4q+3 are the consecutive units 8q + 4h + 32t .. +3.
+__device__ __forceinline__ f32x16 bias_rows(const float* lb, int h, int t) {
+  f32x16 c;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float4 v = *reinterpret_cast<const float4*>(lb + 8 * q + 4 * h + 32 * t);
+    c[4 * q] = v.x;
+    c[4 * q + 1] = v.y;
+    c[4 * q + 2] = v.z;
+    c[4 * q + 3] = v.w;
+  }
+  return c;
+}
+
+// BF16 of relu of accumulator elements j0 .. j0+7 as one MFMA operand.
+__device__ __forceinline__ bf16x8 pack8_relu(const f32x16& z, int j0) {
+  return __builtin_bit_cast(
+      bf16x8, (u32x4){pack_relu_bf16(z[j0], z[j0 + 1]), pack_relu_bf16(z[j0 + 2], z[j0 + 3]),
+                      pack_relu_bf16(z[j0 + 4], z[j0 + 5]), pack_relu_bf16(z[j0 + 6], z[j0 + 7])});
+}
+__device__ __forceinline__ bf16x8 pack8(const f32x16& v, int j0) {
+  return __builtin_bit_cast(
+      bf16x8, (u32x4){pack_bf16(v[j0], v[j0 + 1]), pack_bf16(v[j0 + 2], v[j0 + 3]),
+                      pack_bf16(v[j0 + 4], v[j0 + 5]), pack_bf16(v[j0 + 6], v[j0 + 7])});
+}
+__device__ __forceinline__ f32x16 splat16(float v) {
+  f32x16 r;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) r[j] = v;
+  return r;
+}
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// The network's operands of a batch block in LDS, loaded once: W2 fragments
+// (t, kb) of the forward products (columns l%32 + 32t, eight rows) and of the
+// backward one (rows l%32 + 32t, eight columns), the hidden biases, W3.
+template <bool TRAIN>
+struct NetLds {
+  u32x4 w2f[8][64];
+  u32x4 w2b[TRAIN ? 8 : 1][64];
+  float lb[2 * kH];
+  float w3[kH];
+};
+template <bool TRAIN>
+__device__ inline void load_net(const Mlp& w, NetLds<TRAIN>& N) {
+  static_assert(64 * kMlpWaves == 8 * 64, "one fragment per thread");
+  const int f = threadIdx.x / 64, lane = threadIdx.x % 64, t = f / 4, kb = f % 4;
+  const int c = lane % 32 + 32 * t, h = lane / 32;
+  bf16x8 vf, vb;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int u = unit_of(kb, h, e);
+    vf[e] = (short)w.w2[u * kH + c];
+    if (TRAIN) vb[e] = (short)w.w2[c * kH + u];
+  }
+  N.w2f[f][lane] = __builtin_bit_cast(u32x4, vf);
+  if (TRAIN) N.w2b[f][lane] = __builtin_bit_cast(u32x4, vb);
+  if (threadIdx.x < 2 * kH)
+    N.lb[threadIdx.x] = w.p[(threadIdx.x < kH ? oB1 : oB2 - kH) + threadIdx.x];
+  if (threadIdx.x < kH) N.w3[threadIdx.x] = from_bf16(w.w3[threadIdx.x]);
+}
+
+// This lane's eight features (8h .. 8h+7, zero past the last) of sample s.  The
+// feature array is only known to be aligned to its elements.
+struct Feat {
+  float v[8];
+};
+__device__ __forceinline__ Feat load_feat(const float* __restrict__ x, long s, int h) {
+  typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+  static_assert(kIn == 10, "eight features for one half of a wave, two for the other");
+  const f32x2u* p = reinterpret_cast<const f32x2u*>(x + s * kIn + 8 * h);
+  Feat f = {};
+  const f32x2u a = p[0];
+  f.v[0] = a[0];
+  f.v[1] = a[1];
+  if (h == 0) {
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+      const f32x2u b = p[q];
+      f.v[2 * q] = b[0];
+      f.v[2 * q + 1] = b[1];
+    }
+  }
+  return f;
+}
+__device__ __forceinline__ bf16x8 pack_feat(const Feat& f) {
+  return __builtin_bit_cast(bf16x8, (u32x4){pack_bf16(f.v[0], f.v[1]), pack_bf16(f.v[2], f.v[3]),
+                                            pack_bf16(f.v[4], f.v[5]), pack_bf16(f.v[6], f.v[7])});
+}
+// W1 fragment t: unit l%32 + 32t, features 8h .. 8h+7
+__device__ __forceinline__ bf16x8 w1_frag(const Mlp& w, int t, int lane) {
   bf16x8 v;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (short)p[e];
+  for (int e = 0; e < 8; ++e) v[e] = (short)w.w1[(8 * (lane / 32) + e) * kH + lane % 32 + 32 * t];
   return v;
 }
 
-// BF16 (nearest even) of accumulator elements j0 .. j0+7 as one MFMA operand.
-__device__ inline bf16x8 pack8_bf16(const f32x16& v, int j0) {
-  bf16x8 r;
+// Hidden layers, hidden x samples: h1 as the operand over the hidden units
+// (b1[kb]) and the pre-activations z2 of the second layer.
+template <bool TRAIN>
+__device__ __forceinline__ void forward_regs(const NetLds<TRAIN>& N, const bf16x8 a1[2], bf16x8 xb,
+                                             int lane, bf16x8 b1[4], f32x16 z2[2]) {
+  const int h = lane / 32;
+  f32x16 z1[2];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) r[e] = (short)to_bf16(v[j0 + e]);
-  return r;
+  for (int t = 0; t < 2; ++t) z1[t] = mfma(a1[t], xb, bias_rows(N.lb, h, t));
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) b1[kb] = pack8_relu(z1[kb / 2], 8 * (kb % 2));
+  z2[0] = bias_rows(N.lb + kH, h, 0);
+  z2[1] = bias_rows(N.lb + kH, h, 1);
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      z2[t] = mfma(__builtin_bit_cast(bf16x8, N.w2f[4 * t + kb][lane]), b1[kb], z2[t]);
 }
 
-// D-layout row of accumulator element j for this lane.
-__device__ inline int drow(int j, int lane) { return 8 * (j / 4) + 4 * (lane / 32) + (j % 4); }
-
-// X of one 32-sample tile from a feature array (rows beyond n are zero).
-template <class L_>
-__device__ inline void stage_x(const float* __restrict__ x, long m0, long n, L_& L, int lane) {
-  for (int e = lane; e < 32 * kInP; e += 64) {
-    const int m = e / kInP, k = e % kInP;
-    const long s = m0 + m;
-    L.x[m][k] = to_bf16((k < kIn && s < n) ? x[s * kIn + k] : 0.f);
-  }
+// The output o of the lane's sample, in both halves: BF16 h2 times BF16 W3
+// (packed pairs w3[t][q], the lane's rows), FP32 sum.
+__device__ __forceinline__ float output_regs(const f32x16 z2[2], const uint32_t w3[2][8], float b3) {
+  float part = 0.f;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      part = __builtin_amdgcn_fdot2_f32_bf16(
+          __builtin_bit_cast(bf16x2, pack_relu_bf16(z2[t][2 * q], z2[t][2 * q + 1])),
+          __builtin_bit_cast(bf16x2, w3[t][q]), part, false);
+  return part + __shfl_xor(part, 32) + b3;
+}
+__device__ __forceinline__ void load_w3(const Mlp& w, int h, uint32_t w3[2][8]) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      w3[t][q] = (uint32_t)w.w3[hid_unit(2 * q, h) + 32 * t] |
+                 ((uint32_t)w.w3[hid_unit(2 * q + 1, h) + 32 * t] << 16);
 }
 
-// Forward pass of one 32-sample tile whose BF16 features are in L.x (written
-// before the call by any lane of the wave): fills L.h1/h2, returns the ReLU
-// activations in D layout and, on lanes 0..31, the output o of sample lane.
-// Only the calling wave's LDS is used.
-template <class L_>
-__device__ inline void forward_tile(const Mlp& w, L_& L, int lane, f32x16 h1[2], f32x16 h2[2],
-                                    float& out_o) {
-  wave_lds_sync();
-  const int col = lane % 32, kh = 8 * (lane / 32);
-  // layer 1: h1 = relu(X W1 + b1)
-  const bf16x8 a1 = load8(&L.x[col][kh]);
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(w.b1 + (t * 64 + lane) * 8);
-    f32x16 acc = {};
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, acc, 0, 0, 0);
-    const float bias = w.p[oB1 + 32 * t + col];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float h = fmaxf(acc[j] + bias, 0.f);
-      acc[j] = h;
-      L.h1[drow(j, lane)][32 * t + col] = to_bf16(h);
-    }
-    h1[t] = acc;
+// Batch inference: out = softplus(o) of every sample.
+__global__ __launch_bounds__(64 * kMlpWaves, 2) void k_predict(Mlp w, const float* __restrict__ x,
+                                                               long n, float* __restrict__ out) {
+  __shared__ NetLds<false> N;
+  load_net<false>(w, N);
+  __syncthreads();
+  const int lane = threadIdx.x % 64;
+  const bf16x8 a1[2] = {w1_frag(w, 0, lane), w1_frag(w, 1, lane)};
+  uint32_t w3[2][8];
+  load_w3(w, lane / 32, w3);
+  const float b3 = w.p[oB3];
+  const long step = (long)gridDim.x * kMlpWaves * 32;
+  for (long m0 = ((long)blockIdx.x * kMlpWaves + threadIdx.x / 64) * 32; m0 < n; m0 += step) {
+    const long s = std::min(m0 + lane % 32, n - 1);
+    bf16x8 b1[4];
+    f32x16 z2[2];
+    forward_regs<false>(N, a1, pack_feat(load_feat(x, s, lane / 32)), lane, b1, z2);
+    const float o = output_regs(z2, w3, b3);
+    if (lane < 32 && m0 + lane < n) out[m0 + lane] = softplus(o);
   }
-  wave_lds_sync();
-  // layer 2: h2 = relu(h1 W2 + b2)
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    f32x16 acc = {};
-#pragma unroll
-    for (int kb = 0; kb < kH / 16; ++kb) {
-      const bf16x8 a = load8(&L.h1[col][16 * kb + kh]);
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(w.b2 + ((t * 4 + kb) * 64 + lane) * 8);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    const float bias = w.p[oB2 + 32 * t + col];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float h = fmaxf(acc[j] + bias, 0.f);
-      acc[j] = h;
-      L.h2[drow(j, lane)][32 * t + col] = to_bf16(h);
-    }
-    h2[t] = acc;
-  }
-  wave_lds_sync();
-  // output: o = h2 . W3 + b3 as one more product, B holding W3 in all 32
-  // columns (K = hidden units); column 0 goes back to lanes 0..31 through LDS
-  f32x16 acc = {};
-#pragma unroll
-  for (int kb = 0; kb < kH / 16; ++kb) {
-    const bf16x8 a = load8(&L.h2[col][16 * kb + kh]);
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(w.w3 + 16 * kb + kh);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-  }
-  if (col == 0)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) L.o[drow(j, lane)] = acc[j];
-  wave_lds_sync();
-  out_o = lane < 32 ? L.o[lane] + w.p[oB3] : 0.f;
 }
 
 // Training: one partial gradient (and loss sum) per block.  Loss = mean over
-// the n samples of (softplus(o) - y)^2.
-template <bool TRAIN>
-__global__ __launch_bounds__(64 * kWaves) void k_mlp(Mlp w, const float* __restrict__ x,
-                                                      const float* __restrict__ y, long n,
-                                                      float* __restrict__ out,
-                                                      float* __restrict__ partial,
-                                                      int tiles_per_wave) {
-  __shared__ WaveLds lds[kWaves];
-  __shared__ float bp[TRAIN ? kWaves : 1][kNParam + 1];  // the waves' partial gradients
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  WaveLds& L = lds[wave];
-  const long gw = (long)blockIdx.x * kWaves + wave;  // global wave index
-  const int col = lane % 32, kh = 8 * (lane / 32);
+// the n samples of (softplus(o) - y)^2.  Per 32-sample tile 41 products and
+// about 700 VALU operations (the ReLUs, masks and BF16 packing), which bound it
+// at two waves per SIMD.  393,216 samples: 34.6 us; 101 us for a form that passed
+// activations between the layers through LDS in two-byte writes (one wave per
+// SIMD, 140 KB of LDS a block).
+__global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float* __restrict__ x,
+                                                             const float* __restrict__ y, long n,
+                                                             float* __restrict__ partial) {
+  __shared__ NetLds<true> N;
+  __shared__ __align__(16) float gs[kMlpWaves][32];  // dL/do per sample of a wave's tile
+  __shared__ float bp[kMlpWaves / 2][kNParam + 1];   // the waves' partial gradients
+  load_net<true>(w, N);
+  __syncthreads();
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, col = lane % 32, h = lane / 32;
+  const bf16x8 a1[2] = {w1_frag(w, 0, lane), w1_frag(w, 1, lane)};
+  uint32_t w3[2][8];
+  load_w3(w, h, w3);
+  const float b3 = w.p[oB3], inv_n = 1.f / (float)n;
+  bf16x8 ident;  // feature x feature unit matrix, to turn X into samples x features
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ident[e] = (short)(8 * h + e == col ? 0x3f80 : 0);
   f32x16 gW2[2][2] = {};  // dW2 tiles [k-tile][n-tile] (rows k, cols n)
   f32x16 gW1[2] = {};     // dW1 tiles [n-tile] (rows i < 16 meaningful)
   float gb1[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gw3[2] = {0.f, 0.f}, gb3 = 0.f, loss = 0.f;
-  const float inv_n = 1.f / (float)n;
-  const long nwaves = (long)gridDim.x * kWaves;
-  for (int tile = 0; tile < tiles_per_wave; ++tile) {
-    const long m0 = (gw + tile * nwaves) * 32;
-    f32x16 h1[2], h2[2];
-    float o;
-    stage_x(x, m0, n, L, lane);
-    forward_tile(w, L, lane, h1, h2, o);
-    if (!TRAIN) {
-      if (lane < 32 && m0 + lane < n) out[m0 + lane] = softplus(o);
-      wave_lds_sync();
-      continue;
+  const long step = (long)gridDim.x * kMlpWaves * 32;
+  long m0 = ((long)blockIdx.x * kMlpWaves + wave) * 32;
+  Feat nf = {};
+  float ny = 0.f;
+  auto fetch = [&](long m) {  // past the end: the last sample, whose g is zeroed
+    const long s = std::min(m + col, n - 1);
+    nf = load_feat(x, s, h);
+    ny = y[s];
+  };
+  if (m0 < n) fetch(m0);
+  for (; m0 < n; m0 += step) {
+    const bf16x8 xb = pack_feat(nf);
+    const float yt = ny;
+    if (m0 + step < n) fetch(m0 + step);
+    bf16x8 b1[4];
+    f32x16 z2[2];
+    forward_regs<true>(N, a1, xb, lane, b1, z2);
+    const float o = output_regs(z2, w3, b3);
+    // dL/do of the lane's sample (both halves)
+    float g = 0.f;
+    if (m0 + col < n) {
+      const float d = softplus(o) - yt;
+      if (h == 0) loss += d * d;
+      g = 2.f * d * inv_n * sigmoid(o);
     }
-    // dL/do
-    if (lane < 32) {
-      const long s = m0 + lane;
-      float g = 0.f;
-      if (s < n) {
-        const float d = softplus(o) - y[s];
-        loss += d * d;
-        g = 2.f * d * inv_n * sigmoid(o);
-      }
-      L.g[lane] = g;
+    if (h == 0) {
+      gb3 += g;
+      gs[wave][col] = g;
     }
-    wave_lds_sync();
-    // output layer gradients and delta2 = g w3 relu'(z2), in the D layout
-    // (the lane's column nn, samples drow(j, lane))
-    f32x16 d2r[2];
+    // delta2 = g w3 relu'(z2), hidden x samples: the operand over the units
+    bf16x8 d2[4];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const int nn = 32 * t + col;
-      const float w3n = from_bf16(w.w3[nn]);
+      const f32x16 wr = bias_rows(N.w3, h, t);
+      f32x16 d;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int m = drow(j, lane);
-        const float g = L.g[m];
-        const float h = h2[t][j];
-        gw3[t] += from_bf16(to_bf16(h)) * g;
-        const float d2 = h > 0.f ? g * w3n : 0.f;
-        gb2[t] += d2;
-        d2r[t][j] = d2;
-        L.d2[m][nn] = to_bf16(d2);
-      }
+      for (int j = 0; j < 16; ++j) d[j] = z2[t][j] > 0.f ? g * wr[j] : 0.f;
+      d2[2 * t] = pack8(d, 0);
+      d2[2 * t + 1] = pack8(d, 8);
     }
-    if (lane == 0)
-      for (int m = 0; m < 32; ++m) gb3 += L.g[m];
     wave_lds_sync();
-    // dW2 += h1^T d2 : rows k (h1 column), cols n, K = samples.  Both operands
-    // come from the D-layout registers: K-slot e of the lane's half in block ks
-    // is sample drow(8 ks + e, lane), the same in A and B.
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        a[t] = pack8_bf16(h1[t], 8 * ks);
-        b[t] = pack8_bf16(d2r[t], 8 * ks);
-      }
-#pragma unroll
-      for (int tk = 0; tk < 2; ++tk)
-#pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
-          gW2[tk][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[tk], b[tn], gW2[tk][tn], 0, 0, 0);
-    }
-    // delta1 = (d2 W2^T) relu'(z1) : rows m, cols k, K = n
-    f32x16 d1r[2];
+    // g of the samples hid_unit(j, h), the rows of a samples x hidden tile
+    const f32x16 gr = bias_rows(gs[wave], h, 0);
+    // samples x hidden: h1 as the operand over the samples and its mask
+    bf16x8 h1[2][2];
+    bool on[2][16];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      f32x16 acc = {};
+      const f32x16 z = mfma(xb, a1[t], splat16(N.lb[col + 32 * t]));
 #pragma unroll
-      for (int kb = 0; kb < kH / 16; ++kb) {
-        const bf16x8 a = load8(&L.d2[col][16 * kb + kh]);
-        const bf16x8 b = load8(&w.w2[(32 * t + col) * kH + 16 * kb + kh]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+      for (int j = 0; j < 16; ++j) on[t][j] = z[j] > 0.f;
+      h1[t][0] = pack8_relu(z, 0);
+      h1[t][1] = pack8_relu(z, 8);
+    }
+    // h2 and delta2 the same; the gradients of W3, b2 and W2
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x16 z = splat16(N.lb[kH + col + 32 * t]);
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+        z = mfma(b1[kb], __builtin_bit_cast(bf16x8, N.w2f[4 * t + kb][lane]), z);
+      const float w3n = N.w3[col + 32 * t];
+      f32x16 d;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const uint32_t hp = pack_relu_bf16(z[2 * q], z[2 * q + 1]);
+        gw3[t] += __builtin_bit_cast(float, hp << 16) * gr[2 * q];
+        gw3[t] += __builtin_bit_cast(float, hp & 0xffff0000u) * gr[2 * q + 1];
       }
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const float h = h1[t][j];
-        const float d1 = h > 0.f ? acc[j] : 0.f;
-        gb1[t] += d1;
-        acc[j] = d1;
+        d[j] = z[j] > 0.f ? gr[j] * w3n : 0.f;
+        gb2[t] += d[j];
       }
-      d1r[t] = acc;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const bf16x8 b = pack8(d, 8 * ks);
+#pragma unroll
+        for (int tk = 0; tk < 2; ++tk) gW2[tk][t] = mfma(h1[tk][ks], b, gW2[tk][t]);
+      }
     }
-    // dW1 += X^T d1 : rows i (< 16), cols k, K = samples in the order of dW2
+    // X over the samples; delta1 = (delta2 W2^T) relu'(z1), samples x hidden;
+    // the gradients of b1 and W1
+    const f32x16 xo = mfma(xb, ident, f32x16{});
+    const bf16x8 xa[2] = {pack8(xo, 0), pack8(xo, 8)};
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 a;
+    for (int t = 0; t < 2; ++t) {
+      f32x16 d = {};
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        a[e] = col < kInP ? (short)L.x[drow(8 * ks + e, lane)][col] : (short)0;
+      for (int kb = 0; kb < 4; ++kb)
+        d = mfma(d2[kb], __builtin_bit_cast(bf16x8, N.w2b[4 * t + kb][lane]), d);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        d[j] = on[t][j] ? d[j] : 0.f;
+        gb1[t] += d[j];
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) gW1[t] = mfma(xa[ks], pack8(d, 8 * ks), gW1[t]);
+    }
+    wave_lds_sync();  // gs is rewritten by the next tile
+  }
+  // the waves' partials: the first half of them into LDS, the second half on
+  // top, then all four together; lanes l and l+32 hold the same columns' other
+  // rows, which the sums over samples add up
+  float* P = bp[wave % (kMlpWaves / 2)];
+  auto put = [&](bool add) {
+    auto at = [&](int i, float v) { P[i] = add ? P[i] + v : v; };
+#pragma unroll
+    for (int tk = 0; tk < 2; ++tk)
 #pragma unroll
       for (int tn = 0; tn < 2; ++tn)
-        gW1[tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pack8_bf16(d1r[tn], 8 * ks), gW1[tn],
-                                                          0, 0, 0);
-    }
-    wave_lds_sync();
-  }
-  if (!TRAIN) return;
-  // this wave's partial into LDS: lanes l and l+32 hold different rows of the
-  // same columns; the per-column sums (biases, W3) are combined through LDS
-  float* P = bp[wave];
 #pragma unroll
-  for (int tk = 0; tk < 2; ++tk)
+        for (int j = 0; j < 16; ++j)
+          at(oW2 + (32 * tk + hid_unit(j, h)) * kH + 32 * tn + col, gW2[tk][tn][j]);
 #pragma unroll
     for (int tn = 0; tn < 2; ++tn)
 #pragma unroll
-      for (int j = 0; j < 16; ++j)
-        P[oW2 + (32 * tk + drow(j, lane)) * kH + 32 * tn + col] = gW2[tk][tn][j];
+      for (int j = 0; j < 8; ++j) at(oW1 + hid_unit(j, h) * kH + 32 * tn + col, gW1[tn][j]);
+    auto colsum = [&](float v, int off) {
+      const float s = v + __shfl_xor(v, 32);
+      if (h == 0) at(off + col, s);
+    };
 #pragma unroll
-  for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int i = drow(j, lane);
-      if (i < kInP) P[oW1 + i * kH + 32 * tn + col] = gW1[tn][j];
+    for (int t = 0; t < 2; ++t) {
+      colsum(gb1[t], oB1 + 32 * t);
+      colsum(gb2[t], oB2 + 32 * t);
+      colsum(gw3[t], oW3 + 32 * t);
     }
-  auto colsum = [&](float v, int t, int off) {
-    L.red[lane] = v;
-    wave_lds_sync();
-    if (lane < 32) P[off + 32 * t + lane] = L.red[lane] + L.red[lane + 32];
-    wave_lds_sync();
+    float l = loss, b = gb3;  // of the lanes below 32
+#pragma unroll
+    for (int q = 16; q > 0; q >>= 1) {
+      l += __shfl_xor(l, q);
+      b += __shfl_xor(b, q);
+    }
+    if (lane == 0) {
+      at(oB3, b);
+      at(kNParam, l);
+    }
   };
-  for (int t = 0; t < 2; ++t) {
-    colsum(gb1[t], t, oB1);
-    colsum(gb2[t], t, oB2);
-    colsum(gw3[t], t, oW3);
-  }
-  L.red[lane] = lane < 32 ? loss : 0.f;
-  wave_lds_sync();
-  if (lane == 0) {
-    float l = 0.f;
-    for (int q = 0; q < 32; ++q) l += L.red[q];
-    P[oB3] = gb3;
-    P[kNParam] = l;
-  }
-  // the block's partial: its waves' partials summed in wave order
+  if (wave < kMlpWaves / 2) put(false);
+  __syncthreads();
+  if (wave >= kMlpWaves / 2) put(true);
   __syncthreads();
   float* Q = partial + (long)blockIdx.x * (kNParam + 1);
-  for (int i = threadIdx.x; i <= kNParam; i += 64 * kWaves) {
+  for (int i = threadIdx.x; i <= kNParam; i += 64 * kMlpWaves) {
     float v = bp[0][i];
 #pragma unroll
-    for (int q = 1; q < kWaves; ++q) v += bp[q][i];
+    for (int q = 1; q < kMlpWaves / 2; ++q) v += bp[q][i];
     Q[i] = v;
   }
 }
 
-// Sum of the per-block partials in a fixed order, in two levels: chunk c of
-// kRedChunk partials into chunks[c], then the chunks in order into grad
-// (grad[i] for i < kNParam, the loss sum last).
-__global__ __launch_bounds__(256) void k_grad_reduce(const float* __restrict__ partial,
-                                                     long nparts, float* __restrict__ chunks) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const long c = blockIdx.y;
-  if (i > kNParam) return;
-  const long q1 = std::min(nparts, (c + 1) * kRedChunk);
+// The blocks' partials summed in a fixed order into grad (the loss sum last):
+// 64 parameters per block, whose threads take a quarter of the partials each,
+// 16 loads in flight.  With ADAM also the update (Kingma & Ba, 2015) of the FP32
+// master parameters and the BF16 weights; the padded rows 10..15 of W1 stay zero.
+struct Adam {
+  float* p;
+  float* m1;
+  float* m2;
+  uint16_t* wb;
+  float lr, b1, b2, eps, c1, c2;
+};
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_grad_sum(const float* __restrict__ partial, long nparts,
+                                                  float* __restrict__ grad, Adam A) {
+  __shared__ float red[4][64];
+  const int c = threadIdx.x % 64, q = threadIdx.x / 64;
+  const int i = blockIdx.x * 64 + c;
+  const long per = (nparts + 3) / 4, q1 = std::min(nparts, (q + 1) * per);
   float s = 0.f;
-  for (long q = c * kRedChunk; q < q1; ++q) s += partial[q * (kNParam + 1) + i];
-  chunks[c * (kNParam + 1) + i] = s;
-}
-__global__ __launch_bounds__(256) void k_grad_final(const float* __restrict__ chunks, long nchunk,
-                                                    float* __restrict__ grad) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i > kNParam) return;
-  float s = 0.f;
-  for (long c = 0; c < nchunk; ++c) s += chunks[c * (kNParam + 1) + i];
-  grad[i] = s;
-}
-
-// Adam (Kingma & Ba, 2015) on the FP32 master parameters; refreshes the BF16
-// weights.  The padded rows 10..15 of W1 stay zero.  The gradient is the
-// chunk sums of k_grad_reduce added in k_grad_final's order (so the same
-// bits), also stored in grad with the loss sum.
-__global__ __launch_bounds__(256) void k_adam(float* __restrict__ p, float* __restrict__ m1,
-                                              float* __restrict__ m2,
-                                              const float* __restrict__ chunks, long nchunk,
-                                              float* __restrict__ grad, float lr, float b1,
-                                              float b2, float eps, float c1, float c2,
-                                              uint16_t* __restrict__ wb) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i > kNParam) return;
-  float gs = 0.f;
-  for (long c = 0; c < nchunk; ++c) gs += chunks[c * (kNParam + 1) + i];
-  grad[i] = gs;
-  if (i == kNParam) return;  // the loss sum
+  if (i <= kNParam)
+    for (long r = q * per; r < q1; r += 16) {
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = r + u < q1 ? partial[(r + u) * (kNParam + 1) + i] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s += v[u];
+    }
+  red[q][c] = s;
+  __syncthreads();
+  if (q || i > kNParam) return;
+  const float g = ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
+  grad[i] = g;
+  if (!ADAM || i == kNParam) return;  // the loss sum
   const bool pad = i < oB1 && (i / kH) >= kIn;
-  float v = p[i];
+  float v = A.p[i];
   if (!pad) {
-    const float gi = gs;
-    const float a = b1 * m1[i] + (1.f - b1) * gi;
-    const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = b;
-    v -= lr * (a / c1) / (sqrtf(b / c2) + eps);
-    p[i] = v;
+    const float a = A.b1 * A.m1[i] + (1.f - A.b1) * g;
+    const float b = A.b2 * A.m2[i] + (1.f - A.b2) * g * g;
+    A.m1[i] = a;
+    A.m2[i] = b;
+    v -= A.lr * (a / A.c1) / (sqrtf(b / A.c2) + A.eps);
+    A.p[i] = v;
   }
-  store_bf16_weight(wb, i, pad ? 0.f : v);
+  store_bf16_weight(A.wb, i, pad ? 0.f : v);
 }
 
 __global__ void k_refresh_bf16(const float* __restrict__ p, uint16_t* __restrict__ wb) {
@@ -692,32 +782,14 @@ __global__ __launch_bounds__(256) void k_apply_deferred(Geom g, const T* __restr
 // u(8(kb%2) + e, h) + 32(kb/2) makes every lane's own results its next
 // operand: no LDS and no barrier between the layers.  The biases start the
 // accumulators; the output dot is split over the halves and joined with one
-// lane exchange.  Same rounding points as forward_tile (BF16 features,
+// lane exchange.  Same rounding points as the batch kernels (BF16 features,
 // weights and activations; FP32 sums); only the summation order differs.
 //
 // Input k-slots: half 0 holds features 0..4 (du/dx, du/dy, du/dz, dv/dx,
 // dv/dy) in slots 0..4, half 1 features 5..8 (dv/dz, dw/dx, dw/dy, dw/dz) in
 // slots 8..11 and the wall distance in slot 12; the other slots are zero.
-__device__ __forceinline__ int hid_unit(int j, int h) { return 8 * (j / 4) + 4 * h + (j % 4); }
 __device__ __forceinline__ int slot_input(int s) {  // feature of input k-slot s, -1: zero
   return s < 5 ? s : (s < 8 ? -1 : (s < 13 ? s - 3 : -1));
-}
-
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// Two FP32 values rounded to BF16 (nearest, ties to even) in one dword, lo | hi << 16.
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
-}
-// BF16 of relu(lo), relu(hi), packed: a negative value rounds to a BF16 with
-// its sign bit set, which a 16-bit signed max against 0 clears to +0, so this
-// is the BF16 of max(x, 0) in two instructions for the pair.
-__device__ __forceinline__ uint32_t pack_relu_bf16(float lo, float hi) {
-  const s16x2 q = __builtin_bit_cast(s16x2, pack_bf16(lo, hi));
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(q, (s16x2){0, 0}));
 }
 
 struct RegMlp {
@@ -726,22 +798,6 @@ struct RegMlp {
   uint32_t w3[2][8];    // BF16 W3 of the lane's layer-2 rows j = 2m, 2m+1, packed
   float b3;
 };
-
-// The hidden biases b1 (lb[0..63]) and b2 (lb[64..127]) are read from LDS into
-// the accumulator rows of lane half h, row block t, when a tile starts: the
-// rows j = 4q .. 4q+3 are the consecutive units 8q + 4h + 32t .. +3.
-__device__ __forceinline__ f32x16 bias_rows(const float* lb, int h, int t) {
-  f32x16 c;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float4 v = *reinterpret_cast<const float4*>(lb + 8 * q + 4 * h + 32 * t);
-    c[4 * q] = v.x;
-    c[4 * q + 1] = v.y;
-    c[4 * q + 2] = v.z;
-    c[4 * q + 3] = v.w;
-  }
-  return c;
-}
 
 __device__ inline void load_reg_mlp(const Mlp& w, int lane, RegMlp& r) {
   const int h = lane / 32, m = lane % 32;
@@ -757,7 +813,7 @@ __device__ inline void load_reg_mlp(const Mlp& w, int lane, RegMlp& r) {
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int unit = hid_unit(8 * (kb % 2) + e, h) + 32 * (kb / 2);
+        const int unit = unit_of(kb, h, e);
         r.a2[t][kb][e] = (short)w.w2[unit * kH + u];
       }
 #pragma unroll
@@ -1172,9 +1228,8 @@ struct pll_closure {
   float* m2 = nullptr;
   uint16_t* wb = nullptr;  // BF16 W1 | W2 | W3
   float* partial = nullptr;
-  long npartial_blocks = 0;  // partial gradients, one per k_mlp block
+  long npartial_blocks = 0;  // partial gradients, one per k_train block
   float* grad = nullptr;    // kNParam + 1 (loss sum last)
-  float* chunks = nullptr;  // first-level gradient sums, (kMaxWaves / kRedChunk) x (kNParam + 1)
   long step = 0;
   hipStream_t stream = nullptr;
   int device = 0;              // the device current at creation (that of stream)
@@ -1187,7 +1242,7 @@ struct pll_closure {
 namespace {
 
 Mlp weights(const pll_closure* c) {
-  return Mlp{c->p, c->wb + kWb1, c->wb + kWb2, c->wb + kWb3, c->wb + kWbB1, c->wb + kWbB2};
+  return Mlp{c->p, c->wb + kWb1, c->wb + kWb2, c->wb + kWb3};
 }
 
 int ensure_partial(pll_closure* c, long nblocks) {
@@ -1199,57 +1254,41 @@ int ensure_partial(pll_closure* c, long nblocks) {
   return PLL_OK;
 }
 
-// Waves of a k_mlp grid for n samples (a multiple of kWaves, at most
-// kMaxWaves) and the 32-sample tiles each wave runs (wave q takes tiles q,
-// q + nwaves, ...).
-long waves_for(long n) {
-  const long tiles = (n + 31) / 32;
-  const long waves = std::min(tiles, kMaxWaves);
-  return (waves + kWaves - 1) / kWaves * kWaves;
-}
-int tiles_per_wave(long n, long nwaves) {
-  const long tiles = (n + 31) / 32;
-  return (int)((tiles + nwaves - 1) / nwaves);
+// Blocks of a training or inference grid for n samples: one 32-sample tile per
+// wave, at most kMaxWaves waves (which then take every nwaves-th tile).
+long mlp_blocks(long n) {
+  const long waves = std::min((n + 31) / 32, kMaxWaves);
+  return (waves + kMlpWaves - 1) / kMlpWaves;
 }
 
-// The gradient into chunk sums; with `final` also summed into c->grad (the
-// training step leaves the last level to k_adam).  Returns the chunk count.
-long gradient_chunks(pll_closure* c, const float* x, const float* y, long n, bool final, int* rc) {
-  const long nw = waves_for(n);
-  *rc = ensure_partial(c, nw / kWaves);
-  if (*rc) return 0;
-  hipLaunchKernelGGL((k_mlp<true>), dim3((unsigned)(nw / kWaves)), dim3(64 * kWaves), 0, c->stream,
-                     weights(c), x, y, n, static_cast<float*>(nullptr), c->partial,
-                     tiles_per_wave(n, nw));
-  const long nblk = nw / kWaves;  // one partial per block
-  const long nchunk = (nblk + kRedChunk - 1) / kRedChunk;
-  hipLaunchKernelGGL(k_grad_reduce, dim3((kNParam + 1 + 255) / 256, (unsigned)nchunk), dim3(256), 0,
-                     c->stream, c->partial, nblk, c->chunks);
-  if (final)
-    hipLaunchKernelGGL(k_grad_final, dim3((kNParam + 1 + 255) / 256), dim3(256), 0, c->stream,
-                       c->chunks, nchunk, c->grad);
-  const hipError_t e = hipGetLastError();
-  *rc = e == hipSuccess ? PLL_OK : hip_fail(e, "closure gradient kernels");
-  return nchunk;
+// The blocks' partial gradients and their sum; with A in a training step's
+// update.
+void launch_gradient(const pll_closure* c, const float* x, const float* y, long n, float* partial,
+                     float* grad, const Adam* A) {
+  const long nblk = mlp_blocks(n);
+  hipLaunchKernelGGL(k_train, dim3((unsigned)nblk), dim3(64 * kMlpWaves), 0, c->stream, weights(c),
+                     x, y, n, partial);
+  hipLaunchKernelGGL((A ? k_grad_sum<true> : k_grad_sum<false>), dim3((kNParam + 1 + 63) / 64),
+                     dim3(256), 0, c->stream, partial, nblk, grad, A ? *A : Adam{});
 }
 
-int gradient(pll_closure* c, const float* x, const float* y, long n) {
-  int rc = PLL_OK;
-  gradient_chunks(c, x, y, n, true, &rc);
-  return rc;
+int gradient(pll_closure* c, const float* x, const float* y, long n, const Adam* A) {
+  const int rc = ensure_partial(c, mlp_blocks(n));
+  if (rc) return rc;
+  launch_gradient(c, x, y, n, c->partial, c->grad, A);
+  PLL_HIP_TRY(hipGetLastError());
+  return PLL_OK;
 }
 
 // ---- allocation-free gradient ------------------------------------------------
 // The buffers of pll_closure_gradient_noalloc live in one file-scope device
 // array, one copy per GPU for the life of the process: the per-block partial
-// gradients of the largest training grid (kMaxWaves / kWaves blocks), the
-// first-level chunk sums and the summed gradient with the loss, each
-// kNParam + 1 floats -- 6.1 MB.  Every call on a GPU shares that GPU's copy;
+// gradients of the largest training grid (kMaxWaves / kMlpWaves blocks) and the
+// summed gradient with the loss, each kNParam + 1 floats -- 5.5 MB.  Every call on a GPU shares that GPU's copy;
 // each call writes every element it reads before reading it, so nothing has
 // to start at zero, and calls that overlap on one GPU race.
-constexpr long kScratchPartials = kMaxWaves / kWaves;
-constexpr long kScratchChunks = kMaxWaves / kRedChunk;
-constexpr long kScratchFloats = (kScratchPartials + kScratchChunks + 1) * (kNParam + 1);
+constexpr long kScratchPartials = kMaxWaves / kMlpWaves;
+constexpr long kScratchFloats = (kScratchPartials + 1) * (kNParam + 1);
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 // Device address of `scratch` on each GPU, resolved once per device with that
@@ -1608,7 +1647,6 @@ int pll_closure_create(uint64_t seed, pll_closure** out) {
   const size_t pb = (size_t)kNParam * sizeof(float);
   if (hipMalloc(&c->p, pb) != hipSuccess || hipMalloc(&c->m1, pb) != hipSuccess ||
       hipMalloc(&c->m2, pb) != hipSuccess || hipMalloc(&c->grad, pb + sizeof(float)) != hipSuccess ||
-      hipMalloc(&c->chunks, (size_t)(kMaxWaves / kRedChunk) * (pb + sizeof(float))) != hipSuccess ||
       hipMalloc(&c->wb, (size_t)kWbLen * sizeof(uint16_t)) != hipSuccess)
     return bail(fail(PLL_ERR_NOMEM, "closure parameters"));
   // Glorot-uniform weights, zero biases (the output bias starts at softplus^-1(1))
@@ -1639,7 +1677,7 @@ int pll_closure_create(uint64_t seed, pll_closure** out) {
 int pll_closure_destroy(pll_closure* c) {
   if (!c) return PLL_OK;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  void* bufs[] = {c->p, c->m1, c->m2, c->wb, c->partial, c->grad, c->chunks};
+  void* bufs[] = {c->p, c->m1, c->m2, c->wb, c->partial, c->grad};
   for (void* q : bufs)
     if (q) (void)hipFree(q);
   if (c->ready) (void)hipEventDestroy(c->ready);
@@ -1674,25 +1712,15 @@ int pll_closure_gradient_noalloc(pll_closure* c, const float* x, const float* y,
   PLL_HIP_TRY(hipGetDevice(&dev));
   if (dev != c->device)
     return fail(PLL_ERR_STATE, "pll_closure_gradient_noalloc: the closure's device must be current");
-  const long nw = waves_for(n), nblk = nw / kWaves;
-  const long nchunk = (nblk + kRedChunk - 1) / kRedChunk;
-  if (nblk > kScratchPartials || nchunk > kScratchChunks)
+  if (mlp_blocks(n) > kScratchPartials)
     return fail(PLL_ERR_ARG, "pll_closure_gradient_noalloc: the training grid exceeds the scratch "
                              "array (at most kMaxWaves waves)");
   float* base = nullptr;
   int rc = scratch_on(dev, &base);
   if (rc) return rc;
-  float* partial = base;
-  float* chunks = base + kScratchPartials * (kNParam + 1);
-  float* grad = chunks + kScratchChunks * (kNParam + 1);
+  float* grad = base + kScratchPartials * (kNParam + 1);
   // the kernels of pll_closure_gradient, on the scratch array
-  hipLaunchKernelGGL((k_mlp<true>), dim3((unsigned)nblk), dim3(64 * kWaves), 0, c->stream,
-                     weights(c), x, y, n, static_cast<float*>(nullptr), partial,
-                     tiles_per_wave(n, nw));
-  hipLaunchKernelGGL(k_grad_reduce, dim3((kNParam + 1 + 255) / 256, (unsigned)nchunk), dim3(256), 0,
-                     c->stream, partial, nblk, chunks);
-  hipLaunchKernelGGL(k_grad_final, dim3((kNParam + 1 + 255) / 256), dim3(256), 0, c->stream, chunks,
-                     nchunk, grad);
+  launch_gradient(c, x, y, n, base, grad, nullptr);
   PLL_HIP_TRY(hipGetLastError());
   float lsum = 0.f;
   if (grad_host)
@@ -1707,7 +1735,7 @@ int pll_closure_gradient_noalloc(pll_closure* c, const float* x, const float* y,
 int pll_closure_gradient(pll_closure* c, const float* x, const float* y, long n, float* grad_host,
                          double* loss) {
   if (!c || !x || !y || n <= 0) return fail(PLL_ERR_ARG, "bad arguments");
-  int rc = gradient(c, x, y, n);
+  int rc = gradient(c, x, y, n, nullptr);
   if (rc) return rc;
   std::vector<float> g(kNParam + 1);
   PLL_HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1719,27 +1747,21 @@ int pll_closure_gradient(pll_closure* c, const float* x, const float* y, long n,
 
 int pll_closure_train_step(pll_closure* c, const float* x, const float* y, long n, double lr) {
   if (!c || !x || !y || n <= 0 || !(lr > 0)) return fail(PLL_ERR_ARG, "bad arguments");
-  int rc = PLL_OK;
-  const long nchunk = gradient_chunks(c, x, y, n, false, &rc);
+  const double b1 = 0.9, b2 = 0.999;
+  const double t = (double)(c->step + 1);
+  const Adam A{c->p,      c->m1,     c->m2, c->wb, (float)lr, (float)b1, (float)b2, 1e-8f,
+               (float)(1.0 - std::pow(b1, t)), (float)(1.0 - std::pow(b2, t))};
+  const int rc = gradient(c, x, y, n, &A);
   if (rc) return rc;
   c->step += 1;
-  const double b1 = 0.9, b2 = 0.999;
-  const float c1 = (float)(1.0 - std::pow(b1, (double)c->step));
-  const float c2 = (float)(1.0 - std::pow(b2, (double)c->step));
-  hipLaunchKernelGGL(k_adam, dim3((kNParam + 1 + 255) / 256), dim3(256), 0, c->stream, c->p,
-                     c->m1, c->m2, c->chunks, nchunk, c->grad, (float)lr, (float)b1, (float)b2,
-                     1e-8f, c1, c2, c->wb);
-  PLL_HIP_TRY(hipGetLastError());
   c->version += 1;
   return PLL_OK;
 }
 
 int pll_closure_predict(pll_closure* c, const float* x, long n, float* out) {
   if (!c || !x || !out || n <= 0) return fail(PLL_ERR_ARG, "bad arguments");
-  const long nw = waves_for(n);
-  hipLaunchKernelGGL((k_mlp<false>), dim3((unsigned)(nw / kWaves)), dim3(64 * kWaves), 0, c->stream,
-                     weights(c), x, static_cast<const float*>(nullptr), n, out,
-                     static_cast<float*>(nullptr), tiles_per_wave(n, nw));
+  hipLaunchKernelGGL(k_predict, dim3((unsigned)mlp_blocks(n)), dim3(64 * kMlpWaves), 0, c->stream,
+                     weights(c), x, n, out);
   PLL_HIP_TRY(hipGetLastError());
   return PLL_OK;
 }
