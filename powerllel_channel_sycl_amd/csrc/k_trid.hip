@@ -131,14 +131,18 @@ __global__ __launch_bounds__(kTx* kTy) void k_trid(int nx, int ny, int nz, T* __
 
 // ---------------------------------------------------------------------------
 // The same solve inside the step, partitioned so that the work array makes one
-// HBM pass each way.  A block owns kCw adjacent columns of one row j; each
-// column is cut into S segments of M planes, one thread per segment, and the
-// segment's right-hand side and reciprocal pivots stay in registers.  The
-// pivots are not read from a table: each segment continues the elimination's
-// pivot recurrence (init_poisson_solver, src/mod_poisson_solver.cc:273-282)
-// from the pivot of the plane below it, which the table `pstart` holds, with
-// the reference's operations (FP64 division), so every pivot is the one the
-// full table holds, bit for bit; the reciprocal is 0 for a zero pivot:
+// HBM pass each way.  The columns (2m, 2m+1) x (2n, 2n+1) of the perm packing
+// share one eigenvalue (m, n >= 1; columns and rows 0 and 1 are classes of their
+// own), so a thread owns a whole eigenvalue class, up to four columns: the
+// pivots, the multipliers and the coefficients' LDS reads are formed once for
+// all four, the four recurrences overlap, and loads are pairs.  A class's columns
+// are cut into S segments of M planes, one thread per segment, and the segment's
+// values and reciprocal pivots stay in registers.  The pivots are not read from
+// a table: each segment continues the elimination's pivot recurrence
+// (init_poisson_solver, src/mod_poisson_solver.cc:273-282) from the pivot of the
+// plane below it, which the table `pstart` holds, with the reference's
+// operations (FP64 division), so every pivot is the one the full table holds,
+// bit for bit; the reciprocal is 0 for a zero pivot:
 //   A. forward elimination of the segment from a zero incoming value, with the
 //      running product g of the negated multipliers (the segment end's
 //      dependence on the incoming value);
@@ -150,57 +154,60 @@ __global__ __launch_bounds__(kTx* kTy) void k_trid(int nx, int ny, int nz, T* __
 // The segment boundaries are combined with other roundings than the
 // sequential sweep, and the pivots are applied as reciprocals, so the result
 // differs from k_trid's by FP64 round-off (it is not bit-identical).
-// FP32-mixed runs the recurrence with less than one division's work per plane
-// instead of two divisions: the multiplier is a[k] times the reciprocal of the
-// pivot below (already formed), and the reciprocal is the hardware estimate
-// refined by one Newton step (which squares its relative error: far below the
-// 6e-8 rounding of the FP32 work array).  The recurrence is the kernel's
-// longest dependent chain, and this form of it saves 16 % of the FP32-mixed
-// solve at 768x384x384 (375 -> 316 us; a second Newton step costs 7 us); the
-// FP64 solve keeps the divisions (its pivots stay bit-exact, and a reciprocal
-// saved it nothing).
+// FP32-mixed runs the recurrence without divisions: the multiplier is a[k] times
+// the reciprocal of the pivot below (already formed), and the reciprocal is the
+// hardware estimate refined by one Newton step (which squares its relative
+// error: far below the 6e-8 rounding of the FP32 work array).
+// One thread per column was bound by the pivots' arithmetic and the coefficients'
+// LDS reads (FP32 2.0 TB/s).  One per class: FP32 1536x768x512 2377 -> 1420 us,
+// 768x384x384 316 -> 249, 384x256x192 79 -> 53; FP64 768x384x384 474 -> 413,
+// 256x192x128 34 -> 23 us.
 __device__ __forceinline__ double rcp_newton(double q) {
   const double r = __builtin_amdgcn_rcp(q);
   return __builtin_fma(r, __builtin_fma(-q, r, 1.0), r);
 }
 constexpr int kSegPlanes = 768;  // the deepest column the segments hold
-// Planes per segment M (8, 16 or 24) and segments per column (at most S = 16,
-// or 32 for columns deeper than 384 planes): short segments where they suffice
-// keep the registers of a thread (its M values and M+1 reciprocal pivots) low.
-constexpr int seg_planes(int nz) {
-  return nz <= 128 ? 8 : (nz <= 256 ? 16 : (nz <= 384 ? 24 : (nz <= 512 ? 16 : 24)));
-}
-constexpr int seg_count_max(int nz) { return nz <= 384 ? 16 : 32; }
-static_assert(seg_planes(kSegPlanes) * seg_count_max(kSegPlanes) >= kSegPlanes &&
-                  seg_planes(512) * seg_count_max(512) >= 512 &&
-                  seg_planes(384) * seg_count_max(384) >= 384,
+// Planes per segment M and most segments per column S.  Short segments keep the
+// registers (4 M values, M+1 reciprocals) at four waves per SIMD; M = 12 where
+// M = 8 would make blocks that leave a CU's wave slots idle (768x384x384: FP64 413
+// against 464 us, FP32 249 against 299 us).
+constexpr int seg_planes(int nz) { return nz <= 256 || (nz > 384 && nz <= 512) ? 8 : 12; }
+constexpr int seg_count_max(int nz) { return nz <= 128 ? 16 : (nz <= 384 ? 32 : 64); }
+constexpr bool segs_hold(int nz) { return seg_planes(nz) * seg_count_max(nz) >= nz; }
+static_assert(segs_hold(128) && segs_hold(256) && segs_hold(384) && segs_hold(512) &&
+                  segs_hold(kSegPlanes),
               "the segments hold every column they take");
+// Classes per block: 128 bytes of a row, or half that in FP32 columns of more than
+// 32 segments (512 threads a block).
+template <typename T, int S>
+constexpr int seg_classes() {
+  return std::is_same<T, float>::value && S <= 32 ? 16 : 8;
+}
 
-// The sequential combination of the S segment-end values, Y_q = hat_q + dep_q *
-// Y_{q-1} (forward, REV false) or from the top (REV true), by the threads of
-// one segment (one per column); the LDS reads are issued four at a time ahead
-// of the dependent chain.
+// The sequential combination of the segment-end values in place, Y_q = end_q +
+// dep_q * Y_{q-1} (forward) or from the top (REV), by one thread per column
+// (column t = component * CW + class); the LDS reads are issued four at a time
+// ahead of the dependent chain.
 template <int CW, int S, bool REV>
-__device__ __forceinline__ void combine(const double (*hat)[CW], const double (*dep)[CW],
-                                        double (*inc)[CW], int nseg, int col) {
+__device__ __forceinline__ void combine(double (*end)[4 * CW], const double (*dep)[CW], int nseg,
+                                        int t) {
   double y = 0.0;
-#pragma unroll
-  for (int q0 = 0; q0 < S; q0 += 4) {
+  for (int q0 = 0; q0 < nseg; q0 += 4) {
     double h[4], d[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int q = REV ? nseg - 1 - (q0 + u) : q0 + u;
       if (q0 + u < nseg) {
-        h[u] = hat[q][col];
-        d[u] = dep[q][col];
+        h[u] = end[q][t];
+        d[u] = dep[q][t % CW];
       }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int q = REV ? nseg - 1 - (q0 + u) : q0 + u;
       if (q0 + u < nseg) {
-        y = h[u] + d[u] * y;
-        inc[q][col] = y;
+        y = __builtin_fma(d[u], y, h[u]);
+        end[q][t] = y;
       }
     }
   }
@@ -217,127 +224,204 @@ struct SegCoef {
   int pin;  // the (0,0) column's last pivot is pinned to 0
 };
 
+// Hides where a register's value came from.
+template <typename V>
+__device__ __forceinline__ void pin(V& v) {
+  asm volatile("" : "+v"(v));
+}
+
+// Blocks: tiles of CW column pairs for each row pair (pair 0 standing for the
+// classes 0), then the same tiles of row 1, then tiles of CW row classes of
+// column 1.
+template <int CW>
+__host__ __device__ constexpr unsigned seg_blocks(int nx, int ny) {
+  return (unsigned)((nx / 2 + CW - 1) / CW) * (ny / 2 + 1) + (ny / 2 + CW) / CW;
+}
+
 template <typename T, int M, int CW, int S>
-__global__ __launch_bounds__(CW* S) void k_trid_seg(int nx, int ny, int nz, int nseg,
-                                                        T* __restrict__ var,
-                                                        const double* __restrict__ a,
-                                                        const double* __restrict__ c,
-                                                        SegCoef sg, int cxn, int cyn) {
-  __shared__ double hat[S][CW];  // segment-end value from a zero incoming value
-  __shared__ double dep[S][CW];  // its dependence on the incoming value
-  __shared__ double inc[S][CW];  // the true value at the segment end
-  __shared__ double sa[kSegPlanes], sb[kSegPlanes], sc[kSegPlanes];
-  const int t = threadIdx.x, col = t % CW, s = t / CW;
-  const int i = blockIdx.x * CW + col, j = blockIdx.y;
-  for (int k = t; k < nz; k += CW * nseg) {
-    sa[k] = a[k];
-    sb[k] = sg.b[k];
-    sc[k] = c[k];
+__global__ __launch_bounds__(CW* S, (sizeof(T) == 8 && M > 8 ? 3 : 4)) void k_trid_seg(int nx, int ny, int nz, int nseg,
+                                                    T* __restrict__ var,
+                                                    const double* __restrict__ a,
+                                                    const double* __restrict__ c, SegCoef sg,
+                                                    int cxn, int cyn) {
+  struct alignas(2 * sizeof(T)) Pair {
+    T x, y;
+  };
+  __shared__ double end[S][4 * CW];  // segment-end values: from a zero incoming value, then true
+  __shared__ double dep[S][CW];      // their dependence on the incoming value
+  __shared__ double sa[M * S], sb[M * S], sc[M * S];
+  const int t = threadIdx.x, cl = t % CW, s = t / CW;
+  for (int k = t; k < nseg * M; k += CW * nseg) {  // zero past the last plane
+    sa[k] = k < nz ? a[k] : 0.0;
+    sb[k] = k < nz ? sg.b[k] : 0.0;
+    sc[k] = k < nz ? c[k] : 0.0;
   }
-  const bool on = i < nx;
+  // the thread's class (ci, cj) and its columns, i0 and i0+1 of rows j0 and
+  // j0+1, of which it keeps those in `keep` (bit 2 dy + dx).  The others, of a
+  // column or row 0 or 1, are another thread's: they are loaded, perhaps while
+  // that thread stores them, and what becomes of them is not used.
+  const int nxp = nx / 2, nyp = ny / 2, tpr = (nxp + CW - 1) / CW;
+  const int b = (int)xcd_remap(blockIdx.x, gridDim.x);
+  const bool col1 = b >= tpr * (nyp + 1);
+  const int e = (b - tpr * (nyp + 1)) * CW + cl;
+  const int xp = col1 ? 0 : (b % tpr) * CW + cl, yp = col1 ? e : b / tpr;
+  const bool on = xp < nxp && yp <= nyp;
+  const int i0 = 2 * xp, j0 = yp < nyp ? 2 * yp : 0;
+  const int ci = col1 ? 1 : compact_index(on ? i0 : 0);
+  const int cj = on ? (yp < nyp ? compact_index(j0) : 1) : 0;
+  const int keep = ((col1 ? 2 : (xp ? 3 : 1)) & 3) * (yp == nyp ? 4 : (yp ? 5 : 1));
   const long nxy = (long)nx * ny;
   const int k0 = s * M;
-  const int n = on ? min(M, nz - k0) : 0;
-  T* v = var + (long)j * nx + i;
-  const int ci = compact_index(on ? i : 0), cj = compact_index(j);
+  const int n = on ? min(M, nz - k0) : 0, last = nz - 1 - k0;  // planes; the last row
+  long off = (long)k0 * nxy + (on ? (long)j0 * nx + i0 : 0);
   // the segment's values (in the field precision: FP32-mixed rounds the
   // forward-eliminated values to FP32 between the sweeps, as k_trid does),
-  // loaded first; then the reciprocal pivots of planes k0-1 .. k0+n-1
-  T x[M];
-  double rb[M + 1];
+  // loaded first; 0 past the last plane
+  T x[4][M];
+  {
+    const T* q = var + off;
 #pragma unroll
-  for (int m = 0; m < M; ++m)
-    if (m < n) x[m] = v[(long)(k0 + m) * nxy];
-  const double lxy = sg.elx[ci] + sg.ely[cj];
-  double piv = k0 > 0 && n > 0 ? sg.pstart[(long)s * cxn * cyn + (long)cj * cxn + ci] : 0.0;
-  rb[0] = piv != 0.0 ? 1.0 / piv : 0.0;
-  __syncthreads();  // sa, sb, sc
-  // init_poisson_solver's recurrence (src/mod_poisson_solver.cc:273-282); a
-  // zero pivot only ends a column, so rb[m - 1] is 1/piv wherever k > 0
-  constexpr bool kMixed = std::is_same<T, float>::value;
-#pragma unroll
-  for (int m = 1; m <= M; ++m)
-    if (m <= n) {
-      const int k = k0 + m - 1;
-      double q = sb[k] + lxy;
-      if (k > 0) {
-        const double a_tmp = kMixed ? sa[k] * rb[m - 1] : sa[k] / piv;
-        q -= (a_tmp * sc[k - 1]);
+    for (int m = 0; m < M; ++m, q += nxy) {
+      Pair r0{T(0), T(0)}, r1{T(0), T(0)};
+      if (m < n) {
+        r0 = *reinterpret_cast<const Pair*>(q);
+        r1 = *reinterpret_cast<const Pair*>(q + nx);
       }
-      if (sg.pin && k == nz - 1 && ci == 0 && cj == 0) q = 0.0;
-      rb[m] = q != 0.0 ? (kMixed ? rcp_newton(q) : 1.0 / q) : 0.0;
-      piv = q;
+      x[0][m] = r0.x;
+      x[1][m] = r0.y;
+      x[2][m] = r1.x;
+      x[3][m] = r1.y;
     }
+  }
+  const double lxy = sg.elx[ci] + sg.ely[cj];
+  double piv = k0 > 0 && n > 0 ? sg.pstart[(long)s * cxn * cyn + (long)cj * cxn + ci] : 1.0;
+  double rb[M + 1];  // reciprocal pivots of planes k0-1 .. k0+M-1, 0 where there is no plane
+  rb[0] = k0 > 0 && piv != 0.0 ? 1.0 / piv : 0.0;
+  __syncthreads();  // sa, sb, sc
+  // init_poisson_solver's recurrence (src/mod_poisson_solver.cc:273-282): a[0]
+  // is 0, and a zero pivot only ends a column
+  constexpr bool kMixed = std::is_same<T, float>::value;
+  // the coefficients are read kAhead planes at a time, not all ahead
+  constexpr int kAhead = 4;
+  const auto step_fence = [] { __builtin_amdgcn_sched_barrier(0); };
+  const int pinned = sg.pin && ci == 0 && cj == 0 ? last + 1 : 0;
+#pragma unroll
+  for (int m = 1; m <= M; ++m) {
+    if (m % kAhead == 1) step_fence();
+    const int k = k0 + m - 1;
+    const double a_tmp = kMixed ? sa[k] * rb[m - 1] : sa[k] / piv;
+    double q = sb[k] + lxy;
+    q -= (a_tmp * sc[m > 1 ? k - 1 : max(k - 1, 0)]);
+    if (m == pinned) q = 0.0;
+    rb[m] = m <= n && q != 0.0 ? (kMixed ? rcp_newton(q) : 1.0 / q) : 0.0;
+    piv = q;
+  }
+  // past the last plane the values, multipliers and reciprocals are 0, and a[0]
+  // and c[nz-1] are 0: the sweeps need no test for a column's ends
+  // between the sweeps the values stay in the field precision, not as the
+  // doubles that the last sweep made of them
+  const auto pin_values = [&] {
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int m = 0; m < M; ++m) pin(x[f][m]);
+  };
   // A: forward elimination from a zero incoming value
   {
-    double y = 0.0, g = 1.0;
+    double y[4] = {0.0, 0.0, 0.0, 0.0}, g = 1.0;
 #pragma unroll
-    for (int m = 0; m < M; ++m)
-      if (m < n) {
-        const int k = k0 + m;
-        if (k == 0) {
-          y = (double)x[0];
-          g = 0.0;
-        } else {
-          const double l = sa[k] * rb[m];
-          y = (double)x[m] - l * y;
-          g = -l * g;
-        }
-      }
-    if (on) {
-      hat[s][col] = y;
-      dep[s][col] = g;
+    for (int m = 0; m < M; ++m) {
+      if (m % kAhead == 0) step_fence();
+      const double l = sa[k0 + m] * rb[m];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) y[f] = __builtin_fma(-l, y[f], (double)x[f][m]);
+      g = -l * g;
     }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) end[s][f * CW + cl] = y[f];
+    dep[s][cl] = g;
   }
   __syncthreads();
-  if (s == 0) combine<CW, S, false>(hat, dep, inc, nseg, col);
+  if (t < 4 * CW) combine<CW, S, false>(end, dep, nseg, t);
+  // few segments leave fewer threads than columns
+  for (int u = t + CW * nseg; u < 4 * CW; u += CW * nseg) combine<CW, S, false>(end, dep, nseg, u);
   __syncthreads();
+  pin_values();
   // B: forward elimination from the true incoming value; the last row
   {
-    double y = s > 0 && on ? inc[s - 1][col] : 0.0;
+    double y[4];
 #pragma unroll
-    for (int m = 0; m < M; ++m)
-      if (m < n) {
-        const int k = k0 + m;
-        y = k == 0 ? (double)x[0] : (double)x[m] - (sa[k] * rb[m]) * y;
-        if (k == nz - 1) y = y * rb[m + 1];  // the reciprocal table holds 0 for a zero pivot
-        x[m] = (T)y;
-      }
-  }
-  __syncthreads();  // inc is rewritten below
-  // C: back substitution from a zero value above the segment
-  {
-    double xv = 0.0, h = 1.0;
+    for (int f = 0; f < 4; ++f) y[f] = s > 0 ? end[s - 1][f * CW + cl] : 0.0;
 #pragma unroll
-    for (int m = M - 1; m >= 0; --m)
-      if (m < n) {
-        const int k = k0 + m;
-        if (k == nz - 1) {
-          xv = (double)x[m];
-          h = 0.0;
-        } else {
-          const double q = sc[k] * rb[m + 1];
-          xv = (double)x[m] * rb[m + 1] - q * xv;
-          h = -q * h;
-        }
+    for (int m = 0; m < M; ++m) {
+      if (m % kAhead == 0) step_fence();
+      const double l = sa[k0 + m] * rb[m];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) y[f] = __builtin_fma(-l, y[f], (double)x[f][m]);
+      if (m == last) {  // the reciprocal is 0 for a zero pivot
+#pragma unroll
+        for (int f = 0; f < 4; ++f) y[f] *= rb[m + 1];
+        rb[m + 1] = 1.0;  // the back substitution takes the row as it is
       }
-    if (on) {
-      hat[s][col] = xv;
-      dep[s][col] = h;
+#pragma unroll
+      for (int f = 0; f < 4; ++f) x[f][m] = (T)y[f];
     }
   }
+  __syncthreads();  // end is rewritten below
+  // C: back substitution from a zero value above the segment
+  {
+    double xv[4] = {0.0, 0.0, 0.0, 0.0}, h = 1.0;
+#pragma unroll
+    for (int m = M - 1; m >= 0; --m) {
+      if (m % kAhead == kAhead - 1) step_fence();
+      const double q = sc[k0 + m] * rb[m + 1];
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+        xv[f] = __builtin_fma((double)x[f][m], rb[m + 1], -(q * xv[f]));
+      h = -q * h;
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) end[s][f * CW + cl] = xv[f];
+    dep[s][cl] = h;
+  }
   __syncthreads();
-  if (s == 0) combine<CW, S, true>(hat, dep, inc, nseg, col);
+  if (t < 4 * CW) combine<CW, S, true>(end, dep, nseg, t);
+  for (int u = t + CW * nseg; u < 4 * CW; u += CW * nseg) combine<CW, S, true>(end, dep, nseg, u);
   __syncthreads();
+  pin_values();
   // D: back substitution from the true value above the segment
   {
-    double xv = s + 1 < nseg && on ? inc[s + 1][col] : 0.0;
+    double xv[4];
 #pragma unroll
-    for (int m = M - 1; m >= 0; --m)
+    for (int f = 0; f < 4; ++f) xv[f] = s + 1 < nseg ? end[s + 1][f * CW + cl] : 0.0;
+#pragma unroll
+    for (int m = M - 1; m >= 0; --m) {
+      if (m % kAhead == kAhead - 1) step_fence();
+      const double q = sc[k0 + m] * rb[m + 1];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        xv[f] = __builtin_fma((double)x[f][m], rb[m + 1], -(q * xv[f]));
+        x[f][m] = (T)xv[f];
+      }
+    }
+  }
+  pin(off);  // the addresses are formed again rather than kept from the loads
+  T* q = var + off;
+  if (keep == 15) {
+#pragma unroll
+    for (int m = 0; m < M; ++m, q += nxy)
       if (m < n) {
-        const int k = k0 + m;
-        xv = k == nz - 1 ? (double)x[m] : (double)x[m] * rb[m + 1] - (sc[k] * rb[m + 1]) * xv;
-        v[(long)k * nxy] = (T)xv;
+        *reinterpret_cast<Pair*>(q) = Pair{x[0][m], x[1][m]};
+        *reinterpret_cast<Pair*>(q + nx) = Pair{x[2][m], x[3][m]};
+      }
+  } else {
+#pragma unroll
+    for (int m = 0; m < M; ++m, q += nxy)
+      if (m < n) {
+        if (keep & 1) q[0] = x[0][m];
+        if (keep & 2) q[1] = x[1][m];
+        if (keep & 4) q[nx] = x[2][m];
+        if (keep & 8) q[nx + 1] = x[3][m];
       }
   }
 }
@@ -437,48 +521,38 @@ int launch_trid(pll_context* c) {
 }
 
 namespace {
-// Columns per block, planes per segment and segments per column of the
-// partitioned solve: FP32-mixed takes 32 columns of up to 16 segments (128-byte
-// rows; 16 columns ran 374 against 316 us at 768x384x384) and 16 columns of 32
-// segments (512-thread blocks; 32 columns, 1024 threads, ran 9 % slower at
-// 1536x768x512), FP64 16 columns.
-template <typename T, int S>
-constexpr int seg_cols() {
-  return std::is_same<T, float>::value && S <= 16 ? 32 : 16;
-}
 template <typename T, int M, int S>
 void trid_seg(pll_context* c) {
-  constexpr int kCw = seg_cols<T, S>();
-  const int nseg = (c->g.nz + M - 1) / M;
-  const dim3 grid((c->g.nx + kCw - 1) / kCw, c->g.ny);
-  const int nz = c->g.nz;
+  constexpr int kCw = seg_classes<T, S>();
+  const int nz = c->g.nz, nseg = (nz + M - 1) / M;
   const SegCoef sg{c->d_seg, c->d_seg + nz, c->d_seg + nz + c->cxn,
                    c->d_seg + nz + c->cxn + c->cyn, c->seg_pin};
-  hipLaunchKernelGGL((k_trid_seg<T, M, kCw, S>), grid, dim3(kCw * nseg), 0, c->stream, c->g.nx,
-                     c->g.ny, nz, nseg, static_cast<T*>(c->spec), c->d_a, c->d_c, sg, c->cxn,
-                     c->cyn);
+  hipLaunchKernelGGL((k_trid_seg<T, M, kCw, S>), dim3(seg_blocks<kCw>(c->g.nx, c->g.ny)),
+                     dim3(kCw * nseg), 0, c->stream, c->g.nx, c->g.ny, nz, nseg,
+                     static_cast<T*>(c->spec), c->d_a, c->d_c, sg, c->cxn, c->cyn);
 }
 template <typename T>
 void trid_seg_t(pll_context* c) {
+  static_assert(seg_planes(256) == 8 && seg_planes(384) == 12 && seg_planes(512) == 8 &&
+                    seg_planes(kSegPlanes) == 12,
+                "the instances below");
   const int nz = c->g.nz;
-  if (nz <= 384) {
-    switch (seg_planes(nz)) {
-      case 8: trid_seg<T, 8, 16>(c); break;
-      case 16: trid_seg<T, 16, 16>(c); break;
-      default: trid_seg<T, 24, 16>(c); break;
-    }
-  } else if (nz <= 512) {
-    trid_seg<T, 16, 32>(c);
-  } else {
-    trid_seg<T, 24, 32>(c);
-  }
+  if (nz <= 128)
+    trid_seg<T, 8, 16>(c);
+  else if (nz <= 256)
+    trid_seg<T, 8, 32>(c);
+  else if (nz <= 384)
+    trid_seg<T, 12, 32>(c);
+  else if (nz <= 512)
+    trid_seg<T, 8, 64>(c);
+  else
+    trid_seg<T, 12, 64>(c);
 }
 }  // namespace
 
 int launch_trid_step(pll_context* c) {
-  // columns deeper than the segments hold take the sequential kernel
-  // (FP32-mixed at 1536x768x512: 2397 us partitioned against 2533 us
-  // sequential, since its recurrence runs on reciprocals)
+  // columns deeper than the segments hold take the sequential kernel (2533 against
+  // 1420 us in FP32-mixed at 1536x768x512)
   if (!c->d_seg || c->g.nz > kSegPlanes) return launch_trid(c);
   TimerScope ts(c, K_TRID);
   if (c->prec == PLL_FP64)
