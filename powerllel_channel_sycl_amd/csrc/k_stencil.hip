@@ -557,9 +557,9 @@ __global__ __launch_bounds__(kRkTx * kLateTy, 4) void k_rk_late(
 }
 
 // Tile rows of k_rk12: one block of them fills a CU either way.  FP64 12 (160
-// VGPRs: three waves per SIMD; with two barriers a plane 8 and 10 rows ran 3021
-// and 2679 against 2348 us at 768x384x384, 16 rows spill), FP32 16 (1302 against
-// 1312 us with 8 and 1440 with 12; 6934 against 7111 us with 8 at 1536x768x512).
+// VGPRs: three waves per SIMD; 16 rows spill), FP32 16.  Measured with two barriers
+// a plane: FP64 8 and 10 rows 3021 and 2679 against 2348 us at 768x384x384, FP32
+// 8 and 12 rows 1312 and 1440 against 1302.
 template <typename T>
 constexpr int kRk12Ty() {
   return std::is_same<T, double>::value ? 12 : 16;
@@ -588,20 +588,19 @@ constexpr int kRk12Slots = 256;  // blocks of k_rk12 that run at once: one per C
 // commit of source plane q+2, so the waves of a block drift apart within it and
 // one's LDS reads overlap another's arithmetic.  The carry holds what plane k-1
 // would be read for, so each ring is two planes and the one being written.  The
-// fetch only issues the loads of a plane; the projection, forcing and boundary
-// rules apply at its commit, and stage 2's results are stored after the commit:
-// arithmetic on the loaded values in the fetch, or stores ahead of the commit,
-// would make a wave wait there.
+// projection, forcing and boundary rules apply at a plane's commit, and stage 2's
+// results are stored after the commit: arithmetic on the loaded values in the
+// fetch, or stores ahead of the commit, would make a wave wait there.
 //
-// Bound by issue and LDS together at one block per CU: FP64 at 768x384x384 keeps
-// the VALU 44 % and the LDS 52 % busy at three waves per SIMD, with 56 B a point
-// of HBM traffic (2.8 TB/s).  2229 us for both stages there against 1646 + 2331
-// us for the two kernels it replaces (stage 2 with calcRHS; calcRHS in the
-// transform's loads costs 440 us more); 2348 us with two barriers a plane, 3058
-// with the reference's operation order as well.  135 us against 121 + 176 at
-// 256x192x128.  FP32: 1243 us (1456 with 8 rows, two barriers and
-// coefficients loaded per lane), 222 against 309 us at 384x256x192, half of which is
-// the chunk rule of rk12_grid.
+// What bounds it is the chain of a plane at one block per CU (leaving stage 2 out
+// saved 3 % in FP64 and nothing in FP32 when the loads were issued after stage 1):
+// so a plane's loads are issued first, each thread loads a pair of cells (6 or 7
+// wide loads instead of up to 14), and the waves that load are not those with ring
+// cells.  At 768x384x384 FP64 2261 -> 2010-2040 us (3.4 TB/s of 61 B a point),
+// FP32 1243 -> 1070; 256x192x128 FP64 128 -> 115, 384x256x192 FP32 213 -> 186,
+// 1536x768x512 FP32 6850 -> 6040.  Loads two planes ahead in a second set of
+// registers ran slower (FP32 1178: the registers are full and all waves load).
+// The two kernels that it replaces took 1646 + 2331 us (FP64, 768x384x384).
 template <typename T, int TY, bool U1OUT, bool CRF>
 __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
     Geom g, const T* __restrict__ su, const T* __restrict__ sv, const T* __restrict__ sw,
@@ -612,10 +611,14 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
   constexpr int TX = kRkTx, NT = TX * TY;
   constexpr int RX = TX + 2, RY = TY + 2, RPL = RX * RY;  // u1 region: tile + 1
   constexpr int UX = TX + 4, UY = TY + 4, UPL = UX * UY;  // source: tile + 2
-  constexpr int NPF = (UPL + NT - 1) / NT;
   constexpr int NRING = RPL - NT;  // region cells outside the tile
   static_assert(NRING == 2 * RX + 2 * TY && NRING <= NT, "one ring cell per thread");
-  __shared__ T ssrc[3][3][UPL];  // [field][plane % 3][cell]; cell (cx, cy) = (i0-1+cx, j0-1+cy)
+  // the source is loaded in pairs of x neighbours by waves that have no ring cells
+  constexpr int F0 = (NRING + 63) / 64 * 64;
+  static_assert(F0 + UPL / 2 <= NT && UX % 2 == 0, "one pair of source cells per thread");
+  using V2 = T __attribute__((ext_vector_type(2)));
+  typedef V2 V2u __attribute__((aligned(sizeof(T))));
+  __shared__ __align__(16) T ssrc[3][3][UPL];  // [field][plane % 3][cell]; cell (cx, cy) = (i0-1+cx, j0-1+cy)
   __shared__ ZCarry<T> szb[NRING];  // the ring cells' carry: few threads have one
   __shared__ T su1[3][3][RPL];   // [field][plane % 3][cell]; cell (rx, ry) = (i0+rx, j0+ry)
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
@@ -632,40 +635,39 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
     return;
   }
   auto wrap = [](int x, int n) { return ((x - 1) % n + n) % n + 1; };
-  int gaddr[NPF];  // plane-relative address of the periodic image (-1: past the tile)
-#pragma unroll
-  for (int n = 0; n < NPF; ++n) {
-    const int e = t + n * NT;
-    gaddr[n] = e < UPL ? wrap(i0 - 1 + e % UX, g.nx) + (int)g.sx * wrap(j0 - 1 + e / UX, g.ny) : -1;
-  }
-  T ru[NPF], rv[NPF], rw[NPF], rp0[NPF], rpe[NPF], rpn[NPF], rpt[NPF];
+  // plane-relative address of the pair's periodic image: its first cell's x is
+  // odd and nx even, so no pair straddles the wrap
+  const int e = 2 * (t - F0);
+  const bool loads = t >= F0 && e < UPL;
+  const int gaddr =
+      loads ? wrap(i0 - 1 + e % UX, g.nx) + (int)g.sx * wrap(j0 - 1 + e / UX, g.ny) : 0;
+  V2 ru{}, rv{}, rw{}, rp{}, rpn{}, rpt{};
+  T rpe = T(0);
   auto fetch = [&](int kk) {
     const bool ghost = kk == 0 || kk == g.nz + 1;
-    const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
-    const long o = g.sxy * ks;
-#pragma unroll
-    for (int n = 0; n < NPF; ++n)
-      if (gaddr[n] >= 0) {
-        const long a = gaddr[n] + o;
-        ru[n] = su[a];
-        rv[n] = sv[a];
-        rw[n] = sw[a];
-        rp0[n] = pp[a];
-        rpe[n] = pp[a + 1];
-        rpn[n] = pp[a + g.sx];
-        rpt[n] = pp[a + g.sxy];
-      }
+    const long o = g.sxy * (ghost ? (kk == 0 ? 1 : g.nz) : kk);
+    if (loads) {
+      auto at = [&](const T* f, long d) { return *reinterpret_cast<const V2u*>(f + (o + d) + gaddr); };
+      ru = at(su, 0);
+      rv = at(sv, 0);
+      rw = at(sw, 0);
+      rp = at(pp, 0);
+      rpe = pp[o + 2 + gaddr];
+      rpn = at(pp, g.sx);
+      rpt = at(pp, g.sxy);
+    }
   };
   auto commit = [&](int kk, int slot) {
     const bool ghost = kk == 0 || kk == g.nz + 1;
     const int ks = ghost ? (kk == 0 ? 1 : g.nz) : kk;
     const bool wzero = kk == 0 || kk >= g.nz;
     const T dzci = uniform_load(q0.m.dzc_inv, ks);
+    if (loads) {
+      V2 su2, sv2, sw2;
 #pragma unroll
-    for (int n = 0; n < NPF; ++n)
-      if (gaddr[n] >= 0) {
-        const T p0 = rp0[n];
-        T qu = ru[n] - (rpe[n] - p0) * q0.dtdxi;
+      for (int n = 0; n < 2; ++n) {
+        const T p0 = rp[n], pe = n ? rpe : rp[1];
+        T qu = ru[n] - (pe - p0) * q0.dtdxi;
         T qv = rv[n] - (rpn[n] - p0) * q0.dtdyi;
         // same association as k_correct: ((p(k+1) - p(k)) * dt) * dzc_inv(k)
         T qw = rw[n] - (rpt[n] - p0) * q0.dt * dzci;
@@ -675,11 +677,14 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
           qu = T(2) * q0.bc_u - qu;  // src/mod_updateBound.cc:92,123
           qv = T(2) * T(0) - qv;
         }
-        const int e = t + n * NT;
-        ssrc[0][slot][e] = qu;
-        ssrc[1][slot][e] = qv;
-        ssrc[2][slot][e] = qw;
+        su2[n] = qu;
+        sv2[n] = qv;
+        sw2[n] = qw;
       }
+      *reinterpret_cast<V2*>(&ssrc[0][slot][e]) = su2;
+      *reinterpret_cast<V2*>(&ssrc[1][slot][e]) = sv2;
+      *reinterpret_cast<V2*>(&ssrc[2][slot][e]) = sw2;
+    }
   };
   // this thread's stage-1 cells: A = its own tile point, B = one ring cell (t < NRING)
   const int ra = (ty + 1) * RX + tx + 1;
@@ -748,6 +753,7 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
     const int k = q - 2;  // stage-2 plane
     // the next iteration's stage 1 reads source planes q+1, q+2
     const bool more = q < qe && q < g.nz;
+    if (more) fetch(q + 2);
     const T pu = nextu, pv = nextv, pw = nextw;
     nextu = za.u;
     nextv = za.v;
@@ -774,9 +780,6 @@ __global__ __launch_bounds__(kRkTx* TY) void k_rk12(
       ghost_top(ra);
       if (has_b) ghost_top(rb);
     }
-    // fetched here rather than before stage 1: its registers are then not
-    // live across both stages
-    if (more) fetch(q + 2);
     T nu = T(0), nv = T(0), nw = T(0);
     if (k >= k0 && active) {
       // u1 planes k = q-2 and q-1 are in the slots of q+1 and q+2
@@ -1342,14 +1345,15 @@ int rk_t(pll_context* c, int stage, int acc, int bcload) {
 // ring's start), so the chunk is the one with the least rounds x (chunk + 3);
 // of equal costs the shortest, whose last round is spread the most.  Against
 // chunks for about 1024 blocks: 230 against 255 us at 384x256x192 (FP32), 30
-// against 39 us at 160x96x96.
+// against 39 us at 160x96x96; against chunks of four planes and more 22 against 27
+// us at 64x64x64, 17 against 26 at 24x20x12.
 TileGrid rk12_grid(const pll_context* c, int ty, int slots) {
   TileGrid t;
   t.ntx = (c->g.nx + kRkTx - 1) / kRkTx;
   t.nty = (c->g.ny + ty - 1) / ty;
   const long cols = (long)t.ntx * t.nty;
   long best = 0;
-  for (int kc = std::min(4, c->g.nz); kc <= c->g.nz; ++kc) {
+  for (int kc = 1; kc <= c->g.nz; ++kc) {
     const long nkc = (c->g.nz + kc - 1) / kc;
     const long cost = ((cols * nkc + slots - 1) / slots) * (kc + 3);
     if (best && cost >= best) continue;
