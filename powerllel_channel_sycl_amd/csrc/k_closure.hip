@@ -92,15 +92,6 @@ __device__ inline void store_bf16_weight(uint16_t* __restrict__ wb, int i, float
     wb[kWb3 + i - oW3] = b;
 }
 
-// Orders a wave's LDS writes before its lanes' later LDS reads of them.  A
-// wave's LDS instructions execute in order, so this only has to keep the
-// compiler from moving memory operations across it.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---- register-resident network ---------------------------------------------
 // A 32 x 32 accumulator leaves lane l (half h = l/32) with one column and the
 // 16 rows hid_unit(j, h) (+32 per row block).  Used as the next product's A or B

@@ -15,11 +15,10 @@
 // columns at a time.
 //
 // Complex transforms use the Stockham autosort formulation, in place in one
-// LDS buffer with the butterflies in registers: lengths in common use are
-// compiled in, every other product of 2, 3 and 5 runs from a plan.  Twiddles
+// LDS buffer with the butterflies in registers: products of 2, 3 and 5 up to 768
+// are compiled in (fft_fixed.hpp), longer ones run from a plan.  Twiddles
 // are computed on the host in long double and rounded to the field precision.
-#include "fft_radix.hpp"
-#include "pll_internal.hpp"
+#include "fft_fixed.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -31,530 +30,15 @@ namespace pll {
 namespace {
 
 // ============================================================================
-// Compile-time transforms for the lengths of the supported grids.  One
-// padded LDS buffer per block; each pass reads its butterfly inputs into
-// registers, synchronises, and writes the outputs back in place, so every
-// thread does at most one radix-R butterfly per pass.  Index arithmetic is
-// constant-folded and the 6/8/12/16 butterflies keep the pass count at 2-3.
-// ============================================================================
-template <int L>
-struct Shape {
-  static constexpr int np = 0;
-  static constexpr int r[1] = {0};
-};
-#define PLL_SHAPE(LEN, ...)                          \
-  template <>                                        \
-  struct Shape<LEN> {                                \
-    static constexpr int r[] = {__VA_ARGS__};        \
-    static constexpr int np = sizeof(r) / sizeof(int); \
-  };
-PLL_SHAPE(4, 4)
-PLL_SHAPE(6, 6)
-PLL_SHAPE(12, 12)
-PLL_SHAPE(20, 4, 5)
-PLL_SHAPE(32, 8, 4)
-PLL_SHAPE(48, 8, 6)
-PLL_SHAPE(64, 8, 8)
-PLL_SHAPE(128, 16, 8)
-PLL_SHAPE(192, 16, 12)
-PLL_SHAPE(256, 16, 16)
-PLL_SHAPE(384, 8, 8, 6)
-PLL_SHAPE(768, 8, 8, 12)
-#undef PLL_SHAPE
-
-template <class SH>
-constexpr int shape_rmin() {
-  int m = 1 << 30;
-  for (int p = 0; p < SH::np; ++p) m = SH::r[p] < m ? SH::r[p] : m;
-  return m;
-}
-template <class SH, int P>
-constexpr int shape_span() {
-  int s = 1;
-  for (int p = 0; p < P; ++p) s *= SH::r[p];
-  return s;
-}
-// threads per sequence: every thread owns one butterfly of the smallest radix
-template <int L>
-constexpr int tps() {
-  return L / shape_rmin<Shape<L>>();
-}
-// one pad slot per 16 complex values spreads strided accesses over the banks
-__device__ __forceinline__ int pad(int x) { return x + (x >> 4); }
-constexpr int padded(int n) { return n + (n >> 4) + 1; }
-constexpr int kLdsMax = 64 * 1024;
-
-// rows per block of the x transforms (about 256 threads, LDS <= 64 KiB)
-template <typename T, int L>
-constexpr int x_rows() {
-  int nb = tps<L>() >= 256 ? 1 : 256 / tps<L>();
-  while (nb > 1 && padded(nb * L) * 2 * (int)sizeof(T) > kLdsMax) nb /= 2;
-  return nb;
-}
-// sequences per block of the y transforms: 128-byte rows, at most 1024 threads
-// and 64 KiB of LDS
-template <typename T, int L>
-constexpr int y_seqs() {
-  int q = 128 / (2 * (int)sizeof(T));
-  while (q > 1 && (q * tps<L>() > 1024 || padded(L * q) * 2 * (int)sizeof(T) > kLdsMax)) q /= 2;
-  return q;
-}
-
-
-template <typename T, int S, int L, int R, int NS, int ES>
-__device__ __forceinline__ void stockham_pass(cpx<T>* buf, const cpx<T>* __restrict__ twL,
-                                              int soff, int jj) {
-  constexpr int LR = L / R;
-  cpx<T> v[R];
-  const bool active = jj < LR;
-  if (active) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = buf[pad(soff + (jj + r * LR) * ES)];
-  }
-  __syncthreads();
-  if (active) {
-    const int k = jj % NS;
-    if (NS > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        cpx<T> w = twL[r * k * (L / (NS * R))];
-        if (S > 0) w.im = -w.im;
-        v[r] = cmul(v[r], w);
-      }
-    }
-    dft<T, R, S>(v);
-    const int base = (jj / NS) * NS * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) buf[pad(soff + (base + r * NS) * ES)] = v[r];
-  }
-  __syncthreads();
-}
-
-template <typename T, int S, int L, int ES, int P = 0>
-__device__ __forceinline__ void stockham(cpx<T>* buf, const cpx<T>* __restrict__ twL, int soff,
-                                         int jj) {
-  using SH = Shape<L>;
-  if constexpr (P < SH::np) {
-    stockham_pass<T, S, L, SH::r[P], shape_span<SH, P>(), ES>(buf, twL, soff, jj);
-    stockham<T, S, L, ES, P + 1>(buf, twL, soff, jj);
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ T& real_at(cpx<T>* buf, int e) {
-  return reinterpret_cast<T*>(buf)[2 * pad(e >> 1) + (e & 1)];
-}
-
-// the largest divisor of n that is at most m
-constexpr int chunk_of(int n, int m) {
-  int c = m < n ? m : n;
-  while (n % c) --c;
-  return c;
-}
-
-// The velocity divergence of calcRHS (src/mod_calcRHS.cc:7-33), for a forward
-// x transform that reads it straight from u, v, w instead of from p.
-template <typename T>
-struct RhsSrc {
-  const T* u;
-  const T* v;
-  const T* w;
-  const T* dzf_inv;
-  T dti, dtidxi, dtidyi;
-  // the velocity's boundary update did not run: the backward neighbours in
-  // the halo are read from their periodic images and w is the wall value 0
-  // on planes 0 and nz (src/mod_updateBound.cc:32-144)
-  int bcfold;
-};
-
-// forceVel's bulk mean and force of u (src/mod_calcVel.cc:287,297) from n block
-// partials of stage 2, as a block of its own in the forward transform that
-// follows: a launch of one block costs more than its work (5-6 us, of which a
-// step of 256x192x128 has 284).
-struct MeanJob {
-  const double* partial;
-  long n;  // 0: nothing to do
-  double nxg, nyg, vel_force;
-  double* mean;
-  double* force;
-};
-__device__ __forceinline__ void mean_job(const MeanJob& m) {
-  __shared__ double red[64];
-  const int W = blockDim.x < 64 ? (int)blockDim.x : 64, t = threadIdx.x;
-  if (t < W) {
-    double s = 0.0;
-    for (long i = t; i < m.n; i += 8 * W) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = i + u * W < m.n ? m.partial[i + u * W] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    red[t] = s;
-  }
-  __syncthreads();
-  if (t == 0) {
-    double s = 0.0;
-    for (int i = 0; i < W; ++i) s += red[i];
-    const double mean = s / m.nxg / m.nyg;
-    *m.mean = mean;
-    *m.force = m.vel_force - mean;
-  }
-}
-
-template <typename T>
-RhsSrc<T> rhs_src(const pll_context* c) {
-  const double dti = 1.0 / c->dt;  // src/mod_calcRHS.cc:11-13
-  return RhsSrc<T>{static_cast<const T*>(c->fld[PLL_U]), static_cast<const T*>(c->fld[PLL_V]),
-                   static_cast<const T*>(c->fld[PLL_W]),
-                   static_cast<const T*>(c->d_mesh) + (c->g.nz + 2),  // dzf_inv
-                   (T)dti, (T)(dti * c->dx_inv), (T)(dti * c->dy_inv), c->rhs_bcfold};
-}
-
-// execute_fft_fwd_xpen (src/mod_fft.cc:60-88), L = nx/2 points per row.  With
-// RHS the rows are calcRHS's output computed on load (nothing is stored in p).
-template <typename T, int L, bool RHS>
-__global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xf(Geom g, const T* __restrict__ p,
-                                                               T* __restrict__ spec,
-                                                               const cpx<T>* __restrict__ twL,
-                                                               const cpx<T>* __restrict__ rtw,
-                                                               long nrows, RhsSrc<T> rs,
-                                                               MeanJob mj) {
-  unsigned bid = blockIdx.x, nblk = gridDim.x;
-  if (RHS && mj.n) {
-    if (bid == 0) {
-      mean_job(mj);
-      return;
-    }
-    --bid;
-    --nblk;
-  }
-  constexpr int TPS = tps<L>(), NB = x_rows<T, L>(), NT = NB * TPS, N = 2 * L;
-  __shared__ cpx<T> buf[padded(NB * L)];
-  __shared__ long rowbase[NB];
-  __shared__ T rowdz[NB];
-  __shared__ long rowvs[NB];     // offset of the v row below (j-1, or its image)
-  __shared__ unsigned char roww[NB];  // bit 0: w below is the wall 0; bit 1: w is the wall 0
-  const long row0 = (long)xcd_remap(bid, nblk) * NB;
-  if (threadIdx.x < NB) {
-    const long r = row0 + threadIdx.x;
-    const int j = (int)(r % g.ny), k = (int)(r / g.ny);
-    rowbase[threadIdx.x] = r < nrows ? g.idx(1, j + 1, k + 1) : -1;
-    if (RHS) {
-      rowdz[threadIdx.x] = r < nrows ? rs.dti * rs.dzf_inv[k + 1] : T(0);
-      const bool f = rs.bcfold != 0;
-      rowvs[threadIdx.x] = (f && j == 0) ? (long)(g.ny - 1) * g.sx : -g.sx;
-      roww[threadIdx.x] = (unsigned char)((f && k == 0 ? 1 : 0) | (f && k + 1 == g.nz ? 2 : 0));
-    }
-  }
-  __syncthreads();
-  // NB*N values, NLD per thread, loaded in chunks of CH whose loads are all
-  // issued before the first is used
-  constexpr int NLD = NB * N / NT, CH = RHS ? chunk_of(NLD, 6) : NLD;
-  static_assert((NB * N) % NT == 0 && NLD % CH == 0, "whole rows per block");
-#pragma unroll
-  for (int u0 = 0; u0 < NLD; u0 += CH) {
-    T a0[CH], a1[CH], a2[CH], a3[CH], a4[CH], a5[CH];
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int e = threadIdx.x + (u0 + u) * NT;
-      const int s = e / N, i = e % N;
-      const long b = rowbase[s];
-      a0[u] = a1[u] = a2[u] = a3[u] = a4[u] = a5[u] = T(0);
-      if (b >= 0) {
-        const long c = b + i;
-        if (RHS) {
-          const long cw = (i == 0 && rs.bcfold) ? b + (N - 1) : c - 1;  // u(0) = u(nx)
-          const unsigned char wf = roww[s];
-          a0[u] = rs.u[c];
-          a1[u] = rs.u[cw];
-          a2[u] = rs.v[c];
-          a3[u] = rs.v[c + rowvs[s]];
-          if (!(wf & 2)) a4[u] = rs.w[c];
-          if (!(wf & 1)) a5[u] = rs.w[c - g.sxy];
-        } else {
-          a0[u] = p[c];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int e = threadIdx.x + (u0 + u) * NT;
-      const int s = e / N, i = e % N;
-      T val = a0[u];
-      if (RHS) {
-        // src/mod_calcRHS.cc:21-28, same association as k_calc_rhs
-        val = (a0[u] - a1[u]) * rs.dtidxi + (a2[u] - a3[u]) * rs.dtidyi + (a4[u] - a5[u]) * rowdz[s];
-      }
-      real_at(buf, s * L * 2 + i) = val;
-    }
-  }
-  __syncthreads();
-  const int s = threadIdx.x / TPS, jj = threadIdx.x % TPS;
-  stockham<T, -1, L, 1>(buf, twL, s * L, jj);
-  const long r = row0 + s;
-  if (r >= nrows) return;
-  cpx<T>* out = reinterpret_cast<cpx<T>*>(spec + r * N);
-  for (int kk = jj; kk < L; kk += TPS) {
-    const cpx<T> zk = buf[pad(s * L + kk)];
-    if (kk == 0) {
-      out[0] = cpx<T>{zk.re + zk.im, zk.re - zk.im};  // X0, X(n/2)
-    } else {
-      const cpx<T> zm = buf[pad(s * L + (L - kk))];
-      const T er = T(0.5) * (zk.re + zm.re), ei = T(0.5) * (zk.im - zm.im);
-      const T orr = T(0.5) * (zk.im + zm.im), oi = T(-0.5) * (zk.re - zm.re);
-      const cpx<T> w = rtw[kk];
-      out[kk] = cpx<T>{er + (w.re * orr - w.im * oi), ei + (w.re * oi + w.im * orr)};
-    }
-  }
-}
-
-// execute_fft_bwd_xpen (src/mod_fft.cc:90-120): perm rows -> p interior * norm.
-// With HALO (the step sequence, where updateBoundP follows at once) a row is
-// stored as aligned pairs p(0..nx+1), the two x-halo cells holding their
-// periodic values p(nx) and p(1), and a row whose copies updateBoundP puts on
-// the y halo or a wall's ghost plane is stored there too (row_images), so that
-// boundary update (src/mod_updateBound.cc:253-296) needs no pass of its own.
-// Offsets of row (j, k)'s copies (0: none): y the periodic image on the y halo,
-// z the zero-gradient ghost plane (src/mod_updateBound.cc:253-296).
-struct RowImage {
-  long y, z;
-};
-__device__ __forceinline__ RowImage row_images(const Geom& g, int j, int k) {
-  return RowImage{j == 0 ? (long)g.ny * g.sx : (j == g.ny - 1 ? -(long)g.ny * g.sx : 0),
-                  k == 0 ? -g.sxy : (k == g.nz - 1 ? g.sxy : 0)};
-}
-template <typename V>
-__device__ __forceinline__ void store_images(V* at, long stride, const RowImage& im, V val) {
-  at[0] = val;
-  if (im.y) at[im.y / stride] = val;
-  if (im.z) at[im.z / stride] = val;
-  if (im.y && im.z) at[(im.y + im.z) / stride] = val;
-}
-
-template <typename T, int L, bool HALO>
-__global__ __launch_bounds__((x_rows<T, L>() * tps<L>())) void k_xb(Geom g, const T* __restrict__ spec,
-                                                               T* __restrict__ p,
-                                                               const cpx<T>* __restrict__ twL,
-                                                               const cpx<T>* __restrict__ rtw,
-                                                               long nrows, T norm) {
-  constexpr int TPS = tps<L>(), NB = x_rows<T, L>(), NT = NB * TPS, N = 2 * L;
-  constexpr int RMIN = shape_rmin<Shape<L>>();
-  __shared__ cpx<T> buf[padded(NB * L)];
-  __shared__ long rowbase[NB];
-  __shared__ RowImage rowimg[NB];
-  const long row0 = (long)xcd_remap(blockIdx.x, gridDim.x) * NB;
-  if (threadIdx.x < NB) {
-    const long r = row0 + threadIdx.x;
-    const int j = (int)(r % g.ny), k = (int)(r / g.ny);
-    rowbase[threadIdx.x] = r < nrows ? g.idx(HALO ? 0 : 1, j + 1, k + 1) : -1;
-    if (HALO) rowimg[threadIdx.x] = row_images(g, j, k);
-  }
-  const cpx<T>* specc = reinterpret_cast<const cpx<T>*>(spec);
-  {
-    constexpr int NLD = NB * L / NT;
-    static_assert((NB * L) % NT == 0, "whole rows per block");
-    cpx<T> t[NLD];
-#pragma unroll
-    for (int u = 0; u < NLD; ++u) {
-      const int e = threadIdx.x + u * NT;
-      const long r = row0 + e / L;
-      t[u] = r < nrows ? specc[r * L + e % L] : cpx<T>{T(0), T(0)};
-    }
-#pragma unroll
-    for (int u = 0; u < NLD; ++u) buf[pad(threadIdx.x + u * NT)] = t[u];
-  }
-  __syncthreads();
-  const int s = threadIdx.x / TPS, jj = threadIdx.x % TPS;
-  // perm slot kk holds (Re Xkk, Im Xkk); slot 0 holds (X0, X(n/2))
-  cpx<T> z[RMIN];
-#pragma unroll
-  for (int u = 0; u < RMIN; ++u) {
-    const int kk = jj + u * TPS;
-    const cpx<T> a = buf[pad(s * L + kk)];
-    cpx<T> xk, xm;
-    if (kk == 0) {
-      xk = cpx<T>{a.re, T(0)};
-      xm = cpx<T>{a.im, T(0)};
-    } else {
-      xk = a;
-      xm = buf[pad(s * L + (L - kk))];
-    }
-    const cpx<T> sm{xk.re + xm.re, xk.im - xm.im};  // Xk + conj(X(h-k))
-    const cpx<T> d{xk.re - xm.re, xk.im + xm.im};   // Xk - conj(X(h-k))
-    const cpx<T> w{rtw[kk].re, -rtw[kk].im};        // exp(+2 pi i k/n)
-    const cpx<T> wd = cmul(w, d);
-    z[u] = cpx<T>{sm.re - wd.im, sm.im + wd.re};
-  }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < RMIN; ++u) buf[pad(s * L + jj + u * TPS)] = z[u];
-  __syncthreads();
-  stockham<T, +1, L, 1>(buf, twL, s * L, jj);
-  if (HALO) {
-    // pair q = (p(2q), p(2q+1)); p(i) is element i-1 of the row, p(0) = p(nx), p(nx+1) = p(1)
-    constexpr int NP = L + 1, NST = (NB * NP + NT - 1) / NT;
-    cpx<T> t[NST];
-#pragma unroll
-    for (int u = 0; u < NST; ++u) {
-      const int e = threadIdx.x + u * NT;
-      const int s2 = e / NP, q = e % NP;
-      if (e < NB * NP) {
-        const int e0 = q == 0 ? N - 1 : 2 * q - 1, e1 = q == L ? 0 : 2 * q;
-        t[u] = cpx<T>{norm * real_at(buf, s2 * N + e0), norm * real_at(buf, s2 * N + e1)};
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < NST; ++u) {
-      const int e = threadIdx.x + u * NT;
-      const int s2 = e / NP, q = e % NP;
-      if (e < NB * NP && rowbase[s2] >= 0)
-        store_images(reinterpret_cast<cpx<T>*>(p + rowbase[s2]) + q, 2, rowimg[s2], t[u]);
-    }
-  } else {
-    constexpr int NST = NB * N / NT;
-    static_assert((NB * N) % NT == 0, "whole rows per block");
-    T t[NST];
-#pragma unroll
-    for (int u = 0; u < NST; ++u) t[u] = norm * real_at(buf, threadIdx.x + u * NT);
-#pragma unroll
-    for (int u = 0; u < NST; ++u) {
-      const int e = threadIdx.x + u * NT;
-      const long b = rowbase[e / N];
-      if (b >= 0) p[b + e % N] = t[u];
-    }
-  }
-}
-
-// A y tile between global memory and LDS: NE complex slots, slot e = j*Q + q2
-// is the pair of columns (2 q2, 2 q2 + 1) of row j.  Each thread first issues
-// all of its loads (or LDS reads), then all of its LDS writes (or stores), so
-// a thread keeps ceil(NE/NT) memory operations in flight instead of one.
-template <typename T, int NE, int NT, int Q>
-__device__ __forceinline__ void load_tile(cpx<T>* buf, const T* plane, int nx) {
-  constexpr int NLD = (NE + NT - 1) / NT;
-  cpx<T> t[NLD];
-#pragma unroll
-  for (int u = 0; u < NLD; ++u) {
-    const int e = threadIdx.x + u * NT;
-    if (NE % NT == 0 || e < NE)
-      t[u] = reinterpret_cast<const cpx<T>*>(plane + (long)(e / Q) * nx)[e % Q];
-  }
-#pragma unroll
-  for (int u = 0; u < NLD; ++u) {
-    const int e = threadIdx.x + u * NT;
-    if (NE % NT == 0 || e < NE) buf[pad(e)] = t[u];
-  }
-}
-template <typename T, int NE, int NT, int Q>
-__device__ __forceinline__ void store_tile(const cpx<T>* buf, T* plane, int nx) {
-  constexpr int NLD = (NE + NT - 1) / NT;
-  cpx<T> t[NLD];
-#pragma unroll
-  for (int u = 0; u < NLD; ++u) {
-    const int e = threadIdx.x + u * NT;
-    if (NE % NT == 0 || e < NE) t[u] = buf[pad(e)];
-  }
-#pragma unroll
-  for (int u = 0; u < NLD; ++u) {
-    const int e = threadIdx.x + u * NT;
-    if (NE % NT == 0 || e < NE) reinterpret_cast<cpx<T>*>(plane + (long)(e / Q) * nx)[e % Q] = t[u];
-  }
-}
-
-// execute_fft_fwd_ypen (src/mod_fft.cc:122-153) on a tile of 2Q perm columns.
-template <typename T, int L>
-__global__ __launch_bounds__((y_seqs<T, L>() * tps<L>())) void k_yf(Geom g, T* __restrict__ spec,
-                                                                  const cpx<T>* __restrict__ twL,
-                                                                  int ntiles) {
-  constexpr int TPS = tps<L>(), Q = y_seqs<T, L>(), NT = Q * TPS, W = 2 * Q;
-  __shared__ cpx<T> buf[padded(L * Q)];
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = (int)(b % (unsigned)ntiles), k = (int)(b / (unsigned)ntiles);
-  T* plane = spec + (long)k * g.nx * g.ny + (long)tile * W;
-  // a slot holds the values of columns (2q, 2q+1) of one row: one 2-element load
-  load_tile<T, L * Q, NT, Q>(buf, plane, g.nx);
-  __syncthreads();
-  const int q = threadIdx.x % Q, jj = threadIdx.x / Q;
-  stockham<T, -1, L, Q>(buf, twL, q, jj);
-#pragma unroll
-  for (int mu = 0; mu <= L / 2 / TPS; ++mu) {
-    const int m = jj + mu * TPS;
-    if (m > L / 2) break;
-    const cpx<T> zm = buf[pad(m * Q + q)];
-    const cpx<T> zc = buf[pad(((L - m) % L) * Q + q)];
-    const T ar = T(0.5) * (zm.re + zc.re), ai = T(0.5) * (zm.im - zc.im);
-    const T br = T(0.5) * (zm.im + zc.im), bi = T(-0.5) * (zm.re - zc.re);
-    if (m == 0) {
-      reinterpret_cast<cpx<T>*>(plane)[q] = cpx<T>{ar, br};
-    } else if (m == L / 2) {
-      reinterpret_cast<cpx<T>*>(plane + g.nx)[q] = cpx<T>{ar, br};
-    } else {
-      reinterpret_cast<cpx<T>*>(plane + (long)(2 * m) * g.nx)[q] = cpx<T>{ar, br};
-      reinterpret_cast<cpx<T>*>(plane + (long)(2 * m + 1) * g.nx)[q] = cpx<T>{ai, bi};
-    }
-  }
-}
-
-// execute_fft_bwd_ypen (src/mod_fft.cc:155-187), unscaled.
-template <typename T, int L>
-__global__ __launch_bounds__((y_seqs<T, L>() * tps<L>())) void k_yb(Geom g, T* __restrict__ spec,
-                                                                  const cpx<T>* __restrict__ twL,
-                                                                  int ntiles) {
-  constexpr int TPS = tps<L>(), Q = y_seqs<T, L>(), NT = Q * TPS, W = 2 * Q;
-  __shared__ cpx<T> buf[padded(L * Q)];
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = (int)(b % (unsigned)ntiles), k = (int)(b / (unsigned)ntiles);
-  T* plane = spec + (long)k * g.nx * g.ny + (long)tile * W;
-  // Global row j, column pair q holds (perm_a[j], perm_b[j]) of columns 2q and
-  // 2q+1.  Rows 2m and 2m+1 (m = 1..L/2-1) give the complex inputs Z[m] and
-  // Z[L-m] of the pair's transform: with A = (e0.re, e1.re), B = (e0.im,
-  // e1.im), Z = A + iB below L/2 and conj(A) + i conj(B) above; rows 0 and 1
-  // hold Z[0] and Z[L/2].  Each thread loads its row pairs and writes the
-  // unpacked values to LDS directly.
-  {
-    constexpr int NE = (L / 2) * Q, NLD = (NE + NT - 1) / NT;
-    cpx<T> e0[NLD], e1[NLD];
-#pragma unroll
-    for (int u = 0; u < NLD; ++u) {
-      const int e = threadIdx.x + u * NT;
-      if (NE % NT == 0 || e < NE) {
-        const int mm = e / Q, q2 = e % Q;
-        e0[u] = reinterpret_cast<const cpx<T>*>(plane + (long)(2 * mm) * g.nx)[q2];
-        e1[u] = reinterpret_cast<const cpx<T>*>(plane + (long)(2 * mm + 1) * g.nx)[q2];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < NLD; ++u) {
-      const int e = threadIdx.x + u * NT;
-      if (NE % NT == 0 || e < NE) {
-        const int mm = e / Q, q2 = e % Q;
-        if (mm == 0) {
-          buf[pad(q2)] = e0[u];
-          buf[pad((L / 2) * Q + q2)] = e1[u];
-        } else {
-          buf[pad(mm * Q + q2)] = cpx<T>{e0[u].re - e1[u].im, e1[u].re + e0[u].im};
-          buf[pad((L - mm) * Q + q2)] = cpx<T>{e0[u].re + e1[u].im, e0[u].im - e1[u].re};
-        }
-      }
-    }
-  }
-  __syncthreads();
-  const int q = threadIdx.x % Q, jj = threadIdx.x / Q;
-  stockham<T, +1, L, Q>(buf, twL, q, jj);
-  store_tile<T, L * Q, NT, Q>(buf, plane, g.nx);
-}
-
-// ============================================================================
 // Run-time-plan transforms for every other length: the same one-buffer Stockham
 // passes with the radices of an FftPlan (fft_plan in fft_radix.hpp: the fewest
 // passes of radices 2..16, then the largest smallest radix), one butterfly per
 // thread and pass, so L = 100 takes two passes (10, 10) and one LDS buffer.
-// They are bound by HBM like the fixed-length kernels, so what matters is loads
-// in flight: kGenChunk loads per thread are issued before the first LDS write,
-// and blocks of about 256 threads and at most 32 KiB of LDS leave five or more
-// of them on a CU.  Against radix 4/2/3/5 passes ping-ponging in 64 KiB blocks:
-// the FP64 step at 200x90x176 294 -> 246 us (its four transforms 136 -> 88 us).
+// What matters is loads in flight: kGenChunk loads per thread are issued before
+// the first LDS write, and blocks of about 256 threads and at most 32 KiB of LDS
+// leave five or more of them on a CU.  Against radix 4/2/3/5 passes ping-ponging in
+// 64 KiB blocks the FP64 step at 200x90x176 took 246 instead of 294 us (its four
+// transforms 88 instead of 136; compiled in, 61).
 // ============================================================================
 // n / d by multiplication, m = ceil(2^32 / d): exact for n * d < 2^32, d > 1
 __device__ __forceinline__ int div_by(int n, unsigned m) { return (int)__umulhi((unsigned)n, m); }
@@ -978,14 +462,6 @@ int setup_t(pll_context* c) {
   return PLL_OK;
 }
 
-// The bulk mean that stage 2 left partials of, for the transform that runs next.
-MeanJob take_mean(pll_context* c) {
-  const long n = c->mean_pending;
-  c->mean_pending = 0;
-  return MeanJob{c->d_partial, n, (double)c->g.nx, (double)c->g.ny, c->vel_force[0], c->d_scalar,
-                 c->d_scalar + 3};
-}
-
 int round_wave(int n) { return (n + 63) / 64 * 64; }
 
 XShape x_shape(const pll_context* c) {
@@ -1039,109 +515,20 @@ int y_generic(pll_context* c, bool fwd) {
   return PLL_OK;
 }
 
-// ---- fixed-length kernels ------------------------------------------------------------
-template <typename T, int L>
-int x_fixed(pll_context* c, bool fwd, bool rhs = false) {
-  constexpr int NB = x_rows<T, L>(), NT = NB * tps<L>();
-  const long nrows = (long)c->g.ny * c->g.nz;
-  const unsigned blocks = (unsigned)((nrows + NB - 1) / NB);
-  const cpx<T>* tw = static_cast<const cpx<T>*>(c->d_twl_x);
-  const cpx<T>* rtw = static_cast<const cpx<T>*>(c->d_rtw_x);
-  if (fwd && rhs) {
-    const RhsSrc<T> rs = rhs_src<T>(c);
-    const MeanJob mj = take_mean(c);
-    TimerScope ts(c, K_FFT_X_FWD_RHS);
-    hipLaunchKernelGGL((k_xf<T, L, true>), dim3(blocks + (mj.n ? 1 : 0)), dim3(NT), 0, c->stream, c->g,
-                       static_cast<const T*>(nullptr), static_cast<T*>(c->spec), tw, rtw, nrows, rs, mj);
-  } else if (fwd) {
-    TimerScope ts(c, K_FFT_X_FWD);
-    hipLaunchKernelGGL((k_xf<T, L, false>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
-                       static_cast<const T*>(c->fld[PLL_P]), static_cast<T*>(c->spec), tw, rtw,
-                       nrows, RhsSrc<T>{}, MeanJob{});
-  } else {
-    const double norm = 1.0 / (c->g.nx * c->g.ny);  // src/mod_fft.cc:57
-    TimerScope ts(c, K_FFT_X_BWD);
-    if (rhs) {  // inside the step: updateBoundP follows, x halos may be written
-      hipLaunchKernelGGL((k_xb<T, L, true>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
-                         static_cast<const T*>(c->spec), static_cast<T*>(c->fld[PLL_P]), tw, rtw,
-                         nrows, (T)norm);
-    } else {
-      hipLaunchKernelGGL((k_xb<T, L, false>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
-                         static_cast<const T*>(c->spec), static_cast<T*>(c->fld[PLL_P]), tw, rtw,
-                         nrows, (T)norm);
-    }
-  }
-  PLL_HIP_TRY(hipGetLastError());
-  return PLL_OK;
-}
-
-template <typename T, int L>
-bool y_fixed_fits(const pll_context* c) {
-  return c->g.nx % (2 * y_seqs<T, L>()) == 0;
-}
-
-template <typename T, int L>
-int y_fixed(pll_context* c, bool fwd) {
-  constexpr int Q = y_seqs<T, L>(), NT = Q * tps<L>();
-  const int ntiles = c->g.nx / (2 * Q);
-  const unsigned blocks = (unsigned)ntiles * c->g.nz;
-  const cpx<T>* tw = static_cast<const cpx<T>*>(c->d_twl_y);
-  if (fwd) {
-    TimerScope ts(c, K_FFT_Y_FWD);
-    hipLaunchKernelGGL((k_yf<T, L>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
-                       static_cast<T*>(c->spec), tw, ntiles);
-  } else {
-    TimerScope ts(c, K_FFT_Y_BWD);
-    hipLaunchKernelGGL((k_yb<T, L>), dim3(blocks), dim3(NT), 0, c->stream, c->g,
-                       static_cast<T*>(c->spec), tw, ntiles);
-  }
-  PLL_HIP_TRY(hipGetLastError());
-  return PLL_OK;
-}
-
-#define PLL_X_SIZES(X) X(4) X(12) X(32) X(48) X(128) X(192) X(384) X(768)
-#define PLL_Y_SIZES(X) X(6) X(20) X(48) X(64) X(192) X(256) X(384) X(768)
-
-template <typename T>
-bool x_has_fixed(int L) {
-#define PLL_CASE(n) if (L == n) return true;
-  PLL_X_SIZES(PLL_CASE)
-#undef PLL_CASE
-  return false;
-}
-
-template <typename T>
-bool y_has_fixed(const pll_context* c, int L) {
-#define PLL_CASE(n) if (L == n) return y_fixed_fits<T, n>(c);
-  PLL_Y_SIZES(PLL_CASE)
-#undef PLL_CASE
-  return false;
-}
-
 // step: calcRHS in the forward loads, periodic halos in the inverse's stores
 template <typename T>
 int x_t(pll_context* c, bool fwd, bool step = false) {
-  if (c->x_fixed) {
-    switch (c->g.nx / 2) {
-#define PLL_CASE(n) case n: return x_fixed<T, n>(c, fwd, step);
-      PLL_X_SIZES(PLL_CASE)
-#undef PLL_CASE
-      default: break;
-    }
-  }
+  if (c->x_fixed)
+    return fwd ? fft_fixed<T, FftPass::x_fwd>(c, c->g.nx / 2, step)
+               : fft_fixed<T, FftPass::x_bwd>(c, c->g.nx / 2, step);
   return x_generic<T>(c, fwd, step);
 }
 
 template <typename T>
 int y_t(pll_context* c, bool fwd) {
-  if (c->y_fixed) {
-    switch (c->g.ny) {
-#define PLL_CASE(n) case n: return y_fixed<T, n>(c, fwd);
-      PLL_Y_SIZES(PLL_CASE)
-#undef PLL_CASE
-      default: break;
-    }
-  }
+  if (c->y_fixed)
+    return fwd ? fft_fixed<T, FftPass::y_fwd>(c, c->g.ny, false)
+               : fft_fixed<T, FftPass::y_bwd>(c, c->g.ny, false);
   return y_generic<T>(c, fwd);
 }
 
@@ -1161,8 +548,8 @@ template <typename T>
 int setup_fixed(pll_context* c) {
   const char* env = std::getenv("PLL_FFT_GENERIC");
   const bool force_generic = env && env[0] == '1';
-  c->x_fixed = !force_generic && x_has_fixed<T>(c->g.nx / 2);
-  c->y_fixed = !force_generic && y_has_fixed<T>(c, c->g.ny);
+  c->x_fixed = !force_generic && fixed_length(c->g.nx / 2);
+  c->y_fixed = !force_generic && fixed_length(c->g.ny);
   int rc;
   if ((rc = unit_table<T>(c, c->g.nx / 2, &c->d_twl_x))) return rc;
   if ((rc = unit_table<T>(c, c->g.ny, &c->d_twl_y))) return rc;

@@ -38,6 +38,15 @@ __device__ __forceinline__ T uniform_load(const T* p, long k) {
   return reinterpret_cast<C*>(reinterpret_cast<uintptr_t>(p))[k];
 }
 
+// Orders a wave's LDS writes before its lanes' later LDS reads of them.  A
+// wave's LDS instructions execute in order, so this only has to keep the
+// compiler from moving memory operations across it.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Stockham plan of a complex transform of length L held in LDS.
 constexpr int kMaxPass = 8;
 struct FftPlan {
@@ -257,6 +266,10 @@ int launch_check_nan(pll_context* c, int field, int* passed);
 
 // transforms and the tridiagonal solve (k_fft.hip, k_trid.hip)
 int fft_setup(pll_context* c);
+// One pass of the transforms with a compiled-in length n (k_fft_fixed.hip).
+enum class FftPass { x_fwd, x_bwd, y_fwd, y_bwd };
+template <typename T, FftPass PASS>
+int fft_fixed(pll_context* c, int n, bool step);
 int launch_fft_x_fwd(pll_context* c);
 // calcRHS fused into the forward x transform (reads u, v, w; p is not written);
 // takes along the bulk mean that force_from_partials left
