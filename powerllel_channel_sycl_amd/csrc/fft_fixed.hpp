@@ -363,6 +363,21 @@ __device__ __forceinline__ void store_images(V* at, long stride, const RowImage&
   if (im.y && im.z) at[(im.y + im.z) / stride] = val;
 }
 
+// Elements 2n and 2n+1 of a row of p with interior at `out`, its x halos and images.
+template <typename T>
+__device__ __forceinline__ void store_halo(T* out, const RowImage& im, int n, int L, cpx<T> v) {
+  auto at = [&](long d) {
+    T* o = out + d;
+    store_two(o + 2 * n, v);
+    if (n == 0) o[2 * L] = v.re;   // p(nx+1) = p(1)
+    if (n == L - 1) o[-1] = v.im;  // p(0) = p(nx)
+  };
+  at(0);
+  if (im.y) at(im.y);
+  if (im.z) at(im.z);
+  if (im.y && im.z) at(im.y + im.z);
+}
+
 template <typename T, int L, bool HALO>
 __global__ __launch_bounds__((x_rows<L>() * tps<L>())) void k_xb(Geom g, const T* __restrict__ spec,
                                                                T* __restrict__ p,
@@ -412,16 +427,7 @@ __global__ __launch_bounds__((x_rows<L>() * tps<L>())) void k_xb(Geom g, const T
       store_two(out + 2 * n, v);
       return;
     }
-    auto at = [&](long d) {
-      T* o = out + d;
-      store_two(o + 2 * n, v);
-      if (n == 0) o[N] = v.re;       // p(nx+1) = p(1)
-      if (n == L - 1) o[-1] = v.im;  // p(0) = p(nx)
-    };
-    at(0);
-    if (im.y) at(im.y);
-    if (im.z) at(im.z);
-    if (im.y && im.z) at(im.y + im.z);
+    store_halo(out, im, n, L, v);
   };
   if constexpr (NP == 1) {
     if (r >= nrows) return;

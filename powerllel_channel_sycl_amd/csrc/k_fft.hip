@@ -389,6 +389,211 @@ __global__ __launch_bounds__(kGenThreads) void k_gyb(Geom g, T* __restrict__ spe
     reinterpret_cast<cpx<T>*>(plane + (long)j * g.nx)[q] = buf[pad(j * Q + q)];
 }
 
+// ============================================================================
+// Whole planes: on the smallest x-y planes one kernel each way runs both transforms
+// of the step (calcRHS in the loads, p's boundary update in the stores).  A step of
+// such a grid is a chain of launches, 3-4 us each for the host: four instead of
+// six.  24x20x12 (FP64, 10 steps): 172 against 237 us where several runs share the
+// host's launches, 358 against 359 us for one run alone.
+// Complex slot j Lx + q of the buffer is element q of row j to the x transforms and,
+// after their split, the column pair (2q, 2q+1) of row j to the y transforms.
+// ============================================================================
+// The largest plane that they take, in complex slots nx/2 ny: one block a plane is a
+// longer chain of passes than two kernels of many blocks, and beyond 512 slots a
+// run alone loses more to it than the launches cost (FP64 32x32x64 37.4 -> 36.1 us a
+// step, 48x48x32 34.3 -> 38.6, 64x64x64 41.7 -> 47.0).
+constexpr int kPlaneSlots = 512;
+struct PlaneShape {
+  int bx, lby;            // rows, log2 of the column pairs that the block transforms at a time
+  unsigned mtps, mL, mH;  // dividing by plan_x.tps (tps = 1: unused), Lx and Lx/2 + 1
+};
+
+// Both directions of x on the plane's rows, rows of a batch side by side.
+template <typename T, int S>
+__device__ __forceinline__ void plane_x(cpx<T>* buf, const Geom& g, const FftPlan& px,
+                                        const PlaneShape& ps, const cpx<T>* __restrict__ tw) {
+  const int s = px.tps > 1 ? div_by(threadIdx.x, ps.mtps) : (int)threadIdx.x;
+  const int jj = (int)threadIdx.x - s * px.tps;
+  for (int r0 = 0; r0 < g.ny; r0 += ps.bx)
+    plan_fft<T, S>(buf, px, tw, (r0 + s) * px.L, 1, jj, s < ps.bx && r0 + s < g.ny);
+}
+template <typename T, int S>
+__device__ __forceinline__ void plane_y(cpx<T>* buf, const FftPlan& px, const FftPlan& py,
+                                        const PlaneShape& ps, const cpx<T>* __restrict__ tw) {
+  const int by = 1 << ps.lby, q = (int)threadIdx.x & (by - 1), jj = (int)threadIdx.x >> ps.lby;
+  for (int q0 = 0; q0 < px.L; q0 += by)
+    plan_fft<T, S>(buf, py, tw, q0 + q, px.L, jj, jj < py.tps && q0 + q < px.L);
+}
+
+// src/mod_calcRHS.cc:7-33, then src/mod_fft.cc:60-88 and :122-153
+template <typename T>
+__global__ __launch_bounds__(kPlaneSlots / 2) void k_plane_fwd(
+    Geom g, T* __restrict__ spec, FftPlan px, FftPlan py, PlaneShape ps,
+    const cpx<T>* __restrict__ twx, const cpx<T>* __restrict__ rtw,
+    const cpx<T>* __restrict__ twy, RhsSrc<T> rs, MeanJob mj) {
+  int k = blockIdx.x;  // plane k+1
+  if (mj.n) {
+    if (k == 0) {
+      mean_job(mj);
+      return;
+    }
+    --k;
+  }
+  extern __shared__ __align__(16) unsigned char smem[];
+  cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
+  const int L = px.L, N = 2 * L, NT = blockDim.x, total = g.ny * L;
+  const bool f = rs.bcfold != 0;
+  const bool below0 = f && k == 0, top0 = f && k + 1 == g.nz;  // w is the wall 0
+  const T dz = rs.dti * rs.dzf_inv[k + 1];
+  const long b0 = g.idx(1, 1, k + 1);
+  constexpr int CH = 2;
+  for (int e0 = threadIdx.x; e0 < total; e0 += CH * NT) {
+    T ul[CH];
+    cpx<T> uu[CH], vv[CH], vb[CH], ww[CH], wb[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT;
+      if (e < total) {
+        const int j = div_by(e, ps.mL), i = 2 * (e - j * L);
+        const long c = b0 + (long)j * g.sx;
+        uu[u] = load_two(rs.u + c + i);
+        ul[u] = rs.u[c + (i == 0 && f ? N - 1 : i - 1)];  // u(0) = u(nx)
+        vv[u] = load_two(rs.v + c + i);
+        vb[u] = load_two(rs.v + c + (f && j == 0 ? (long)(g.ny - 1) * g.sx : -g.sx) + i);
+        ww[u] = load_two(rs.w + c + i);
+        wb[u] = load_two(rs.w + c - g.sxy + i);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT;
+      if (e < total) {
+        if (top0) ww[u] = cpx<T>{T(0), T(0)};
+        if (below0) wb[u] = cpx<T>{T(0), T(0)};
+        // src/mod_calcRHS.cc:21-28, same association as k_calc_rhs
+        buf[pad(e)] = cpx<T>{(uu[u].re - ul[u]) * rs.dtidxi + (vv[u].re - vb[u].re) * rs.dtidyi +
+                                 (ww[u].re - wb[u].re) * dz,
+                             (uu[u].im - uu[u].re) * rs.dtidxi + (vv[u].im - vb[u].im) * rs.dtidyi +
+                                 (ww[u].im - wb[u].im) * dz};
+      }
+    }
+  }
+  __syncthreads();
+  plane_x<T, -1>(buf, g, px, ps, twx);
+  // split the rows in place: one thread takes slots kk and L - kk
+  const int H = L / 2 + 1;
+  for (int e = threadIdx.x; e < g.ny * H; e += NT) {
+    const int j = div_by(e, ps.mH), kk = e - j * H;
+    auto half = [&](cpx<T> zk, cpx<T> zm, int n) {
+      const T er = T(0.5) * (zk.re + zm.re), ei = T(0.5) * (zk.im - zm.im);
+      const T orr = T(0.5) * (zk.im + zm.im), oi = T(-0.5) * (zk.re - zm.re);
+      const cpx<T> w = rtw[n];
+      return cpx<T>{er + (w.re * orr - w.im * oi), ei + (w.re * oi + w.im * orr)};
+    };
+    cpx<T>& lo = buf[pad(j * L + kk)];
+    const cpx<T> a = lo;
+    if (kk == 0) {
+      lo = cpx<T>{a.re + a.im, a.re - a.im};  // X0, X(n/2)
+    } else if (2 * kk <= L) {
+      cpx<T>& hi = buf[pad(j * L + (L - kk))];
+      const cpx<T> b = hi;
+      lo = half(a, b, kk);
+      if (2 * kk != L) hi = half(b, a, L - kk);
+    }
+  }
+  __syncthreads();
+  plane_y<T, -1>(buf, px, py, ps, twy);
+  cpx<T>* out = reinterpret_cast<cpx<T>*>(spec + (long)k * g.nx * g.ny);
+  for (int e = threadIdx.x; e < (g.ny / 2 + 1) * L; e += NT) {
+    const int m = div_by(e, ps.mL), q = e - m * L;
+    const cpx<T> zm = buf[pad(m * L + q)];
+    const cpx<T> zc = buf[pad((m == 0 ? 0 : g.ny - m) * L + q)];
+    const cpx<T> re{T(0.5) * (zm.re + zc.re), T(0.5) * (zm.im + zc.im)};
+    const cpx<T> im{T(0.5) * (zm.im - zc.im), T(-0.5) * (zm.re - zc.re)};
+    if (m == 0) {
+      out[q] = re;
+    } else if (2 * m == g.ny) {
+      out[L + q] = re;
+    } else {
+      out[2 * m * L + q] = re;
+      out[(2 * m + 1) * L + q] = im;
+    }
+  }
+}
+
+// src/mod_fft.cc:155-187 and :90-120, then src/mod_updateBound.cc:253-296
+template <typename T>
+__global__ __launch_bounds__(kPlaneSlots / 2) void k_plane_bwd(
+    Geom g, const T* __restrict__ spec, T* __restrict__ p, FftPlan px, FftPlan py, PlaneShape ps,
+    const cpx<T>* __restrict__ twx, const cpx<T>* __restrict__ rtw,
+    const cpx<T>* __restrict__ twy, T norm) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  cpx<T>* buf = reinterpret_cast<cpx<T>*>(smem);
+  const int k = blockIdx.x, L = px.L, NT = blockDim.x;
+  // rows 2m and 2m+1 unpack into the complex inputs Z[m] and Z[ny-m] (k_yb)
+  const cpx<T>* in = reinterpret_cast<const cpx<T>*>(spec + (long)k * g.nx * g.ny);
+  constexpr int CH = 2;
+  const int half = g.ny / 2 * L;
+  for (int e0 = threadIdx.x; e0 < half; e0 += CH * NT) {
+    cpx<T> r0[CH], r1[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT;
+      if (e < half) {
+        const int m = div_by(e, ps.mL), q = e - m * L;
+        r0[u] = in[2 * m * L + q];
+        r1[u] = in[(2 * m + 1) * L + q];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int e = e0 + u * NT;
+      if (e < half) {
+        const int m = div_by(e, ps.mL), q = e - m * L;
+        if (m == 0) {
+          buf[pad(q)] = r0[u];
+          buf[pad(g.ny / 2 * L + q)] = r1[u];
+        } else {
+          buf[pad(m * L + q)] = cpx<T>{r0[u].re - r1[u].im, r1[u].re + r0[u].im};
+          buf[pad((g.ny - m) * L + q)] = cpx<T>{r0[u].re + r1[u].im, r0[u].im - r1[u].re};
+        }
+      }
+    }
+  }
+  __syncthreads();
+  plane_y<T, +1>(buf, px, py, ps, twy);
+  // perm slot kk holds (Re Xkk, Im Xkk); slot 0 holds (X0, X(n/2)).  One thread
+  // merges slots kk and L - kk.
+  const int H = L / 2 + 1;
+  for (int e = threadIdx.x; e < g.ny * H; e += NT) {
+    const int j = div_by(e, ps.mH), kk = e - j * H;
+    auto merge = [&](cpx<T> xk, cpx<T> xm, int n) {
+      const cpx<T> sm{xk.re + xm.re, xk.im - xm.im};  // Xk + conj(X(h-k))
+      const cpx<T> d{xk.re - xm.re, xk.im + xm.im};   // Xk - conj(X(h-k))
+      const cpx<T> w{rtw[n].re, -rtw[n].im};          // exp(+2 pi i k/n)
+      const cpx<T> wd = cmul(w, d);
+      return cpx<T>{sm.re - wd.im, sm.im + wd.re};
+    };
+    cpx<T>& lo = buf[pad(j * L + kk)];
+    const cpx<T> a = lo;
+    if (kk == 0) {
+      lo = merge(cpx<T>{a.re, T(0)}, cpx<T>{a.im, T(0)}, 0);
+    } else if (2 * kk <= L) {
+      cpx<T>& hi = buf[pad(j * L + (L - kk))];
+      const cpx<T> b = hi;
+      lo = merge(a, b, kk);
+      if (2 * kk != L) hi = merge(b, a, L - kk);
+    }
+  }
+  __syncthreads();
+  plane_x<T, +1>(buf, g, px, ps, twx);
+  for (int e = threadIdx.x; e < g.ny * L; e += NT) {
+    const int j = div_by(e, ps.mL), n = e - j * L;
+    const cpx<T> z = buf[pad(e)];
+    store_halo(p + g.idx(1, j + 1, k + 1), row_images(g, j, k), n, L, cpx<T>{norm * z.re, norm * z.im});
+  }
+}
+
 // ---- host side -------------------------------------------------------------------
 unsigned magic(int d) { return (unsigned)((0x100000000ULL + (unsigned)d - 1) / (unsigned)d); }
 
@@ -544,6 +749,42 @@ int unit_table(pll_context* c, int L, void** dst) {
   return upload_table<T>(c, t, dst);
 }
 
+void setup_plane(pll_context* c) {
+  const long slots = (long)c->g.nx / 2 * c->g.ny;
+  // two slots a thread; plans of so short rows and columns take no more threads
+  c->plane_threads = slots <= kPlaneSlots
+                         ? std::max(round_wave((int)(slots + 1) / 2),
+                                    round_wave(std::max(c->plan_x.tps, c->plan_y.tps)))
+                         : 0;
+}
+template <typename T>
+int plane_t(pll_context* c, bool fwd) {
+  const int L = c->g.nx / 2, nt = c->plane_threads;
+  PlaneShape ps{nt / c->plan_x.tps, 0, c->plan_x.tps > 1 ? magic(c->plan_x.tps) : 0,
+                magic(L), magic(L / 2 + 1)};
+  while ((c->plan_y.tps << (ps.lby + 1)) <= nt && (1 << ps.lby) < L) ++ps.lby;
+  const cpx<T>* twx = static_cast<const cpx<T>*>(c->d_twl_x);
+  const cpx<T>* twy = static_cast<const cpx<T>*>(c->d_twl_y);
+  const cpx<T>* rtw = static_cast<const cpx<T>*>(c->d_rtw_x);
+  T* spec = static_cast<T*>(c->spec);
+  const size_t lds = (size_t)padded(c->g.ny * L) * 2 * sizeof(T);
+  if (fwd) {
+    const MeanJob mj = take_mean(c);
+    TimerScope ts(c, K_PLANE_FWD);
+    hipLaunchKernelGGL((k_plane_fwd<T>), dim3(c->g.nz + (mj.n ? 1 : 0)), dim3(nt), lds,
+                       c->stream, c->g, spec, c->plan_x, c->plan_y, ps, twx, rtw, twy, rhs_src<T>(c),
+                       mj);
+  } else {
+    const double norm = 1.0 / (c->g.nx * c->g.ny);  // src/mod_fft.cc:57
+    TimerScope ts(c, K_PLANE_BWD);
+    hipLaunchKernelGGL((k_plane_bwd<T>), dim3(c->g.nz), dim3(nt), lds, c->stream, c->g,
+                       static_cast<const T*>(spec), static_cast<T*>(c->fld[PLL_P]), c->plan_x,
+                       c->plan_y, ps, twx, rtw, twy, (T)norm);
+  }
+  PLL_HIP_TRY(hipGetLastError());
+  return PLL_OK;
+}
+
 template <typename T>
 int setup_fixed(pll_context* c) {
   const char* env = std::getenv("PLL_FFT_GENERIC");
@@ -553,6 +794,7 @@ int setup_fixed(pll_context* c) {
   int rc;
   if ((rc = unit_table<T>(c, c->g.nx / 2, &c->d_twl_x))) return rc;
   if ((rc = unit_table<T>(c, c->g.ny, &c->d_twl_y))) return rc;
+  if (!force_generic) setup_plane(c);
   return PLL_OK;
 }
 
@@ -577,6 +819,12 @@ int launch_fft_y_bwd(pll_context* c) { return c->prec == PLL_FP64 ? y_t<double>(
 
 int launch_poisson_step(pll_context* c, bool rhs) {
   int rc;
+  if (rhs && c->plane_threads) {
+    const bool f64 = c->prec == PLL_FP64;
+    if ((rc = f64 ? plane_t<double>(c, true) : plane_t<float>(c, true))) return rc;
+    if ((rc = launch_trid_step(c))) return rc;
+    return f64 ? plane_t<double>(c, false) : plane_t<float>(c, false);
+  }
   if ((rc = rhs ? launch_fft_x_fwd_rhs(c) : launch_fft_x_fwd(c))) return rc;
   if ((rc = launch_fft_y_fwd(c))) return rc;
   if ((rc = launch_trid_step(c))) return rc;

@@ -15,7 +15,7 @@ const char* const kKernelNames[K_COUNT] = {
     "rk1",         "rk2",       "calc_rhs",   "fft_x_fwd",    "fft_y_fwd", "solve_trid",
     "fft_y_bwd",   "fft_x_bwd", "correct_vel", "mean_partial", "mean_final", "force_add",
     "bc_vel",      "bc_p",      "check",      "init",         "misc",
-    "fft_x_fwd_rhs", "rk_closure", "rk12"};
+    "fft_x_fwd_rhs", "rk_closure", "rk12", "fft_plane_fwd", "fft_plane_bwd"};
 
 namespace {
 thread_local std::string g_last_error;

@@ -98,6 +98,8 @@ enum KernelId {
   K_FFT_X_FWD_RHS,  // calcRHS fused into the forward x transform
   K_RK_CLOSURE,     // RK stage with the learned eddy viscosity
   K_RK12,           // both RK stages of a step inside a run
+  K_PLANE_FWD,      // calcRHS and both forward transforms of a small plane
+  K_PLANE_BWD,      // both inverse transforms and p's boundary update
   K_COUNT
 };
 extern const char* const kKernelNames[K_COUNT];
@@ -153,6 +155,7 @@ struct pll_context {
   int rhs_bcfold = 0;  // calcRHS in the x transform reads halos through the boundary rules
   int x_batch = 1;  // rows per block of the run-time-plan x transforms
   int y_tile = 0;   // log2 of the column pairs per block of the y transforms
+  int plane_threads = 0;  // threads of the whole-plane transforms (0: not used)
 
   // reductions
   double* d_partial = nullptr;

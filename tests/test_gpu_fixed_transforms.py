@@ -101,3 +101,11 @@ def test_steps_match_the_routines(nx, ny, nz, precision):
     for a, b in zip(*out):
         # velocities of order one: FP64 round-off; FP32 the step's accumulated rounding
         assert np.max(np.abs(a - b)) < (1e-12 if precision == "fp64" else 1e-5)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32_mixed"])
+@pytest.mark.parametrize("nx,ny,nz", [(4, 4, 2), (24, 20, 12), (30, 18, 6), (6, 162, 4), (250, 4, 4),
+                                      (32, 32, 8), (64, 16, 6)])
+def test_steps_of_whole_planes_match_the_routines(nx, ny, nz, precision):
+    """Planes of up to 512 complex slots, odd nx/2 and the limit among them."""
+    test_steps_match_the_routines(nx, ny, nz, precision)
