@@ -145,11 +145,22 @@ __device__ __forceinline__ f32x16 bias_rows(const float* lb, int h, int t) {
   return c;
 }
 
+// NAN0: with the FP32 maximum instead, for which a NaN is 0 (batch inference; in
+// training, where a NaN input spoils the gradient in any case, it would cost 7 %).
+template <bool NAN0>
+__device__ __forceinline__ uint32_t pack_relu(float lo, float hi) {
+  if constexpr (NAN0)
+    return pack_bf16(fmaxf(lo, 0.f), fmaxf(hi, 0.f));
+  else
+    return pack_relu_bf16(lo, hi);
+}
+
 // BF16 of relu of accumulator elements j0 .. j0+7 as one MFMA operand.
+template <bool NAN0>
 __device__ __forceinline__ bf16x8 pack8_relu(const f32x16& z, int j0) {
   return __builtin_bit_cast(
-      bf16x8, (u32x4){pack_relu_bf16(z[j0], z[j0 + 1]), pack_relu_bf16(z[j0 + 2], z[j0 + 3]),
-                      pack_relu_bf16(z[j0 + 4], z[j0 + 5]), pack_relu_bf16(z[j0 + 6], z[j0 + 7])});
+      bf16x8, (u32x4){pack_relu<NAN0>(z[j0], z[j0 + 1]), pack_relu<NAN0>(z[j0 + 2], z[j0 + 3]),
+                      pack_relu<NAN0>(z[j0 + 4], z[j0 + 5]), pack_relu<NAN0>(z[j0 + 6], z[j0 + 7])});
 }
 __device__ __forceinline__ bf16x8 pack8(const f32x16& v, int j0) {
   return __builtin_bit_cast(
@@ -240,7 +251,7 @@ __device__ __forceinline__ void forward_regs(const NetLds<TRAIN>& N, const bf16x
 #pragma unroll
   for (int t = 0; t < 2; ++t) z1[t] = mfma(a1[t], xb, bias_rows(N.lb, h, t));
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) b1[kb] = pack8_relu(z1[kb / 2], 8 * (kb % 2));
+  for (int kb = 0; kb < 4; ++kb) b1[kb] = pack8_relu<!TRAIN>(z1[kb / 2], 8 * (kb % 2));
   z2[0] = bias_rows(N.lb + kH, h, 0);
   z2[1] = bias_rows(N.lb + kH, h, 1);
 #pragma unroll
@@ -252,6 +263,7 @@ __device__ __forceinline__ void forward_regs(const NetLds<TRAIN>& N, const bf16x
 
 // The output o of the lane's sample, in both halves: BF16 h2 times BF16 W3
 // (packed pairs w3[t][q], the lane's rows), FP32 sum.
+template <bool TRAIN>
 __device__ __forceinline__ float output_regs(const f32x16 z2[2], const uint32_t w3[2][8], float b3) {
   float part = 0.f;
 #pragma unroll
@@ -259,7 +271,7 @@ __device__ __forceinline__ float output_regs(const f32x16 z2[2], const uint32_t 
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       part = __builtin_amdgcn_fdot2_f32_bf16(
-          __builtin_bit_cast(bf16x2, pack_relu_bf16(z2[t][2 * q], z2[t][2 * q + 1])),
+          __builtin_bit_cast(bf16x2, pack_relu<!TRAIN>(z2[t][2 * q], z2[t][2 * q + 1])),
           __builtin_bit_cast(bf16x2, w3[t][q]), part, false);
   return part + __shfl_xor(part, 32) + b3;
 }
@@ -289,7 +301,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_predict(Mlp w, const floa
     bf16x8 b1[4];
     f32x16 z2[2];
     forward_regs<false>(N, a1, pack_feat(load_feat(x, s, lane / 32)), lane, b1, z2);
-    const float o = output_regs(z2, w3, b3);
+    const float o = output_regs<false>(z2, w3, b3);
     if (lane < 32 && m0 + lane < n) out[m0 + lane] = softplus(o);
   }
 }
@@ -336,7 +348,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
     bf16x8 b1[4];
     f32x16 z2[2];
     forward_regs<true>(N, a1, xb, lane, b1, z2);
-    const float o = output_regs(z2, w3, b3);
+    const float o = output_regs<true>(z2, w3, b3);
     // dL/do of the lane's sample (both halves)
     float g = 0.f;
     if (m0 + col < n) {
@@ -370,8 +382,8 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
       const f32x16 z = mfma(xb, a1[t], splat16(N.lb[col + 32 * t]));
 #pragma unroll
       for (int j = 0; j < 16; ++j) on[t][j] = z[j] > 0.f;
-      h1[t][0] = pack8_relu(z, 0);
-      h1[t][1] = pack8_relu(z, 8);
+      h1[t][0] = pack8_relu<false>(z, 0);
+      h1[t][1] = pack8_relu<false>(z, 8);
     }
     // h2 and delta2 the same; the gradients of W3, b2 and W2
 #pragma unroll
