@@ -109,3 +109,17 @@ def test_steps_match_the_routines(nx, ny, nz, precision):
 def test_steps_of_whole_planes_match_the_routines(nx, ny, nz, precision):
     """Planes of up to 512 complex slots, odd nx/2 and the limit among them."""
     test_steps_match_the_routines(nx, ny, nz, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32_mixed"])
+@pytest.mark.parametrize("nx,ny,nz", [(18, 10, 8), (200, 90, 12), (90, 54, 20)])
+def test_steps_with_run_time_plans_match_the_routines(nx, ny, nz, precision, monkeypatch):
+    monkeypatch.setenv("PLL_FFT_GENERIC", "1")
+    test_steps_match_the_routines(nx, ny, nz, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32_mixed"])
+@pytest.mark.parametrize("nx,ny,nz", [(1600, 6, 4), (12, 800, 4)])
+def test_steps_of_long_lengths_match_the_routines(nx, ny, nz, precision):
+    """Lengths beyond the compiled-in ones."""
+    test_steps_match_the_routines(nx, ny, nz, precision)
