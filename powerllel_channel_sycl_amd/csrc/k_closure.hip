@@ -145,22 +145,16 @@ __device__ __forceinline__ f32x16 bias_rows(const float* lb, int h, int t) {
   return c;
 }
 
-// NAN0: with the FP32 maximum instead, for which a NaN is 0 (batch inference; in
-// training, where a NaN input spoils the gradient in any case, it would cost 7 %).
-template <bool NAN0>
+// The batch kernels' form: the FP32 maximum, for which a NaN is 0 whatever its sign.
 __device__ __forceinline__ uint32_t pack_relu(float lo, float hi) {
-  if constexpr (NAN0)
-    return pack_bf16(fmaxf(lo, 0.f), fmaxf(hi, 0.f));
-  else
-    return pack_relu_bf16(lo, hi);
+  return pack_bf16(fmaxf(lo, 0.f), fmaxf(hi, 0.f));
 }
 
 // BF16 of relu of accumulator elements j0 .. j0+7 as one MFMA operand.
-template <bool NAN0>
 __device__ __forceinline__ bf16x8 pack8_relu(const f32x16& z, int j0) {
   return __builtin_bit_cast(
-      bf16x8, (u32x4){pack_relu<NAN0>(z[j0], z[j0 + 1]), pack_relu<NAN0>(z[j0 + 2], z[j0 + 3]),
-                      pack_relu<NAN0>(z[j0 + 4], z[j0 + 5]), pack_relu<NAN0>(z[j0 + 6], z[j0 + 7])});
+      bf16x8, (u32x4){pack_relu(z[j0], z[j0 + 1]), pack_relu(z[j0 + 2], z[j0 + 3]),
+                      pack_relu(z[j0 + 4], z[j0 + 5]), pack_relu(z[j0 + 6], z[j0 + 7])});
 }
 __device__ __forceinline__ bf16x8 pack8(const f32x16& v, int j0) {
   return __builtin_bit_cast(
@@ -251,7 +245,7 @@ __device__ __forceinline__ void forward_regs(const NetLds<TRAIN>& N, const bf16x
 #pragma unroll
   for (int t = 0; t < 2; ++t) z1[t] = mfma(a1[t], xb, bias_rows(N.lb, h, t));
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) b1[kb] = pack8_relu<!TRAIN>(z1[kb / 2], 8 * (kb % 2));
+  for (int kb = 0; kb < 4; ++kb) b1[kb] = pack8_relu(z1[kb / 2], 8 * (kb % 2));
   z2[0] = bias_rows(N.lb + kH, h, 0);
   z2[1] = bias_rows(N.lb + kH, h, 1);
 #pragma unroll
@@ -263,7 +257,6 @@ __device__ __forceinline__ void forward_regs(const NetLds<TRAIN>& N, const bf16x
 
 // The output o of the lane's sample, in both halves: BF16 h2 times BF16 W3
 // (packed pairs w3[t][q], the lane's rows), FP32 sum.
-template <bool TRAIN>
 __device__ __forceinline__ float output_regs(const f32x16 z2[2], const uint32_t w3[2][8], float b3) {
   float part = 0.f;
 #pragma unroll
@@ -271,7 +264,7 @@ __device__ __forceinline__ float output_regs(const f32x16 z2[2], const uint32_t 
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       part = __builtin_amdgcn_fdot2_f32_bf16(
-          __builtin_bit_cast(bf16x2, pack_relu<!TRAIN>(z2[t][2 * q], z2[t][2 * q + 1])),
+          __builtin_bit_cast(bf16x2, pack_relu(z2[t][2 * q], z2[t][2 * q + 1])),
           __builtin_bit_cast(bf16x2, w3[t][q]), part, false);
   return part + __shfl_xor(part, 32) + b3;
 }
@@ -301,15 +294,17 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_predict(Mlp w, const floa
     bf16x8 b1[4];
     f32x16 z2[2];
     forward_regs<false>(N, a1, pack_feat(load_feat(x, s, lane / 32)), lane, b1, z2);
-    const float o = output_regs<false>(z2, w3, b3);
+    const float o = output_regs(z2, w3, b3);
     if (lane < 32 && m0 + lane < n) out[m0 + lane] = softplus(o);
   }
 }
 
 // Training: one partial gradient (and loss sum) per block.  Loss = mean over
-// the n samples of (softplus(o) - y)^2.  Per 32-sample tile 41 products and
-// about 700 VALU operations (the ReLUs, masks and BF16 packing), which bound it
-// at two waves per SIMD.  393,216 samples: 34.6 us; 101 us for a form that passed
+// the n samples of (softplus(o) - y)^2.  Per 32-sample tile 40 products and
+// about 750 VALU operations (the ReLUs, masks and BF16 packing), which bound it
+// at two waves per SIMD.  393,216 samples: 37.5 us, of which 3 us are the FP32
+// maxima of the ReLUs (a 16-bit maximum of the packed pairs is half as many
+// operations, but lets a positive NaN through); 101 us for a form that passed
 // activations between the layers through LDS in two-byte writes (one wave per
 // SIMD, 140 KB of LDS a block).
 __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float* __restrict__ x,
@@ -317,6 +312,9 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
                                                              float* __restrict__ partial) {
   __shared__ NetLds<true> N;
   __shared__ __align__(16) float gs[kMlpWaves][32];  // dL/do per sample of a wave's tile
+  // X of a wave's tile as features x samples, samples in the order of the k-slots
+  // (ks, h, e); 80-byte rows spread the reads over the banks
+  __shared__ __align__(16) uint16_t xt[kMlpWaves][kInP][40];
   __shared__ float bp[kMlpWaves / 2][kNParam + 1];   // the waves' partial gradients
   load_net<true>(w, N);
   __syncthreads();
@@ -325,9 +323,8 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
   uint32_t w3[2][8];
   load_w3(w, h, w3);
   const float b3 = w.p[oB3], inv_n = 1.f / (float)n;
-  bf16x8 ident;  // feature x feature unit matrix, to turn X into samples x features
-#pragma unroll
-  for (int e = 0; e < 8; ++e) ident[e] = (short)(8 * h + e == col ? 0x3f80 : 0);
+  // the k-slot of sample col: hid_unit(8 ks + e, half) == col
+  const int slot = 16 * (col / 16) + 8 * (col / 4 % 2) + 4 * (col / 8 % 2) + col % 4;
   f32x16 gW2[2][2] = {};  // dW2 tiles [k-tile][n-tile] (rows k, cols n)
   f32x16 gW1[2] = {};     // dW1 tiles [n-tile] (rows i < 16 meaningful)
   float gb1[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gw3[2] = {0.f, 0.f}, gb3 = 0.f, loss = 0.f;
@@ -335,20 +332,23 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
   long m0 = ((long)blockIdx.x * kMlpWaves + wave) * 32;
   Feat nf = {};
   float ny = 0.f;
-  auto fetch = [&](long m) {  // past the end: the last sample, whose g is zeroed
+  auto fetch = [&](long m) {  // past the end: zero features, and g is zeroed
     const long s = std::min(m + col, n - 1);
     nf = load_feat(x, s, h);
     ny = y[s];
+    if (m + 32 > n && m + col >= n) nf = Feat{};
   };
   if (m0 < n) fetch(m0);
   for (; m0 < n; m0 += step) {
     const bf16x8 xb = pack_feat(nf);
     const float yt = ny;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) xt[wave][8 * h + e][slot] = (uint16_t)xb[e];
     if (m0 + step < n) fetch(m0 + step);
     bf16x8 b1[4];
     f32x16 z2[2];
     forward_regs<true>(N, a1, xb, lane, b1, z2);
-    const float o = output_regs<true>(z2, w3, b3);
+    const float o = output_regs(z2, w3, b3);
     // dL/do of the lane's sample (both halves)
     float g = 0.f;
     if (m0 + col < n) {
@@ -382,8 +382,8 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
       const f32x16 z = mfma(xb, a1[t], splat16(N.lb[col + 32 * t]));
 #pragma unroll
       for (int j = 0; j < 16; ++j) on[t][j] = z[j] > 0.f;
-      h1[t][0] = pack8_relu<false>(z, 0);
-      h1[t][1] = pack8_relu<false>(z, 8);
+      h1[t][0] = pack8_relu(z, 0);
+      h1[t][1] = pack8_relu(z, 8);
     }
     // h2 and delta2 the same; the gradients of W3, b2 and W2
 #pragma unroll
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
       f32x16 d;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const uint32_t hp = pack_relu_bf16(z[2 * q], z[2 * q + 1]);
+        const uint32_t hp = pack_relu(z[2 * q], z[2 * q + 1]);
         gw3[t] += __builtin_bit_cast(float, hp << 16) * gr[2 * q];
         gw3[t] += __builtin_bit_cast(float, hp & 0xffff0000u) * gr[2 * q + 1];
       }
@@ -412,10 +412,13 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
         for (int tk = 0; tk < 2; ++tk) gW2[tk][t] = mfma(h1[tk][ks], b, gW2[tk][t]);
       }
     }
-    // X over the samples; delta1 = (delta2 W2^T) relu'(z1), samples x hidden;
-    // the gradients of b1 and W1
-    const f32x16 xo = mfma(xb, ident, f32x16{});
-    const bf16x8 xa[2] = {pack8(xo, 0), pack8(xo, 8)};
+    // X over the samples (exchanged through LDS: as a product with a unit matrix
+    // an infinite feature or a NaN would reach every feature of its sample);
+    // delta1 = (delta2 W2^T) relu'(z1), samples x hidden; the gradients of b1 and W1
+    bf16x8 xa[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)  // rows 16.. of the product are not used
+      xa[ks] = *reinterpret_cast<const bf16x8*>(&xt[wave][col % kInP][16 * ks + 8 * h]);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       f32x16 d = {};
@@ -430,7 +433,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_train(Mlp w, const float*
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) gW1[t] = mfma(xa[ks], pack8(d, 8 * ks), gW1[t]);
     }
-    wave_lds_sync();  // gs is rewritten by the next tile
+    wave_lds_sync();  // gs and xt are rewritten by the next tile
   }
   // the waves' partials: the first half of them into LDS, the second half on
   // top, then all four together; lanes l and l+32 hold the same columns' other
