@@ -3,9 +3,11 @@
 // the runtime checks.  All kernels are templated on the field type T (double
 // for the FP64 path, float for the FP32-mixed path).
 //
-// FP64 parity: the library is compiled with -ffp-contract=off and every
-// expression below keeps the association of the reference formula it cites,
-// so an FP64 launch reproduces the reference arithmetic bit for bit.
+// FP64 parity: the library is compiled with -ffp-contract=off, and the separate
+// stages and routines keep the association of the reference formulas they cite,
+// so an FP64 launch of them reproduces the reference arithmetic bit for bit.
+// Inside a run the two stages of a step are fused (k_rk12, tendency_fast), in
+// another order of operations and as accurately.
 #include "pll_internal.hpp"
 #include "stencil_ops.hpp"
 
@@ -40,17 +42,17 @@ struct PlaneAcc {
 
 // The momentum operator with fewer operations, scaled by S = dt (stage 2 halves
 // its result): algebraically equal to S*(visc - conv) of tendency_z, with the
-// mesh factors gathered into per-plane coefficients (RkCoef), the viscous terms
-// written as second differences and products fused into FMAs: about 85
-// operations for the three components instead of 150.  It rounds differently
-// from the reference's order (no less accurately), so only the FP32-mixed
-// stages and the fused stages inside a run use it.
+// mesh factors gathered into per-plane coefficients (RkCoef) and products fused
+// into FMAs: about 95 operations for the three components instead of 150 in
+// FP64, 85 in FP32.  It rounds differently from the reference's order, so only
+// the FP32-mixed stages and the fused stages inside a run use it; against 80-bit
+// arithmetic a run's FP64 error is that of the reference's order.
 template <typename T>
 struct RkCoef {
   T a1, a2, b1, b2;  // (u,v) face interpolation to k+1/2 and k-1/2
   T zuv, cp, cm;     // S*0.25*dzf_inv(k); S*re_inv*dzc_inv(k|k-1)*dzf_inv(k)
   T zw, dp, dm;      // S*0.25*dzc_inv(k); S*re_inv*dzf_inv(k+1|k)*dzc_inv(k)
-  T cdu, cdw;        // diagonal of the viscous operator: 2 vx + 2 vy + cp + cm (u, v), + dp + dm (w)
+  T cdu, cdw;        // FP32's diagonal of the viscous operator: 2 vx + 2 vy + cp + cm (u, v), + dp + dm (w)
 };
 template <typename T>
 __device__ __forceinline__ RkCoef<T> load_coef(const RkCoef<T>* p, int k) {
@@ -100,6 +102,11 @@ __device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W
                                               T& iv, T& iw, ZConv<T>& zc) {
   // not held to the reference's rounding: let products fuse into FMAs
 #pragma clang fp contract(fast)
+  // The viscous part, in FP64 as second differences: they are exact where
+  // neighbours are close, and leave a uniform field as it is.  FP32 takes the
+  // neighbours' sums minus the diagonal, which is fewer operations (FP64 would gain
+  // 1 % of a step by it).
+  constexpr bool kDiff = sizeof(T) == 8;
   // FP64: one component at a time, or the compiler reads the LDS values of all
   // three ahead and the registers of a wave no longer fit three waves per SIMD
   // (k_rk12 at 768x384x384: 2442 us without the fence, 2348 us with it; FP32
@@ -119,8 +126,11 @@ __device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W
     zc.u = ct;
     T conv = cu.cx * (ae * ae - aw * aw) + cu.cy * (an * vn - as * vs) + q.zuv * (ct - cb);
     if (CRF) conv += cu.crf * (ae - aw);
-    // viscous part as neighbour sums minus the diagonal: fewer operations
-    iu = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.cp * qt + q.cm * qb - q.cdu * q0 - conv;
+    if constexpr (kDiff)
+      iu = cu.vx * ((qe - q0) - (q0 - qw)) + cu.vy * ((qn - q0) - (q0 - qs)) +
+           q.cp * (qt - q0) - q.cm * (q0 - qb) - conv;
+    else
+      iu = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.cp * qt + q.cm * qb - q.cdu * q0 - conv;
   }
   fence();
   {
@@ -135,7 +145,11 @@ __device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W
     zc.v = ct;
     T conv = cu.cx * (ue * ae - uw * aw) + cu.cy * (an * an - as * as) + q.zuv * (ct - cb);
     if (CRF) conv += cu.crf * (ae - aw);
-    iv = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.cp * qt + q.cm * qb - q.cdu * q0 - conv;
+    if constexpr (kDiff)
+      iv = cu.vx * ((qe - q0) - (q0 - qw)) + cu.vy * ((qn - q0) - (q0 - qs)) +
+           q.cp * (qt - q0) - q.cm * (q0 - qb) - conv;
+    else
+      iv = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.cp * qt + q.cm * qb - q.cdu * q0 - conv;
   }
   fence();
   {
@@ -152,7 +166,11 @@ __device__ __forceinline__ void tendency_fast(const A& U, const A& V, const A& W
     zc.w = ct;
     T conv = cu.cx * (ue * ae - uw * aw) + cu.cy * (vn * an - vs * as) + q.zw * (ct - cb);
     if (CRF) conv += cu.crf * (ae - aw);
-    iw = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.dp * qt + q.dm * qb - q.cdw * q0 - conv;
+    if constexpr (kDiff)
+      iw = cu.vx * ((qe - q0) - (q0 - qw)) + cu.vy * ((qn - q0) - (q0 - qs)) +
+           q.dp * (qt - q0) - q.dm * (q0 - qb) - conv;
+    else
+      iw = cu.vx * (qe + qw) + cu.vy * (qn + qs) + q.dp * qt + q.dm * qb - q.cdw * q0 - conv;
   }
 }
 
@@ -202,8 +220,10 @@ struct CarryAcc {
   }
 };
 
-// Stage 1: o = s + dt*F(s); stage 2: o = ((s + old) + dt*F(s))/2, with the
-// carry replaced by the next plane's.
+// Stage 1: o = s + dt*F(s); stage 2: o = ((s + dt*F(s)) + old)/2, with the
+// carry replaced by the next plane's.  The reference adds in this order too
+// (src/mod_calcVel.cc:194,216,238): s + old, added first, would round at
+// twice the magnitude twice.
 template <typename T, int STAGE, bool CRF, int SX>
 __device__ __forceinline__ void stage_update(const PlaneAcc<T, SX>& U, const PlaneAcc<T, SX>& V,
                                              const PlaneAcc<T, SX>& W, const RkParam<T>& q, int k,
@@ -220,9 +240,9 @@ __device__ __forceinline__ void stage_update(const PlaneAcc<T, SX>& U, const Pla
     o2 = z.v + iv;
     o3 = z.w + iw;
   } else {
-    o1 = ((z.u + ou) + iu) * T(0.5);
-    o2 = ((z.v + ov) + iv) * T(0.5);
-    o3 = ((z.w + ow) + iw) * T(0.5);
+    o1 = ((z.u + iu) + ou) * T(0.5);
+    o2 = ((z.v + iv) + ov) * T(0.5);
+    o3 = ((z.w + iw) + ow) * T(0.5);
   }
 }
 
