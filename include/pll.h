@@ -241,8 +241,9 @@ int pll_closure_get_scales(pll_closure *c, double *gscale, double *yscale, doubl
  * divergence of the eddy-viscosity stress 2 nu_t S_ij to the momentum
  * tendency (src/mod_calcVel.cc:27-242), with nu_t evaluated by the network
  * inside the stage kernel; pll_step then runs the unfused sequence
- * src/main.cc:117-153.  Training the closure while attached is ordered
- * before the context's next stage. */
+ * src/main.cc:117-153.  Training the closure (or setting its parameters) while
+ * attached is ordered after the context's stages already enqueued and before
+ * its next one. */
 int pll_closure_attach(pll_context *ctx, pll_closure *c);
 /* Save a closure (parameters and scales) to a file / create one from such a
  * file: "PLLCLOS1", int32 parameter count, the FP32 parameters, the three FP64

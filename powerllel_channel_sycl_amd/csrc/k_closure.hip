@@ -22,6 +22,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <random>
@@ -1241,6 +1242,7 @@ struct pll_closure {
   int device = 0;              // the device current at creation (that of stream)
   hipEvent_t ready = nullptr;  // orders a context's closure stages after training
   long version = 0;            // bumped by every asynchronous change of the weights
+  std::shared_ptr<ClosureOrder> order = std::make_shared<ClosureOrder>();
   // feature and output scales: inputs g*gs and (wall distance)*ys, nu_t = nus*softplus(o)
   double gs = 1.0, ys = 1.0, nus = 1.0;
 };
@@ -1267,23 +1269,48 @@ long mlp_blocks(long n) {
   return (waves + kMlpWaves - 1) / kMlpWaves;
 }
 
+// A context's enqueued stages: what the closure's stream runs next waits for them.
+// With the order's lock held.
+int wait_for_reader(const ClosureOrder& o, pll_context* ctx) {
+  if (!ctx->closure_reading || !o.stream) return PLL_OK;
+  PLL_HIP_TRY(hipEventRecord(ctx->closure_read, ctx->stream));
+  PLL_HIP_TRY(hipStreamWaitEvent(o.stream, ctx->closure_read, 0));
+  ctx->closure_reading = false;
+  return PLL_OK;
+}
+// Before a change of the weights on the closure's stream.  With the order's lock held.
+int wait_for_readers(pll_closure* c) {
+  for (pll_context* ctx : c->order->readers)
+    if (const int rc = wait_for_reader(*c->order, ctx)) return rc;
+  return PLL_OK;
+}
+
 // The blocks' partial gradients and their sum; with A in a training step's
 // update.
-void launch_gradient(const pll_closure* c, const float* x, const float* y, long n, float* partial,
-                     float* grad, const Adam* A) {
+int launch_gradient(pll_closure* c, const float* x, const float* y, long n, float* partial,
+                    float* grad, const Adam* A) {
   const long nblk = mlp_blocks(n);
+  const dim3 blocks((kNParam + 1 + 63) / 64);
   hipLaunchKernelGGL(k_train, dim3((unsigned)nblk), dim3(64 * kMlpWaves), 0, c->stream, weights(c),
                      x, y, n, partial);
-  hipLaunchKernelGGL((A ? k_grad_sum<true> : k_grad_sum<false>), dim3((kNParam + 1 + 63) / 64),
-                     dim3(256), 0, c->stream, partial, nblk, grad, A ? *A : Adam{});
+  if (A) {
+    std::lock_guard<std::mutex> lock(c->order->m);
+    const int rc = wait_for_readers(c);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_grad_sum<true>, blocks, dim3(256), 0, c->stream, partial, nblk, grad, *A);
+    PLL_HIP_TRY(hipGetLastError());
+    c->step += 1;
+    c->version += 1;
+  } else {
+    hipLaunchKernelGGL(k_grad_sum<false>, blocks, dim3(256), 0, c->stream, partial, nblk, grad, Adam{});
+  }
+  PLL_HIP_TRY(hipGetLastError());
+  return PLL_OK;
 }
 
 int gradient(pll_closure* c, const float* x, const float* y, long n, const Adam* A) {
   const int rc = ensure_partial(c, mlp_blocks(n));
-  if (rc) return rc;
-  launch_gradient(c, x, y, n, c->partial, c->grad, A);
-  PLL_HIP_TRY(hipGetLastError());
-  return PLL_OK;
+  return rc ? rc : launch_gradient(c, x, y, n, c->partial, c->grad, A);
 }
 
 // ---- allocation-free gradient ------------------------------------------------
@@ -1368,13 +1395,6 @@ T* fld(const pll_context* c, int f) {
 template <typename T>
 int rk_closure_t(pll_context* c, int stage, int fold, int corr, int acc, int bcload) {
   pll_closure* cl = c->closure;
-  if (c->closure_version != cl->version) {
-    // the weights changed on the closure's stream (training) since this
-    // context last waited for them
-    PLL_HIP_TRY(hipEventRecord(cl->ready, cl->stream));
-    PLL_HIP_TRY(hipStreamWaitEvent(c->stream, cl->ready, 0));
-    c->closure_version = cl->version;
-  }
   const Geom g = c->g;
   const int ntx = (g.nx + kLx - 1) / kLx, nty = (g.ny + kLy - 1) / kLy, ntz = (g.nz + kLz - 1) / kLz;
   const dim3 grid((unsigned)ntx * nty * ntz), block(64 * kWaves);
@@ -1415,11 +1435,21 @@ int rk_closure_t(pll_context* c, int stage, int fold, int corr, int acc, int bcl
   }
   const double* dzflzi = c->d_mesh64 + 3 * (c->g.nz + 2);
   {
+    std::unique_lock<std::mutex> lock(c->closure_order->m);
+    if (c->closure_version != cl->version) {
+      // the weights changed on the closure's stream (training) since this
+      // context last waited for them
+      PLL_HIP_TRY(hipEventRecord(cl->ready, cl->stream));
+      PLL_HIP_TRY(hipStreamWaitEvent(c->stream, cl->ready, 0));
+      c->closure_version = cl->version;
+    }
     TimerScope ts(c, K_RK_CLOSURE);
     hipLaunchKernelGGL((k_nut<T>), dim3((unsigned)nblk), block, 0, c->stream, g, su, sv, sw,
                        mesh_t<T>(c), feat_mesh<T>(c), (float)c->dx_inv, (float)c->dy_inv,
                        (float)(0.25 * c->dx_inv), (float)(0.25 * c->dy_inv), weights(cl),
                        (float)cl->gs, (float)cl->ys, nus, c->d_nut, ncell);
+    c->closure_reading = true;
+    lock.unlock();
     if (stage == 1)
       hipLaunchKernelGGL((k_rk_les<T, 1>), grid, block, 0, c->stream, g, su, sv, sw,
                          fld<T>(c, PLL_U1), fld<T>(c, PLL_V1), fld<T>(c, PLL_W1), mesh_t<T>(c), dxi,
@@ -1515,6 +1545,20 @@ int launch_rk_closure(pll_context* c, int stage, int fold, int corr, int acc, in
   return c->prec == PLL_FP64 ? rk_closure_t<double>(c, stage, fold, corr, acc, bcload)
                              : rk_closure_t<float>(c, stage, fold, corr, acc, bcload);
 }
+int closure_detach(pll_context* c) {
+  if (!c->closure_order) return PLL_OK;
+  int rc;
+  {
+    std::lock_guard<std::mutex> lock(c->closure_order->m);
+    rc = wait_for_reader(*c->closure_order, c);
+    auto& r = c->closure_order->readers;
+    r.erase(std::remove(r.begin(), r.end(), c), r.end());
+  }
+  c->closure_order.reset();
+  c->closure = nullptr;
+  c->closure_reading = false;
+  return rc;
+}
 bool closure_fused_available(const pll_context* c) {
   return closure_stage_blocks(c) <= c->npartial;
 }
@@ -1594,9 +1638,18 @@ int pll_closure_attach(pll_context* ctx, pll_closure* c) {
     if (rc) return rc;
     if (!ctx->d_nut) PLL_HIP_TRY(ctx_malloc(ctx, &ctx->d_nut, (size_t)ctx->nspec * sizeof(float)));
     PLL_HIP_TRY(hipMemsetAsync(ctx->d_nut, 0, (size_t)ctx->nspec * sizeof(float), ctx->stream));
+    if (!ctx->closure_read)
+      PLL_HIP_TRY(hipEventCreateWithFlags(&ctx->closure_read, hipEventDisableTiming));
   }
-  ctx->closure = c;
+  const int rc = closure_detach(ctx);
+  if (rc) return rc;
   ctx->closure_version = -1;
+  if (c) {
+    std::lock_guard<std::mutex> lock(c->order->m);
+    c->order->readers.push_back(ctx);
+    ctx->closure_order = c->order;
+    ctx->closure = c;
+  }
   return PLL_OK;
 }
 
@@ -1648,6 +1701,7 @@ int pll_closure_create(uint64_t seed, pll_closure** out) {
   if (e != hipSuccess) return bail(hip_fail(e, "hipGetDevice"));
   e = hipStreamCreate(&c->stream);
   if (e != hipSuccess) return bail(hip_fail(e, "closure stream"));
+  c->order->stream = c->stream;
   e = hipEventCreateWithFlags(&c->ready, hipEventDisableTiming);
   if (e != hipSuccess) return bail(hip_fail(e, "closure event"));
   const size_t pb = (size_t)kNParam * sizeof(float);
@@ -1682,6 +1736,11 @@ int pll_closure_create(uint64_t seed, pll_closure** out) {
 
 int pll_closure_destroy(pll_closure* c) {
   if (!c) return PLL_OK;
+  {
+    std::lock_guard<std::mutex> lock(c->order->m);
+    (void)wait_for_readers(c);
+    c->order->stream = nullptr;
+  }
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void* bufs[] = {c->p, c->m1, c->m2, c->wb, c->partial, c->grad};
   for (void* q : bufs)
@@ -1703,6 +1762,9 @@ int pll_closure_get_params(pll_closure* c, float* host) {
 
 int pll_closure_set_params(pll_closure* c, const float* host) {
   if (!c || !host) return fail(PLL_ERR_ARG, "null argument");
+  std::lock_guard<std::mutex> lock(c->order->m);
+  const int rc = wait_for_readers(c);
+  if (rc) return rc;
   PLL_HIP_TRY(hipStreamSynchronize(c->stream));
   PLL_HIP_TRY(hipMemcpy(c->p, host, (size_t)kNParam * sizeof(float), hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_refresh_bf16, dim3((kNParam + 255) / 256), dim3(256), 0, c->stream, c->p,
@@ -1726,8 +1788,7 @@ int pll_closure_gradient_noalloc(pll_closure* c, const float* x, const float* y,
   if (rc) return rc;
   float* grad = base + kScratchPartials * (kNParam + 1);
   // the kernels of pll_closure_gradient, on the scratch array
-  launch_gradient(c, x, y, n, base, grad, nullptr);
-  PLL_HIP_TRY(hipGetLastError());
+  if ((rc = launch_gradient(c, x, y, n, base, grad, nullptr))) return rc;
   float lsum = 0.f;
   if (grad_host)
     PLL_HIP_TRY(hipMemcpyAsync(grad_host, grad, (size_t)kNParam * sizeof(float),
@@ -1757,11 +1818,7 @@ int pll_closure_train_step(pll_closure* c, const float* x, const float* y, long 
   const double t = (double)(c->step + 1);
   const Adam A{c->p,      c->m1,     c->m2, c->wb, (float)lr, (float)b1, (float)b2, 1e-8f,
                (float)(1.0 - std::pow(b1, t)), (float)(1.0 - std::pow(b2, t))};
-  const int rc = gradient(c, x, y, n, &A);
-  if (rc) return rc;
-  c->step += 1;
-  c->version += 1;
-  return PLL_OK;
+  return gradient(c, x, y, n, &A);
 }
 
 int pll_closure_predict(pll_closure* c, const float* x, long n, float* out) {

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -104,6 +106,16 @@ enum KernelId {
 };
 extern const char* const kKernelNames[K_COUNT];
 
+// Orders the readers of a closure's weights (the stages of the contexts that it is
+// attached to, on their streams) and its writers (training and set_params, on
+// the closure's): a stage waits for the last writer, a writer for every stage
+// enqueued before it.  Held by the closure and its contexts, whichever goes first.
+struct ClosureOrder {
+  std::mutex m;  // a stage's launch and a writer's, whole
+  hipStream_t stream = nullptr;  // the closure's; null when it is gone
+  std::vector<pll_context*> readers;
+};
+
 // Pending event pair of one timed launch.
 struct PendingTimer {
   int kid;
@@ -174,6 +186,9 @@ struct pll_context {
   // eddy-viscosity stress with the network evaluated in the stage kernel
   pll_closure* closure = nullptr;
   long closure_version = -1;  // the closure's weight version this stream has waited for
+  std::shared_ptr<pll::ClosureOrder> closure_order;
+  hipEvent_t closure_read = nullptr;  // recorded behind the stages that a writer waits for
+  bool closure_reading = false;       // stages enqueued since the last writer
   void* d_feat = nullptr;   // feature coefficients per plane (field precision), 3*(nz+2)
   float* d_nut = nullptr;   // eddy viscosity of the last closure stage, nx*ny*nz
 
@@ -240,6 +255,8 @@ int launch_rk(pll_context* c, int stage, int fold, int corr = 0, int acc = 0, in
 // corr, acc, bcload as for launch_rk
 int launch_rk_closure(pll_context* c, int stage, int fold = 0, int corr = 0, int acc = 0,
                       int bcload = 0);
+// Takes the context off its closure's readers; a writer still waits for its stages.
+int closure_detach(pll_context* c);
 // the closure stages' bulk-mean partials fit d_partial (the fused step sequence)
 bool closure_fused_available(const pll_context* c);
 // forceVel's bulk mean of u and its force from n FP64 block partials in
