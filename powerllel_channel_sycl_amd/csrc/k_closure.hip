@@ -1234,8 +1234,7 @@ struct pll_closure {
   float* m1 = nullptr;  // Adam moments
   float* m2 = nullptr;
   uint16_t* wb = nullptr;  // BF16 W1 | W2 | W3
-  float* partial = nullptr;
-  long npartial_blocks = 0;  // partial gradients, one per k_train block
+  float* partial = nullptr; // partial gradients of the largest training grid (kMaxPartials)
   float* grad = nullptr;    // kNParam + 1 (loss sum last)
   long step = 0;
   hipStream_t stream = nullptr;
@@ -1253,21 +1252,13 @@ Mlp weights(const pll_closure* c) {
   return Mlp{c->p, c->wb + kWb1, c->wb + kWb2, c->wb + kWb3};
 }
 
-int ensure_partial(pll_closure* c, long nblocks) {
-  if (nblocks <= c->npartial_blocks) return PLL_OK;
-  if (c->partial) (void)hipFree(c->partial);
-  c->partial = nullptr;
-  PLL_HIP_TRY(hipMalloc(&c->partial, (size_t)nblocks * (kNParam + 1) * sizeof(float)));
-  c->npartial_blocks = nblocks;
-  return PLL_OK;
-}
-
 // Blocks of a training or inference grid for n samples: one 32-sample tile per
 // wave, at most kMaxWaves waves (which then take every nwaves-th tile).
 long mlp_blocks(long n) {
   const long waves = std::min((n + 31) / 32, kMaxWaves);
   return (waves + kMlpWaves - 1) / kMlpWaves;
 }
+constexpr long kMaxPartials = kMaxWaves / kMlpWaves;  // one per block
 
 // A context's enqueued stages: what the closure's stream runs next waits for them.
 // With the order's lock held.
@@ -1308,20 +1299,14 @@ int launch_gradient(pll_closure* c, const float* x, const float* y, long n, floa
   return PLL_OK;
 }
 
-int gradient(pll_closure* c, const float* x, const float* y, long n, const Adam* A) {
-  const int rc = ensure_partial(c, mlp_blocks(n));
-  return rc ? rc : launch_gradient(c, x, y, n, c->partial, c->grad, A);
-}
-
 // ---- allocation-free gradient ------------------------------------------------
 // The buffers of pll_closure_gradient_noalloc live in one file-scope device
 // array, one copy per GPU for the life of the process: the per-block partial
-// gradients of the largest training grid (kMaxWaves / kMlpWaves blocks) and the
-// summed gradient with the loss, each kNParam + 1 floats -- 5.5 MB.  Every call on a GPU shares that GPU's copy;
-// each call writes every element it reads before reading it, so nothing has
+// gradients of the largest training grid (kMaxPartials) and the summed gradient
+// with the loss, each kNParam + 1 floats -- 5.5 MB.  Every call on a GPU shares
+// that GPU's copy; each call writes every element it reads before reading it, so nothing has
 // to start at zero, and calls that overlap on one GPU race.
-constexpr long kScratchPartials = kMaxWaves / kMlpWaves;
-constexpr long kScratchFloats = (kScratchPartials + 1) * (kNParam + 1);
+constexpr long kScratchFloats = (kMaxPartials + 1) * (kNParam + 1);
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 // Device address of `scratch` on each GPU, resolved once per device with that
@@ -1707,6 +1692,7 @@ int pll_closure_create(uint64_t seed, pll_closure** out) {
   const size_t pb = (size_t)kNParam * sizeof(float);
   if (hipMalloc(&c->p, pb) != hipSuccess || hipMalloc(&c->m1, pb) != hipSuccess ||
       hipMalloc(&c->m2, pb) != hipSuccess || hipMalloc(&c->grad, pb + sizeof(float)) != hipSuccess ||
+      hipMalloc(&c->partial, kMaxPartials * (pb + sizeof(float))) != hipSuccess ||
       hipMalloc(&c->wb, (size_t)kWbLen * sizeof(uint16_t)) != hipSuccess)
     return bail(fail(PLL_ERR_NOMEM, "closure parameters"));
   // Glorot-uniform weights, zero biases (the output bias starts at softplus^-1(1))
@@ -1780,13 +1766,13 @@ int pll_closure_gradient_noalloc(pll_closure* c, const float* x, const float* y,
   PLL_HIP_TRY(hipGetDevice(&dev));
   if (dev != c->device)
     return fail(PLL_ERR_STATE, "pll_closure_gradient_noalloc: the closure's device must be current");
-  if (mlp_blocks(n) > kScratchPartials)
+  if (mlp_blocks(n) > kMaxPartials)
     return fail(PLL_ERR_ARG, "pll_closure_gradient_noalloc: the training grid exceeds the scratch "
                              "array (at most kMaxWaves waves)");
   float* base = nullptr;
   int rc = scratch_on(dev, &base);
   if (rc) return rc;
-  float* grad = base + kScratchPartials * (kNParam + 1);
+  float* grad = base + kMaxPartials * (kNParam + 1);
   // the kernels of pll_closure_gradient, on the scratch array
   if ((rc = launch_gradient(c, x, y, n, base, grad, nullptr))) return rc;
   float lsum = 0.f;
@@ -1802,7 +1788,7 @@ int pll_closure_gradient_noalloc(pll_closure* c, const float* x, const float* y,
 int pll_closure_gradient(pll_closure* c, const float* x, const float* y, long n, float* grad_host,
                          double* loss) {
   if (!c || !x || !y || n <= 0) return fail(PLL_ERR_ARG, "bad arguments");
-  int rc = gradient(c, x, y, n, nullptr);
+  const int rc = launch_gradient(c, x, y, n, c->partial, c->grad, nullptr);
   if (rc) return rc;
   std::vector<float> g(kNParam + 1);
   PLL_HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1818,7 +1804,7 @@ int pll_closure_train_step(pll_closure* c, const float* x, const float* y, long 
   const double t = (double)(c->step + 1);
   const Adam A{c->p,      c->m1,     c->m2, c->wb, (float)lr, (float)b1, (float)b2, 1e-8f,
                (float)(1.0 - std::pow(b1, t)), (float)(1.0 - std::pow(b2, t))};
-  return gradient(c, x, y, n, &A);
+  return launch_gradient(c, x, y, n, c->partial, c->grad, &A);
 }
 
 int pll_closure_predict(pll_closure* c, const float* x, long n, float* out) {
