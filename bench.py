@@ -8,7 +8,8 @@ BC, projection, constant-flow forcing, halo/BC).
 
 Metric: Mpoint-steps/s = nx*ny*nz*steps / seconds / 1e6, inputs resident in
 HBM; three windows of --steps steps are timed and the median is reported.  The roofline entry reports the dominant kernel's algorithmic bytes per
-launch over its average HIP-event duration against the 8 TB/s HBM peak.  The
+launch over its average HIP-event duration against the 8 TB/s HBM peak, and
+those of the kernels of one step inside a run over the step's time.  The
 CPU baseline is the FP64 oracle (the CPU restatement of the reference
 algorithm) timed for a few steps (--cpu-steps, default six) of the same grid on
 this host's cores (CPU model, thread count and visible cores are reported).
@@ -38,33 +39,36 @@ WORKLOADS = {
 }
 DEFAULT_WORKLOAD = "retau550_768x384x384"
 
-# Algorithmic (compulsory) HBM bytes per grid point per launch.  Inside a run
-# both RK stages run in one kernel (rk12) with the previous step's projection
-# applied on load: it reads u, v, w, p and writes u, v, w; u1 stays on chip.
-# calcRHS runs inside the forward x transform (reads u, v, w, writes the work
-# array); each other transform and the tridiagonal solve read and write the work
-# array once; correctVel (last step of a run) reads p, u, v, w and writes u, v, w;
-# the separate bulk mean reads u; the force update reads and writes u.  The
-# separate stages (rk1, rk2: first step of a run) are listed with the deferred
-# projection's p among their reads (FP64 stage 1, FP32 stage 2), and rk2_rhs is
-# FP64 stage 2 with calcRHS and the projection in one kernel: forms that earlier
-# measurements were made in and that no run launches any more.
-BYTES_PER_POINT = {
-    "fp64": {"rk1": 56, "rk2": 72, "calc_rhs": 32, "rk2_rhs": 88, "rk12": 56,
+# Algorithmic (compulsory) HBM bytes per grid point of each kernel that is
+# launched.  Inside a run both RK stages run in one kernel (rk12) with the previous
+# step's projection applied on load: it reads u, v, w, p and writes u, v, w; u1
+# stays on chip.  calcRHS runs inside the forward x transform (reads u, v, w, writes
+# the work array); each other transform and the tridiagonal solve read and write the
+# work array once.  The separate stages (first step of a run) read u, v, w and
+# write u1, v1, w1 (rk1), and read u1, v1, w1, u, v, w and write u, v, w (rk2);
+# correctVel (last step of a run) reads p, u, v, w and writes u, v, w; the separate
+# bulk mean reads u; the force update reads and writes u.
+LAUNCH_BYTES = {
+    "fp64": {"rk1": 48, "rk2": 72, "calc_rhs": 32, "rk12": 56,
              "fft_x_fwd": 16, "fft_x_fwd_rhs": 32,
              "fft_y_fwd": 16, "solve_trid": 16, "fft_y_bwd": 16, "fft_x_bwd": 16,
              "correct_vel": 56, "mean_partial": 8, "force_add": 16},
-    "fp32_mixed": {"rk1": 28, "rk2": 40, "rk12": 28, "calc_rhs": 16, "fft_x_fwd": 8,
-                   "fft_x_fwd_rhs": 16,
-                   "fft_y_fwd": 8, "solve_trid": 8, "fft_y_bwd": 8, "fft_x_bwd": 8,
-                   "correct_vel": 28, "mean_partial": 4, "force_add": 8},
 }
+LAUNCH_BYTES["fp32_mixed"] = {k: b // 2 for k, b in LAUNCH_BYTES["fp64"].items()}
+# A step inside a run: rk12, calcRHS in the forward x transform, three more
+# transforms and the solve.
+RUN_STEP = ("rk12", "fft_x_fwd_rhs", "fft_y_fwd", "solve_trid", "fft_y_bwd", "fft_x_bwd")
+# The same with the separate stages as they were when the deferred projection
+# was among their reads (FP64 stage 1, FP32 stage 2) and FP64 stage 2 held calcRHS
+# (rk2_rhs): the bytes that older figures of those kernels were formed with.
+BYTES_PER_POINT = {"fp64": {**LAUNCH_BYTES["fp64"], "rk1": 56, "rk2_rhs": 88},
+                   "fp32_mixed": {**LAUNCH_BYTES["fp32_mixed"], "rk1": 28, "rk2": 40}}
 # Timed windows of --steps steps each; the reported time is their median.
 WINDOWS = 3
 
 # The compulsory bytes per point of each routine of the reference's RK2 step
-# (src/main.cc:116-154, FP64, one launch each): their sum is the roofline of the
-# whole step; FP32-mixed halves it.
+# (src/main.cc:116-154, FP64, one launch each; FP32-mixed halves them): what the
+# step would move without fusing anything.
 ROUTINE_BYTES_FP64 = {"rk1": 48, "rk2": 72, "calc_rhs": 32, "fft_x_fwd": 16, "fft_y_fwd": 16,
                       "solve_trid": 16, "fft_y_bwd": 16, "fft_x_bwd": 16, "correct_vel": 56,
                       "mean_partial": 8, "force_add": 16}
@@ -175,7 +179,7 @@ def closure_kernels_probe(reps=5):
     profiles: a fine FP32-mixed 384x256x192 channel filtered onto the coarse
     FP64 96x64x64 one with the training samples of one snapshot
     (pll_closure_samples: k_filter, k_samples), Adam steps on them
-    (pll_closure_train_step: k_mlp, k_grad_reduce, k_adam), and the two RK
+    (pll_closure_train_step: k_train, k_grad_sum), and the two RK
     stages of the coarse grid with the closure attached (pll_time_int_vel_rk1
     / _rk2: k_nut, k_rk_les) with the boundary updates between them."""
     import torch
@@ -360,7 +364,7 @@ def measure(wl, precision, steps, warmup):
     div = ch.calcMaxDiv()[0]
     ch.close()
     scale = 1.0 if precision == "fp64" else 0.5
-    table = BYTES_PER_POINT[precision]
+    table = LAUNCH_BYTES[precision]
     kernels = {}
     total = sum(ms for ms, n in times.values() if n)
     for name, (ms, n) in times.items():
@@ -380,7 +384,9 @@ def measure(wl, precision, steps, warmup):
     measured = MEASURED_HBM_B_PER_POINT.get(precision, {}).get(dom)
     traffic = (round(measured * npts) if measured is not None and wl == DEFAULT_WORKLOAD
                else None)
-    step_gbs = STEP_BYTES_FP64 * scale * npts / (ms_step * 1e-3) / 1e9
+    step_bytes = sum(table[k] for k in RUN_STEP)
+    step_gbs = step_bytes * npts / (ms_step * 1e-3) / 1e9
+    unfused_gbs = STEP_BYTES_FP64 * scale * npts / (ms_step * 1e-3) / 1e9
     return {
         "value": round(npts * steps / sec / 1e6, 2),
         "ms_per_step": round(ms_step, 4),
@@ -389,7 +395,9 @@ def measure(wl, precision, steps, warmup):
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic, "step_achieved": round(step_gbs, 1),
                      "step_frac": round(step_gbs / HBM_PEAK_GBS, 4),
-                     "bytes_per_point_step": STEP_BYTES_FP64 * scale},
+                     "bytes_per_point_step": step_bytes,
+                     # the rate at which the unfused sequence would have to move its bytes
+                     "unfused_equivalent_GBps": round(unfused_gbs, 1)},
         "kernels": kernels,
         "check": {"bulk_u": mean_u, "max_div": div},
     }
