@@ -392,10 +392,10 @@ __global__ __launch_bounds__(kRkTx * kRkTy) void k_rk(Geom g, const T* __restric
         dv[a] = V(0, 0, 0) + iv;
         dw[a] = W(0, 0, 0) + iw;
       } else {
-        const T nu = ((U(0, 0, 0) + ou) + iu) * 0.5f;
+        const T nu = ((U(0, 0, 0) + iu) + ou) * 0.5f;  // k_rk12's order
         du[a] = nu;
-        dv[a] = ((V(0, 0, 0) + ov) + iv) * 0.5f;
-        dw[a] = ((W(0, 0, 0) + ow) + iw) * 0.5f;
+        dv[a] = ((V(0, 0, 0) + iv) + ov) * 0.5f;
+        dw[a] = ((W(0, 0, 0) + iw) + ow) * 0.5f;
         if (acc) msum += (double)nu * uniform_load(dzflzi, k);
       }
     }
