@@ -698,23 +698,21 @@ __global__ __launch_bounds__(256) void k_samples(
 // ---- the deferred projection, forcing and boundary update -----------------
 // In the closure's step sequence the previous step's velocity has neither its
 // projection nor its forcing nor its boundary update: its values are rebuilt
-// from the stored ones as k_rk's folded loads do.  With `bcload`: x/y halo
-// cells read their periodic image, the ghost planes 0 and nz+1 follow the
-// boundary rules from planes 1 and nz (2 bc - u, -v;
-// src/mod_updateBound.cc:92,123) and w is 0 on planes 0, nz and nz+1 (:137);
-// with `corr` the value first becomes u - dt grad(p) (src/mod_calcVel.cc:272-274,
-// k_correct's association), then the deferred forcing of each component in
-// fmask (device scalars force[0..2]) is added.  Without `bcload` the stored
-// value is read.  p's x halos must hold their periodic values (the step's
+// from the stored ones as k_rk12's loads do.  x/y halo cells read their periodic
+// image, the ghost planes 0 and nz+1 follow the boundary rules from planes 1 and
+// nz (2 bc - u, -v; src/mod_updateBound.cc:92,123) and w is 0 on planes 0, nz and
+// nz+1 (:137); before that the value becomes u - dt grad(p)
+// (src/mod_calcVel.cc:272-274, k_correct's association) and the deferred forcing of
+// each component in fmask (device scalars force[0..2]) is added.  p's x halos must
+// hold their periodic values (the step's
 // inverse x transform writes them); its y halo is read at its image and its z
 // ghost planes are not needed (w is 0 on the planes that would read them), so
 // updateBoundP need not have run.
 template <typename T>
 struct VelRules {
-  int bcload, corr;
-  const T* p;              // previous pressure, valid halos (corr)
-  const T* dzc_inv;        // (corr)
-  T dtdxi, dtdyi, dt;      // (corr)
+  const T* p;              // previous pressure, valid halos
+  const T* dzc_inv;
+  T dtdxi, dtdyi, dt;
   const double* force;     // deferred forcing of u, v, w (fmask)
   int fmask;
   T bc_u;                  // u's wall value, src/mod_updateBound.cc:80
@@ -724,7 +722,6 @@ struct VelRules {
 template <typename T>
 __device__ __forceinline__ T rule_load(const T* __restrict__ q, int fc, int i, int j, int k,
                                        const Geom& g, const VelRules<T>& r) {
-  if (!r.bcload) return q[g.idx(i, j, k)];
   const int ii = i == 0 ? g.nx : (i == g.nx + 1 ? 1 : i);
   const int jj = j == 0 ? g.ny : (j == g.ny + 1 ? 1 : j);
   const bool ghost = k == 0 || k == g.nz + 1;
@@ -732,15 +729,13 @@ __device__ __forceinline__ T rule_load(const T* __restrict__ q, int fc, int i, i
   if (fc == 2 && (k == 0 || k >= g.nz)) return T(0);
   const long a = g.idx(ii, jj, ks);
   T v = q[a];
-  if (r.corr) {
-    const T p0 = r.p[a];
-    if (fc == 0)
-      v = v - (r.p[a + 1] - p0) * r.dtdxi;
-    else if (fc == 1)
-      v = v - (r.p[jj == g.ny ? a - (long)(g.ny - 1) * g.sx : a + g.sx] - p0) * r.dtdyi;
-    else
-      v = v - (r.p[a + g.sxy] - p0) * r.dt * r.dzc_inv[ks];
-  }
+  const T p0 = r.p[a];
+  if (fc == 0)
+    v = v - (r.p[a + 1] - p0) * r.dtdxi;
+  else if (fc == 1)
+    v = v - (r.p[jj == g.ny ? a - (long)(g.ny - 1) * g.sx : a + g.sx] - p0) * r.dtdyi;
+  else
+    v = v - (r.p[a + g.sxy] - p0) * r.dt * r.dzc_inv[ks];
   if ((r.fmask >> fc) & 1) v = v + (T)r.force[fc];
   if (ghost) v = fc == 0 ? T(2) * r.bc_u - v : T(2) * T(0) - v;
   return v;
@@ -870,29 +865,6 @@ constexpr int kLx = 32, kLy = 8, kLz = 1;
 constexpr int kEx = kLx + 2, kEy = kLy + 2, kEz = kLz + 2, kExt = kEx * kEy * kEz;
 static_assert(kLx * kLy == 64 * kWaves, "one thread per (i, j) column of the tile");
 
-// The 16 field values one half of a sample's inputs reads, as (field, offset
-// from the cell a = idx(i,j,k)).  Both halves take three 4-point central
-// differences ((p0 + p1) - (p2 + p3), Q0..Q2) and two face differences
-// (p0 - p1, D0 and D1), in cell_gradient's operand order:
-//   half 0: Q0 du/dy, Q1 du/dz, Q2 dv/dx, D0 du/dx, D1 dv/dy
-//   half 1: Q0 dv/dz, Q1 dw/dx, Q2 dw/dy, D0 dw/dz (D1 unused, reads w[a], w[a-sz])
-// so the two halves of a wave run the same instructions on different addresses.
-template <typename T>
-__device__ inline void les_half_loads(const T* u, const T* v, const T* w, long sx, long sz,
-                                      int half, const T* fp[16], long fo[16]) {
-  const long o0[16] = {sx, sx - 1, -sx, -sx - 1, sz, sz - 1, -sz, -sz - 1,
-                       1,  1 - sx, -1,  -1 - sx, 0,  -1,     0,   -sx};
-  const long o1[16] = {sz, sz - sx, -sz, -sz - sx, 1,  1 - sz, -1,  -1 - sz,
-                       sx, sx - sz, -sx, -sx - sz, 0,  -sz,    0,   -sz};
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const T* f0 = (s < 8 || s == 12 || s == 13) ? u : v;
-    const T* f1 = s < 4 ? v : w;
-    fp[s] = half ? f1 : f0;
-    fo[s] = half ? o1[s] : o0[s];
-  }
-}
-
 // The values of one field that the closure stage reads around a cell: slot 0
 // the cell, 1..6 its face neighbours (+x, -x, +y, -y, +z, -z), 7 and 8 two
 // diagonal neighbours, which differ by field (u: (-1,1,0), (-1,0,1); v:
@@ -949,15 +921,6 @@ struct RegAcc {
   __device__ __forceinline__ T operator()(int di, int dj, int dk) const {
     return r[stencil_slot(f, di, dj, dk)];
   }
-};
-
-// One tile's inputs for a lane: the fetched field values, the plane
-// coefficients of its cell, and whether the sample is a cell of the domain.
-template <typename T>
-struct LesIn {
-  T v[16];
-  T hz, dfi, zs, yw;
-  bool valid;
 };
 
 // The eddy viscosity of every cell of a stage's source field, in chunks of
@@ -1372,13 +1335,13 @@ T* fld(const pll_context* c, int f) {
   return static_cast<T*>(c->fld[f]);
 }
 
-// The closure stage.  Stage 1 with fold (and corr) first applies the previous
-// step's forcing (and projection) and boundary update in one pass
-// (k_apply_deferred), and with bcload writes u1's boundary update itself;
-// stage 2 with acc sums the bulk-mean partials of its new u for the next
-// step's forcing.  The sources are read as stored, halos included.
+// The closure stage.  Stage 1 with deferred first applies the previous step's
+// projection, forcing and boundary update in one pass (k_apply_deferred), and
+// with halo writes u1's boundary update itself; stage 2 with acc sums the
+// bulk-mean partials of its new u for the next step's forcing.  The sources are
+// read as stored, halos included.
 template <typename T>
-int rk_closure_t(pll_context* c, int stage, int fold, int corr, int acc, int bcload) {
+int rk_closure_t(pll_context* c, int stage, int deferred, int acc, int halo) {
   pll_closure* cl = c->closure;
   const Geom g = c->g;
   const int ntx = (g.nx + kLx - 1) / kLx, nty = (g.ny + kLy - 1) / kLy, ntz = (g.nz + kLz - 1) / kLz;
@@ -1395,16 +1358,16 @@ int rk_closure_t(pll_context* c, int stage, int fold, int corr, int acc, int bcl
   const long nblk = std::min((ncell + kNutChunk - 1) / kNutChunk, 512L);
   if (acc && (stage != 2 || (long)grid.x > c->npartial))
     return fail(PLL_ERR_STATE, "the bulk-mean partials are stage 2's and must fit the scratch");
-  if (corr && !fold) return fail(PLL_ERR_STATE, "deferred projection needs folded loads");
-  if (bcload && stage != 1) return fail(PLL_ERR_STATE, "the closure's stage 2 reads an updated u1");
+  if ((deferred || halo) && stage != 1)
+    return fail(PLL_ERR_STATE, "the closure's stage 2 reads an updated u1");
   const T bc_u = (T)(0.0 - c->u_crf);  // src/mod_updateBound.cc:80
-  if (stage == 1 && fold) {
+  if (deferred) {
     // the previous step's projection, forcing and boundary update into the
     // spare velocity buffers, which then become u, v, w
     if (!c->fld_alt[0] || !c->fld_alt[1] || !c->fld_alt[2])
       return fail(PLL_ERR_STATE, "no spare velocity buffers");
     const int fmask = (c->is_forced[0] ? 1 : 0) | (c->is_forced[1] ? 2 : 0) | (c->is_forced[2] ? 4 : 0);
-    const VelRules<T> r{1, corr, fld<T>(c, PLL_P), mesh_t<T>(c).dzc_inv,
+    const VelRules<T> r{fld<T>(c, PLL_P), mesh_t<T>(c).dzc_inv,
                         (T)(c->dt * c->dx_inv), (T)(c->dt * c->dy_inv),  // src/mod_calcVel.cc:256-258
                         dt, c->d_scalar + 3, fmask, bc_u};
     const long n = (long)(g.nx + 2) * (g.ny + 2) * (g.nz + 2);
@@ -1438,7 +1401,7 @@ int rk_closure_t(pll_context* c, int stage, int fold, int corr, int acc, int bcl
     if (stage == 1)
       hipLaunchKernelGGL((k_rk_les<T, 1>), grid, block, 0, c->stream, g, su, sv, sw,
                          fld<T>(c, PLL_U1), fld<T>(c, PLL_V1), fld<T>(c, PLL_W1), mesh_t<T>(c), dxi,
-                         dyi, rei, dt, ucrf, c->d_nut, ntx, nty, bcload, bc_u, 0, dzflzi,
+                         dyi, rei, dt, ucrf, c->d_nut, ntx, nty, halo, bc_u, 0, dzflzi,
                          c->d_partial);
     else
       hipLaunchKernelGGL((k_rk_les<T, 2>), grid, block, 0, c->stream, g, su, sv, sw,
@@ -1523,12 +1486,12 @@ int filter(pll_context* f, pll_context* c) {
 }  // namespace
 
 namespace pll {
-int launch_rk_closure(pll_context* c, int stage, int fold, int corr, int acc, int bcload) {
+int launch_rk_closure(pll_context* c, int stage, int deferred, int acc, int halo) {
   int rc = feat_setup_any(c);
   if (rc) return rc;
   if (!c->d_nut) PLL_HIP_TRY(ctx_malloc(c, &c->d_nut, (size_t)c->nspec * sizeof(float)));
-  return c->prec == PLL_FP64 ? rk_closure_t<double>(c, stage, fold, corr, acc, bcload)
-                             : rk_closure_t<float>(c, stage, fold, corr, acc, bcload);
+  return c->prec == PLL_FP64 ? rk_closure_t<double>(c, stage, deferred, acc, halo)
+                             : rk_closure_t<float>(c, stage, deferred, acc, halo);
 }
 int closure_detach(pll_context* c) {
   if (!c->closure_order) return PLL_OK;

@@ -1605,9 +1605,8 @@ int rk_setup(pll_context* c) {
   return PLL_DISPATCH(c, rk_coef_setup<double>(c), rk_coef_setup<float>(c));
 }
 
-int launch_rk(pll_context* c, int stage, int fold, int corr, int acc, int bcload) {
-  if (c->closure) return launch_rk_closure(c, stage, fold, corr, acc, bcload);
-  if (fold || corr) return fail(PLL_ERR_STATE, "the separate stages take no deferred updates");
+int launch_rk(pll_context* c, int stage, int acc, int bcload) {
+  if (c->closure) return launch_rk_closure(c, stage, 0, acc, 0);
   return PLL_DISPATCH(c, rk_t<double>(c, stage, acc, bcload), rk_t<float>(c, stage, acc, bcload));
 }
 int launch_calc_rhs(pll_context* c) { return PLL_DISPATCH(c, rhs_t<double>(c), rhs_t<float>(c)); }

@@ -297,8 +297,8 @@ int poisson_impl(pll_context* c) {
 
 // One step of src/main.cc:116-154.  When only u is forced (or nothing is),
 // within a multi-step run the projection, the force update and the final
-// boundary update of a step (:145-153) are folded into the next step's RK loads
-// (`corr`, `fold`) and the bulk mean of the forcing is reduced by stage 2 from
+// boundary update of a step (:145-153) are left to the next step's RK loads
+// (`fold`) and the bulk mean of the forcing is reduced by stage 2 from
 // the predictor; the last step of a run applies them explicitly, so every run
 // ends in the reference's state.
 int finish_step(pll_context* c);
@@ -315,10 +315,9 @@ int step_impl(pll_context* c, bool first, bool last) {
     // boundary update written by stage 1, the predictor's bulk mean for the
     // forcing summed by stage 2, and calcRHS inside the forward x transform
     // (which rebuilds u's boundary on load)
-    const int corr = fold;
     const int acc = c->is_forced[0] ? 1 : 0;
-    if ((rc = launch_rk(c, 1, fold, corr, 0, 1))) return rc;  // :145-153, :117, :121
-    if ((rc = launch_rk(c, 2, 0, 0, acc, 0))) return rc;      // :125
+    if ((rc = launch_rk_closure(c, 1, fold, 0, 1))) return rc;  // :145-153, :117, :121
+    if ((rc = launch_rk(c, 2, acc))) return rc;                 // :125
     c->rhs_bcfold = 1;
     rc = launch_poisson_step(c, true);  // :133-141
     c->rhs_bcfold = 0;
@@ -328,9 +327,9 @@ int step_impl(pll_context* c, bool first, bool last) {
   if (c->closure) {
     // the closure stages (eddy viscosity evaluated in the stage kernel), then
     // the reference sequence src/main.cc:121-153 unfused
-    if ((rc = launch_rk(c, 1, 0))) return rc;  // :117
+    if ((rc = launch_rk(c, 1))) return rc;  // :117
     if ((rc = launch_bc_vel(c, 1))) return rc;  // :121
-    if ((rc = launch_rk(c, 2, 0))) return rc;  // :125
+    if ((rc = launch_rk(c, 2))) return rc;  // :125
     if ((rc = launch_bc_vel(c, 0))) return rc;  // :129
     if ((rc = launch_calc_rhs(c))) return rc;   // :133
     if ((rc = launch_poisson_step(c, false))) return rc;  // :137-141
@@ -349,8 +348,8 @@ int step_impl(pll_context* c, bool first, bool last) {
     if (fold) {
       if ((rc = launch_rk12(c, acc, last))) return rc;  // :117-125
     } else {
-      if ((rc = launch_rk(c, 1, 0))) return rc;             // :117
-      if ((rc = launch_rk(c, 2, 0, 0, acc, 1))) return rc;  // :125
+      if ((rc = launch_rk(c, 1))) return rc;          // :117
+      if ((rc = launch_rk(c, 2, acc, 1))) return rc;  // :125
     }
     c->rhs_bcfold = 1;
     rc = launch_poisson_step(c, true);  // :133-141
@@ -361,9 +360,9 @@ int step_impl(pll_context* c, bool first, bool last) {
     return last ? finish_run(c, 2) : PLL_OK;
   }
   // unfused: v or w is forced
-  if ((rc = launch_rk(c, 1, 0))) return rc;     // src/main.cc:117
+  if ((rc = launch_rk(c, 1))) return rc;        // src/main.cc:117
   if ((rc = launch_bc_vel(c, 1))) return rc;    // :121
-  if ((rc = launch_rk(c, 2, 0))) return rc;     // :125
+  if ((rc = launch_rk(c, 2))) return rc;        // :125
   if ((rc = launch_bc_vel(c, 0))) return rc;    // :129
   if ((rc = launch_calc_rhs(c))) return rc;     // :133
   if ((rc = launch_poisson_step(c, false))) return rc;  // :137-141
@@ -559,12 +558,12 @@ int pll_transform2crf(pll_context* c, double vel_crf) {
 
 int pll_time_int_vel_rk1(pll_context* c) {
   if (!c) return fail(PLL_ERR_ARG, "null context");
-  return launch_rk(c, 1, 0);
+  return launch_rk(c, 1);
 }
 
 int pll_time_int_vel_rk2(pll_context* c) {
   if (!c) return fail(PLL_ERR_ARG, "null context");
-  return launch_rk(c, 2, 0);
+  return launch_rk(c, 2);
 }
 
 int pll_correct_vel(pll_context* c) {

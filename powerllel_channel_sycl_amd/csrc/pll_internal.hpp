@@ -244,17 +244,15 @@ struct TimerScope {
 
 // ---- launchers (implemented in the .hip files) -------------------------------------
 // stencils and pointwise kernels (k_stencil.hip)
-// fold: stage 1 applies the previous step's deferred force and rebuilds the
-// halos on load; stage 2 adds the deferred force to its point value of u.
-// corr: apply the deferred projection on load; acc (stage 2): bulk mean of the
-// new u into d_scalar[0], force into d_scalar[3]
-// bcload (stage 2, FP32): rebuild the source's halos on load (u1's boundary
-// update not run)
-int launch_rk(pll_context* c, int stage, int fold, int corr = 0, int acc = 0, int bcload = 0);
-// the stage of a context with an attached closure (k_closure.hip); fold,
-// corr, acc, bcload as for launch_rk
-int launch_rk_closure(pll_context* c, int stage, int fold = 0, int corr = 0, int acc = 0,
-                      int bcload = 0);
+// A stage on its own; with a closure attached, the closure's.  acc (stage 2): the
+// bulk mean of the new u is left for the next transform (force_from_partials);
+// bcload (plain stage 2): rebuild the source's halos on load (u1's boundary update
+// not run)
+int launch_rk(pll_context* c, int stage, int acc = 0, int bcload = 0);
+// The stage of a context with an attached closure (k_closure.hip).  deferred (stage
+// 1): the previous step's projection, forcing and boundary update first; halo
+// (stage 1): u1's boundary update is written too; acc as above.
+int launch_rk_closure(pll_context* c, int stage, int deferred, int acc, int halo);
 // Takes the context off its closure's readers; a writer still waits for its stages.
 int closure_detach(pll_context* c);
 // the closure stages' bulk-mean partials fit d_partial (the fused step sequence)
