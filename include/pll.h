@@ -213,16 +213,17 @@ int pll_closure_destroy(pll_closure *c);
 int pll_closure_num_params(void);
 int pll_closure_get_params(pll_closure *c, float *host);
 int pll_closure_set_params(pll_closure *c, const float *host);
-/* Gradient of the mean squared error of softplus(o) against y (host copy), and the loss. */
+/* Gradient of the mean squared error of softplus(o) against y (host copy), and the loss.
+ * A pre-activation that is NaN counts as 0 here, in train_step and in predict. */
 int pll_closure_gradient(pll_closure *c, const float *x, const float *y, long n, float *grad_host,
                          double *loss);
 /* pll_closure_gradient without allocating: no counterpart in the reference;
  * for callers that cannot allocate device memory (code under HIP graph
- * capture, tight training loops).  The kernels' partial gradients, chunk sums
- * and result live in one static device array of 6.1 MB per GPU (every
- * training grid fits: at most 1024 waves); the call allocates nothing on the
- * device or host.  All calls on one GPU share that array, so calls that
- * overlap on one GPU (other streams, other threads, other closures) race.
+ * capture, tight training loops).  The kernels' partial gradients and result
+ * live in one static device array of 5.5 MB per GPU (every training grid fits:
+ * at most 256 blocks, 2048 waves); the call allocates nothing on the device or
+ * host.  All calls on one GPU share that array, so calls that overlap on one
+ * GPU (other streams, other threads, other closures) race.
  * The closure's device (current at pll_closure_create) must be current. */
 int pll_closure_gradient_noalloc(pll_closure *c, const float *x, const float *y, long n,
                                  float *grad_host, double *loss);
@@ -240,10 +241,12 @@ int pll_closure_get_scales(pll_closure *c, double *gscale, double *yscale, doubl
  * closure).  With a closure attached, timeIntVelRK1/RK2 and pll_step add the
  * divergence of the eddy-viscosity stress 2 nu_t S_ij to the momentum
  * tendency (src/mod_calcVel.cc:27-242), with nu_t evaluated by the network
- * inside the stage kernel; pll_step then runs the unfused sequence
- * src/main.cc:117-153.  Training the closure (or setting its parameters) while
- * attached is ordered after the context's stages already enqueued and before
- * its next one. */
+ * on every cell of a stage's source before the stage; pll_step then runs a
+ * deferred sequence of its own (the previous step's projection, forcing and
+ * boundary update in one pass before stage 1), or src/main.cc:117-153 routine
+ * by routine where v or w is forced.  Training the closure or setting its
+ * parameters while attached is ordered after the context's stages already
+ * enqueued and before its next one. */
 int pll_closure_attach(pll_context *ctx, pll_closure *c);
 /* Save a closure (parameters and scales) to a file / create one from such a
  * file: "PLLCLOS1", int32 parameter count, the FP32 parameters, the three FP64

@@ -303,7 +303,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_predict(Mlp w, const floa
 // Training: one partial gradient (and loss sum) per block.  Loss = mean over
 // the n samples of (softplus(o) - y)^2.  Per 32-sample tile 40 products and
 // about 750 VALU operations (the ReLUs, masks and BF16 packing), which bound it
-// at two waves per SIMD.  393,216 samples: 37.5 us, of which 3 us are the FP32
+// at two waves per SIMD.  393,216 samples: 37.8 us, of which 3 us are the FP32
 // maxima of the ReLUs (a 16-bit maximum of the packed pairs is half as many
 // operations, but lets a positive NaN through); 101 us for a form that passed
 // activations between the layers through LDS in two-byte writes (one wave per

@@ -16,7 +16,7 @@
 //
 // Complex transforms use the Stockham autosort formulation, in place in one
 // LDS buffer with the butterflies in registers: products of 2, 3 and 5 up to 768
-// are compiled in (fft_fixed.hpp), longer ones run from a plan.  Twiddles
+// (but 625) are compiled in (fft_fixed.hpp), others run from a plan.  Twiddles
 // are computed on the host in long double and rounded to the field precision.
 #include "fft_fixed.hpp"
 

@@ -625,8 +625,8 @@ constexpr int kRk12Slots = 256;  // blocks of k_rk12 that run at once: one per C
 // saved 3 % in FP64 and nothing in FP32 when the loads were issued after stage 1):
 // so a plane's loads are issued first, each thread loads a pair of cells (6 or 7
 // wide loads instead of up to 14), and the waves that load are not those with ring
-// cells.  At 768x384x384 FP64 2261 -> 2010-2040 us (3.4 TB/s of 61 B a point),
-// FP32 1243 -> 1070; 256x192x128 FP64 128 -> 115, 384x256x192 FP32 213 -> 186,
+// cells.  At 768x384x384 FP64 2261 -> 2010-2040 us, with the viscous terms as second
+// differences 2040-2120 (3.3 TB/s of 61 B a point), FP32 1243 -> 1070; 256x192x128 FP64 128 -> 115, 384x256x192 FP32 213 -> 186,
 // 1536x768x512 FP32 6850 -> 6040.  Loads two planes ahead in a second set of
 // registers ran slower (FP32 1178: the registers are full and all waves load).
 // The two kernels that it replaces took 1646 + 2331 us (FP64, 768x384x384).

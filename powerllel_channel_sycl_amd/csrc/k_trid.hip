@@ -170,7 +170,10 @@ constexpr int kSegPlanes = 768;  // the deepest column the segments hold
 // Planes per segment M and most segments per column S.  Short segments keep the
 // registers (4 M values, M+1 reciprocals) at four waves per SIMD; M = 12 where
 // M = 8 would make blocks that leave a CU's wave slots idle (768x384x384: FP64 413
-// against 464 us, FP32 249 against 299 us).
+// against 464 us, FP32 249 against 299 us).  M = 12 takes 168 registers in FP64
+// (three waves) and 134 in FP32, which is held to four waves all the same: 8
+// registers spill, but two blocks of 512 threads fit a CU instead of one
+// (768x384x384, 10 steps 25.3 against 25.6 ms).
 constexpr int seg_planes(int nz) { return nz <= 256 || (nz > 384 && nz <= 512) ? 8 : 12; }
 constexpr int seg_count_max(int nz) { return nz <= 128 ? 16 : (nz <= 384 ? 32 : 64); }
 constexpr bool segs_hold(int nz) { return seg_planes(nz) * seg_count_max(nz) >= nz; }
