@@ -133,7 +133,6 @@ int download(pll_context* c, const void* src, double* host, long n) {
 void release(pll_context* c) {
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  c->closure_reading = false;
   (void)closure_detach(c);
   if (c->closure_read) (void)hipEventDestroy(c->closure_read);
   for (auto& t : c->pending) {
