@@ -512,12 +512,15 @@ __global__ __launch_bounds__(256) void k_grad_sum(const float* __restrict__ part
 #pragma unroll
       for (int u = 0; u < 16; ++u) v[u] = r + u < q1 ? partial[(r + u) * (kNParam + 1) + i] : 0.f;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) s += v[u];
+      for (int h = 8; h > 0; h >>= 1)
+#pragma unroll
+        for (int u = 0; u < h; ++u) v[u] += v[u + h];
+      s += v[0];
     }
   red[q][c] = s;
   __syncthreads();
   if (q || i > kNParam) return;
-  const float g = ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
+  const float g = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
   grad[i] = g;
   if (!ADAM || i == kNParam) return;  // the loss sum
   const bool pad = i < oB1 && (i / kH) >= kIn;
