@@ -203,27 +203,28 @@ struct MeanJob {
   double* mean;
   double* force;
 };
+__device__ __forceinline__ double sum8(const double* s) {
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
 __device__ __forceinline__ void mean_job(const MeanJob& m) {
-  __shared__ double red[64];
+  __shared__ double red[64], top[8];
   const int W = blockDim.x < 64 ? (int)blockDim.x : 64, t = threadIdx.x;
   if (t < W) {
-    double s[8] = {};
+    double s = 0.0;
     for (long i = t; i < m.n; i += 8 * W) {
       double v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] = i + u * W < m.n ? m.partial[i + u * W] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s[u] += v[u];
+      s += sum8(v);
     }
-    red[t] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    red[t] = s;
+    for (int i = t + W; i < 64; i += W) red[i] = 0.0;
   }
   __syncthreads();
-  for (int h = 32; h > 0; h >>= 1) {
-    if (t < h && t + h < W) red[t] += red[t + h];
-    __syncthreads();
-  }
+  if (t < 8) top[t] = sum8(red + 8 * t);  // a block has at least 8 threads
+  __syncthreads();
   if (t == 0) {
-    const double mean = red[0] / m.nxg / m.nyg;
+    const double mean = sum8(top) / m.nxg / m.nyg;
     *m.mean = mean;
     *m.force = m.vel_force - mean;
   }
